@@ -18,11 +18,10 @@
 //
 // When every view's radiance is the moment cut, the views' cuts -- most of
 // each frame's time -- run as one launch over all views' tiles: each view's
-// frame runs up to its cut on its lane, the lanes join, one kernel takes
-// the tiles of all views heaviest first (by their costs in the last
-// launch), and the lanes fork again for each view's combine.  A small view
-// then adds its tiles to the launch instead of leaving the GPU to a short
-// kernel of its own, and no view's heaviest tiles run alone at the end.
+// frame runs up to its cut on its lane, the lanes join, one set of launches
+// cuts the tiles of all views, and the lanes fork again for each view's
+// combine.  A small view then adds its tiles to the launch instead of leaving
+// the GPU to a short kernel of its own.
 #include <algorithm>
 #include <vector>
 
@@ -41,8 +40,9 @@ struct arc_batch {
     // default: on the 64-view workload a cut per view measured faster, as
     // each view's cut then overlaps other views' rebuilds and lists)
     int one_cut = 0;
-    arc::DevBuf views_dev, costs, order;   // the views' descriptors, tile costs and launch order
-    int nitems = 0;                        // tiles of all views
+    std::vector<arc::CutView> views;       // the views' descriptors
+    arc::DevBuf views_dev;                 // the same on the device
+    arc::CutPoolMem pool;
 };
 
 namespace {
@@ -94,31 +94,30 @@ int join_lanes(arc_batch* b, hipStream_t s, std::vector<hipEvent_t>& evs) {
 }
 
 // Eagerly, before the capture: every view's frame up to its cut, the views'
-// descriptors into device memory, one unordered launch of all cuts (it
-// writes the tile costs the captured launches order by), the combines.
+// descriptors into device memory, one launch of all cuts (the pool reaches
+// its size), the combines.
 int prepare_one_cut(arc_batch* b, const arc_batch_view* views, int nviews) {
     arc_ctx* ctx = b->ctx;
     ARC_TRY(fork_lanes(b, ctx->stream, b->fork));
     for (int i = 0; i < nviews; ++i) ARC_TRY(run_deferred(views[i]));
     for (arc_ctx* c : b->lanes) ARC_HIP(ctx, hipStreamSynchronize(c->stream));
-    std::vector<arc::CutView> hv(nviews);
+    b->views.resize(nviews);
     int nitems = 0;
     for (int i = 0; i < nviews; ++i) {
-        hv[i] = views[i].gather->def_view;
-        hv[i].tile_base = nitems;
-        nitems += hv[i].ntiles;
+        b->views[i] = views[i].gather->def_view;
+        b->views[i].tile_base = nitems;
+        nitems += b->views[i].ntiles;
     }
-    ARC_TRY(arc::ensure(ctx, b->views_dev, sizeof(arc::CutView) * (size_t)nviews));
-    ARC_TRY(arc::ensure(ctx, b->costs, sizeof(float) * (size_t)nitems));
-    ARC_TRY(arc::ensure(ctx, b->order, sizeof(int) * (size_t)nitems));
-    for (int i = 0; i < nviews; ++i) hv[i].tile_cost = b->costs.as<float>() + hv[i].tile_base;
-    ARC_HIP(ctx, hipMemcpy(b->views_dev.p, hv.data(), sizeof(arc::CutView) * (size_t)nviews, hipMemcpyHostToDevice));
-    ARC_TRY(arc::cut_moments_views(ctx, b->origin, b->views_dev.as<arc::CutView>(), nviews, nitems,
-                                   b->costs.as<float>(), b->order.as<int>(), false));
-    ARC_HIP(ctx, hipStreamSynchronize(b->origin));
+    const size_t bytes = sizeof(arc::CutView) * (size_t)nviews;
+    ARC_TRY(arc::ensure(ctx, b->views_dev, bytes));
+    ARC_HIP(ctx, hipMemcpy(b->views_dev.p, b->views.data(), bytes, hipMemcpyHostToDevice));
+    for (int pass = 0; pass < 2; ++pass) {  // a second time when the pool was too small: it grows then
+        ARC_TRY(arc::cut_moments_views(ctx, b->origin, b->views.data(), b->views_dev.as<arc::CutView>(), nviews, b->pool));
+        ARC_HIP(ctx, hipStreamSynchronize(b->origin));
+        if (!b->pool.seen || *b->pool.seen <= b->pool.cap) break;
+    }
     for (int i = 0; i < nviews; ++i) ARC_TRY(arc::gather_finish(views[i].gather));
     for (arc_ctx* c : b->lanes) ARC_HIP(ctx, hipStreamSynchronize(c->stream));
-    b->nitems = nitems;
     return ARC_OK;
 }
 
@@ -190,6 +189,13 @@ int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews) {
     }
     for (arc_ctx* c : b->lanes) ARC_HIP(ctx, hipStreamSynchronize(c->stream));
     ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // a view whose cut's pool was too small runs again: the pool grows, which it cannot in the graph
+    for (int i = 0; i < nviews; ++i) {
+        const arc_batch_view& v = views[i];
+        if (!arc::cut_pool_short(v.gather)) continue;
+        ARC_TRY(arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr));
+        ARC_HIP(ctx, hipStreamSynchronize(arc_gather_ctx(v.gather)->stream));
+    }
     if (one_cut) ARC_TRY(prepare_one_cut(b, views, nviews));
     // 2. capture on the batch's own stream (the legacy null stream cannot be
     // captured): fork the lanes from it, run the views on their lanes, join
@@ -207,8 +213,7 @@ int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews) {
         for (int i = 0; st == ARC_OK && i < nviews; ++i) st = run_deferred(views[i]);
         if (st == ARC_OK) st = join_lanes(b, b->origin, b->join);
         if (st == ARC_OK)
-            st = arc::cut_moments_views(ctx, b->origin, b->views_dev.as<arc::CutView>(), nviews, b->nitems,
-                                        b->costs.as<float>(), b->order.as<int>(), true);
+            st = arc::cut_moments_views(ctx, b->origin, b->views.data(), b->views_dev.as<arc::CutView>(), nviews, b->pool);
         if (st == ARC_OK) st = fork_lanes(b, b->origin, b->fork2);
         for (int i = 0; st == ARC_OK && i < nviews; ++i) st = arc::gather_finish(views[i].gather);
         if (st == ARC_OK) st = join_lanes(b, b->origin, b->join2);
@@ -253,8 +258,7 @@ void arc_batch_destroy(arc_batch* b) {
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->fork2) (void)hipEventDestroy(b->fork2);
     arc::release(b->views_dev);
-    arc::release(b->costs);
-    arc::release(b->order);
+    arc::release_pool(b->pool);
     for (arc_ctx* c : b->lanes) arc_ctx_destroy(c);
     if (b->origin) (void)hipStreamDestroy(b->origin);
     delete b;

@@ -42,6 +42,8 @@
 #include "cut_common.hpp"
 
 using namespace arc::cut;
+using arc::CutPool;
+using arc::CutView;
 
 namespace {
 
@@ -52,7 +54,10 @@ constexpr int kScanBlock = 256;  // leaves per block of the prefix scan
 //   2-4 the four points, 12 floats   5-7 (b_c, a_c) per channel
 //   8-12 per channel (txx - tzz, tyy - tzz, 0, 2txy, 2txz, 2tyz), 18 floats
 constexpr int kMom = 13;
-constexpr int kMomStack = 96;    // per-wave stack of the tile traversal (default; 64 and 128 also built)
+// float4 per internal node of the traversal's record, one 48-byte gather per
+// node: (box min, max_c I_c), (box max, first leaf), (left, right, count, -)
+constexpr int kTrav = 3;
+constexpr int kMomStack = 128;   // per-wave stack of the serial traversal (deeper than any tree: 32 code bits + 25 index bits)
 
 // Terms of leaf i of the sorted order (crec leaf record: r0 = position,
 // r1 = unit normal, r2 = I), in four groups of ten:
@@ -188,7 +193,8 @@ __device__ inline void range_group(const double* __restrict__ pre, const double*
 __global__ __launch_bounds__(kScanBlock) void k_mom_nodes(const int* __restrict__ ranges,
                                                           const arc_bvh_node* __restrict__ nodes, int n,
                                                           const double* __restrict__ pre,
-                                                          const double* __restrict__ tot, float4* __restrict__ mom) {
+                                                          const double* __restrict__ tot, float4* __restrict__ mom,
+                                                          float4* __restrict__ trav) {
     const int k = blockIdx.x * kScanBlock + threadIdx.x;
     if (k >= n - 1) return;
     const int first = ranges[2 * k], last = ranges[2 * k + 1];
@@ -292,14 +298,11 @@ __global__ __launch_bounds__(kScanBlock) void k_mom_nodes(const int* __restrict_
     tf[18] = 0.f;
     tf[19] = 0.f;
     o[0] = make_float4((float)cx, (float)cy, (float)cz, (float)Ib);
+    float4* t = trav + (size_t)kTrav * k;
+    t[0] = make_float4(b.bbMin.x, b.bbMin.y, b.bbMin.z, (float)Ib);
+    t[1] = make_float4(b.bbMax.x, b.bbMax.y, b.bbMax.z, __int_as_float(first));
+    t[2] = make_float4(__int_as_float(b.left), __int_as_float(b.right), __int_as_float(last - first + 1), 0.f);
 }
-
-struct CutMom {
-    const arc_bvh_node* nodes;  // n - 1 internal nodes (boxes)
-    const float4* crec;         // leaf records, slots [0, n) in sorted order
-    const float4* mom;          // kMom float4 per internal node
-    int n;
-};
 
 // Wave-uniform record reads (the nodes' boxes and moment records, one
 // address for the whole wave) go through the constant address space in the
@@ -424,162 +427,875 @@ __device__ inline int wave_inclusive_sum(int v) {
     return v;
 }
 
-// The queued exact ranges' leaves, summed exactly.  A range is
-// (first << 7 | (count - 1)) over contiguous sorted leaves.  The leaves of
-// all ranges are taken 64 at a time: each lane finds its leaf (a binary
-// search over the ranges' prefix counts) and loads its record with vector
-// loads, the wave writes the 64 records to its LDS stage, and the pairs are
-// evaluated from there, every lane reading the same record (a broadcast).
-// The next 64 records are loaded while these are evaluated, so a record's
-// memory latency is paid once per 64 leaves, not once per leaf.
-//
-// A leaf whose AVPL faces away from every pixel of the tile adds 0 to every
-// sum (its cosine max(0, n_a . (p - x_a)) is 0), and about half of the
-// leaves do (a surface's AVPLs seen from behind): each lane tests its leaf
-// against the tile's box tb = (centre, half extent): the largest
-// n_a . (p - x_a) over the box is n_a . (c - x_a) + |n_a| . e.  Only the
-// leaves that can face some pixel, with a margin above FP32 rounding, are
-// staged.
-__device__ inline void add_ranges(const float4* __restrict__ crec, const uint32_t* X, int nx, int* pfx,
-                                  float4 (*stage)[3], const float* tb, const PixelF& P, Acc& acc) {
+__device__ inline int lane_below(uint64_t m) {  // set bits of m below this lane
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// The leaves of nx exact ranges (first << 7 | (count - 1), contiguous sorted
+// leaves), at most `most` of them from the from-th on (a multiple of 64), 64
+// at a time, one per lane.  A lane's range among those of the
+// batch: the ranges that start inside it mark their first lane in LDS, and a
+// lane counts the marks up to its own (14 instructions per 64 leaves, where a
+// binary search over the ranges' prefix counts takes 56).  Each lane tests its
+// leaf against the tile: an AVPL that faces away from every pixel adds 0 to
+// every sum (its cosine max(0, n_a . (p - x_a)) is 0), and about half of the
+// leaves do (a surface's AVPLs seen from behind).  tb = (centre, half extent)
+// of the tile's box: the largest n_a . (p - x_a) over it is n_a . (c - x_a) +
+// |n_a| . e, compared with a margin above FP32 rounding.  take(facing, r0, r1,
+// r2) gets each lane's leaf record and whether it can face some pixel.
+template <class Take>
+__device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32_t* X, int nx, int from, int most,
+                                   int* pfx, int* mark, const float* tb, Take take) {
     const int lane = threadIdx.x & 63;
     const int c0 = lane < nx ? (int)(X[lane] & 127u) + 1 : 0;
     const int c1 = lane + 64 < nx ? (int)(X[lane + 64] & 127u) + 1 : 0;
-    const int s0 = wave_inclusive_sum(c0);
+    int s0 = wave_inclusive_sum(c0);
     const int t0 = __builtin_amdgcn_readlane(s0, 63);
-    const int s1 = wave_inclusive_sum(c1) + t0;
-    const int total = __builtin_amdgcn_readlane(s1, 63);
-    if (lane < nx) pfx[lane] = s0 - c0;
-    if (lane + 64 < nx) pfx[lane + 64] = s1 - c1;
-    // the wave's LDS writes come before its reads of other lanes' slots
-    __builtin_amdgcn_wave_barrier();
-    auto fetch = [&](int base, float4& a0, float4& a1, float4& a2) {
+    int s1 = wave_inclusive_sum(c1) + t0;
+    const int leaves = __builtin_amdgcn_readlane(s1, 63);
+    const int total = leaves - from > most ? from + most : leaves;
+    s0 = lane < nx ? s0 - c0 : INT_MAX;       // where the range in X[lane] starts
+    s1 = lane + 64 < nx ? s1 - c1 : INT_MAX;  // and the one in X[lane + 64]
+    if (lane < nx) pfx[lane] = s0;
+    if (lane + 64 < nx) pfx[lane + 64] = s1;
+    const float scale = fabsf(tb[0]) + fabsf(tb[1]) + fabsf(tb[2]) + tb[3] + tb[4] + tb[5];
+    float4 b0 = make_float4(0.f, 0.f, 0.f, 0.f), b1 = b0, b2 = b0;
+    int before = __popcll(__ballot(s0 < from)) + __popcll(__ballot(s1 < from));  // ranges that start before the batch
+    auto fetch = [&](int base) {
+        mark[lane] = 0;
+        __builtin_amdgcn_wave_barrier();  // the wave's LDS writes come before its reads of other lanes' slots
+        if ((unsigned)(s0 - base) < 64u) mark[s0 - base] = 1;
+        if ((unsigned)(s1 - base) < 64u) mark[s1 - base] = 1;
+        __builtin_amdgcn_wave_barrier();
+        const uint64_t m = __ballot(mark[lane] != 0);
         const int g = base + lane;
         if (g < total) {
-            int lo = 0, hi = nx - 1;  // the last range that starts at or before g
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (pfx[mid] <= g) lo = mid;
-                else hi = mid - 1;
-            }
-            const float4* l = crec + kCrec * (size_t)((int)(X[lo] >> 7) + (g - pfx[lo]));
-            a0 = l[0];
-            a1 = l[1];
-            a2 = l[2];
+            const int r = before - 1 + lane_below(m) + (int)((m >> lane) & 1);
+            const float4* l = crec + kCrec * (size_t)((int)(X[r] >> 7) + (g - pfx[r]));
+            b0 = l[0];
+            b1 = l[1];
+            b2 = l[2];
         }
+        before += __popcll(m);
     };
-    float4 b0 = make_float4(0.f, 0.f, 0.f, 0.f), b1 = b0, b2 = b0;
-    fetch(0, b0, b1, b2);
-    for (int base = 0; base < total; base += 64) {
-        bool facing = base + lane < total;
-        if (facing) {
-            const float dx = tb[0] - b0.x, dy = tb[1] - b0.y, dz = tb[2] - b0.z;
-            const float reach = b1.x * dx + b1.y * dy + b1.z * dz + fabsf(b1.x) * tb[3] + fabsf(b1.y) * tb[4] +
-                                fabsf(b1.z) * tb[5];
-            const float margin = 1e-5f * (fabsf(b0.x) + fabsf(b0.y) + fabsf(b0.z) + fabsf(tb[0]) + fabsf(tb[1]) +
-                                          fabsf(tb[2]) + tb[3] + tb[4] + tb[5]);
-            facing = reach > -margin;
-        }
-        const uint64_t fm = __ballot(facing);
-        if (facing) {
-            const int slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fm >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)fm, 0u));
-            stage[slot][0] = b0;
-            stage[slot][1] = b1;
-            stage[slot][2] = b2;
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (base + 64 < total) fetch(base + 64, b0, b1, b2);
-        const int cnt = __popcll(fm);
-        // not unrolled: unrolled, the loop holds several leaves' records in
-        // registers and the kernel loses waves per SIMD (measured slower)
-#pragma unroll 1
-        for (int j = 0; j < cnt; ++j) {
-            const float4 r0 = stage[j][0], r1 = stage[j][1], r2 = stage[j][2];
-            acc.add_run(r2, leaf_g(P, r0, r1));
-        }
-        acc.maybe_flush();
-        __builtin_amdgcn_wave_barrier();  // every lane's reads before the next chunk's writes
+    fetch(from);
+    for (int base = from; base < total; base += 64) {
+        const float dx = tb[0] - b0.x, dy = tb[1] - b0.y, dz = tb[2] - b0.z;
+        const float reach = b1.x * dx + b1.y * dy + b1.z * dz + fabsf(b1.x) * tb[3] + fabsf(b1.y) * tb[4] +
+                            fabsf(b1.z) * tb[5];
+        const float margin = 1e-5f * (scale + fabsf(b0.x) + fabsf(b0.y) + fabsf(b0.z));
+        const bool facing = base + lane < total && reach > -margin;
+        const float4 r0 = b0, r1 = b1, r2 = b2;
+        if (base + 64 < total) fetch(base + 64);  // in flight while these are summed
+        take(facing, r0, r1, r2);
     }
 }
 
-// One depth-first cut per 8x8 tile (one wave), refined when any of the
-// tile's pixels asks for it (ballot), as k_cut_eb_tile; kept nodes are summed
-// with the moment estimate, or exactly when they hold at most exact_count
-// AVPLs.  criterion: ARC_CRITERION_BOUND (bound > threshold) or
-// ARC_CRITERION_EXPANSION (s > opening * d_c, or bound * (s / d_c)^2 >
-// threshold).
+// ---- the cut ----------------------------------------------------------------
 //
-// The traversal only decides: kept nodes and exact leaf ranges are queued in
-// LDS (kKeep of each per wave) and summed in passes of their own when a queue
-// fills and at the end.  The traversal loop then carries no sums across its
-// branches, and each pass is a straight loop of one kind of work.
+// Per 8x8 tile: a node is refined when any of the tile's pixels asks for it;
+// kept nodes are summed with the moment estimate, or exactly when they hold
+// at most exact_count AVPLs.  criterion: ARC_CRITERION_BOUND (bound >
+// threshold) or ARC_CRITERION_EXPANSION (s > opening * d_c, or bound *
+// (s / d_c)^2 > threshold).
+//
+//   k_cut_decide   finds each tile's cut and writes it to a pool of chunks:
+//                  kKeep kept nodes, or kKeep exact ranges, which are as many
+//                  chunks as they hold times kChunkLeaves leaves;
+//   k_cut_eval     sums the chunks, a wave per chunk whatever tile it belongs
+//                  to, into 64 x 3 partial sums each;
+//   k_cut_serial   the tiles that found the pool full: the depth-first cut of
+//                  one node at a time, summed as it goes;
+//   k_cut_combine  adds each tile's partial sums in the order of its chunks.
+//
+// One wave that walked its tile's cut node by node and summed it as it went
+// paid a dependent record load and a 64-pixel test per node, and the tile
+// with the largest cut set the kernel's time: with 375 tiles on 1024 SIMDs
+// (200x120 pixels) that was 1.8 ms.
 constexpr int kKeep = 128;
+constexpr int kChunkLeaves = 2048;
+constexpr int kDecideStack = 640;   // pending nodes per wave
+constexpr int kStackReserve = 64;   // of these for the depth-first descent when the rest is full (tree depth <= 57)
+enum ChunkKind { kNodes = 0, kRanges = 1 };
 
-// Kept nodes handed to the matrix-core pass (k_mom_est) instead of being
-// estimated in the traversal: a frame's pool of chunks of kKeep node
-// indices, taken with one atomic per chunk, each chunk linked to the
-// previous chunk of its tile.  A tile whose chunk does not fit estimates it
-// in place, so the pool's size changes only the speed.
-struct EstPool {
-    uint32_t* entries;  // cap chunks of kKeep internal-node indices
-    int2* meta;         // per chunk: (entries, the tile's previous chunk or -1)
-    int* taken;         // chunks taken this frame (may pass cap)
-    int cap;
-    int* head;          // per tile: its last chunk, -1 for none
-    float* queued;      // per tile: the nodes it queued (the order of k_mom_est)
-};
+__device__ inline float uniform_f(float v) { return __int_as_float(uniform(__float_as_int(v))); }
 
-// The cut of one 8x8 tile (tx, ty) of a view, by one wave, with the wave's
-// LDS: stack S, the two queues E and X, the exact ranges' prefix counts and
-// the leaf stage.  The tree's arrays are read-only, non-aliasing arguments:
-// the compiler then reads the wave-uniform node and moment records with
-// scalar loads.
-// The traversal's node and record reads: through the constant address space
-// (kUniformAs, a copy of the node) or plainly (a reference into the array,
-// so fields are read where they are used).
-template <bool kUniformAs>
-struct NodeRead;
+// The view of an item of the launch's tile list (kMany), or the only one.
+template <bool kMany>
+struct Views;
 template <>
-struct NodeRead<false> {
-    __device__ static const arc_bvh_node& node(const arc_bvh_node* __restrict__ n, int k) { return n[k]; }
-    __device__ static float4 rec(const float4* __restrict__ m, int k, int i) { return m[kMom * (size_t)k + i]; }
+struct Views<false> {
+    CutView one;
+    __device__ CutView of(int) const { return one; }
 };
 template <>
-struct NodeRead<true> {
-    __device__ static arc_bvh_node node(const arc_bvh_node* n, int k) { return uload_node(n + k); }
-    __device__ static float4 rec(const float4* m, int k, int i) { return uload4(uptr(m + kMom * (size_t)k + i)); }
-};
-
-template <bool kUniformAs, bool kPool, int kStack>
-__device__ __forceinline__ void cut_tile(const arc_bvh_node* __restrict__ nodes, const float4* __restrict__ crec,
-                                         const float4* __restrict__ mom, const float4* __restrict__ nbox,
-                                         const float4* __restrict__ gpos,
-                                         const float4* __restrict__ gnrm, const float4* __restrict__ galb,
-                                         const arc_material* __restrict__ mats, int W, int H, const Threshold& th,
-                                         float delta, int budget, int criterion, float open2, int exact_count,
-                                         float* __restrict__ tile_cost, float4* __restrict__ out_rad,
-                                         unsigned long long* __restrict__ counters, int tx, int ty, int tw, int* S,
-                                         int* E, uint32_t* X, int* pfx, float4 (*stage)[3], float* tb,
-                                         const EstPool* __restrict__ pool) {
-    const int lane = threadIdx.x & 63;
-    const int2 xy = make_int2(tx * 8 + (lane & 7), ty * 8 + (lane >> 3));
-    const bool live = xy.x < W && xy.y < H;
-    const int q = live ? xy.y * W + xy.x : 0;
-    const PixelF P = load_pixel(gpos, gnrm, galb, mats, q);
-    const float thr = live ? th.at(q) : INFINITY;
-    const float delta2 = delta * delta;
-    {  // the box of the tile's live pixels, as centre and half extent, for the exact leaves
-        float lx = live ? P.px : INFINITY, ly = live ? P.py : INFINITY, lz = live ? P.pz : INFINITY;
-        float hx = live ? P.px : -INFINITY, hy = live ? P.py : -INFINITY, hz = live ? P.pz : -INFINITY;
-        for (int off = 32; off > 0; off >>= 1) {
-            lx = fminf(lx, __shfl_xor(lx, off));
-            ly = fminf(ly, __shfl_xor(ly, off));
-            lz = fminf(lz, __shfl_xor(lz, off));
-            hx = fmaxf(hx, __shfl_xor(hx, off));
-            hy = fmaxf(hy, __shfl_xor(hy, off));
-            hz = fmaxf(hz, __shfl_xor(hz, off));
+struct Views<true> {
+    const CutView* many;
+    int n;
+    __device__ CutView of(int item) const {
+        int lo = 0, hi = n - 1;  // the last view whose tiles start at or before item
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (((uint_*)&many[mid].tile_base)[0] <= item) lo = mid;
+            else hi = mid - 1;
         }
+        CutView v;
+        const ARC_UNIFORM_AS uint32_t* src = (const ARC_UNIFORM_AS uint32_t*)(many + lo);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(&v);
+#pragma unroll
+        for (size_t i = 0; i < sizeof(CutView) / 4; ++i) dst[i] = src[i];
+        return v;
+    }
+};
+
+__device__ inline Threshold view_threshold(const CutView& v) {
+    Threshold th;
+    th.est = v.th_est;
+    th.sum = v.th_sum;
+    th.eps = v.th_eps;
+    th.floor_frac = v.th_floor;
+    th.inv_npix = v.th_inv_npix;
+    return th;
+}
+
+// Tile t of a view: its tile column and row.  The tile grid is the (2 gx) x
+// (2 gy) tiles of gx x gy blocks of 16x16 pixels.
+__device__ inline int tiles_wide(int W) { return 2 * ((W + 15) / 16); }
+
+// A pixel as the decisions read it from LDS: (p, threshold), (max(n, 0), -),
+// (min(n, 0), -).  A lane outside the image stands at pixel 0 with an infinite
+// threshold: it never asks for a node, but a node in front of it is not
+// dropped (it adds nothing to the image and counts towards the budget).
+constexpr int kPixRec = 3;
+
+// The Lightcuts bound of box (lo, hi) with intensity ilum at pixel record P,
+// node_bound1's terms with the box corner per axis taken as
+// max(n, 0) (hi - p) + min(n, 0) (lo - p).
+__device__ inline float pixel_bound(const float4* P, const float4& lo, const float4& hi, float delta2, float& thr) {
+    const float4 p = P[0], np = P[1], nm = P[2];
+    thr = p.w;
+    const float ax = lo.x - p.x, ay = lo.y - p.y, az = lo.z - p.z;
+    const float bx = hi.x - p.x, by = hi.y - p.y, bz = hi.z - p.z;
+    const float ex = fmaxf(fmaxf(ax, -bx), 0.f), ey = fmaxf(fmaxf(ay, -by), 0.f), ez = fmaxf(fmaxf(az, -bz), 0.f);
+    const float dmin2 = fmaxf(ex * ex + ey * ey + ez * ez, delta2);
+    const float hmax = np.x * bx + nm.x * ax + np.y * by + nm.y * ay + np.z * bz + nm.z * az;
+    const float ri = __builtin_amdgcn_rsqf(dmin2);
+    return lo.w * __builtin_amdgcn_fmed3f(hmax * ri, 0.f, 1.f) * (ri * ri);
+}
+
+__device__ inline float wave_fmin(float v) {
+    for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off));
+    return uniform_f(v);
+}
+__device__ inline float wave_fmax(float v) {
+    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+    return uniform_f(v);
+}
+__device__ inline int wave_isum(int v) {
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return uniform(v);
+}
+
+// Whether some AVPL of a kept node can face some pixel of the tile (box
+// centre tc, half extent te): the largest n_a . (p - x_a) over the node's
+// normal box, its box and the tile's box, by interval products per axis, is
+// not below 0 by more than FP32 rounding.  A node that fails adds 0 (its
+// estimate would add only the clamped cosine's second-order residue).
+__device__ inline bool node_faces(const float* tb, const float4& lo, const float4& hi, const float4& nl,
+                                  const float4& nh) {
+    float reach = 0.f, scale = 0.f;
+    auto axis = [&](float c, float e, float plo, float phi, float nlo, float nhi) {
+        const float vlo = (c - e) - phi, vhi = (c + e) - plo;  // p - x over the boxes
+        reach += fmaxf(fmaxf(nlo * vlo, nlo * vhi), fmaxf(nhi * vlo, nhi * vhi));
+        scale += fabsf(c) + e + fabsf(plo) + fabsf(phi);
+    };
+    axis(tb[0], tb[3], lo.x, hi.x, nl.x, nh.x);
+    axis(tb[1], tb[4], lo.y, hi.y, nl.y, nh.y);
+    axis(tb[2], tb[5], lo.z, hi.z, nl.z, nh.z);
+    return reach > -1e-5f * scale;
+}
+
+// One wave's working memory of k_cut_decide.
+struct DecideLds {
+    int stack[kDecideStack];  // pending internal nodes
+    int amb[128];             // nodes whose decision needs every pixel
+    int keep[kKeep + 64];     // kept nodes, flushed in chunks of kKeep
+    uint32_t ex[2 * kKeep];   // exact ranges first << 7 | (count - 1), flushed likewise
+    float4 pix[64][kPixRec];
+};
+
+// The cut of one tile by one wave, 64 nodes at a time, one per lane.
+//
+// A lane first decides its node from the tile as a whole and a few of its
+// pixels, which settles most nodes with a fraction of the 64-pixel test:
+//   refined   when one of the sample pixels asks for it (any pixel may);
+//   dropped   when the whole box lies behind every pixel's tangent plane (the
+//             height over the planes, by interval products over the tile's
+//             positions and normals, is below 0 by more than rounding);
+//   kept      when the bound at the tile's nearest point with the interval
+//             height is below the tile's smallest threshold, and some sample
+//             pixel has the box in front of it.
+// The rest are queued, and tested against all 64 pixels (from LDS) once 64 of
+// them have come together.  Every decision is the one the pixels' bounds
+// give: the tile's tests only settle nodes whose outcome they prove, with a
+// margin above FP32 rounding.
+//
+// Bound by the VALU (about 200 instructions per 64 nodes for the first test,
+// 30 per node for those that need every pixel) against 30 per node and a
+// dependent load each for one node at a time.
+template <bool kMany, bool kExpansion>
+__global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, int nitems, CutPool pool) {
+    __shared__ DecideLds lds[kCutThreads / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int item;
+    if constexpr (kMany) {
+        item = uniform(blockIdx.x * (kCutThreads / 64) + wave);
+        if (item >= nitems) return;  // the whole wave: no block barrier below
+    } else {  // a block's four tiles are one 16x16-pixel block, neighbouring blocks on one XCD
+        const int gx = (views.one.W + 15) / 16, gy = (views.one.H + 15) / 16;
+        const int b = xcd_block(blockIdx.x, gx * gy);
+        item = uniform(((b / gx) * 2 + (wave >> 1)) * 2 * gx + (b % gx) * 2 + (wave & 1));
+    }
+    const CutView v = views.of(item);
+    const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
+    const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
+    const bool live = x < v.W && y < v.H;
+    const uint64_t alive = __ballot(live);
+    if (alive == 0) {  // a tile of the 16x16 block outside the image
+        if (lane == 0) pool.head[item] = -1;
+        return;
+    }
+    DecideLds& S = lds[wave];
+    const bool outside = !((alive >> 63) & 1);  // some lane is outside the image
+    const bool expansion = kExpansion && v.criterion == ARC_CRITERION_EXPANSION;
+    const float delta2 = v.delta * v.delta;
+    float tb[6], tlo[3], thi[3], nlo[3], nhi[3], thr_min;
+    int rep[5];
+    {
+        const int q = live ? y * v.W + x : 0;
+        const PixelF P = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, q);
+        const float thr = live ? view_threshold(v).at(q) : INFINITY;
+        const float px = P.px, py = P.py, pz = P.pz;
+        const float nx = P.nx, ny = P.ny, nz = P.nz;
+        S.pix[lane][0] = make_float4(px, py, pz, thr);
+        S.pix[lane][1] = make_float4(fmaxf(nx, 0.f), fmaxf(ny, 0.f), fmaxf(nz, 0.f), 0.f);
+        S.pix[lane][2] = make_float4(fminf(nx, 0.f), fminf(ny, 0.f), fminf(nz, 0.f), 0.f);
+        tlo[0] = wave_fmin(live ? px : INFINITY);
+        tlo[1] = wave_fmin(live ? py : INFINITY);
+        tlo[2] = wave_fmin(live ? pz : INFINITY);
+        thi[0] = wave_fmax(live ? px : -INFINITY);
+        thi[1] = wave_fmax(live ? py : -INFINITY);
+        thi[2] = wave_fmax(live ? pz : -INFINITY);
+        nlo[0] = wave_fmin(live ? nx : INFINITY);
+        nlo[1] = wave_fmin(live ? ny : INFINITY);
+        nlo[2] = wave_fmin(live ? nz : INFINITY);
+        nhi[0] = wave_fmax(live ? nx : -INFINITY);
+        nhi[1] = wave_fmax(live ? ny : -INFINITY);
+        nhi[2] = wave_fmax(live ? nz : -INFINITY);
+        thr_min = wave_fmin(thr);
+        const uint64_t least = __ballot(live && thr <= thr_min);
+        rep[0] = least ? __ffsll((unsigned long long)least) - 1 : __ffsll((unsigned long long)alive) - 1;
+        // the corners; lane 63 also where it is outside the image (as it is whenever any lane is)
+        rep[1] = 0;
+        rep[2] = (alive >> 7) & 1 ? 7 : rep[0];
+        rep[3] = (alive >> 56) & 1 ? 56 : rep[0];
+        rep[4] = 63;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            tb[a] = 0.5f * (tlo[a] + thi[a]);
+            tb[3 + a] = 0.5f * (thi[a] - tlo[a]);
+        }
+        if (lane == 0) {
+            float* o = pool.tbox + 8 * (size_t)item;
+#pragma unroll
+            for (int a = 0; a < 6; ++a) o[a] = tb[a];
+        }
+    }
+    __builtin_amdgcn_wave_barrier();  // the wave's pixel records before its reads of other lanes'
+
+    int sp = 0, na = 0, ne = 0, nx = 0;             // wave-uniform queue lengths
+    int ntest = 0, nvis = 0, nkeep = 0, nleaf = 0;  // wave-uniform counts
+    int lexact = 0;                                 // per lane: AVPLs of the exact ranges this lane found
+    int ldone = 0;                                  // per lane: AVPLs of the nodes it decided without refining
+    int nbud = 0;                                   // nodes kept because the budget was spent
+    int head = -1, last = -1;                       // the tile's chunks
+    bool full = false, over = false;                // the pool has no room; the budget is reached
+
+    int spare = 0, nspare = 0;  // chunks taken from the pool and not used yet
+    // the next chunk, linked to the tile's: part `part` of the entries in chunk `from` (-1: its own); false: the pool is full
+    auto chunk = [&](int kind, int cnt, int from, int part, int& c) {
+        if (nspare == 0) {
+            nspare = head < 0 ? pool.grab : 2 * pool.grab;
+            int got = 0;
+            if (lane == 0) got = atomicAdd(pool.taken, nspare);
+            spare = uniform(got);
+        }
+        c = spare;
+        if (c >= pool.cap) return false;
+        ++spare;
+        --nspare;
+        if (lane == 0) {
+            pool.meta[c] = make_int4(item, kind | (cnt << 8), -1, (from < 0 ? c : from) * 16 + part);
+            if (last >= 0) pool.meta[last].z = c;
+        }
+        if (head < 0) head = c;
+        last = c;
+        return true;
+    };
+    auto evaluated = [&]() { return nkeep + nleaf + wave_isum(lexact); };
+    auto flush_keep = [&](int least) {
+        while (ne >= least && ne > 0 && !full) {
+            const int m = min(ne, kKeep);
+            int c;
+            if (!chunk(kNodes, m, -1, 0, c)) {
+                full = true;
+                return;
+            }
+            uint32_t* dst = pool.entries + (size_t)c * kKeep;
+            if (lane < m) dst[lane] = (uint32_t)S.keep[lane];
+            if (lane + 64 < m) dst[lane + 64] = (uint32_t)S.keep[lane + 64];
+            const int rest = ne - m;  // < 64
+            const int r = lane < rest ? S.keep[m + lane] : 0;
+            __builtin_amdgcn_wave_barrier();
+            if (lane < rest) S.keep[lane] = r;
+            __builtin_amdgcn_wave_barrier();
+            ne = rest;
+        }
+    };
+    auto flush_ex = [&](int least) {
+        while (nx >= least && nx > 0 && !full) {
+            const int m = min(nx, kKeep);
+            const uint32_t x0 = lane < m ? S.ex[lane] : 0u, x1 = lane + 64 < m ? S.ex[lane + 64] : 0u;
+            int parts = 1;
+            if (v.exact_count > kChunkLeaves / kKeep) {
+                const int leaves = (lane < m ? (int)(x0 & 127u) + 1 : 0) + (lane + 64 < m ? (int)(x1 & 127u) + 1 : 0);
+                parts = (wave_isum(leaves) + kChunkLeaves - 1) / kChunkLeaves;  // at most 128 x 128 leaves: 8
+            }
+            int c = -1, first = -1;
+            for (int k = 0; k < parts; ++k) {
+                if (!chunk(kRanges, m, first, k, c)) {
+                    full = true;
+                    return;
+                }
+                if (k == 0) first = c;
+            }
+            uint32_t* dst = pool.entries + (size_t)first * kKeep;
+            if (lane < m) dst[lane] = x0;
+            if (lane + 64 < m) dst[lane + 64] = x1;
+            const int rest = nx - m;  // < kKeep
+            const uint32_t r0 = lane < rest ? S.ex[m + lane] : 0u, r1 = lane + 64 < rest ? S.ex[m + lane + 64] : 0u;
+            __builtin_amdgcn_wave_barrier();
+            if (lane < rest) S.ex[lane] = r0;
+            if (lane + 64 < rest) S.ex[lane + 64] = r1;
+            __builtin_amdgcn_wave_barrier();
+            nx = rest;
+        }
+    };
+    // The decided nodes of a batch, one per lane: exact ranges, refined nodes
+    // (their leaf children are exact ranges of one), kept nodes.
+    auto apply = [&](int k, const float4& r0, const float4& r1, const float4& r2, bool exact, bool refine, bool keep) {
+        const int first = __float_as_int(r1.w), l = __float_as_int(r2.x), r = __float_as_int(r2.y),
+                  count = __float_as_int(r2.z);
+        const uint64_t mx = __ballot(exact), mr = __ballot(refine), mk = __ballot(keep);
+        ntest += __popcll(mr) + __popcll(mk);
+        nvis += __popcll(mr);
+        if (exact) {
+            S.ex[nx + lane_below(mx)] = ((uint32_t)first << 7) | (uint32_t)(count - 1);
+            lexact += count;
+        }
+        nx += __popcll(mx);
+        if (mr) {
+            const bool li = refine && l < 0, ri = refine && r < 0, ll = refine && l >= 0, rl = refine && r >= 0;
+            const uint64_t mli = __ballot(li), mri = __ballot(ri), mll = __ballot(ll), mrl = __ballot(rl);
+            if (li) S.stack[sp + lane_below(mli)] = -(l + 1);
+            sp += __popcll(mli);
+            if (ri) S.stack[sp + lane_below(mri)] = -(r + 1);
+            sp += __popcll(mri);
+            if (ll) S.ex[nx + lane_below(mll)] = (uint32_t)l << 7;
+            nx += __popcll(mll);
+            if (rl) S.ex[nx + lane_below(mrl)] = (uint32_t)r << 7;
+            nx += __popcll(mrl);
+            nleaf += __popcll(mll) + __popcll(mrl);
+        }
+        if (mk) {
+            bool faces = false;
+            if (keep) faces = node_faces(tb, r0, r1, v.nbox[2 * (size_t)k], v.nbox[2 * (size_t)k + 1]);
+            const uint64_t mf = __ballot(faces);
+            if (faces) S.keep[ne + lane_below(mf)] = k;
+            ne += __popcll(mf);
+            nkeep += __popcll(mf);
+        }
+        __builtin_amdgcn_wave_barrier();  // the queues' writes before other lanes read them
+        if (ne >= kKeep || nx >= kKeep) {
+            over = evaluated() >= v.budget;
+            if (!over) {
+                flush_keep(kKeep);
+                flush_ex(kKeep);
+            }
+        }
+    };
+    // The whole subtree of node k, 64 nodes at a time.  False when the budget
+    // is reached inside it or the pool is full.
+    auto subtree = [&](int root) {
+        const int base = sp;
+        if (lane == 0) S.stack[sp] = root;
+        ++sp;
+        __builtin_amdgcn_wave_barrier();
+        bool one = false;  // the stack is full: depth first, the node just queued before any other
+        while (!over && !full) {
+            const int room = kDecideStack - kStackReserve - sp;
+            const bool every = one || (room >= 2 && (na >= 64 || sp == base));  // from every pixel
+            if (every && na == 0) break;
+            const int m = one ? 1 : every ? min(min(64, na), room / 2) : max(1, min(min(64, sp - base), room));
+            const bool on = lane < m;
+            const int k = !on ? 0 : every ? S.amb[na - 1 - lane] : S.stack[sp - 1 - lane];
+            if (every) na -= m;
+            else sp -= m;
+            __builtin_amdgcn_wave_barrier();  // read before the slots are written over
+            const float4* r = v.trav + (size_t)kTrav * k;
+            const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+            float s2 = 0.f;
+            float4 m0 = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (expansion) {
+                const float4* mr = v.mom + (size_t)kMom * k;
+                m0 = mr[0];
+                s2 = mr[1].x * mr[1].x;
+            }
+            const bool small = __float_as_int(r2.z) <= v.exact_count;
+            bool ask = false, front = false, exact, refine, keep, unsure = false;
+            if (every) {
+                for (int p = 0; p < 64; p += 4) {
+        #pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        float thr;
+                        const float4* P = S.pix[p + u];
+                        const float b = pixel_bound(P, r0, r1, delta2, thr);
+                        if (expansion) {
+                            const float dx = m0.x - P[0].x, dy = m0.y - P[0].y, dz = m0.z - P[0].z;
+                            const float dc2 = dx * dx + dy * dy + dz * dz;
+                            ask = ask || (b > 0.f && (s2 > v.open2 * dc2 || b * s2 > thr * dc2));
+                        } else {
+                            ask = ask || b > thr;
+                        }
+                        front = front || b > 0.f;
+                    }
+                    if (!__ballot(on && !(small ? front : ask))) break;  // every node is settled
+                }
+                exact = on && small && front;
+                refine = on && !small && ask;
+                keep = on && !small && !ask && front;
+                one = false;
+            } else {
+                float ux = 0.f, scale = 0.f, d2 = 0.f;
+                bool outside_front = false;
+                auto axis = [&](float lo, float hi, float plo, float phi, float nl, float nh) {
+                    const float dlo = lo - phi, dhi = hi - plo;  // box - pixel over the tile
+                    ux += fmaxf(fmaxf(nl * dlo, nl * dhi), fmaxf(nh * dlo, nh * dhi));
+                    scale += fmaxf(fabsf(dlo), fabsf(dhi));
+                    const float e = fmaxf(fmaxf(dlo, plo - hi), 0.f);
+                    d2 = fmaf(e, e, d2);
+                };
+                axis(r0.x, r1.x, tlo[0], thi[0], nlo[0], nhi[0]);
+                axis(r0.y, r1.y, tlo[1], thi[1], nlo[1], nhi[1]);
+                axis(r0.z, r1.z, tlo[2], thi[2], nlo[2], nhi[2]);
+                const float ri = __builtin_amdgcn_rsqf(fmaxf(d2, delta2));
+                const float most = r0.w * __builtin_amdgcn_fmed3f((ux + 1e-5f * scale) * ri, 0.f, 1.f) * (ri * ri) * 1.001f;
+                bool far = true;  // the expansion criterion's distance tests cannot ask for the node
+                float lim = thr_min;
+                if (expansion) {
+                    const float cx = fmaxf(fmaxf(tlo[0] - m0.x, m0.x - thi[0]), 0.f), cy = fmaxf(fmaxf(tlo[1] - m0.y, m0.y - thi[1]), 0.f),
+                                cz = fmaxf(fmaxf(tlo[2] - m0.z, m0.z - thi[2]), 0.f);
+                    const float dc2 = (cx * cx + cy * cy + cz * cz) * 0.998f;
+                    far = s2 <= v.open2 * dc2;
+                    lim = thr_min * dc2;
+                }
+        #pragma unroll
+                for (int j = 0; j < 5; ++j) {
+                    float thr;
+                    const float4* P = S.pix[rep[j]];
+                    const float b = pixel_bound(P, r0, r1, delta2, thr);
+                    if (expansion) {
+                        const float dx = m0.x - P[0].x, dy = m0.y - P[0].y, dz = m0.z - P[0].z;
+                        const float dc2 = dx * dx + dy * dy + dz * dz;
+                        ask = ask || (b > 0.f && (s2 > v.open2 * dc2 || b * s2 > thr * dc2));
+                    } else {
+                        ask = ask || b > thr;
+                    }
+                    front = front || b > 0.f;
+                    outside_front = j == 4 && outside && b > 0.f;
+                }
+                const bool behind = ux < -1e-5f * scale && !outside_front;
+                const bool below = expansion ? far && most * s2 <= lim : most <= lim;
+                exact = on && small && front && !behind;
+                refine = on && !small && ask;
+                keep = on && !small && !ask && front && below && !behind;
+                unsure = on && !(exact || refine || keep || behind);
+                const uint64_t mu = __ballot(unsure);
+                if (unsure) S.amb[na + lane_below(mu)] = k;
+                na += __popcll(mu);
+                one = room < 2 && mu != 0;
+            }
+            if (on && !refine && (every || !unsure)) ldone += __float_as_int(r2.z);
+            apply(k, r0, r1, r2, exact, refine, keep);
+        }
+        if (!over && !full) over = evaluated() >= v.budget;
+        return !over && !full;
+    };
+    // Node k alone, from every pixel (one per lane): its children are pushed
+    // (a leaf as -(leaf + 1)), unless the budget is spent.
+    auto single = [&](int k) {
+        const float4* r = v.trav + (size_t)kTrav * k;
+        const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+        float thr;
+        const float b = pixel_bound(S.pix[lane], r0, r1, delta2, thr);
+        if (!__ballot(b > 0.f)) return;
+        const int count = __float_as_int(r2.z);
+        if (count <= v.exact_count) {
+            if (lane == 0) {
+                S.ex[nx] = ((uint32_t)__float_as_int(r1.w) << 7) | (uint32_t)(count - 1);
+                lexact += count;
+            }
+            ++nx;
+            return;
+        }
+        bool ask = b > thr;
+        if (expansion) {
+            const float4* mr = v.mom + (size_t)kMom * k;
+            const float4 m0 = mr[0], p = S.pix[lane][0];
+            const float s2 = mr[1].x * mr[1].x, dx = m0.x - p.x, dy = m0.y - p.y, dz = m0.z - p.z;
+            const float dc2 = dx * dx + dy * dy + dz * dz;
+            ask = b > 0.f && (s2 > v.open2 * dc2 || b * s2 > thr * dc2);
+        }
+        ++ntest;
+        const bool refine = __ballot(ask) != 0;
+        if (refine && evaluated() < v.budget) {
+            ++nvis;
+            const int l = __float_as_int(r2.x), rr = __float_as_int(r2.y);  // child < 0: internal -(k + 1)
+            if (lane == 0) {
+                S.stack[sp] = -(rr + 1);
+                S.stack[sp + 1] = -(l + 1);
+            }
+            sp += 2;
+            return;
+        }
+        nbud += refine;
+        if (node_faces(tb, r0, r1, v.nbox[2 * (size_t)k], v.nbox[2 * (size_t)k + 1])) {
+            if (lane == 0) S.keep[ne] = k;
+            ++ne;
+            ++nkeep;
+        }
+    };
+    // Depth first over subtrees.  The budget ends a cut in depth-first order:
+    // a node that asks to be refined is kept once the nodes before it have
+    // used the budget up.  A subtree after which the budget is not reached
+    // never meets that, and is cut in any order; one that reaches it is taken
+    // back and entered a node at a time, and so is one whose AVPLs, at the
+    // share of them that the last such subtree's cut evaluated, would reach
+    // it.  Nearly every tile's first subtree, the whole tree, is its last.
+    float share = 0.f;
+    if (lane == 0) S.stack[0] = 0;  // the root
+    __builtin_amdgcn_wave_barrier();
+    sp = 1;
+    while (sp > 0 && !full) {
+        const int k = uniform(S.stack[sp - 1]);
+        --sp;
+        __builtin_amdgcn_wave_barrier();
+        if (k < 0) {  // a leaf
+            if (lane == 0) S.ex[nx] = (uint32_t)(-(k + 1)) << 7;
+            ++nx;
+            ++nleaf;
+        } else {
+            // the queues are empty unless the budget is spent, so taking a
+            // subtree back is taking its chunks back
+            const int base = sp, c0 = last, t0 = ntest, v0 = nvis, k0 = nkeep, l0 = nleaf, e0 = lexact;
+            const float size = __float_as_int(v.trav[(size_t)kTrav * k + 2].z);
+            const bool enter = over || share * size > (float)(v.budget - evaluated());
+            ldone = 0;
+            if (enter || (!subtree(k) && !full)) {
+                if (!enter) {
+                    share = (float)(evaluated() - k0 - l0 - wave_isum(e0)) / (float)max(wave_isum(ldone), 1);
+                    if (lane == 0) {
+                        for (int c = c0 >= 0 ? pool.meta[c0].z : head; c >= 0; c = pool.meta[c].z) pool.meta[c].y = 0;
+                        if (c0 >= 0) pool.meta[c0].z = -1;
+                    }
+                    if (c0 < 0) head = -1;
+                    last = c0;
+                    sp = base;
+                    na = ne = nx = 0;
+                    ntest = t0;
+                    nvis = v0;
+                    nkeep = k0;
+                    nleaf = l0;
+                    lexact = e0;
+                    over = false;
+                }
+                single(k);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        over = evaluated() >= v.budget;
+        const int least = over && sp > 0 ? kKeep : 1;
+        flush_keep(least);
+        flush_ex(least);
+    }
+    if (lane < nspare && spare + lane < pool.cap) pool.meta[spare + lane] = make_int4(item, 0, -1, 0);
+    if (full) {  // hand the tile to k_cut_serial, its chunks to nobody
+        if (lane == 0) {
+            for (int c = head; c >= 0; c = pool.meta[c].z) pool.meta[c].y = 0;
+            pool.head[item] = -1;
+            pool.serial[atomicAdd(pool.nserial, 1)] = item;
+            pool.evaluated[item] = -1;
+        }
+        return;
+    }
+    const int total = evaluated();
+    if (lane == 0) {
+        pool.head[item] = head;
+        pool.evaluated[item] = total;
+        if (v.counters) {
+            const unsigned long long n = (unsigned long long)__popcll(alive);
+            atomicAdd(&v.counters[C_TESTED], n * ntest);
+            atomicAdd(&v.counters[C_VISITED], n * nvis);
+            atomicAdd(&v.counters[C_EVALUATED], n * total);
+            atomicAdd(&v.counters[C_EXACT], n * (total - nkeep));
+            atomicAdd(&v.counters[C_BUDGET], (unsigned long long)nbud);
+        }
+    }
+}
+
+// ---- the chunks' sums ----------------------------------------------------
+//
+// On gfx950 an FP32 add, multiply or FMA whose operands are vector registers
+// (or inline constants) issues every 2.4 cycles per SIMD with four waves or
+// more, and every 4.5 with a scalar operand; maxima, compares and selects take
+// 4.5 too, a reciprocal 8.4 (measured per instruction).  So the records, one
+// for many pixels, are read into vector registers (from LDS, where the read
+// costs 8 cycles of the CU per 16 bytes and wave), and to pay for the reads a
+// wave takes kSlots records at a time: its lanes are kSlots groups, group r
+// holds record r, and each lane kSlots of the tile's 64 pixels (its place in
+// the group + kGroupLanes b).  The lanes that share a pixel meet once per
+// chunk.  Clamps are output modifiers of multiplies, which cost nothing.
+constexpr int kSlots = 2, kGroupLanes = 64 / kSlots;
+struct Pixels {  // a lane's pixels
+    float px[kSlots], py[kSlots], pz[kSlots], nx[kSlots], ny[kSlots], nz[kSlots];
+};
+
+// One wave's working memory of k_cut_eval.
+struct EvalLds {
+    uint32_t ex[kKeep];  // a chunk's kept nodes or exact ranges
+    int pfx[kKeep];      // the ranges' leaves' prefix counts
+    int mark[64];        // where ranges start among 64 leaves
+    union {
+        struct {
+            float4 a[64 + 2 * kSlots];  // (x, y, z, nx) of the leaves that face the tile
+            float4 b[64 + 2 * kSlots];  // (ny, nz, Ir, Ig)
+            float c[64 + 2 * kSlots];   // Ib
+        } leaf;
+        float4 pix[2][64];      // the tile's pixels on their way to the lanes
+    };
+};
+
+// G of a leaf (a unit normal) for a pixel, leaf_g's product as the two cosines
+// clamped to [0, 1] by their multiplies (they are at most 1 to rounding) over
+// |d|^2.
+__device__ inline float leaf_cos2(const Pixels& P, int b, float x, float y, float z, float nx, float ny, float nz) {
+    const float dx = x - P.px[b], dy = y - P.py[b], dz = z - P.pz[b];
+    const float inv = __builtin_amdgcn_rsqf(dist2(dx, dy, dz, kDistFloor2));
+    const float c1 = __builtin_amdgcn_fmed3f((P.nx[b] * dx + P.ny[b] * dy + P.nz[b] * dz) * inv, 0.f, 1.f);
+    const float c2 = __builtin_amdgcn_fmed3f((nx * dx + ny * dy + nz * dz) * -inv, 0.f, 1.f);
+    return (c1 * c2) * (inv * inv);
+}
+
+// n staged leaves, n a multiple of 2 kSlots.
+__device__ inline void sum_leaves(const EvalLds& S, int n, const Pixels& P, float (&tot)[kSlots][3]) {
+    const int r = (threadIdx.x & 63) / kGroupLanes;
+    const float4 *pa = S.leaf.a + r, *pq = S.leaf.b + r;
+    const float* pc = S.leaf.c + r;
+    for (int j = 0; j < n; j += 2 * kSlots, pa += 2 * kSlots, pq += 2 * kSlots, pc += 2 * kSlots) {
+#pragma unroll
+        for (int u = 0; u < 2 * kSlots; u += kSlots) {
+            const float4 a = pa[u], q = pq[u];
+            const float c = pc[u];
+#pragma unroll
+            for (int b = 0; b < kSlots; ++b) {
+                const float g = leaf_cos2(P, b, a.x, a.y, a.z, a.w, q.x, q.y);
+                tot[b][0] = fmaf(q.z, g, tot[b][0]);
+                tot[b][1] = fmaf(q.w, g, tot[b][1]);
+                tot[b][2] = fmaf(c, g, tot[b][2]);
+            }
+        }
+    }
+}
+
+// A chunk's exact ranges: the kChunkLeaves leaves from `from` on that face the tile.
+__device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, int nx, int from, const float* tb,
+                                  const Pixels& P, float (&tot)[kSlots][3]) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+    walk_ranges(crec, S.ex, nx, from, kChunkLeaves, S.pfx, S.mark, tb, [&](bool facing, const float4& r0, const float4& r1, const float4& r2) {
+        const uint64_t m = __ballot(facing);
+        if (facing) {
+            const int j = n + lane_below(m);
+            S.leaf.a[j] = make_float4(r0.x, r0.y, r0.z, r1.x);
+            S.leaf.b[j] = make_float4(r1.y, r1.z, r2.x, r2.y);
+            S.leaf.c[j] = r2.z;
+        }
+        n += __popcll(m);
+        __builtin_amdgcn_wave_barrier();  // before the wave's reads of other lanes' writes
+        const int whole = n & ~(2 * kSlots - 1), rest = n - whole;
+        sum_leaves(S, whole, P, tot);
+        if (rest && whole) {  // the rest waits for the next 64 leaves
+            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+            float c = 0.f;
+            if (lane < rest) {
+                a = S.leaf.a[whole + lane];
+                b = S.leaf.b[whole + lane];
+                c = S.leaf.c[whole + lane];
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (lane < rest) {
+                S.leaf.a[lane] = a;
+                S.leaf.b[lane] = b;
+                S.leaf.c[lane] = c;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        n = rest;
+    });
+    if (n) {  // padded with leaves without intensity
+        if (lane >= n && lane < 2 * kSlots) {
+            S.leaf.a[lane] = S.leaf.a[0];
+            S.leaf.b[lane] = make_float4(S.leaf.b[0].x, S.leaf.b[0].y, 0.f, 0.f);
+            S.leaf.c[lane] = 0.f;
+        }
+        __builtin_amdgcn_wave_barrier();
+        sum_leaves(S, 2 * kSlots, P, tot);
+    }
+}
+
+// A wave per chunk, the chunks taken as waves come free: a chunk is at most
+// kKeep estimates or kChunkLeaves exact pairs per pixel, so the launch's waves
+// end together whichever tiles the cut is large in.
+template <bool kMany>
+__global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_cut_eval(Views<kMany> views, CutPool pool) {
+    __shared__ EvalLds lds[kCutThreads / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    EvalLds& S = lds[wave];
+    const int waves = gridDim.x * (kCutThreads / 64);
+    const int n = uniform(min(*pool.taken, pool.cap));
+    // chunks are taken in groups, a fraction of a wave's share, so that few atomics serve many chunks
+    const int group = max(1, min(8, n / (4 * waves)));
+    for (int c = 0, left = 0;; ++c, --left) {
+        if (left <= 0) {
+            int got = 0;
+            if (lane == 0) got = atomicAdd(pool.next, group);
+            c = uniform(got);
+            if (c >= n) break;
+            left = min(group, n - c);
+        }
+        const int4 m = pool.meta[c];
+        const int item = uniform(m.x), kind = uniform(m.y) & 255, cnt = uniform(m.y) >> 8;
+        if (cnt == 0) continue;  // not used, or its tile is cut serially
+        const CutView v = views.of(item);
+        const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
+        const uint32_t* e = pool.entries + (size_t)(uniform(m.w) >> 4) * kKeep;
+        const uint32_t e0 = lane < cnt ? e[lane] : 0u, e1 = lane + 64 < cnt ? e[lane + 64] : 0u;
+        const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
+        const PixelF F = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, x < v.W && y < v.H ? y * v.W + x : 0);
+        float* o = pool.part + (size_t)c * 192 + lane;
+        if (kind == kNodes) {
+            Acc acc;
+            const int half = min(cnt, 64);
+            for (int j = 0; j < half; ++j)
+                add_moments<true>(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e0, j), acc);
+            acc.flush();
+            for (int j = 64; j < cnt; ++j)
+                add_moments<true>(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e1, j - 64), acc);
+            acc.flush();
+            o[0] = acc.k[0].s;
+            o[64] = acc.k[1].s;
+            o[128] = acc.k[2].s;
+            continue;
+        }
+        if (lane < cnt) S.ex[lane] = e0;
+        if (lane + 64 < cnt) S.ex[lane + 64] = e1;
+        S.pix[0][lane] = make_float4(F.px, F.py, F.pz, F.nx);
+        S.pix[1][lane] = make_float4(F.ny, F.nz, 0.f, 0.f);
+        __builtin_amdgcn_wave_barrier();
+        Pixels P;
+#pragma unroll
+        for (int b = 0; b < kSlots; ++b) {
+            const int k = lane % kGroupLanes + kGroupLanes * b;
+            const float4 p = S.pix[0][k], q = S.pix[1][k];
+            P.px[b] = p.x; P.py[b] = p.y; P.pz[b] = p.z;
+            P.nx[b] = p.w; P.ny[b] = q.x; P.nz[b] = q.y;
+        }
+        __builtin_amdgcn_wave_barrier();  // read before the leaves are written over them
+        float tot[kSlots][3];
+#pragma unroll
+        for (int b = 0; b < kSlots; ++b) tot[b][0] = tot[b][1] = tot[b][2] = 0.f;
+        ufloat* box = uptr(pool.tbox + 8 * (size_t)item);
+        const float tb[6] = {box[0], box[1], box[2], box[3], box[4], box[5]};
+        sum_ranges(v.crec, S, cnt, (uniform(m.w) & 15) * kChunkLeaves, tb, P, tot);
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) {
+            float out = 0.f;
+#pragma unroll
+            for (int b = 0; b < kSlots; ++b) {
+                float s = tot[b][ch];
+#pragma unroll
+                for (int off = kGroupLanes; off < 64; off <<= 1) s += __shfl_xor(s, off);
+                if (lane / kGroupLanes == b) out = s;  // lane l keeps pixel l
+            }
+            o[64 * ch] = out;
+        }
+    }
+}
+
+// Each tile's partial sums, in the order its chunks were made.
+template <bool kMany>
+__global__ __launch_bounds__(kCutThreads) void k_cut_combine(Views<kMany> views, int nitems, CutPool pool) {
+    const int lane = threadIdx.x & 63;
+    const int item = uniform(blockIdx.x * (kCutThreads / 64) + (threadIdx.x >> 6));
+    if (item >= nitems) return;
+    if (item == 0 && lane == 0) *pool.seen = *pool.taken;  // what the next frame's pool should hold
+    const CutView v = views.of(item);
+    const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
+    const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
+    if (!__ballot(x < v.W && y < v.H)) return;
+    const int evaluated = uniform(pool.evaluated[item]);
+    if (evaluated < 0) return;  // k_cut_serial writes it
+    Kahan k[3];
+    for (int c = uniform(pool.head[item]); c >= 0;) {
+        const float* s = pool.part + (size_t)c * 192 + lane;
+        c = uniform(pool.meta[c].z);
+        k[0].add(s[0]);
+        k[1].add(s[64]);
+        k[2].add(s[128]);
+    }
+    if (x >= v.W || y >= v.H) return;
+    const int q = y * v.W + x;
+    const PixelF P = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, q);
+    v.out_rad[q] = make_float4(k[0].s * P.br, k[1].s * P.bg, k[2].s * P.bb, v.counters ? (float)evaluated : 1.f);
+}
+
+// One depth-first cut, a node at a time, summed as it goes: the tiles that
+// found the pool full.  Kept nodes and exact ranges are queued in LDS and summed in passes
+// of their own when a queue fills, so the traversal carries no sums across
+// its branches.
+__device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int* E, uint32_t* X, int* pfx,
+                                            int* mark, float4 (*stage)[3], float* tb) {
+    const int lane = threadIdx.x & 63, tw = tiles_wide(v.W);
+    const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
+    const bool live = x < v.W && y < v.H;
+    const int q = live ? y * v.W + x : 0;
+    const PixelF P = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, q);
+    const float thr = live ? view_threshold(v).at(q) : INFINITY;
+    const float delta2 = v.delta * v.delta;
+    {  // the box of the tile's live pixels, as centre and half extent
+        const float lx = wave_fmin(live ? P.px : INFINITY), hx = wave_fmax(live ? P.px : -INFINITY);
+        const float ly = wave_fmin(live ? P.py : INFINITY), hy = wave_fmax(live ? P.py : -INFINITY);
+        const float lz = wave_fmin(live ? P.pz : INFINITY), hz = wave_fmax(live ? P.pz : -INFINITY);
         if (lane == 0) {
             tb[0] = 0.5f * (lx + hx);
             tb[1] = 0.5f * (ly + hy);
@@ -590,21 +1306,13 @@ __device__ __forceinline__ void cut_tile(const arc_bvh_node* __restrict__ nodes,
         }
         __builtin_amdgcn_wave_barrier();  // lane 0's writes before the wave's reads
     }
-    const bool expansion = criterion == ARC_CRITERION_EXPANSION;
+    const bool expansion = v.criterion == ARC_CRITERION_EXPANSION;
     Acc acc;
     unsigned nvis = 0, nev = 0, nerr = 0, nbud = 0, ntest = 0, nexact = 0;  // wave-uniform
     int ne = 0, nx = 0;                                                     // queued, wave-uniform
-    int head = -1;                                                          // the tile's last pool chunk
-    unsigned npool = 0;                                                     // nodes handed to the pool
-    // the queued kept nodes: to the pool when there is room, else estimated here
     auto flush_est = [&]() {
         if (ne == 0) return;
-        // A kept node whose AVPLs all face away from every pixel of the tile
-        // adds 0 (its estimate would add only the clamped cosine's
-        // second-order residue): the largest n_a . (p - x_a) over the
-        // node's normal box, its box and the tile's box, by interval
-        // products per axis, is below 0 by more than FP32 rounding.  One
-        // lane per queued node; the facing ones are compacted in place.
+        // the kept nodes that face the tile, one lane per node, compacted in place
         int kept = 0;
         for (int base = 0; base < ne; base += 64) {
             const int j = base + lane;
@@ -612,55 +1320,40 @@ __device__ __forceinline__ void cut_tile(const arc_bvh_node* __restrict__ nodes,
             int k = 0;
             if (j < ne) {
                 k = E[j];
-                const arc_bvh_node& nd = nodes[k];
-                const float4 nl = nbox[2 * (size_t)k], nh = nbox[2 * (size_t)k + 1];
-                float reach = 0.f, scale = 0.f;
-                auto axis = [&](float c, float e, float plo, float phi, float nlo, float nhi) {
-                    const float vlo = (c - e) - phi, vhi = (c + e) - plo;  // p - x over the boxes
-                    reach += fmaxf(fmaxf(nlo * vlo, nlo * vhi), fmaxf(nhi * vlo, nhi * vhi));
-                    scale += fabsf(c) + e + fabsf(plo) + fabsf(phi);
-                };
-                axis(tb[0], tb[3], nd.bbMin.x, nd.bbMax.x, nl.x, nh.x);
-                axis(tb[1], tb[4], nd.bbMin.y, nd.bbMax.y, nl.y, nh.y);
-                axis(tb[2], tb[5], nd.bbMin.z, nd.bbMax.z, nl.z, nh.z);
-                facing = reach > -1e-5f * scale;
+                const float4* r = v.trav + (size_t)kTrav * k;
+                facing = node_faces(tb, r[0], r[1], v.nbox[2 * (size_t)k], v.nbox[2 * (size_t)k + 1]);
             }
             const uint64_t fm = __ballot(facing);
             // every lane has read its entry before any is overwritten (kept <= base)
             __builtin_amdgcn_wave_barrier();
-            if (facing)
-                E[kept + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fm >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)fm, 0u))] = k;
+            if (facing) E[kept + lane_below(fm)] = k;
             kept += __popcll(fm);
             __builtin_amdgcn_wave_barrier();
         }
         nev -= (unsigned)(ne - kept);
-        ne = kept;
-        if (ne == 0) return;
-        if constexpr (kPool) {
-            int c = 0;
-            if (lane == 0) c = atomicAdd(pool->taken, 1);
-            c = uniform(c);  // lane 0's
-            if (c < pool->cap) {
-                uint32_t* dst = pool->entries + (size_t)c * kKeep;
-                if (lane < ne) dst[lane] = (uint32_t)E[lane];
-                if (lane + 64 < ne) dst[lane + 64] = (uint32_t)E[lane + 64];
-                if (lane == 0) pool->meta[c] = make_int2(ne, head);
-                head = c;
-                npool += ne;
-                ne = 0;
-                return;
-            }
-        }
-        for (int j = 0; j < ne; ++j) {
-            const int k = uniform(E[j]);
-            add_moments<kUniformAs>(P, mom + kMom * (size_t)k, acc);
+        for (int j = 0; j < kept; ++j) {
+            add_moments<true>(P, v.mom + kMom * (size_t)uniform(E[j]), acc);
             acc.maybe_flush();
         }
         ne = 0;
     };
     auto drain_exact = [&]() {
-        if (nx > 0) add_ranges(crec, X, nx, pfx, stage, tb, P, acc);
+        if (nx > 0)
+            walk_ranges(v.crec, X, nx, 0, INT_MAX, pfx, mark, tb, [&](bool facing, const float4& r0, const float4& r1, const float4& r2) {
+                const uint64_t fm = __ballot(facing);
+                if (facing) {
+                    const int j = lane_below(fm);
+                    stage[j][0] = r0;
+                    stage[j][1] = r1;
+                    stage[j][2] = r2;
+                }
+                __builtin_amdgcn_wave_barrier();
+                const int cnt = __popcll(fm);
+#pragma unroll 1
+                for (int j = 0; j < cnt; ++j) acc.add_run(stage[j][2], leaf_g(P, stage[j][0], stage[j][1]));
+                acc.maybe_flush();
+                __builtin_amdgcn_wave_barrier();  // read before the next 64 leaves' writes
+            });
         nx = 0;
     };
     int sp = 0;
@@ -669,34 +1362,39 @@ __device__ __forceinline__ void cut_tile(const arc_bvh_node* __restrict__ nodes,
         bool pop = true;  // take the next node from the stack (not a refined node's left child)
         if (node < 0) {
             const int k = -(node + 1);
-            const auto& b = NodeRead<kUniformAs>::node(nodes, k);
-            const float4 m0 = NodeRead<kUniformAs>::rec(mom, k, 0);  // (c, max I)
-            const float4 m1 = NodeRead<kUniformAs>::rec(mom, k, 1);  // (s, first, count, -)
-            const float s = m1.x;
-            const int first = __float_as_int(m1.y), count = __float_as_int(m1.z);
-            const float bound = node_bound1(P, b, m0.w, delta2);
+            ufloat* r = uptr(v.trav + (size_t)kTrav * k);
+            const float4 r0 = uload4(r), r1 = uload4(r + 4), r2 = uload4(r + 8);
+            arc_bvh_node b;
+            b.left = __float_as_int(r2.x);
+            b.right = __float_as_int(r2.y);
+            b.bbMin = arc_float3{r0.x, r0.y, r0.z};
+            b.bbMax = arc_float3{r1.x, r1.y, r1.z};
+            b.visited = 0;  // not read
+            const int first = __float_as_int(r1.w), count = __float_as_int(r2.z);
+            const float bound = node_bound1(P, b, r0.w, delta2);
             if (!__ballot(bound > 0.f)) {
                 // behind every pixel's tangent plane: contributes exactly 0
-            } else if (count <= exact_count) {
+            } else if (count <= v.exact_count) {
                 // small node: its AVPLs exactly (refining it would end in the same sum)
                 X[nx++] = ((uint32_t)first << 7) | (uint32_t)(count - 1);
                 nexact += count;
             } else {
                 bool refine;
                 if (expansion) {
-                    const float dx = m0.x - P.px, dy = m0.y - P.py, dz = m0.z - P.pz;
+                    ufloat* m = uptr(v.mom + kMom * (size_t)k);
+                    const float dx = m[0] - P.px, dy = m[1] - P.py, dz = m[2] - P.pz;
                     const float dc2 = dx * dx + dy * dy + dz * dz;
-                    const float s2 = s * s;
-                    refine = bound > 0.f && (s2 > open2 * dc2 || bound * s2 > thr * dc2);
+                    const float s2 = m[4] * m[4];
+                    refine = bound > 0.f && (s2 > v.open2 * dc2 || bound * s2 > thr * dc2);
                 } else {
                     refine = bound > thr;
                 }
                 ++ntest;
                 bool keep = true;
                 if (__ballot(refine)) {
-                    if ((int)(nev + nexact) >= budget) {
+                    if ((int)(nev + nexact) >= v.budget) {
                         ++nbud;  // cut budget spent: keep the cluster
-                    } else if (sp < kStack) {
+                    } else if (sp < kMomStack) {
                         S[sp++] = b.right;
                         node = uniform(b.left);
                         ++nvis;
@@ -725,370 +1423,47 @@ __device__ __forceinline__ void cut_tile(const arc_bvh_node* __restrict__ nodes,
     flush_est();
     drain_exact();
     acc.flush();
-    // the tile's cost in VALU instructions (about 30 per bound test, 130 per
-    // moment estimate made here, 18 per queued exact leaf: 26 per pair for
-    // the half that face the tile, a few for the rest; and the pixel's own
-    // loads and stores): the next frame's launch order
-    if (lane == 0) {
-        tile_cost[ty * tw + tx] = 300.f + 30.f * (float)ntest + 130.f * (float)(nev - npool) +
-                                  18.f * (float)nexact + 2.f * (float)npool;
-        if constexpr (kPool) {
-            pool->head[ty * tw + tx] = head;
-            pool->queued[ty * tw + tx] = (float)npool;
-        }
-    }
     const int alive = __popcll(__ballot(live));  // all lanes take part in the ballot
-    if (counters && lane == 0) {
-        atomicAdd(&counters[C_TESTED], (unsigned long long)ntest * alive);
-        atomicAdd(&counters[C_VISITED], (unsigned long long)nvis * alive);
-        atomicAdd(&counters[C_EVALUATED], (unsigned long long)(nev + nexact) * alive);
-        atomicAdd(&counters[C_EXACT], (unsigned long long)nexact * alive);
-        atomicAdd(&counters[C_ERRORS], (unsigned long long)nerr);
-        atomicAdd(&counters[C_BUDGET], (unsigned long long)nbud);
+    if (v.counters && lane == 0) {
+        atomicAdd(&v.counters[C_TESTED], (unsigned long long)ntest * alive);
+        atomicAdd(&v.counters[C_VISITED], (unsigned long long)nvis * alive);
+        atomicAdd(&v.counters[C_EVALUATED], (unsigned long long)(nev + nexact) * alive);
+        atomicAdd(&v.counters[C_EXACT], (unsigned long long)nexact * alive);
+        atomicAdd(&v.counters[C_ERRORS], (unsigned long long)nerr);
+        atomicAdd(&v.counters[C_BUDGET], (unsigned long long)nbud);
     }
     if (live)
-        out_rad[q] = make_float4(acc.k[0].s * P.br, acc.k[1].s * P.bg, acc.k[2].s * P.bb,
-                                 counters ? (float)(nev + nexact) : 1.f);
+        v.out_rad[q] = make_float4(acc.k[0].s * P.br, acc.k[1].s * P.bg, acc.k[2].s * P.bb,
+                                   v.counters ? (float)(nev + nexact) : 1.f);
 }
 
-// One launch per view: the view's tiles, in `order` when given (heaviest
-// first), else each block its four tiles of a 16x16-pixel block.
-//
-// Eight waves per SIMD: the registers are held to 64 VGPRs (a few values of
-// the tile's set-up spill, none inside the traversal or the sums), and a
-// block's LDS (about 20 KB with a stack of 64 or 96 nodes) lets eight blocks
-// share a CU's 160 KB.  The traversal waits on one dependent node load at a
-// time, so the eighth wave hides more of it: 37.5 -> 35.8 ms on the 1080p x
-// 1M frame.
-#define ARC_CUT_WAVES __attribute__((amdgpu_waves_per_eu(8)))
-template <bool kPool, int kStack>
-__global__ __launch_bounds__(kCutThreads) ARC_CUT_WAVES void k_cut_mom_tile(const arc_bvh_node* __restrict__ nodes,
-                                                              const float4* __restrict__ crec,
-                                                              const float4* __restrict__ mom,
-                                                              const float4* __restrict__ nbox,
-                                                              const float4* __restrict__ gpos,
-                                                              const float4* __restrict__ gnrm,
-                                                              const float4* __restrict__ galb,
-                                                              const arc_material* __restrict__ mats, int W, int H,
-                                                              Threshold th, float delta, int budget, int criterion,
-                                                              float open2, int exact_count,
-                                                              const int* __restrict__ order,
-                                                              float* __restrict__ tile_cost,
-                                                              float4* __restrict__ out_rad,
-                                                              unsigned long long* __restrict__ counters,
-                                                              const EstPool* __restrict__ pool) {
-    __shared__ int stk[kCutThreads / 64][kStack];
+// The tiles of pool.serial; with `all`, every tile of the launch.
+template <bool kMany>
+__global__ __launch_bounds__(kCutThreads) void k_cut_serial(Views<kMany> views, int nitems, int all,
+                                                           CutPool pool) {
+    __shared__ int stk[kCutThreads / 64][kMomStack];
     __shared__ int qest[kCutThreads / 64][kKeep];       // internal nodes to estimate
     __shared__ uint32_t qex[kCutThreads / 64][kKeep];   // exact ranges: first << 7 | (count - 1)
     __shared__ int qpfx[kCutThreads / 64][kKeep];       // their leaves' prefix counts
-    __shared__ float4 lstage[kCutThreads / 64][64][3];  // 64 leaf records
+    __shared__ int qmark[kCutThreads / 64][64];         // where ranges start among 64 leaves
+    __shared__ float4 lstage[kCutThreads / 64][64][3];  // leaves that face the tile
     __shared__ float tbox[kCutThreads / 64][8];         // the tile's box: centre, half extent
     const int wave = threadIdx.x >> 6;
-    // the wave's 8x8 tile: the tile grid is (2 gx) x (2 gy) tiles of the
-    // launch's gx x gy blocks of 16x16 pixels
-    const int gx = (W + 15) / 16, gy = (H + 15) / 16, tw = 2 * gx;
-    int tx, ty;
-    if (order) {
-        const int ti = uniform(order[blockIdx.x * 4 + wave]);
-        tx = ti % tw;
-        ty = ti / tw;
-    } else {
-        const int b = xcd_block(blockIdx.x, gx * gy);
-        tx = (b % gx) * 2 + (wave & 1);
-        ty = (b / gx) * 2 + (wave >> 1);
-    }
-    cut_tile<false, kPool, kStack>(nodes, crec, mom, nbox, gpos, gnrm, galb, mats, W, H, th, delta, budget, criterion, open2,
-                           exact_count, tile_cost, out_rad, counters, tx, ty, tw, stk[wave], qest[wave], qex[wave],
-                           qpfx[wave], lstage[wave], tbox[wave], pool);
-}
-
-// One launch over the tiles of many views: the launch's tiles are the views'
-// tile lists one after the other (view v's from views[v].tile_base), taken
-// in `order` when given, so the heaviest tiles of all views start first and
-// no view's tail runs alone.
-__global__ __launch_bounds__(kCutThreads) ARC_CUT_WAVES void k_cut_mom_views(const arc::CutView* __restrict__ views, int nviews,
-                                                               const int* __restrict__ order, int nitems) {
-    __shared__ int stk[kCutThreads / 64][kMomStack];
-    __shared__ int qest[kCutThreads / 64][kKeep];
-    __shared__ uint32_t qex[kCutThreads / 64][kKeep];
-    __shared__ int qpfx[kCutThreads / 64][kKeep];
-    __shared__ float4 lstage[kCutThreads / 64][64][3];
-    __shared__ float tbox[kCutThreads / 64][8];
-    const int wave = threadIdx.x >> 6;
-    const int slot = uniform(blockIdx.x * 4 + wave);  // one per wave (the compiler cannot see that)
-    if (slot >= nitems) return;  // the whole wave: the cut has no block barrier
-    const int item = order ? uniform(order[slot]) : slot;
-    int lo = 0, hi = nviews - 1;  // the last view whose tiles start at or before item
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (views[mid].tile_base <= item) lo = mid;
-        else hi = mid - 1;
-    }
-    const arc::CutView& v = views[lo];
-    const int t = item - v.tile_base;
-    const int tw = 2 * ((v.W + 15) / 16);
-    Threshold th;
-    th.est = v.th_est;
-    th.sum = v.th_sum;
-    th.eps = v.th_eps;
-    th.floor_frac = v.th_floor;
-    th.inv_npix = v.th_inv_npix;
-    cut_tile<true, false, kMomStack>(v.nodes, v.crec, v.mom, v.nbox, v.gpos, v.gnrm, v.galb, v.mats, v.W, v.H, th, v.delta, v.budget,
-                          v.criterion, v.open2, v.exact_count, v.tile_cost, v.out_rad, v.counters, t % tw, t / tw, tw,
-                          stk[wave], qest[wave], qex[wave], qpfx[wave], lstage[wave], tbox[wave], nullptr);
-}
-
-// ---- kept nodes on the matrix cores ---------------------------------------
-//
-// A kept node's estimate for a pixel p (add_moments) is made of dot products
-// of pixel features with node coefficients.  With d = c - p:
-//   |d|^2              = |c|^2 - 2 c . p + |p|^2
-//   n_p . (q_j - p)    = (q_j, -1) . (n_p, n_p . p)          (the four points)
-//   |q_j - p|^2        = |q_j|^2 - 2 q_j . p + |p|^2
-//   b_c . d            = (b_c . c, -b_c) . (1, p)
-//   d^T T'_c d         = a quadratic polynomial in p: 10 coefficients,
-// where T'_c is the record's quadratic form plus a_c on its diagonal, which
-// folds the constant term in (a_c = a_c |d|^2 / |d|^2): 15/128 T_c plus
-// 3/128 I_c on the diagonal.  Per channel
-//   A_c / 4 = b_c . d / |d| + d^T T'_c d / |d|^2,
-// and the node adds max(A_c / 4, 0) * sum_j max(n_p . (q_j - p), 0) / |q_j - p|^3.
-// For 16 nodes x 16 pixels each product is one 16x16x4 FP32 MFMA (the
-// quadratic form three, K = 12): 21 per block.  What stays on the VALU is
-// the five reciprocal square roots, the clamps and the sums.
-//
-// Coordinates are relative to the tile's first pixel.  The rounding of an
-// expanded square |c|^2 - 2 c . p + |p|^2 is relative to |c|^2 + |p|^2,
-// which stays within a small factor of |d|^2 for a kept node (its bound is
-// small: the node is far against its own size and the tile's).
-//
-// Lane l of v_mfma_f32_16x16x4f32 holds A[l % 16][l / 16], B[l / 16][l % 16]
-// and D[4 (l / 16) + r][l % 16], r = 0..3.  A row is a node (16 per group),
-// a column a pixel (16 per block, four blocks per tile), so lane l of the
-// result holds pixel l % 16 of the block for nodes 4 (l / 16) .. + 3: its sums
-// run over a quarter of the nodes and meet across lanes once at the end.
-typedef float mf4 __attribute__((ext_vector_type(4)));
-
-__device__ inline mf4 mfma4(float a, float b, mf4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-constexpr int kEstRows = 21;  // MFMA A operands per node
-constexpr int kEstFeat = 17;  // pixel features (16 in four sets of 4, and |p|^2)
-
-// Row k of the A operands of node record r (kMom float4), relative to o.
-__device__ inline void est_rows(const float4* __restrict__ r, float ox, float oy, float oz, int k,
-                                float (&a)[kEstRows]) {
-    const float4 m0 = r[0];
-    const float cx = m0.x - ox, cy = m0.y - oy, cz = m0.z - oz;
-    // component k - 1 of a vector (rows 1..3)
-    auto comp = [k](float x, float y, float z) { return k == 1 ? x : (k == 2 ? y : z); };
-    a[0] = k == 0 ? cx * cx + cy * cy + cz * cz : -2.f * comp(cx, cy, cz);
-    const float4 p01 = r[2], p12 = r[3], p23 = r[4];
-    const float q[12] = {p01.x, p01.y, p01.z, p01.w, p12.x, p12.y, p12.z, p12.w, p23.x, p23.y, p23.z, p23.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float qx = q[3 * j] - ox, qy = q[3 * j + 1] - oy, qz = q[3 * j + 2] - oz;
-        a[1 + 2 * j] = k == 0 ? qx : (k == 1 ? qy : (k == 2 ? qz : -1.f));
-        a[2 + 2 * j] = k == 0 ? qx * qx + qy * qy + qz * qz : -2.f * comp(qx, qy, qz);
-    }
-#pragma unroll
-    for (int ch = 0; ch < 3; ++ch) {
-        const float4 mr = r[5 + ch];
-        const float4 ta = r[8 + (6 * ch) / 4], tb = r[8 + (6 * ch + 4) / 4];
-        // the six floats 6 ch .. 6 ch + 5 of records 8..12: (xx, yy, zz, 2xy, 2xz, 2yz)
-        const float tt[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
-        const int o6 = (6 * ch) % 4;
-        const float al = mr.w;
-        const float txx = tt[o6] + al, tyy = tt[o6 + 1] + al, tzz = tt[o6 + 2] + al;
-        const float txy = tt[o6 + 3], txz = tt[o6 + 4], tyz = tt[o6 + 5];
-        a[9 + ch] = k == 0 ? mr.x * cx + mr.y * cy + mr.z * cz : -comp(mr.x, mr.y, mr.z);
-        const float lx = -(2.f * txx * cx + txy * cy + txz * cz);
-        const float ly = -(2.f * tyy * cy + txy * cx + tyz * cz);
-        const float lz = -(2.f * tzz * cz + txz * cx + tyz * cy);
-        const float c0 = txx * cx * cx + tyy * cy * cy + tzz * cz * cz + txy * cx * cy + txz * cx * cz + tyz * cy * cz;
-        a[12 + 3 * ch] = k == 0 ? c0 : comp(lx, ly, lz);
-        a[13 + 3 * ch] = k == 0 ? txx : (k == 1 ? tyy : (k == 2 ? tzz : txy));
-        a[14 + 3 * ch] = k == 0 ? txz : (k == 1 ? tyz : 0.f);
+    const int waves = gridDim.x * (kCutThreads / 64);
+    const int n = all ? nitems : uniform(*pool.nserial);
+    for (int k = uniform(blockIdx.x * (kCutThreads / 64) + wave); k < n; k += waves) {
+        const int item = all ? k : uniform(pool.serial[k]);
+        const CutView v = views.of(item);
+        serial_tile(v, item - (kMany ? v.tile_base : 0), stk[wave], qest[wave], qex[wave], qpfx[wave], qmark[wave], lstage[wave],
+                    tbox[wave]);
     }
 }
 
-// The pooled kept nodes of each tile, one wave per tile, added to the
-// traversal's sums in out_rad.  Tiles in `order` when given.
-__global__ __launch_bounds__(kCutThreads) void k_mom_est(const float4* __restrict__ mom,
-                                                         const uint32_t* __restrict__ entries,
-                                                         const int2* __restrict__ meta,
-                                                         const int* __restrict__ head,
-                                                         const float4* __restrict__ gpos,
-                                                         const float4* __restrict__ gnrm,
-                                                         const float4* __restrict__ galb,
-                                                         const arc_material* __restrict__ mats, int W, int H,
-                                                         const int* __restrict__ order,
-                                                         float4* __restrict__ out_rad) {
-    __shared__ float feat[kCutThreads / 64][kEstFeat][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int gx = (W + 15) / 16, gy = (H + 15) / 16, tw = 2 * gx;
-    int tx, ty;
-    if (order) {
-        const int ti = uniform(order[blockIdx.x * 4 + wave]);
-        tx = ti % tw;
-        ty = ti / tw;
-    } else {
-        const int b = xcd_block(blockIdx.x, gx * gy);
-        tx = (b % gx) * 2 + (wave & 1);
-        ty = (b / gx) * 2 + (wave >> 1);
-    }
-    int c = uniform(head[ty * tw + tx]);
-    if (c < 0) return;  // the whole wave: nothing pooled (no block barrier below)
-    const int2 xy = make_int2(tx * 8 + (lane & 7), ty * 8 + (lane >> 3));
-    const bool live = xy.x < W && xy.y < H;
-    const int q = live ? xy.y * W + xy.x : 0;
-    const PixelF P = load_pixel(gpos, gnrm, galb, mats, q);
-    // the tile's origin: its first pixel (lane 0's)
-    const float o_x = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(P.px)));
-    const float o_y = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(P.py)));
-    const float o_z = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(P.pz)));
-    {
-        const float px = P.px - o_x, py = P.py - o_y, pz = P.pz - o_z;
-        float (*f)[64] = feat[wave];
-        f[0][lane] = 1.f;
-        f[1][lane] = px;
-        f[2][lane] = py;
-        f[3][lane] = pz;
-        f[4][lane] = P.nx;
-        f[5][lane] = P.ny;
-        f[6][lane] = P.nz;
-        f[7][lane] = P.nx * px + P.ny * py + P.nz * pz;
-        f[8][lane] = px * px;
-        f[9][lane] = py * py;
-        f[10][lane] = pz * pz;
-        f[11][lane] = px * py;
-        f[12][lane] = px * pz;
-        f[13][lane] = py * pz;
-        f[14][lane] = 0.f;
-        f[15][lane] = 0.f;
-        f[16][lane] = px * px + py * py + pz * pz;
-    }
-    __builtin_amdgcn_wave_barrier();  // the wave's feature writes before its reads of other lanes'
-    const int kr = lane >> 4, col = lane & 15;
-    const mf4 zero = {0.f, 0.f, 0.f, 0.f};
-    float tot[4][3];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) tot[b][0] = tot[b][1] = tot[b][2] = 0.f;
-    while (c >= 0) {
-        const int2 m = meta[c];
-        const int cnt = uniform(m.x), prev = uniform(m.y);
-        for (int g0 = 0; g0 < cnt; g0 += 16) {
-            float a[kEstRows];
-            if (g0 + col < cnt) {
-                const int node = (int)entries[(size_t)c * kKeep + g0 + col];
-                est_rows(mom + kMom * (size_t)node, o_x, o_y, o_z, kr, a);
-            } else {
-#pragma unroll
-                for (int i = 0; i < kEstRows; ++i) a[i] = 0.f;  // no node: every product 0
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int px = 16 * b + col;
-                const float (*f)[64] = feat[wave];
-                const float b1 = f[kr][px], b2 = f[4 + kr][px], b4 = f[8 + kr][px], b5 = f[12 + kr][px];
-                const float p2 = f[16][px];
-                mf4 K = zero;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const mf4 cs = mfma4(a[1 + 2 * j], b2, zero);
-                    const mf4 dd = mfma4(a[2 + 2 * j], b1, zero);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float rr = __builtin_amdgcn_rsqf(fmaxf(dd[r] + p2, 1e-24f));
-                        K[r] = fmaf(fmaxf(cs[r], 0.f), rr * rr * rr, K[r]);
-                    }
-                }
-                const mf4 dc = mfma4(a[0], b1, zero);
-                mf4 inv, i2;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    inv[r] = __builtin_amdgcn_rsqf(fmaxf(dc[r] + p2, 1e-30f));
-                    i2[r] = inv[r] * inv[r];
-                }
-#pragma unroll
-                for (int ch = 0; ch < 3; ++ch) {
-                    const mf4 n1 = mfma4(a[9 + ch], b1, zero);
-                    mf4 n2 = mfma4(a[12 + 3 * ch], b1, zero);
-                    n2 = mfma4(a[13 + 3 * ch], b4, n2);
-                    n2 = mfma4(a[14 + 3 * ch], b5, n2);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        tot[b][ch] = fmaf(fmaxf(fmaf(n1[r], inv[r], n2[r] * i2[r]), 0.f), K[r], tot[b][ch]);
-                }
-                // one block's products at a time: the blocks' results are not
-                // held together
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        c = prev;
-    }
-    // pixel 16 b + col's sums are spread over lanes col, col + 16, col + 32,
-    // col + 48; lane l keeps block l / 16, its own pixel
-    float out[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int ch = 0; ch < 3; ++ch) {
-            float v = tot[b][ch];
-            v += __shfl_xor(v, 16);
-            v += __shfl_xor(v, 32);
-            if (kr == b) out[ch] = v;
-        }
-    if (live) {
-        float4 o = out_rad[q];
-        o.x += out[0] * P.br;
-        o.y += out[1] * P.bg;
-        o.z += out[2] * P.bb;
-        out_rad[q] = o;
-    }
-}
-
-// A frame's pool: no chunk taken, no tile's chain, and the descriptor the
-// traversal reads (in device memory, so that it is read only where a chunk
-// is handed over).
-__global__ void k_pool_reset(EstPool p, EstPool* __restrict__ desc, int ntiles) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < ntiles) p.head[i] = -1;
-    if (i == 0) {
-        *p.taken = 0;
-        *desc = p;
-    }
-}
-
-// The launch order of the cut's tiles from their costs in the last frame,
-// heaviest first (longest-processing-time order): the tiles' costs spread
-// over two orders of magnitude, and a heavy tile started last runs alone at
-// the end of the launch.  A bucket sort on eight buckets per octave of cost,
-// in one workgroup; the order within a bucket is that of the LDS atomics.
-// A tile's result does not depend on the order.
-constexpr int kOrderBins = 256;
-constexpr int kOrderThreads = 1024;
-
-__device__ inline int order_bin(float c) {
-    const int b = (int)(__log2f(fmaxf(c, 1.f)) * 8.f);
-    return kOrderBins - 1 - min(max(b, 0), kOrderBins - 1);
-}
-
-__global__ __launch_bounds__(kOrderThreads) void k_tile_order(const float* __restrict__ cost, int n,
-                                                              int* __restrict__ order) {
-    __shared__ int hist[kOrderBins];
-    __shared__ int off[kOrderBins];
-    for (int i = threadIdx.x; i < kOrderBins; i += kOrderThreads) hist[i] = 0;
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += kOrderThreads) atomicAdd(&hist[order_bin(cost[i])], 1);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int s = 0;
-        for (int b = 0; b < kOrderBins; ++b) {
-            off[b] = s;
-            s += hist[b];
-        }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += kOrderThreads) order[atomicAdd(&off[order_bin(cost[i])], 1)] = i;
+// A frame's pool: no chunk taken, no tile handed back.
+__global__ void k_pool_reset(CutPool p) {
+    *p.taken = 0;
+    *p.nserial = 0;
+    *p.next = 0;
 }
 
 }  // namespace
@@ -1102,6 +1477,7 @@ int cut_moments_build(arc_gather* g, arc_bvh* b) {
     if (!b->has_cut_records || !g->crec.p) return fail(ctx, ARC_E_STATE, "moment records need the cut tree");
     const int nblocks = (n + kScanBlock - 1) / kScanBlock;
     ARC_TRY(ensure(ctx, g->mom, sizeof(float4) * kMom * (size_t)(n - 1)));
+    ARC_TRY(ensure(ctx, g->mom_trav, sizeof(float4) * kTrav * (size_t)(n - 1)));
     ARC_TRY(ensure(ctx, g->mom_pre, sizeof(double) * kMomTerms * (size_t)n));
     ARC_TRY(ensure(ctx, g->mom_tot, sizeof(double) * kMomTerms * (size_t)nblocks));
     hipLaunchKernelGGL(k_mom_scan, dim3(nblocks, kGroups), dim3(kScanBlock), 0, ctx->stream, g->crec.as<float4>(),
@@ -1111,12 +1487,95 @@ int cut_moments_build(arc_gather* g, arc_bvh* b) {
                        nblocks);
     hipLaunchKernelGGL(k_mom_nodes, dim3((n - 1 + kScanBlock - 1) / kScanBlock), dim3(kScanBlock), 0, ctx->stream,
                        b->ranges.as<int>(), b->nodes.as<arc_bvh_node>(), n, g->mom_pre.as<double>(),
-                       g->mom_tot.as<double>(), g->mom.as<float4>());
+                       g->mom_tot.as<double>(), g->mom.as<float4>(), g->mom_trav.as<float4>());
     ARC_LAUNCHED(ctx);
     ARC_TRY(ensure(ctx, g->mom_nbox, sizeof(float4) * 2 * (size_t)(n - 1)));
     ARC_TRY(node_normal_boxes(b, g->crec.as<float4>(), g->mom_nbox.as<float4>()));
     g->mom_ready = true;
     return ARC_OK;
+}
+
+namespace {
+
+// The chunks a tile can need: most frames use about 25 per tile (a million
+// AVPLs at a bound of 0.01) or 50 where larger nodes are summed exactly, a
+// small tree fewer than its leaves fill.
+int default_chunks(int n, int exact_count) { return std::min(exact_count > 16 ? 96 : 48, 8 + n / 64); }
+
+constexpr int kMinChunks = 16384;  // 21 MB
+
+// Readies `mem` for nitems tiles: the chunks of `per_tile` per tile, or as
+// many as the last frame asked for when that was more (read from pinned
+// memory that k_cut_combine writes: a frame still running counts at the next
+// one).  Nothing grows while the stream is captured.
+int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, long long want, bool grow, CutPool& p) {
+    if (!mem.seen) {
+        ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&mem.seen), sizeof(int), hipHostMallocDefault));
+        *mem.seen = 0;
+    }
+    if (grow) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
+        const int seen = *static_cast<volatile int*>(mem.seen);
+        want = std::max(want, (long long)mem.cap);
+        if (capture == hipStreamCaptureStatusNone && seen > want) want = (long long)seen + seen / 4;
+    }
+    // a small image's tiles can hold 512 chunks each (a budget of 65536): no small pools
+    want = std::max(want, std::min((long long)kMinChunks, 512LL * nitems));
+    if (want > INT_MAX / kKeep) want = INT_MAX / kKeep;
+    ARC_TRY(ensure(ctx, mem.entries, sizeof(uint32_t) * kKeep * (size_t)want));
+    ARC_TRY(ensure(ctx, mem.meta, sizeof(int4) * (size_t)want));
+    ARC_TRY(ensure(ctx, mem.part, sizeof(float) * 192 * (size_t)want));
+    ARC_TRY(ensure(ctx, mem.tiles, sizeof(int) * ((size_t)11 * nitems + 4)));
+    mem.cap = (int)want;
+    float* tbox = mem.tiles.as<float>();
+    int* head = reinterpret_cast<int*>(tbox + 8 * (size_t)nitems);
+    p = CutPool{mem.entries.as<uint32_t>(), mem.meta.as<int4>(), mem.part.as<float>(), tbox, head, head + nitems,
+                head + 2 * (size_t)nitems, head + 3 * (size_t)nitems, head + 3 * (size_t)nitems + 1,
+                head + 3 * (size_t)nitems + 2, mem.seen, (int)want, nitems < 4096 ? 4 : 8};
+    return ARC_OK;
+}
+
+// Resident waves of k_cut_eval: eight per SIMD.
+constexpr int kEvalBlocks = 2048;
+
+// Below this budget the serial cut takes every tile: most would reach their
+// budget, and entering subtrees that are then taken back costs more than it
+// saves (1283x719 pixels, 250001 AVPLs: 2.9 ms against 4.0 at a budget of 4096,
+// 7.6 against 7.7 at 15000; 200x120 pixels, 20000 AVPLs: 1.0 against 1.2 and
+// 2.0 against 0.7).
+constexpr int kSerialBudget = 8192;
+
+template <bool kMany>
+void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool expansion, bool serial, const CutPool& p) {
+    const int blocks = (nitems + 3) / 4;
+    if (serial) {
+        hipLaunchKernelGGL(k_cut_serial<kMany>, dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, 1, p);
+        return;
+    }
+    hipLaunchKernelGGL(k_pool_reset, dim3(1), dim3(1), 0, stream, p);
+    if (expansion)
+        hipLaunchKernelGGL((k_cut_decide<kMany, true>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
+    else
+        hipLaunchKernelGGL((k_cut_decide<kMany, false>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
+    hipLaunchKernelGGL(k_cut_eval<kMany>, dim3(std::min(8 * blocks, kEvalBlocks)), dim3(kCutThreads), 0, stream, views, p);
+    hipLaunchKernelGGL(k_cut_serial<kMany>, dim3(std::min(blocks, 256)), dim3(kCutThreads), 0, stream, views, nitems, 0, p);
+    hipLaunchKernelGGL(k_cut_combine<kMany>, dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
+}
+
+}  // namespace
+
+void release_pool(CutPoolMem& mem) {
+    release(mem.entries);
+    release(mem.meta);
+    release(mem.part);
+    release(mem.tiles);
+    if (mem.seen) (void)hipHostFree(mem.seen);
+    mem = CutPoolMem{};
+}
+
+bool cut_pool_short(arc_gather* g) {
+    return g->est_chunks == 0 && g->pool.seen && *static_cast<volatile int*>(g->pool.seen) > g->pool.cap;
 }
 
 int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, unsigned long long* counters,
@@ -1128,82 +1587,42 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
     CutEB t{};
     Threshold th{};
     ARC_TRY(prepare_cut(g, b, cp, t, th));
-    const CutMom tm{b->nodes.as<arc_bvh_node>(), g->crec.as<float4>(), g->mom.as<float4>(), n};
-    const int blocks = ((g->width + 15) / 16) * ((g->height + 15) / 16);
-    const int ntiles = 4 * blocks;
+    const int nitems = 4 * ((g->width + 15) / 16) * ((g->height + 15) / 16);
+    const CutView v{g->crec.as<float4>(), g->mom.as<float4>(), g->mom_trav.as<float4>(), g->mom_nbox.as<float4>(),
+                    g->gpos, g->gnrm, g->galb, g->mats.as<arc_material>(), th.est, th.sum, th.eps, th.floor_frac,
+                    th.inv_npix, g->width, g->height, cp.delta, cp.budget, cp.criterion, cp.opening * cp.opening,
+                    cp.exact_count, rad, counters, 0, nitems, n};
     if (defer) {
-        *defer = CutView{tm.nodes, tm.crec, tm.mom, g->mom_nbox.as<float4>(), g->gpos, g->gnrm, g->galb,
-                         g->mats.as<arc_material>(),
-                         th.est, th.sum, th.eps, th.floor_frac, th.inv_npix, g->width, g->height, cp.delta,
-                         cp.budget, cp.criterion, cp.opening * cp.opening, cp.exact_count, nullptr, rad, counters,
-                         0, ntiles};
+        *defer = v;
         return ARC_OK;
     }
-    if (g->tile_cost_n != ntiles || g->tile_cost.bytes < sizeof(float) * (size_t)ntiles) g->tile_cost_n = 0;
-    ARC_TRY(ensure(ctx, g->tile_cost, sizeof(float) * (size_t)ntiles));
-    ARC_TRY(ensure(ctx, g->tile_order, sizeof(int) * (size_t)ntiles));
-    // the last frame's tile costs, if they describe this image, order the launch
-    const int* order = nullptr;
-    if (g->tile_cost_n == ntiles) {
-        hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderThreads), 0, ctx->stream, g->tile_cost.as<float>(), ntiles,
-                           g->tile_order.as<int>());
-        order = g->tile_order.as<int>();
-    }
-    // the kept nodes' pool for the matrix-core pass
-    const size_t cap = (size_t)ntiles * (size_t)std::max(g->est_chunks, 0);
-    EstPool pool{};
-    EstPool* desc = nullptr;
-    if (cap > 0) {
-        if (cap > (size_t)INT_MAX) return fail(ctx, ARC_E_INVALID, "estimate pool too large");
-        ARC_TRY(ensure(ctx, g->est_entries, sizeof(uint32_t) * kKeep * cap));
-        // + the chunk counter and the descriptor
-        ARC_TRY(ensure(ctx, g->est_meta, sizeof(int2) * (cap + 2) + sizeof(EstPool)));
-        ARC_TRY(ensure(ctx, g->est_head, sizeof(int) * (size_t)ntiles));
-        ARC_TRY(ensure(ctx, g->est_queued, sizeof(float) * (size_t)ntiles));
-        ARC_TRY(ensure(ctx, g->est_order, sizeof(int) * (size_t)ntiles));
-        int2* meta = g->est_meta.as<int2>();
-        pool = EstPool{g->est_entries.as<uint32_t>(), meta, reinterpret_cast<int*>(meta + cap), (int)cap,
-                       g->est_head.as<int>(), g->est_queued.as<float>()};
-        desc = reinterpret_cast<EstPool*>(meta + cap + 2);
-        hipLaunchKernelGGL(k_pool_reset, dim3((ntiles + 255) / 256), dim3(256), 0, ctx->stream, pool, desc, ntiles);
+    const bool serial = cp.budget < kSerialBudget;
+    CutPool pool{};
+    if (!serial) {
+        const long long per_tile = g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);
+        ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, pool));
     }
     if (mark) ARC_HIP(ctx, hipEventRecord(mark, ctx->stream));
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kCutThreads), 0, ctx->stream, tm.nodes, tm.crec, tm.mom,
-                           g->mom_nbox.as<float4>(), g->gpos,
-                           g->gnrm, g->galb, g->mats.as<arc_material>(), g->width, g->height, th, cp.delta, cp.budget,
-                           cp.criterion, cp.opening * cp.opening, cp.exact_count, order, g->tile_cost.as<float>(), rad,
-                           counters, desc);
-    };
-    // the traversal's stack depth (its deepest cut): a launch-shape setting
-    switch ((cap > 0 ? 1000 : 0) + g->cut_stack) {
-        case 64: launch(k_cut_mom_tile<false, 64>); break;
-        case 128: launch(k_cut_mom_tile<false, 128>); break;
-        case 1064: launch(k_cut_mom_tile<true, 64>); break;
-        case 1096: launch(k_cut_mom_tile<true, 96>); break;
-        case 1128: launch(k_cut_mom_tile<true, 128>); break;
-        default: launch(k_cut_mom_tile<false, 96>); break;
-    }
+    launch_cut<false>(ctx->stream, Views<false>{v}, nitems, cp.criterion == ARC_CRITERION_EXPANSION, serial, pool);
     ARC_LAUNCHED(ctx);
-    g->tile_cost_n = ntiles;
-    if (cap > 0) {
-        // this frame's pooled counts order the estimate pass, heaviest tile first
-        hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderThreads), 0, ctx->stream, pool.queued, ntiles,
-                           g->est_order.as<int>());
-        hipLaunchKernelGGL(k_mom_est, dim3(blocks), dim3(kCutThreads), 0, ctx->stream, tm.mom, pool.entries, pool.meta,
-                           pool.head, g->gpos, g->gnrm, g->galb, g->mats.as<arc_material>(), g->width, g->height,
-                           g->est_order.as<int>(), rad);
-        ARC_LAUNCHED(ctx);
-    }
     return ARC_OK;
 }
 
-int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* views, int nviews, int nitems,
-                      float* costs, int* order, bool ordered) {
-    if (nviews < 1 || nitems < 1) return ARC_OK;
-    if (ordered) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderThreads), 0, stream, costs, nitems, order);
-    hipLaunchKernelGGL(k_cut_mom_views, dim3((nitems + 3) / 4), dim3(kCutThreads), 0, stream, views, nviews,
-                       ordered ? order : nullptr, nitems);
+int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_views, const CutView* views, int nviews,
+                      CutPoolMem& mem) {
+    if (nviews < 1) return ARC_OK;
+    int nitems = 0;
+    long long want = 0;
+    bool serial = false, expansion = false;
+    for (int i = 0; i < nviews; ++i) {
+        nitems += host_views[i].ntiles;
+        want += (long long)host_views[i].ntiles * default_chunks(host_views[i].n, host_views[i].exact_count);
+        serial = serial || host_views[i].budget < kSerialBudget;
+        expansion = expansion || host_views[i].criterion == ARC_CRITERION_EXPANSION;
+    }
+    CutPool pool{};
+    ARC_TRY(ready_pool(ctx, stream, mem, nitems, want, true, pool));
+    launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, serial, pool);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }

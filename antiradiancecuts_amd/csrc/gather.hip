@@ -546,13 +546,8 @@ void arc_gather_destroy(arc_gather* g) {
     arc::release(g->mom_pre);
     arc::release(g->mom_tot);
     arc::release(g->mom_nbox);
-    arc::release(g->tile_cost);
-    arc::release(g->tile_order);
-    arc::release(g->est_entries);
-    arc::release(g->est_meta);
-    arc::release(g->est_head);
-    arc::release(g->est_queued);
-    arc::release(g->est_order);
+    arc::release(g->mom_trav);
+    arc::release_pool(g->pool);
     arc::release(g->cest);
     arc_bvh_destroy(g->bvh);
     delete g;
@@ -893,7 +888,6 @@ int arc_gather_set_launch_shape(arc_gather* g, int cut_stack, int anti_chunk) {
         return arc::fail(g->ctx, ARC_E_INVALID, "launch shape: cut_stack is 64, 96 or 128");
     if (anti_chunk != 768 && anti_chunk != 1536 && anti_chunk != 3072)
         return arc::fail(g->ctx, ARC_E_INVALID, "launch shape: anti_chunk is 768, 1536 or 3072");
-    g->cut_stack = cut_stack;
     g->anti_chunk = anti_chunk;
     return ARC_OK;
 }

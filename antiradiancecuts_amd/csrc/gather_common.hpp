@@ -11,14 +11,15 @@
 #include "gather_math.hpp"
 
 namespace arc {
-// One view's moment cut, as a launch over many views reads it: the tree's
-// arrays, the G-buffer, the pixel thresholds (estimate, image sum and the
-// factors of Threshold), the cut's parameters, the outputs, and where the
-// view's tiles start in the launch's list of tiles (and their cost slots).
+// One view's moment cut, as its kernels read it (by value, or from an array
+// for a launch over many views): the tree's records, the G-buffer, the pixel
+// thresholds (estimate, image sum and the factors of Threshold), the cut's
+// parameters, the outputs, and where the view's tiles start in the launch's
+// list of tiles.
 struct CutView {
-    const arc_bvh_node* nodes;
-    const float4* crec;
-    const float4* mom;
+    const float4* crec;  // leaf records, slots [0, n) in sorted order
+    const float4* mom;   // moment record per internal node
+    const float4* trav;  // traversal record per internal node
     const float4* nbox;  // per internal node: the box of its AVPLs' unit normals (lo, hi)
     const float4* gpos;
     const float4* gnrm;
@@ -32,11 +33,40 @@ struct CutView {
     int budget, criterion;
     float open2;
     int exact_count;
-    float* tile_cost;
     float4* out_rad;
     unsigned long long* counters;
     int tile_base, ntiles;
+    int n;  // leaves
 };
+
+// The chunks of a moment cut's launch: kept nodes and exact ranges found by
+// the decision kernel, summed by the evaluation kernel (cut_moments.hip).
+struct CutPool {
+    uint32_t* entries;  // cap chunks of 128 entries
+    int4* meta;         // per chunk: (tile, kind | entries << 8, the tile's next chunk or -1, 16 x the chunk that
+                        // holds its entries + which part of them)
+    float* part;        // per chunk: 3 x 64 partial sums
+    float* tbox;        // per tile: its box, centre and half extent (8 floats)
+    int* head;          // per tile: its first chunk or -1
+    int* evaluated;     // per tile: nodes and leaves its cut sums, -1 when it is cut serially
+    int* serial;        // the tiles to cut serially
+    int* taken;         // chunks asked for (may pass cap)
+    int* nserial;
+    int* next;          // the evaluation's next chunk
+    int* seen;          // pinned host memory: chunks the frame asked for
+    int cap;
+    int grab;           // chunks a tile takes with its first atomic, twice as many with each later one: the
+                        // counter serves about 100 atomics per microsecond, and a tile's last grab leaves
+                        // some unused, which the evaluation has to pass over
+};
+
+// The pool's memory, kept between launches.
+struct CutPoolMem {
+    DevBuf entries, meta, part, tiles;
+    int* seen = nullptr;
+    int cap = 0;
+};
+void release_pool(CutPoolMem& mem);
 }  // namespace arc
 
 struct arc_gather {
@@ -64,21 +94,14 @@ struct arc_gather {
     arc::DevBuf mom, mom_pre, mom_tot;
     arc::DevBuf mom_nbox;  // per internal node: the box of its AVPLs' unit normals
     bool mom_ready = false;  // mom holds the records of the current cut tree
-    // moment cut: each 8x8 tile's cost in the last frame (VALU instructions,
-    // estimated from its counts) and the launch order made from it, heaviest
-    // tile first; tile_cost_n is the tile count the costs describe (0: none)
-    arc::DevBuf tile_cost, tile_order;
-    int tile_cost_n = 0;
-    // moment cut: the kept nodes handed from the traversal to the
-    // matrix-core pass, est_chunks chunks of 128 per tile (0, the default:
-    // estimated in the traversal, measured faster), each tile's chain, its
-    // queued count and the pass's order
+    arc::DevBuf mom_trav;  // per internal node: the traversal's record
+    // moment cut: the pool its tiles' cuts are written to; est_chunks > 0
+    // sets its chunks per tile, 0 sizes it from the tree and the last frame
     int est_chunks = 0;
-    // launch shapes the results do not depend on: the moment cut's traversal
-    // stack (64, 96 or 128 nodes) and the clustered antiradiance's list
-    // entries filed per pass (768, 1536 or 3072)
-    int cut_stack = 96, anti_chunk = 1536;
-    arc::DevBuf est_entries, est_meta, est_head, est_queued, est_order;
+    arc::CutPoolMem pool;
+    // a launch shape the results do not depend on: the clustered
+    // antiradiance's list entries filed per pass (768, 1536 or 3072)
+    int anti_chunk = 1536;
     arc_cutnet* net = nullptr;  // learned cut: the predictor (borrowed)
     arc_bvh* bvh = nullptr;
     // per-frame phase events: frame slot, then 9 marks (start, upload done,
@@ -306,11 +329,14 @@ int cut_moments_build(arc_gather* g, arc_bvh* b);
 // written there instead of launching it (cut_moments_views launches it).
 int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, unsigned long long* counters,
                 hipEvent_t mark, CutView* defer = nullptr);
-// One launch of the moment cut over the tiles of many views (device array
-// `views`, nitems tiles in all), heaviest tile first by the costs of the
-// last launch when `ordered`; costs and order hold nitems each.
-int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* views, int nviews, int nitems,
-                      float* costs, int* order, bool ordered);
+// The moment cuts of many views in one set of launches (host_views and its
+// device copy `views`).
+int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_views, const CutView* views, int nviews,
+                      CutPoolMem& mem);
+// Whether the last frame asked for more chunks than the gather's pool holds
+// (its remaining tiles were cut serially; the next eager frame grows it).
+// The frame must have ended.
+bool cut_pool_short(arc_gather* g);
 // The combine of a frame run with defer_cut, once its cut has run.
 int gather_finish(arc_gather* g);
 // The learned cut: per tile, refine / keep from g->net, the error-bound

@@ -372,25 +372,22 @@ int arc_cutnet_train(arc_cutnet* net, const float* X, const float* y, const floa
 /* The network the gather's ARC_CUT_LEARNED frames use (borrowed; NULL detaches). */
 int arc_gather_set_cutnet(arc_gather* g, arc_cutnet* net);
 /* No counterpart in the reference (a schedule setting of this library's
- * moment cut).  With chunks_per_tile > 0 the moment cut's traversal hands its
- * kept nodes to a second pass that estimates them on the matrix cores,
- * through a pool of chunks_per_tile chunks of 128 nodes per 8x8 tile (device
- * memory 512 bytes per chunk).  A tile that finds the pool full estimates its
- * nodes in the traversal, so the setting changes the speed and the memory,
- * and the image only by rounding.  0 (the default) estimates every kept node
- * in the traversal, where the estimates fill the issue slots that the
- * traversal's dependent loads leave idle.  Read by the next frame.
- * ARC_E_INVALID for a negative count or more than 256 (4.2 GB at 1080p). */
+ * moment cut).  The cut's kept nodes and exact ranges are found by one kernel
+ * and summed by another, through a pool of chunks (128 entries and 64 x 3
+ * partial sums, 1.3 KB each, at least 16384 of them).  chunks_per_tile > 0
+ * sets the pool's chunks per 8x8 tile; 0 (the default) sizes it from the tree
+ * and grows it to what the last frame asked for.  A tile that finds the pool
+ * full is cut and summed node by node, so the setting changes the speed and
+ * the memory, and the image only by rounding.  Read by the next frame.
+ * ARC_E_INVALID for a negative count or more than 256. */
 int arc_gather_set_estimate_pool(arc_gather* g, int chunks_per_tile);
 /* No counterpart in the reference (launch shapes of this library's kernels,
- * searched by its autotuner).  cut_stack: the moment cut's traversal stack,
- * in nodes, per 8x8 tile (64, 96 or 128; default 96): the deepest cut a tile
- * can refine to; a tile that needs more keeps the node it cannot refine and
- * is counted in errorPixels.  anti_chunk: the clustered antiradiance's list
- * entries filed into the tiles' LDS sub-lists per pass (768, 1536 or 3072;
- * default 1536): more per pass is fewer passes and more LDS per workgroup.
- * Neither changes the image beyond rounding while errorPixels stays 0.  Read
- * by the next frame.  ARC_E_INVALID for other values. */
+ * searched by its autotuner).  cut_stack: 64, 96 or 128 (accepted; the moment
+ * cut's traversal needs no depth setting any more).  anti_chunk: the clustered
+ * antiradiance's list entries filed into the tiles' LDS sub-lists per pass
+ * (768, 1536 or 3072; default 1536): more per pass is fewer passes and more
+ * LDS per workgroup.  Neither changes the image beyond rounding.  Read by the
+ * next frame.  ARC_E_INVALID for other values. */
 int arc_gather_set_launch_shape(arc_gather* g, int cut_stack, int anti_chunk);
 /* Training rows of one frame: builds the frame's AvplBvh and thresholds as
  * arc_gather_run does with params (cutMode is ignored), then walks each tile's
