@@ -13,8 +13,9 @@
 //              64-byte record per triangle in input order; the leaves are
 //              triangle pieces (large triangles split into slabs along their
 //              longest axis), and the tree over them is a binned-SAH build
-//              on the host at scene creation (static geometry: built once,
-//              traversed by every path and pixel);
+//              on the host at scene creation, collapsed to eight-wide nodes
+//              (static geometry: built once, traversed by every path and
+//              pixel by eight lanes per ray);
 //   intersect  Triangle::intersect in FRONT_FACE mode (Triangle.h): Moller-
 //              Trumbore on unnormalised barycentrics with the reference's
 //              |det| < EPS = 1e-4 rejection; the closest hit with t > 0
@@ -35,7 +36,9 @@
 //              front-facing triangle, position (x, y, z, 1) and normal
 //              (n, material) in the G-buffer layout the gather reads.
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "arc_internal.hpp"
@@ -47,19 +50,13 @@ struct arc_trace_scene {
     int ntri = 0;
     int nleaf = 0;                    // leaves: triangle pieces (a large triangle is split)
     arc::DevBuf tri;                  // 4 float4 per triangle, input order
-    arc::DevBuf leaf_tri;             // per leaf: its triangle
-    arc::DevBuf leaf_box;             // per leaf: box lo, hi (2 float4)
-    arc::DevBuf nodes;                // the tree's internal nodes (BvhNode layout, boxes of the pieces)
+    arc::DevBuf nodes;                // the tree's eight-wide nodes, 16 float4 each (wide_nodes)
+    int stack = 1;                    // most nodes a traversal keeps pending
     arc::DevBuf mats;                 // material table, 256 entries
     arc::DevBuf emissive;             // per material: emissive != 0
-    int max_depth = 0;                // deepest internal node (root = 1)
+    int max_depth = 0;                // deepest internal node of the binary tree (root = 1)
     // shooter output
-    arc::DevBuf state, active, stage, path_offset, scan_blocks, out;
-    struct {
-        f3 *pos, *nrm, *rad, *in_dir, *dir;
-        float* pdf;
-        int *bounce, *mat, *draws, *count;
-    } ps{};
+    arc::DevBuf count, stage, path_offset, scan_blocks, out;
 };
 
 namespace {
@@ -71,7 +68,7 @@ constexpr float kOneOverTwoPi = 0.15915494309f;   // ONE_OVER_TWO_PI (Defines.h:
 constexpr float kOneOverPi = 0.318309886f;
 constexpr int kThreads = 256;
 constexpr int kMaxPieces = 8;         // most leaves one triangle is split into
-constexpr int kTraceStack = 48;       // per-lane stack of the closest-hit traversal (LDS)
+constexpr int kTraceStack = 48;       // deepest binary tree taken
 constexpr int kScan = 1024;
 
 struct V {
@@ -101,9 +98,8 @@ struct Tri {  // 4 float4 per triangle
 
 struct SceneDev {
     const float4* tri;               // triangles in input order, 4 float4 each
-    const arc_bvh_node* nodes;       // n - 1 internal nodes
-    const int* leaf_tri;             // leaf -> triangle
-    int n;                           // leaves
+    const float4* nodes;             // eight-wide nodes, 16 float4 each
+    int stack;                       // pending nodes of a traversal, per ray
     const arc_material* mats;        // 256 entries
     const int* emissive;             // 256 entries
 };
@@ -129,98 +125,212 @@ __device__ inline Tri load_tri(const float4* tri, int s) {
     return Tri{r[0], r[1], r[2], r[3]};
 }
 
-// Slab test; returns the entry distance or INFINITY when the box is missed
-// or lies beyond t_max.
-__device__ inline float box_enter(const arc_bvh_node& b, V o, V inv, float t_max) {
-    const float tx0 = (b.bbMin.x - o.x) * inv.x, tx1 = (b.bbMax.x - o.x) * inv.x;
-    const float ty0 = (b.bbMin.y - o.y) * inv.y, ty1 = (b.bbMax.y - o.y) * inv.y;
-    const float tz0 = (b.bbMin.z - o.z) * inv.z, tz1 = (b.bbMax.z - o.z) * inv.z;
-    const float t0 = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.f));
-    const float t1 = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), t_max));
-    return t0 <= t1 ? t0 : INFINITY;
-}
-
 __device__ inline float safe_inv(float w) {
     const float m = fmaxf(fabsf(w), 1e-30f);
     return 1.0f / copysignf(m, w);
 }
 
-// Closest front-facing hit with t > 0 (ties: the lower triangle index, as a
-// loop over the triangles in order finds it).  stk: this lane's LDS stack,
-// entry j at stk[j * kThreads].  Returns the triangle index or -1.  A
-// triangle split into several leaves is tested once per leaf its ray
-// reaches, with the same result each time.
-__device__ int closest_hit(const SceneDev& S, V o, V dir, float det_eps, float& t_best, int* stk) {
-    t_best = INFINITY;
-    int best = -1;
-    if (S.n == 1) {
-        float t;
-        const int ti = S.leaf_tri[0];
-        if (tri_hit(load_tri(S.tri, ti), o, dir, det_eps, t) && t > 0.f) {
-            t_best = t;
-            best = ti;
-        }
-        return best;
+// Closest front-facing hits with t > 0 (ties: the lower triangle index, as a
+// loop over the triangles in order finds it), eight lanes per ray.
+//
+// A step takes one node of the eight-wide tree: each lane of the ray's group
+// tests one child, a triangle piece's triangle at once, and the inner children
+// that the ray enters before its closest hit go to the group's stack in LDS,
+// nearest on top.  The scenes' triangles overlap densely (a ray leaving a
+// surface starts inside hundreds of boxes), so a ray is a long chain of
+// dependent node reads, and for the few rays of a late bounce the chain is all
+// the time: 0.7 ms a ray where one lane walks a two-wide tree.  An eight-wide
+// step replaces about three dependent reads by one of 256 consecutive bytes
+// and tests up to eight triangles together.  Where the chip is full (a
+// G-buffer) the step's vector instructions bound it, about 110, a third of
+// them the triangle test: 1280 x 720 pixels over 100K triangles take 1.40 ms,
+// 2.26 with a lane per ray.  The order of the children comes from whole-number
+// keys compared across DPP: with ds_bpermute and float compares it was half of
+// a step (2.01 ms).
+//
+// The box tests are conservative in FP32: the exit distance carries a factor
+// above the slabs' rounding and the keys', so a box that holds the closest hit
+// is never passed over.
+constexpr int kGroup = 8;                        // lanes per ray
+constexpr int kWave = 64;                        // threads of a block that traces: no wave waits on another
+constexpr int kGroups = kWave / kGroup;          // its rays
+constexpr int kNoChild = 0x7fffffff;
+constexpr float kBoxSlack = 1.000002f;
+
+struct Ray {
+    V o, d, inv;
+    float det_eps;
+    float t;       // closest hit so far, INFINITY for none
+    int tri;       // its triangle, -1 for none
+    int node, sp;  // the node to take next; pending nodes
+    bool on;       // still in the tree
+};
+
+__device__ inline void ray_start(Ray& r, V o, V d, float det_eps) {
+    r.o = o;
+    r.d = d;
+    r.inv = mk(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
+    r.det_eps = det_eps;
+    r.t = INFINITY;
+    r.tri = -1;
+    r.node = 0;
+    r.sp = 0;
+    r.on = true;
+}
+
+// v of lane ^ X, X < 8
+template <int X>
+__device__ inline int lane_xor(int v) {
+    constexpr int kQuad[4] = {0xE4, 0xB1, 0x4E, 0x1B};
+    if (X >= 4) v = __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false);  // lane ^ 7
+    constexpr int q = X >= 4 ? X ^ 7 : X;
+    return q == 0 ? v : __builtin_amdgcn_update_dpp(v, v, kQuad[q], 0xf, 0xf, false);
+}
+
+template <int X>
+__device__ inline void closer_of(float& t, int& ti) {  // the closer of this lane's hit and lane ^ X's
+    const float ot = __int_as_float(lane_xor<X>(__float_as_int(t)));
+    const int oi = lane_xor<X>(ti);
+    if (oi >= 0 && (ot < t || (ot == t && oi < ti))) {
+        t = ot;
+        ti = oi;
     }
-    const V inv = mk(safe_inv(dir.x), safe_inv(dir.y), safe_inv(dir.z));
-    int sp = 0;
-    int node = 0;  // internal node index
-    for (;;) {
-        const arc_bvh_node& b = S.nodes[node];
-        int next[2];
-        float tn[2];
-        const int ch[2] = {b.left, b.right};
-        int cnt = 0;
-        for (int k = 0; k < 2; ++k) {
-            const int c = ch[k];
-            if (c >= 0) {  // leaf: test its triangle at once
-                float t;
-                const int ti = S.leaf_tri[c];
-                if (tri_hit(load_tri(S.tri, ti), o, dir, det_eps, t) && t > 0.f &&
-                    (t < t_best || (t == t_best && ti < best))) {
-                    t_best = t;
-                    best = ti;
-                }
-            } else {
-                const float te = box_enter(S.nodes[-(c + 1)], o, inv, t_best);
-                if (te < INFINITY) {
-                    next[cnt] = -(c + 1);
-                    tn[cnt] = te;
-                    ++cnt;
-                }
-            }
+}
+
+// One child: a hit of its triangle (t, ti) or the entry of its box as a key:
+// the distance's bits, the last three replaced by the lane, so that no two of a
+// group are equal; -1 for none.
+__device__ inline int child_test(const SceneDev& S, const Ray& r, int node, int lane, float& t, int& ti, int& child) {
+    const float4* c = S.nodes + 16 * (size_t)node + 2 * lane;
+    const float4 lo = c[0], hi = c[1];
+    child = __float_as_int(lo.w);
+    const float tx0 = (lo.x - r.o.x) * r.inv.x, tx1 = (hi.x - r.o.x) * r.inv.x;
+    const float ty0 = (lo.y - r.o.y) * r.inv.y, ty1 = (hi.y - r.o.y) * r.inv.y;
+    const float tz0 = (lo.z - r.o.z) * r.inv.z, tz1 = (hi.z - r.o.z) * r.inv.z;
+    const float t0 = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.f));
+    const float t1 = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), r.t));
+    if (child == kNoChild || !(t0 <= t1 * kBoxSlack) || t0 == INFINITY) return -1;
+    if (child < 0) return (__float_as_int(t0) & 0x7ffffff8) | lane;
+    float d;
+    if (tri_hit(load_tri(S.tri, child), r.o, r.d, r.det_eps, d) && d > 0.f) {
+        t = d;
+        ti = child;
+    }
+    return -1;
+}
+
+// Of a group's keys, how many are larger than this lane's.
+__device__ inline int keys_after(int key) {
+    return (lane_xor<1>(key) > key) + (lane_xor<2>(key) > key) + (lane_xor<3>(key) > key) +
+           (lane_xor<4>(key) > key) + (lane_xor<5>(key) > key) + (lane_xor<6>(key) > key) +
+           (lane_xor<7>(key) > key);
+}
+
+// One node of each ray that is on.  stk: the group's stack of (node, entry
+// distance).  All lanes of the wave take part.
+__device__ inline void ray_step(const SceneDev& S, Ray& r, int2* stk) {
+    const int lane = threadIdx.x & (kGroup - 1);
+    float t = INFINITY;
+    int child = 0, ti = -1, key = -1;
+    if (r.on) key = child_test(S, r, r.node, lane, t, ti, child);
+    if (__ballot(ti >= 0)) {  // the group's closest, ties to the lower index
+        closer_of<1>(t, ti);
+        closer_of<2>(t, ti);
+        closer_of<4>(t, ti);
+        if (ti >= 0 && (t < r.t || (t == r.t && ti < r.tri))) {
+            r.t = t;
+            r.tri = ti;
         }
-        if (cnt == 2) {
-            const int nearer = tn[0] <= tn[1] ? 0 : 1;
-            stk[(sp++) * kThreads] = next[1 - nearer];  // depth is checked at build: sp < kTraceStack
-            node = next[nearer];
-            continue;
-        }
-        if (cnt == 1) {
-            node = next[0];
-            continue;
-        }
-        // pop the next pending subtree that can still hold a closer hit
-        bool found = false;
-        while (sp > 0) {
-            const int m = stk[(--sp) * kThreads];
-            if (box_enter(S.nodes[m], o, inv, t_best) < INFINITY) {
-                node = m;
-                found = true;
+    }
+    if (__int_as_float(key) > r.t * kBoxSlack) key = -1;
+    // the entered children in order of distance, the nearest last
+    const int after = keys_after(key);
+    if (key >= 0) stk[r.sp + after] = make_int2(-(child + 1), key);
+    const uint64_t in = __ballot(key >= 0);
+    const unsigned half = threadIdx.x & 32 ? (unsigned)(in >> 32) : (unsigned)in;
+    r.sp += __popc(__builtin_amdgcn_ubfe(half, threadIdx.x & 24, 8));
+    __builtin_amdgcn_wave_barrier();  // the group's writes before its lanes read them
+    if (r.on) {
+        r.on = false;
+        while (r.sp > 0) {  // the next pending subtree that can still hold a closer hit
+            const int2 e = stk[--r.sp];
+            if (__int_as_float(e.y) <= r.t * kBoxSlack) {
+                r.node = e.x;
+                r.on = true;
                 break;
             }
         }
-        if (!found) break;
     }
-    return best;
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ inline float wave_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ inline V wave_value(V v, int lane) {
+    return mk(wave_value(v.x, lane), wave_value(v.y, lane), wave_value(v.z, lane));
+}
+
+// The ray of the group that starts at lane `from`, by the whole wave: each
+// group takes another pending node.  For the last rays of a wave, whose other
+// groups have nothing left to do: the chain of dependent reads shortens by as
+// many as the ray has nodes pending.  stk: the wave's stack, the other groups'
+// parts included (no ray of theirs is in the tree).  Eight nodes are taken at
+// once while their 64 children leave one depth-first descent's room.
+__device__ inline void ray_wide(const SceneDev& S, Ray& mine, int from, int2* stk) {
+    Ray r;
+    r.o = wave_value(mine.o, from);
+    r.d = wave_value(mine.d, from);
+    r.inv = wave_value(mine.inv, from);
+    r.det_eps = mine.det_eps;
+    r.t = INFINITY;
+    r.tri = -1;
+    const int lane = threadIdx.x & (kGroup - 1), grp = threadIdx.x / kGroup;
+    const uint64_t higher = ~0ull << (threadIdx.x | (kGroup - 1)) << 1;  // the groups after this one
+    if (threadIdx.x == 0) stk[0] = make_int2(0, 0);
+    __builtin_amdgcn_wave_barrier();
+    int sp = 1;
+    while (sp > 0) {
+        const int take = sp + kWave <= (kGroups - 1) * S.stack ? min(sp, kGroups) : 1;
+        float t = INFINITY;
+        int child = 0, ti = -1, key = -1;
+        if (grp < take) {
+            const int2 e = stk[sp - 1 - grp];
+            if (__int_as_float(e.y) <= r.t * kBoxSlack) key = child_test(S, r, e.x, lane, t, ti, child);
+        }
+        sp -= take;
+        __builtin_amdgcn_wave_barrier();  // read before it is written
+        if (__ballot(ti >= 0)) {
+            closer_of<1>(t, ti);
+            closer_of<2>(t, ti);
+            closer_of<4>(t, ti);
+            for (int g = 0; g < take; ++g) {
+                const float ot = wave_value(t, g * kGroup);
+                const int oi = __builtin_amdgcn_readlane(ti, g * kGroup);
+                if (oi >= 0 && (ot < r.t || (ot == r.t && oi < r.tri))) {
+                    r.t = ot;
+                    r.tri = oi;
+                }
+            }
+        }
+        if (__int_as_float(key) > r.t * kBoxSlack) key = -1;
+        const int after = keys_after(key);
+        const uint64_t in = __ballot(key >= 0);
+        if (key >= 0) stk[sp + after + __popcll(in & higher)] = make_int2(-(child + 1), key);
+        sp += __popcll(in);
+        __builtin_amdgcn_wave_barrier();
+    }
+    if ((int)(threadIdx.x & ~(kGroup - 1)) == from) {
+        mine.t = r.t;
+        mine.tri = r.tri;
+        mine.on = false;
+    }
 }
 
 // Scene::IntersectRayScene: a hit on an emissive triangle is no hit.
-__device__ inline int scene_hit(const SceneDev& S, V o, V dir, float& t, int* stk) {
-    const int s = closest_hit(S, o, dir, kEps, t, stk);
-    if (s < 0) return -1;
-    const int mat = __float_as_int(S.tri[4 * (size_t)s].w);
-    return S.emissive[mat & 255] ? -1 : s;
+__device__ inline int scene_hit(const SceneDev& S, const Ray& r) {
+    if (r.tri < 0) return -1;
+    return S.emissive[__float_as_int(S.tri[4 * (size_t)r.tri].w) & 255] ? -1 : r.tri;
 }
 
 // ------------------------------------------------------------ sampling --
@@ -314,112 +424,155 @@ struct AvplOut {
     int *mat, *bounce;
 };
 
-// Wavefront form of createPath (AvplShooter.h:77-142): the state of every
-// path lives in HBM between launches, one launch per bounce runs the paths
-// still alive (no lane waits on another lane's longer path), and each
-// launch stages the AVPLs it creates; a final scatter puts every path's
-// AVPLs together in path order.  Draw order per path as in createPath:
-// light position (2), first direction (2), then per bounce roulette (1) and
-// the next direction (2).
-struct PathState {
-    f3 *pos, *nrm, *rad, *in_dir, *dir;
-    float* pdf;
-    int *bounce, *mat, *draws, *count;
-};
-
-struct Staged {  // AVPLs of all bounces, in the order the bounces created them
+struct Staged {  // AVPLs in the order they were created; path -1: no AVPL
     AvplOut a;
     int* path;
 };
 
-__global__ __launch_bounds__(kThreads) void k_path_start(Light L, uint64_t seed, int paths, PathState P,
-                                                         int* __restrict__ active) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= paths) return;
-    Rng rng{seed, (uint64_t)i << 24, 0};
-    // AreaLight::samplePos: glm::linearRand over [-1, 1]^2, x then y
-    const float sx = -1.f + 2.f * rng.next();
-    const float sy = -1.f + 2.f * rng.next();
-    const V pos = L.center + (sx * L.half_w) * L.s + (sy * L.half_h) * L.u;
-    const float pdf0 = 1.f / L.area;
-    const V rad = (1.f / pdf0) * L.radiance;  // rad / pdf
-    const float u1 = rng.next(), u2 = rng.next();
-    float pdf;
-    const V dir = sample_cos_cone(L.front, u1, u2, 1.f, pdf);
-    P.pos[i] = f3{pos.x, pos.y, pos.z};
-    P.nrm[i] = f3{L.front.x, L.front.y, L.front.z};
-    P.rad[i] = f3{rad.x, rad.y, rad.z};
-    P.in_dir[i] = f3{0.f, 0.f, 0.f};
-    P.dir[i] = f3{dir.x, dir.y, dir.z};
-    P.pdf[i] = pdf;
-    P.bounce[i] = 0;
-    P.mat[i] = L.mat;
-    P.draws[i] = (int)rng.k;
-    P.count[i] = 0;
-    active[i] = i;
-}
+// createPath (AvplShooter.h:77-142), a path per group of lanes from its first
+// ray to its last: traced, its AVPL staged, continued or replaced by the next
+// path without leaving the kernel.  (With a launch per bounce, the host waits
+// for the count of live paths 47 times per 100K paths, and a bounce of a
+// handful of rays takes as long as its longest ray: 100K paths over 100K
+// triangles took 33 ms, 2.1 here.)  A wave shades when at
+// most half of its rays are still in the tree, so that few lanes wait for the
+// longest one.  What bounds it is the longest path, up to 47 rays one after the
+// other (5.4 ms with eight lanes for each ray to the end); so a wave with no
+// more than four paths left takes their rays one by one with all its lanes
+// (ray_wide).  Draw order per path as in createPath: light position (2),
+// first direction (2), then per bounce roulette (1) and the next direction
+// (2).  Writes each path's AVPL count; a final scatter puts every path's AVPLs
+// together in path order.  AVPLs past `cap` are counted, not staged.
+constexpr int kWideRays = 4;   // most rays of a wave that it takes one by one
+constexpr int kSlotGrab = 64;  // staging slots a wave takes with one atomic
 
-// One bounce of every live path: trace, create the AVPL, roulette, sample
-// the next direction.  Survivors are appended to next_active.
-__global__ __launch_bounds__(kThreads) void k_path_step(SceneDev S, uint64_t seed, int explicit_direct, PathState P,
-                                                        const int* __restrict__ active, int n_active,
-                                                        int* __restrict__ next_active, int* __restrict__ n_next,
-                                                        Staged st, int stage_base) {
-    __shared__ int stk[kTraceStack * kThreads];
-    const int j = blockIdx.x * kThreads + threadIdx.x;
-    if (j >= n_active) return;
-    const int i = active[j];
-    const V nrm = ld(P.nrm[i]), direction = ld(P.dir[i]);
-    const V org = ld(P.pos[i]) + kEps * nrm;
-    float t;
-    const int s = scene_hit(S, org, direction, t, stk + threadIdx.x);
-    // every active path stages one AVPL slot; a miss leaves it unused (bounce 0)
-    const int slot = stage_base + j;
-    if (s < 0) {
-        st.path[slot] = -1;
-        return;
+__global__ __launch_bounds__(kWave) void k_paths(SceneDev S, Light L, uint64_t seed, int paths, int explicit_direct,
+                                                    int* __restrict__ next_path, unsigned* __restrict__ n_staged, int cap,
+                                                    int* __restrict__ count, Staged st) {
+    extern __shared__ int2 stacks[];
+    const int grp = threadIdx.x / kGroup, lane = threadIdx.x & 63;
+    const bool lead = (threadIdx.x & (kGroup - 1)) == 0;
+    int2* stk = stacks + (size_t)grp * S.stack;
+    int slots = 0, nslots = 0;  // the wave's staging slots
+    int path = (int)blockIdx.x * kGroups + grp;
+    bool wide = false;          // so few paths are left that the wave traces each ray as a whole
+    bool fresh = true, done = false;  // the group starts a path; has none left
+    V pos{}, nrm{}, rad0{}, in_dir{}, direction{};
+    float pdf0 = 0.f;
+    int bounce0 = 0, mat0 = 0;
+    Rng rng{seed, 0, 0};
+    Ray r{};
+    for (;;) {
+        const bool shade = !r.on && !done;
+        bool made = false, ended = fresh && shade;
+        V hit_n{}, hit_pos{}, contrib{}, anti{}, rad{}, next{};
+        float pdf = 0.f;
+        int mat = 0;
+        if (shade && !fresh) {
+            const int s = scene_hit(S, r);
+            ended = true;
+            if (s >= 0) {
+                made = true;
+                const float cos_theta = dot(nrm, direction);
+                // getIncidentRadiance() * cos_theta / pdf, per component
+                contrib = mk(rad0.x * cos_theta / pdf0, rad0.y * cos_theta / pdf0, rad0.z * cos_theta / pdf0);
+                if (bounce0 > 0) contrib = contrib * phong_eval(-1.f * in_dir, direction, nrm, S.mats[mat0 & 255]);
+                const float4* T = S.tri + 4 * (size_t)s;
+                hit_n = mk(T[3].x, T[3].y, T[3].z);
+                const V hit = r.o + r.t * direction;  // Intersection::setPosition(origin + dist * dir)
+                hit_pos = hit - kEps * hit_n;
+                mat = __float_as_int(T[0].w);
+                anti = contrib;
+                if (bounce0 == 0 && explicit_direct) anti = mk(0.f, 0.f, 0.f);
+                const bool stop = rng.next() > kRr;  // Russian roulette
+                rad = stop ? mk(0.f, 0.f, 0.f) : (1.f / kRr) * contrib;
+                if (!stop) {
+                    const float s0 = rng.next(), s1 = rng.next();
+                    next = phong_sample(-1.f * direction, hit_n, S.mats[mat & 255], s0, s1, pdf);
+                    ended = length(next) <= 0.f || pdf < 1e-4f;
+                }
+            }
+        }
+        const uint64_t mm = __ballot(made && lead);
+        if (mm) {  // staging slots for the AVPLs just made
+            const int need = __popcll(mm);
+            if (nslots < need) {
+                if (lane < nslots && (unsigned)(slots + lane) < (unsigned)cap) st.path[slots + lane] = -1;  // not used
+                int got = 0;
+                if (lane == 0) got = (int)atomicAdd(n_staged, (unsigned)kSlotGrab);
+                slots = __builtin_amdgcn_readfirstlane(got);
+                nslots = kSlotGrab;
+            }
+            const int slot = slots + __popcll(mm & ((1ull << lane) - 1ull));
+            if (made && lead && (unsigned)slot < (unsigned)cap) {
+                st.a.pos[slot] = f3{hit_pos.x, hit_pos.y, hit_pos.z};
+                st.a.nrm[slot] = f3{hit_n.x, hit_n.y, hit_n.z};
+                st.a.dir[slot] = f3{direction.x, direction.y, direction.z};
+                st.a.rad[slot] = f3{rad.x, rad.y, rad.z};
+                st.a.anti[slot] = f3{anti.x, anti.y, anti.z};
+                st.a.mat[slot] = mat;
+                st.a.bounce[slot] = bounce0 + 1;
+                st.path[slot] = path;
+            }
+            slots += need;
+            nslots -= need;
+        }
+        if (made) {
+            ++bounce0;
+            pos = hit_pos;
+            nrm = hit_n;
+            rad0 = rad;
+            in_dir = direction;
+            direction = next;
+            pdf0 = pdf;
+            mat0 = mat;
+        }
+        if (shade && ended && !fresh && lead) count[path] = bounce0;
+        const uint64_t me = __ballot(shade && ended && !fresh && lead);
+        if (me) {  // the next paths
+            int got = 0;
+            if (lane == 0) got = atomicAdd(next_path, __popcll(me));
+            got = __builtin_amdgcn_readfirstlane(got);
+            // the group's leader's place among the wave's leaders
+            const int mine = got + __popcll(me & ((1ull << (lane & ~(kGroup - 1))) - 1ull));
+            if (shade && ended && !fresh) path = mine;
+        }
+        if (shade && ended) {
+            if (path >= paths) {
+                done = true;
+            } else {  // AreaLight::samplePos: glm::linearRand over [-1, 1]^2, x then y
+                rng = Rng{seed, (uint64_t)path << 24, 0};
+                const float sx = -1.f + 2.f * rng.next();
+                const float sy = -1.f + 2.f * rng.next();
+                pos = L.center + (sx * L.half_w) * L.s + (sy * L.half_h) * L.u;
+                const float area_pdf = 1.f / L.area;
+                rad0 = (1.f / area_pdf) * L.radiance;  // rad / pdf
+                const float u1 = rng.next(), u2 = rng.next();
+                direction = sample_cos_cone(L.front, u1, u2, 1.f, pdf0);
+                nrm = L.front;
+                in_dir = mk(0.f, 0.f, 0.f);
+                bounce0 = 0;
+                mat0 = L.mat;
+            }
+            fresh = false;
+        }
+        if (shade && !done) ray_start(r, pos + kEps * nrm, direction, kEps);
+        const uint64_t live = __ballot(!done);
+        if (live == 0) break;
+        if (wide) {  // every live ray starts here
+            for (uint64_t m = live & 0x0101010101010101ull; m; m &= m - 1) ray_wide(S, r, __builtin_ctzll(m), stacks);
+            continue;
+        }
+        wide = __popcll(live) <= kWideRays * kGroup;
+        // trace until at most half of the live rays are in the tree; to the
+        // end before the wave takes its last rays one by one
+        for (;;) {
+            const uint64_t on = __ballot(r.on);
+            if (on == 0 || (!wide && 2 * __popcll(on) <= __popcll(live & ~on))) break;
+            ray_step(S, r, stk);
+        }
     }
-    const V rad0 = ld(P.rad[i]);
-    const float pdf0 = P.pdf[i];
-    const float cos_theta = dot(nrm, direction);
-    // getIncidentRadiance() * cos_theta / pdf, per component
-    V contrib = mk(rad0.x * cos_theta / pdf0, rad0.y * cos_theta / pdf0, rad0.z * cos_theta / pdf0);
-    const int bounce0 = P.bounce[i];
-    if (bounce0 > 0) contrib = contrib * phong_eval(-1.f * ld(P.in_dir[i]), direction, nrm, S.mats[P.mat[i] & 255]);
-    const float4* T = S.tri + 4 * (size_t)s;
-    const V hit_n = mk(T[3].x, T[3].y, T[3].z);
-    const V hit = org + t * direction;  // Intersection::setPosition(origin + dist * dir)
-    const V pos = hit - kEps * hit_n;
-    const int bounce = bounce0 + 1, mat = __float_as_int(T[0].w);
-    V anti = contrib;
-    if (bounce == 1 && explicit_direct) anti = mk(0.f, 0.f, 0.f);
-    Rng rng{seed, (uint64_t)i << 24, (uint32_t)P.draws[i]};
-    const bool stop = rng.next() > kRr;  // Russian roulette
-    const V rad = stop ? mk(0.f, 0.f, 0.f) : (1.f / kRr) * contrib;
-    st.a.pos[slot] = f3{pos.x, pos.y, pos.z};
-    st.a.nrm[slot] = f3{hit_n.x, hit_n.y, hit_n.z};
-    st.a.dir[slot] = f3{direction.x, direction.y, direction.z};
-    st.a.rad[slot] = f3{rad.x, rad.y, rad.z};
-    st.a.anti[slot] = f3{anti.x, anti.y, anti.z};
-    st.a.mat[slot] = mat;
-    st.a.bounce[slot] = bounce;
-    st.path[slot] = i;
-    P.count[i] += 1;
-    if (stop) return;
-    const float s0 = rng.next(), s1 = rng.next();
-    float pdf;
-    const V next = phong_sample(-1.f * direction, hit_n, S.mats[mat & 255], s0, s1, pdf);
-    if (length(next) <= 0.f || pdf < 1e-4f) return;
-    P.pos[i] = f3{pos.x, pos.y, pos.z};
-    P.nrm[i] = f3{hit_n.x, hit_n.y, hit_n.z};
-    P.rad[i] = f3{rad.x, rad.y, rad.z};
-    P.in_dir[i] = f3{direction.x, direction.y, direction.z};
-    P.dir[i] = f3{next.x, next.y, next.z};
-    P.pdf[i] = pdf;
-    P.bounce[i] = bounce;
-    P.mat[i] = mat;
-    P.draws[i] = (int)rng.k;
-    next_active[atomicAdd(n_next, 1)] = i;
+    if (lane < nslots && (unsigned)(slots + lane) < (unsigned)cap) st.path[slots + lane] = -1;
 }
 
 // Staged AVPL -> offset[path] + bounce - 1: each path's AVPLs together, in
@@ -492,18 +645,24 @@ struct Camera {
     V pos, right, up, fwd;  // right and up scaled by tan(fovy / 2) (and the aspect)
 };
 
-__global__ __launch_bounds__(kThreads) void k_gbuffer(SceneDev S, Camera cam, int W, int H,
+__global__ __launch_bounds__(kWave) void k_gbuffer(SceneDev S, Camera cam, int W, int H,
                                                       float4* __restrict__ pos4, float4* __restrict__ nrm4) {
-    __shared__ int stk[kTraceStack * kThreads];
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= W * H) return;
-    const int px = i % W, py = i / W;
+    extern __shared__ int2 stacks[];
+    // a block's rays are 4 x 2 pixels
+    const int grp = threadIdx.x / kGroup, bw = (W + 3) / 4;
+    const int px = (int)(blockIdx.x % bw) * 4 + (grp & 3), py = (int)(blockIdx.x / bw) * 2 + (grp >> 2);
+    const bool live = px < W && py < H;
+    const int i = py * W + px;
     const float sx = 2.f * ((float)px + 0.5f) / (float)W - 1.f;
     const float sy = 1.f - 2.f * ((float)py + 0.5f) / (float)H;
     const V dir = normalize(cam.fwd + sx * cam.right + sy * cam.up);
-    float t;
-    // a rasteriser has no |det| floor: any front face counts
-    const int s = closest_hit(S, cam.pos, dir, 0.f, t, stk + threadIdx.x);
+    Ray r;
+    ray_start(r, cam.pos, dir, 0.f);  // a rasteriser has no |det| floor: any front face counts
+    r.on = live;
+    while (__ballot(r.on)) ray_step(S, r, stacks + (size_t)grp * S.stack);
+    if (!live || (threadIdx.x & (kGroup - 1)) != 0) return;
+    const int s = r.tri;
+    const float t = r.t;
     if (s < 0) {
         pos4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         nrm4[i] = make_float4(0.f, 0.f, -1.f, 1.f);
@@ -537,29 +696,38 @@ __global__ __launch_bounds__(kThreads) void k_pack_tris(const f3* __restrict__ p
 }
 
 
-__global__ __launch_bounds__(kThreads) void k_zero_ints(int* __restrict__ p, int n) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) p[i] = 0;
+// A shot's counters: the first path that no group starts with, no AVPL staged.
+__global__ void k_paths_reset(int* __restrict__ counters, int first) {
+    counters[0] = first;
+    counters[1] = 0;
 }
 
-__global__ __launch_bounds__(kThreads) void k_intersect(SceneDev S, const f3* __restrict__ org,
+__global__ __launch_bounds__(kWave) void k_intersect(SceneDev S, const f3* __restrict__ org,
                                                         const f3* __restrict__ dir, int n, float* __restrict__ t,
                                                         int* __restrict__ tri_index) {
-    __shared__ int stk[kTraceStack * kThreads];
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    float th;
-    const int s = scene_hit(S, ld(org[i]), ld(dir[i]), th, stk + threadIdx.x);
-    t[i] = s < 0 ? -1.f : th;
+    extern __shared__ int2 stacks[];
+    const int grp = threadIdx.x / kGroup, i = blockIdx.x * kGroups + grp;
+    const bool live = i < n;
+    Ray r;
+    ray_start(r, ld(org[live ? i : 0]), ld(dir[live ? i : 0]), kEps);
+    r.on = live;
+    while (__ballot(r.on)) ray_step(S, r, stacks + (size_t)grp * S.stack);
+    if (!live || (threadIdx.x & (kGroup - 1)) != 0) return;
+    const int s = scene_hit(S, r);
+    t[i] = s < 0 ? -1.f : r.t;
     tri_index[i] = s;
 }
 
 int blocks(int n) { return (n + kThreads - 1) / kThreads; }
 
 SceneDev scene_dev(arc_trace_scene* sc) {
-    return SceneDev{sc->tri.as<float4>(), sc->nodes.as<arc_bvh_node>(), sc->leaf_tri.as<int>(), sc->nleaf,
-                    sc->mats.as<arc_material>(), sc->emissive.as<int>()};
+    return SceneDev{sc->tri.as<float4>(), sc->nodes.as<float4>(), sc->stack, sc->mats.as<arc_material>(),
+                    sc->emissive.as<int>()};
 }
+
+constexpr int kPathBlocks = 4096;  // waves of k_paths: four per SIMD, what its registers let run at once
+
+size_t stack_bytes(const arc_trace_scene* sc) { return sizeof(int2) * (size_t)kGroups * sc->stack; }
 
 // Binned SAH build over the leaves' boxes (host, once per scene): 16 bins
 // of the centroids along the longest axis of their bounds, the split of
@@ -710,6 +878,88 @@ int tree_depth(const std::vector<arc_bvh_node>& nodes) {
     return best;
 }
 
+// The binary tree as eight-wide nodes: from a node's two children, the inner
+// child of the largest box is replaced by its own children until there are
+// eight or only leaves.  A node is 16 float4: per child (box lo, child) and
+// (box hi, 0), child >= 0 a triangle, < 0 the eight-wide node -(child + 1),
+// kNoChild none.  The boxes are widened by 1e-5 of the scene's largest
+// coordinate, far above the rounding of the triangle test, so no hit at a
+// piece's edge is lost.  `stack` receives the most nodes a depth-first
+// traversal keeps pending.
+void wide_nodes(const std::vector<arc_bvh_node>& nodes, const std::vector<int>& order, const std::vector<float>& plo,
+                const std::vector<float>& phi, const std::vector<int>& ptri, std::vector<float4>& wide, int& stack) {
+    struct Child { int c; float lo[3], hi[3]; };
+    auto child = [&](int c) {
+        Child r;
+        r.c = c;
+        for (int d = 0; d < 3; ++d) {
+            if (c >= 0) {
+                r.lo[d] = plo[3 * (size_t)order[c] + d];
+                r.hi[d] = phi[3 * (size_t)order[c] + d];
+            } else {
+                const arc_bvh_node& n = nodes[-(c + 1)];
+                r.lo[d] = (&n.bbMin.x)[d];
+                r.hi[d] = (&n.bbMax.x)[d];
+            }
+        }
+        return r;
+    };
+    auto area = [](const Child& r) {
+        const float x = r.hi[0] - r.lo[0], y = r.hi[1] - r.lo[1], z = r.hi[2] - r.lo[2];
+        return x * y + y * z + z * x;
+    };
+    float far = 0.f;
+    for (size_t k = 0; k < plo.size(); ++k) far = std::max({far, std::fabs(plo[k]), std::fabs(phi[k])});
+    const float pad = 1e-5f * far;
+    struct Task { int node, wide, pending; };  // binary node (-1: a tree of one leaf), its place, nodes pending above it
+    std::vector<Task> tasks{{nodes.empty() ? -1 : 0, 0, 0}};
+    wide.assign(16, float4{});
+    stack = 1;
+    while (!tasks.empty()) {
+        const Task t = tasks.back();
+        tasks.pop_back();
+        Child c[8];
+        int n = 0;
+        if (t.node < 0) {
+            c[n++] = child(0);
+        } else {
+            c[n++] = child(nodes[t.node].left);
+            c[n++] = child(nodes[t.node].right);
+        }
+        while (n < 8) {
+            int best = -1;
+            for (int k = 0; k < n; ++k)
+                if (c[k].c < 0 && (best < 0 || area(c[k]) > area(c[best]))) best = k;
+            if (best < 0) break;
+            const arc_bvh_node& b = nodes[-(c[best].c + 1)];
+            c[best] = child(b.left);
+            c[n++] = child(b.right);
+        }
+        int inner = 0;
+        for (int k = 0; k < n; ++k) inner += c[k].c < 0;
+        stack = std::max(stack, t.pending + inner);
+        for (int k = 0; k < 8; ++k) {
+            float4 lo{}, hi{};
+            int ref = kNoChild;
+            if (k < n) {
+                if (c[k].c >= 0) {
+                    ref = ptri[order[c[k].c]];
+                } else {
+                    const int w = (int)(wide.size() / 16);
+                    wide.resize(wide.size() + 16);
+                    tasks.push_back({-(c[k].c + 1), w, t.pending + inner - 1});
+                    ref = -(w + 1);
+                }
+                lo = make_float4(c[k].lo[0] - pad, c[k].lo[1] - pad, c[k].lo[2] - pad, 0.f);
+                hi = make_float4(c[k].hi[0] + pad, c[k].hi[1] + pad, c[k].hi[2] + pad, 0.f);
+            }
+            std::memcpy(&lo.w, &ref, sizeof(int));
+            wide[16 * (size_t)t.wide + 2 * k] = lo;
+            wide[16 * (size_t)t.wide + 2 * k + 1] = hi;
+        }
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -766,20 +1016,25 @@ int arc_trace_scene_create(arc_ctx* ctx, const arc_float3* p0, const arc_float3*
         std::nth_element(sorted.begin(), sorted.begin() + ntri / 2, sorted.end());
         const double unit = sorted[ntri / 2];
         struct D3 { double v[3]; };
-        auto clip = [](const std::vector<D3>& in, int a, double c, bool keep_ge) {
-            std::vector<D3> out;
-            for (size_t k = 0; k < in.size(); ++k) {
-                const D3& p = in[k];
-                const D3& q = in[(k + 1) % in.size()];
+        struct Poly {  // a triangle clipped twice has at most 5 corners; 8 leave room for rounding
+            D3 at[8];
+            int n = 0;
+            void add(const D3& p) { if (n < 8) at[n++] = p; }
+        };
+        auto clip = [](const Poly& in, int a, double c, bool keep_ge) {
+            Poly out;
+            for (int k = 0; k < in.n; ++k) {
+                const D3& p = in.at[k];
+                const D3& q = in.at[k + 1 < in.n ? k + 1 : 0];
                 const bool pin = keep_ge ? p.v[a] >= c : p.v[a] <= c;
                 const bool qin = keep_ge ? q.v[a] >= c : q.v[a] <= c;
-                if (pin) out.push_back(p);
+                if (pin) out.add(p);
                 if (pin != qin) {
                     const double t = (c - p.v[a]) / (q.v[a] - p.v[a]);
                     D3 r;
                     for (int d = 0; d < 3; ++d) r.v[d] = p.v[d] + t * (q.v[d] - p.v[d]);
                     r.v[a] = c;
-                    out.push_back(r);
+                    out.add(r);
                 }
             }
             return out;
@@ -808,17 +1063,19 @@ int arc_trace_scene_create(arc_ctx* ctx, const arc_float3* p0, const arc_float3*
             int a = 0;
             for (int d = 1; d < 3; ++d)
                 if (bhi[d] - blo[d] > bhi[a] - blo[a]) a = d;
+            Poly whole;
+            for (const D3& p : v) whole.add(p);
             for (int j = 0; j < k; ++j) {
                 const double lo_a = blo[a] + (bhi[a] - blo[a]) * j / k;
                 const double hi_a = j == k - 1 ? bhi[a] : blo[a] + (bhi[a] - blo[a]) * (j + 1) / k;
-                const std::vector<D3> poly = clip(clip({v[0], v[1], v[2]}, a, lo_a, true), a, hi_a, false);
+                const Poly poly = clip(clip(whole, a, lo_a, true), a, hi_a, false);
                 double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-                for (const D3& q : poly)
+                for (int q = 0; q < poly.n; ++q)
                     for (int d = 0; d < 3; ++d) {
-                        lo[d] = std::min(lo[d], q.v[d]);
-                        hi[d] = std::max(hi[d], q.v[d]);
+                        lo[d] = std::min(lo[d], poly.at[q].v[d]);
+                        hi[d] = std::max(hi[d], poly.at[q].v[d]);
                     }
-                if (poly.empty())  // rounding only: keep the whole triangle box within the slab
+                if (poly.n == 0)  // rounding only: keep the whole triangle box within the slab
                     for (int d = 0; d < 3; ++d) {
                         lo[d] = blo[d];
                         hi[d] = bhi[d];
@@ -841,8 +1098,6 @@ int arc_trace_scene_create(arc_ctx* ctx, const arc_float3* p0, const arc_float3*
     int st = arc::ensure(ctx, sc->mats, sizeof(arc_material) * 256);
     if (st == ARC_OK) st = arc::ensure(ctx, sc->emissive, sizeof(int) * 256);
     if (st == ARC_OK) st = arc::ensure(ctx, sc->tri, sizeof(float4) * 4 * (size_t)ntri);
-    if (st == ARC_OK) st = arc::ensure(ctx, sc->leaf_tri, sizeof(int) * (size_t)np);
-    if (st == ARC_OK) st = arc::ensure(ctx, sc->leaf_box, sizeof(float4) * 2 * (size_t)np);
     arc::DevBuf staging;
     if (st == ARC_OK) st = arc::ensure(ctx, staging, 3 * v3 + sizeof(int) * (size_t)ntri);
     if (st != ARC_OK) {
@@ -868,37 +1123,20 @@ int arc_trace_scene_create(arc_ctx* ctx, const arc_float3* p0, const arc_float3*
     std::vector<int> order;
     std::vector<arc_bvh_node> hn;
     sah_build(plo, phi, order, hn);
-    {
-        std::vector<int> lt(np);
-        std::vector<float4> lb(2 * (size_t)np);
-        for (int k = 0; k < np; ++k) {
-            const int r = order[k];
-            lt[k] = ptri[r];
-            lb[2 * (size_t)k] = make_float4(plo[3 * r], plo[3 * r + 1], plo[3 * r + 2], 0.f);
-            lb[2 * (size_t)k + 1] = make_float4(phi[3 * r], phi[3 * r + 1], phi[3 * r + 2], 0.f);
-        }
-        e = hipMemcpy(sc->leaf_tri.p, lt.data(), sizeof(int) * (size_t)np, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(sc->leaf_box.p, lb.data(), sizeof(float4) * 2 * (size_t)np,
-                                           hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            arc::release(staging);
-            return fail(arc::hip_fail(ctx, e, "arc_trace_scene_create", __FILE__, __LINE__));
-        }
-    }
     hipLaunchKernelGGL(k_pack_tris, dim3(blocks(ntri)), dim3(kThreads), 0, ctx->stream, d0, d1, d2, dm,
                        sc->emissive.as<int>(), ntri, sc->tri.as<float4>());
     if (hipGetLastError() != hipSuccess) st = ARC_E_HIP;
-    if (st == ARC_OK && np > 1) {
-        const int nn = np - 1;
-        st = arc::ensure(ctx, sc->nodes, sizeof(arc_bvh_node) * (size_t)nn);
+    sc->max_depth = tree_depth(hn);
+    if (st == ARC_OK && sc->max_depth >= kTraceStack)
+        st = arc::fail(ctx, ARC_E_UNSUPPORTED, "triangle tree deeper than the traversal stack");
+    if (st == ARC_OK) {
+        std::vector<float4> wide;
+        wide_nodes(hn, order, plo, phi, ptri, wide, sc->stack);
+        st = arc::ensure(ctx, sc->nodes, sizeof(float4) * wide.size());
         if (st == ARC_OK) {
-            e = hipMemcpy(sc->nodes.p, hn.data(), sizeof(arc_bvh_node) * (size_t)nn, hipMemcpyHostToDevice);
+            e = hipMemcpy(sc->nodes.p, wide.data(), sizeof(float4) * wide.size(), hipMemcpyHostToDevice);
             if (e != hipSuccess) st = arc::hip_fail(ctx, e, "arc_trace_scene_create", __FILE__, __LINE__);
         }
-        sc->max_depth = tree_depth(hn);
-        // the traversal keeps at most one pending subtree per level
-        if (st == ARC_OK && sc->max_depth >= kTraceStack)
-            st = arc::fail(ctx, ARC_E_UNSUPPORTED, "triangle tree deeper than the traversal stack");
     }
     if (st == ARC_OK) {
         e = hipStreamSynchronize(ctx->stream);
@@ -914,13 +1152,10 @@ void arc_trace_scene_destroy(arc_trace_scene* sc) {
     if (!sc) return;
     if (sc->ctx && sc->ctx->stream) (void)hipStreamSynchronize(sc->ctx->stream);
     arc::release(sc->tri);
-    arc::release(sc->leaf_tri);
-    arc::release(sc->leaf_box);
     arc::release(sc->nodes);
     arc::release(sc->mats);
     arc::release(sc->emissive);
-    arc::release(sc->state);
-    arc::release(sc->active);
+    arc::release(sc->count);
     arc::release(sc->stage);
     arc::release(sc->path_offset);
     arc::release(sc->scan_blocks);
@@ -933,7 +1168,7 @@ int arc_trace_intersect(arc_trace_scene* sc, const arc_float3* org, const arc_fl
     if (!sc || n < 0 || (n > 0 && (!org || !dir || !t || !tri_index))) return ARC_E_INVALID;
     if (n == 0) return ARC_OK;
     arc_ctx* ctx = sc->ctx;
-    hipLaunchKernelGGL(k_intersect, dim3(blocks(n)), dim3(kThreads), 0, ctx->stream, scene_dev(sc),
+    hipLaunchKernelGGL(k_intersect, dim3((n + kGroups - 1) / kGroups), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc),
                        reinterpret_cast<const f3*>(org), reinterpret_cast<const f3*>(dir), n, t, tri_index);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
@@ -971,28 +1206,11 @@ int arc_trace_shoot(arc_trace_scene* sc, const arc_area_light* light, int num_pa
     const int explicit_direct = (flags & ARC_SHOOT_NO_EXPLICIT_DIRECT) ? 0 : 1;
     if (num_paths == 0) return ARC_OK;
     const size_t np = (size_t)num_paths;
-    // path state, 80 bytes per path
-    ARC_TRY(arc::ensure(ctx, sc->state, np * (5 * sizeof(f3) + 5 * sizeof(int))));
-    {
-        char* b = sc->state.as<char>();
-        f3* v[5];
-        for (int k = 0; k < 5; ++k) v[k] = reinterpret_cast<f3*>(b + (size_t)k * np * sizeof(f3));
-        int* w = reinterpret_cast<int*>(b + 5 * np * sizeof(f3));
-        sc->ps = {v[0], v[1], v[2], v[3], v[4], reinterpret_cast<float*>(w), w + np, w + 2 * np,
-                               w + 3 * np, w + 4 * np};
-    }
-    const PathState P{sc->ps.pos, sc->ps.nrm, sc->ps.rad, sc->ps.in_dir, sc->ps.dir, sc->ps.pdf, sc->ps.bounce,
-                      sc->ps.mat, sc->ps.draws, sc->ps.count};
-    ARC_TRY(arc::ensure(ctx, sc->active, sizeof(int) * (2 * np + 2)));
-    int* act[2] = {sc->active.as<int>(), sc->active.as<int>() + np};
-    int* n_next = sc->active.as<int>() + 2 * np;
+    // per-path AVPL counts, and the shot's counters
+    ARC_TRY(arc::ensure(ctx, sc->count, sizeof(int) * (np + 2)));
+    int* count = sc->count.as<int>();
+    int* counters = count + np;
     const SceneDev S = scene_dev(sc);
-    hipLaunchKernelGGL(k_path_start, dim3(blocks(num_paths)), dim3(kThreads), 0, ctx->stream, L, seed, num_paths, P,
-                       act[0]);
-    ARC_LAUNCHED(ctx);
-    // one launch per bounce over the live paths
-    size_t cap = 0, staged = 0;
-    Staged st{};
     auto stage_at = [&](arc::DevBuf& buf, size_t c) {
         char* b = buf.as<char>();
         Staged r;
@@ -1007,45 +1225,30 @@ int arc_trace_shoot(arc_trace_scene* sc, const arc_area_light* light, int num_pa
         return r;
     };
     const size_t slot_bytes = 5 * sizeof(f3) + 3 * sizeof(int);
-    if (sc->stage.p) {  // reuse the last call's staging area
-        cap = sc->stage.bytes / slot_bytes;
+    const int pblocks = std::min((num_paths + kGroups - 1) / kGroups, kPathBlocks);
+    // a path makes 5 AVPLs at most on average (roulette at 0.8), and a wave
+    // may leave a grab's rest unused
+    size_t cap = std::min(std::max(8 * np + (size_t)kSlotGrab * pblocks, sc->stage.bytes / slot_bytes), (size_t)INT_MAX);
+    Staged st{};
+    unsigned staged = 0;
+    for (;;) {  // a second time when the paths made more AVPLs than that
+        ARC_TRY(arc::ensure(ctx, sc->stage, cap * slot_bytes));
         st = stage_at(sc->stage, cap);
-    }
-    int n_active = num_paths, cur = 0;
-    for (int step = 0; n_active > 0; ++step) {
-        if (step > 4096) return arc::fail(ctx, ARC_E_STATE, "path tracing did not terminate");
-        if (staged + (size_t)n_active > cap) {  // grow the staging area, keeping what it holds
-            const size_t ncap = std::max(staged + (size_t)n_active, std::max((size_t)8 * np, 2 * cap));
-            arc::DevBuf nb;
-            ARC_TRY(arc::ensure(ctx, nb, ncap * slot_bytes));
-            const Staged ns = stage_at(nb, ncap);
-            if (staged > 0) {
-                const void* src[8] = {st.a.pos, st.a.nrm, st.a.dir, st.a.rad, st.a.anti, st.a.mat, st.a.bounce, st.path};
-                void* dst[8] = {ns.a.pos, ns.a.nrm, ns.a.dir, ns.a.rad, ns.a.anti, ns.a.mat, ns.a.bounce, ns.path};
-                const size_t sz[8] = {sizeof(f3), sizeof(f3), sizeof(f3), sizeof(f3), sizeof(f3), 4, 4, 4};
-                for (int k = 0; k < 8; ++k)
-                    ARC_HIP(ctx, hipMemcpyAsync(dst[k], src[k], staged * sz[k], hipMemcpyDeviceToDevice, ctx->stream));
-            }
-            ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            arc::release(sc->stage);
-            sc->stage = nb;
-            cap = ncap;
-            st = ns;
-        }
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(kThreads), 0, ctx->stream, n_next, 1);
-        hipLaunchKernelGGL(k_path_step, dim3(blocks(n_active)), dim3(kThreads), 0, ctx->stream, S, seed,
-                           explicit_direct, P, act[cur], n_active, act[1 - cur], n_next, st, (int)staged);
+        hipLaunchKernelGGL(k_paths_reset, dim3(1), dim3(1), 0, ctx->stream, counters, pblocks * kGroups);
+        hipLaunchKernelGGL(k_paths, dim3(pblocks), dim3(kWave), stack_bytes(sc), ctx->stream, S, L, seed, num_paths,
+                           explicit_direct, counters, reinterpret_cast<unsigned*>(counters + 1), (int)cap, count, st);
         ARC_LAUNCHED(ctx);
-        staged += (size_t)n_active;
-        ARC_HIP(ctx, hipMemcpyAsync(&n_active, n_next, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        ARC_HIP(ctx, hipMemcpyAsync(&staged, counters + 1, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        cur = 1 - cur;
+        if ((size_t)staged <= cap) break;
+        if (staged > (unsigned)INT_MAX) return arc::fail(ctx, ARC_E_UNSUPPORTED, "too many AVPLs");
+        cap = std::min((size_t)staged + (size_t)staged / 8, (size_t)INT_MAX);
     }
     // per-path counts -> offsets -> AVPLs in path order
     const int nb = (num_paths + kScan - 1) / kScan;
     ARC_TRY(arc::ensure(ctx, sc->path_offset, sizeof(int) * (np + 1)));
     ARC_TRY(arc::ensure(ctx, sc->scan_blocks, sizeof(int) * ((size_t)nb + 1)));
-    hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(kScan), 0, ctx->stream, P.count, num_paths,
+    hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(kScan), 0, ctx->stream, count, num_paths,
                        sc->path_offset.as<int>(), sc->scan_blocks.as<int>());
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScan), 0, ctx->stream, sc->scan_blocks.as<int>(), nb);
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScan), 0, ctx->stream, sc->path_offset.as<int>(), num_paths,
@@ -1095,8 +1298,8 @@ int arc_trace_gbuffer(arc_trace_scene* sc, arc_float3 camPos, arc_float3 forward
     const float th = std::tan(0.5f * fovy), aspect = (float)width / (float)height;
     Camera cam{mk(camPos.x, camPos.y, camPos.z), mk(rx * th * aspect, ry * th * aspect, rz * th * aspect),
                mk(ux * th, uy * th, uz * th), mk(fx, fy, fz)};
-    const int npix = width * height;
-    hipLaunchKernelGGL(k_gbuffer, dim3(blocks(npix)), dim3(kThreads), 0, ctx->stream, scene_dev(sc), cam, width,
+    const int gblocks = ((width + 3) / 4) * ((height + 1) / 2);
+    hipLaunchKernelGGL(k_gbuffer, dim3(gblocks), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc), cam, width,
                        height, reinterpret_cast<float4*>(pos4), reinterpret_cast<float4*>(nrm4));
     ARC_LAUNCHED(ctx);
     return ARC_OK;
