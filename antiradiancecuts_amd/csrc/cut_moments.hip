@@ -513,7 +513,14 @@ __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32
 // with the largest cut set the kernel's time: with 375 tiles on 1024 SIMDs
 // (200x120 pixels) that was 1.8 ms.
 constexpr int kKeep = 128;
-constexpr int kChunkLeaves = 2048;
+// A small image over a small tree has few range chunks: with 2048 leaves in one
+// and 5700 chunks for 8192 waves, some CUs held a full set and others none
+// (600x300 pixels, 4000 AVPLs, exact up to 128: 431 us for 120 us of vector
+// work, 0.67 ms a frame; 0.59 with 1024 leaves, 0.60 with 512, whose parts scan
+// their ranges too often).
+constexpr int kChunkLeaves = 1024;
+constexpr int kNextCounters = 8, kNextStride = 32;  // the counters of k_cut_eval's chunks, a cache line each
+constexpr int kPartBits = 5;        // a range chunk is kKeep ranges of at most 128 leaves: at most 32 parts
 constexpr int kDecideStack = 640;   // pending nodes per wave
 constexpr int kStackReserve = 64;   // of these for the depth-first descent when the rest is full (tree depth <= 57)
 enum ChunkKind { kNodes = 0, kRanges = 1 };
@@ -735,7 +742,7 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
         ++spare;
         --nspare;
         if (lane == 0) {
-            pool.meta[c] = make_int4(item, kind | (cnt << 8), -1, (from < 0 ? c : from) * 16 + part);
+            pool.meta[c] = make_int4(item, kind | (cnt << 8), -1, ((from < 0 ? c : from) << kPartBits) + part);
             if (last >= 0) pool.meta[last].z = c;
         }
         if (head < 0) head = c;
@@ -767,9 +774,9 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
             const int m = min(nx, kKeep);
             const uint32_t x0 = lane < m ? S.ex[lane] : 0u, x1 = lane + 64 < m ? S.ex[lane + 64] : 0u;
             int parts = 1;
-            if (v.exact_count > kChunkLeaves / kKeep) {
+            {
                 const int leaves = (lane < m ? (int)(x0 & 127u) + 1 : 0) + (lane + 64 < m ? (int)(x1 & 127u) + 1 : 0);
-                parts = (wave_isum(leaves) + kChunkLeaves - 1) / kChunkLeaves;  // at most 128 x 128 leaves: 8
+                parts = (wave_isum(leaves) + kChunkLeaves - 1) / kChunkLeaves;
             }
             int c = -1, first = -1;
             for (int k = 0; k < parts; ++k) {
@@ -1183,13 +1190,24 @@ __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))
     EvalLds& S = lds[wave];
     const int waves = gridDim.x * (kCutThreads / 64);
     const int n = uniform(min(*pool.taken, pool.cap));
-    // chunks are taken in groups, a fraction of a wave's share, so that few atomics serve many chunks
+    // A wave starts with the chunk of its number and then takes groups of
+    // chunks, a fraction of its share, from one of eight counters: a counter
+    // serves about 100 atomics per microsecond (one for all took 230 us for 23K
+    // chunks).  A counter's groups stand at changing places among eight: a
+    // tile's first chunks are its largest and its last ones not used, and they
+    // come in eights.  Where a group is eight chunks, one counter keeps up,
+    // and all waves work on neighbouring tiles until the end (250001 AVPLs,
+    // 1283x719: 16.0 ms, 16.9 with eight).
     const int group = max(1, min(8, n / (4 * waves)));
-    for (int c = 0, left = 0;; ++c, --left) {
+    const int counters = group == 8 ? 1 : min(kNextCounters, (int)gridDim.x), k = blockIdx.x % counters;
+    int c = blockIdx.x * (kCutThreads / 64) + wave;
+    for (int left = c < n ? 1 : 0;; ++c, --left) {
         if (left <= 0) {
+            if (n <= waves) break;
             int got = 0;
-            if (lane == 0) got = atomicAdd(pool.next, group);
-            c = uniform(got);
+            if (lane == 0) got = atomicAdd(pool.next + kNextStride * k, 1);
+            got = uniform(got);
+            c = waves + (got * counters + (k + (int)((unsigned)got * 0x9E3779B1u >> 29)) % counters) * group;
             if (c >= n) break;
             left = min(group, n - c);
         }
@@ -1198,7 +1216,7 @@ __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))
         if (cnt == 0) continue;  // not used, or its tile is cut serially
         const CutView v = views.of(item);
         const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
-        const uint32_t* e = pool.entries + (size_t)(uniform(m.w) >> 4) * kKeep;
+        const uint32_t* e = pool.entries + (size_t)(uniform(m.w) >> kPartBits) * kKeep;
         const uint32_t e0 = lane < cnt ? e[lane] : 0u, e1 = lane + 64 < cnt ? e[lane + 64] : 0u;
         const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
         const PixelF F = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, x < v.W && y < v.H ? y * v.W + x : 0);
@@ -1236,7 +1254,7 @@ __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))
         for (int b = 0; b < kSlots; ++b) tot[b][0] = tot[b][1] = tot[b][2] = 0.f;
         ufloat* box = uptr(pool.tbox + 8 * (size_t)item);
         const float tb[6] = {box[0], box[1], box[2], box[3], box[4], box[5]};
-        sum_ranges(v.crec, S, cnt, (uniform(m.w) & 15) * kChunkLeaves, tb, P, tot);
+        sum_ranges(v.crec, S, cnt, (uniform(m.w) & ((1 << kPartBits) - 1)) * kChunkLeaves, tb, P, tot);
 #pragma unroll
         for (int ch = 0; ch < 3; ++ch) {
             float out = 0.f;
@@ -1461,9 +1479,11 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_serial(Views<kMany> views, 
 
 // A frame's pool: no chunk taken, no tile handed back.
 __global__ void k_pool_reset(CutPool p) {
-    *p.taken = 0;
-    *p.nserial = 0;
-    *p.next = 0;
+    if (threadIdx.x == 0) {
+        *p.taken = 0;
+        *p.nserial = 0;
+    }
+    p.next[kNextStride * threadIdx.x] = 0;
 }
 
 }  // namespace
@@ -1497,10 +1517,14 @@ int cut_moments_build(arc_gather* g, arc_bvh* b) {
 
 namespace {
 
-// The chunks a tile can need: most frames use about 25 per tile (a million
-// AVPLs at a bound of 0.01) or 50 where larger nodes are summed exactly, a
-// small tree fewer than its leaves fill.
-int default_chunks(int n, int exact_count) { return std::min(exact_count > 16 ? 96 : 48, 8 + n / 64); }
+// The chunks a tile can need.  Most frames use 9 to 11 per tile at 4000 to 8000
+// AVPLs, 25 at 64000 and 25 to 40 at a million where nodes of up to 64 AVPLs
+// are summed exactly; 4 to 11, 43 and 60 to 120 where larger ones are.  (8 + n
+// / 64 of them cost the first frame of a 600x300 image with 4000 AVPLs 0.1 ms
+// of allocation.)
+int default_chunks(int n, int exact_count) {
+    return exact_count > 64 ? std::min(96, 12 + n / 1024) : std::min(48, 14 + n / 2048);
+}
 
 constexpr int kMinChunks = 16384;  // 21 MB
 
@@ -1523,16 +1547,19 @@ int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, lo
     // a small image's tiles can hold 512 chunks each (a budget of 65536): no small pools
     want = std::max(want, std::min((long long)kMinChunks, 512LL * nitems));
     if (want > INT_MAX / kKeep) want = INT_MAX / kKeep;
-    ARC_TRY(ensure(ctx, mem.entries, sizeof(uint32_t) * kKeep * (size_t)want));
-    ARC_TRY(ensure(ctx, mem.meta, sizeof(int4) * (size_t)want));
-    ARC_TRY(ensure(ctx, mem.part, sizeof(float) * 192 * (size_t)want));
-    ARC_TRY(ensure(ctx, mem.tiles, sizeof(int) * ((size_t)11 * nitems + 4)));
+    // one allocation: a new gather's first frame pays for each
+    const size_t chunk = (size_t)want, part = sizeof(float) * 192 * chunk, entries = sizeof(uint32_t) * kKeep * chunk,
+                 meta = sizeof(int4) * chunk;
+    ARC_TRY(ensure(ctx, mem.buf, part + entries + meta +
+                                     sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1))));
     mem.cap = (int)want;
-    float* tbox = mem.tiles.as<float>();
+    char* at = mem.buf.as<char>();
+    float* tbox = reinterpret_cast<float*>(at + part + entries + meta);
     int* head = reinterpret_cast<int*>(tbox + 8 * (size_t)nitems);
-    p = CutPool{mem.entries.as<uint32_t>(), mem.meta.as<int4>(), mem.part.as<float>(), tbox, head, head + nitems,
+    p = CutPool{reinterpret_cast<uint32_t*>(at + part), reinterpret_cast<int4*>(at + part + entries),
+                reinterpret_cast<float*>(at), tbox, head, head + nitems,
                 head + 2 * (size_t)nitems, head + 3 * (size_t)nitems, head + 3 * (size_t)nitems + 1,
-                head + 3 * (size_t)nitems + 2, mem.seen, (int)want, nitems < 4096 ? 4 : 8};
+                head + 3 * (size_t)nitems + 2 + kNextStride, mem.seen, (int)want, nitems < 4096 ? 4 : 8};
     return ARC_OK;
 }
 
@@ -1553,7 +1580,7 @@ void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool 
         hipLaunchKernelGGL(k_cut_serial<kMany>, dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, 1, p);
         return;
     }
-    hipLaunchKernelGGL(k_pool_reset, dim3(1), dim3(1), 0, stream, p);
+    hipLaunchKernelGGL(k_pool_reset, dim3(1), dim3(kNextCounters), 0, stream, p);
     if (expansion)
         hipLaunchKernelGGL((k_cut_decide<kMany, true>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
     else
@@ -1566,10 +1593,7 @@ void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool 
 }  // namespace
 
 void release_pool(CutPoolMem& mem) {
-    release(mem.entries);
-    release(mem.meta);
-    release(mem.part);
-    release(mem.tiles);
+    release(mem.buf);
     if (mem.seen) (void)hipHostFree(mem.seen);
     mem = CutPoolMem{};
 }

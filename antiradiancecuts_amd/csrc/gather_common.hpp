@@ -43,8 +43,8 @@ struct CutView {
 // the decision kernel, summed by the evaluation kernel (cut_moments.hip).
 struct CutPool {
     uint32_t* entries;  // cap chunks of 128 entries
-    int4* meta;         // per chunk: (tile, kind | entries << 8, the tile's next chunk or -1, 16 x the chunk that
-                        // holds its entries + which part of them)
+    int4* meta;         // per chunk: (tile, kind | entries << 8, the tile's next chunk or -1, the chunk that holds
+                        // its entries and which part of them)
     float* part;        // per chunk: 3 x 64 partial sums
     float* tbox;        // per tile: its box, centre and half extent (8 floats)
     int* head;          // per tile: its first chunk or -1
@@ -52,7 +52,7 @@ struct CutPool {
     int* serial;        // the tiles to cut serially
     int* taken;         // chunks asked for (may pass cap)
     int* nserial;
-    int* next;          // the evaluation's next chunk
+    int* next;          // the evaluation's counters of chunks
     int* seen;          // pinned host memory: chunks the frame asked for
     int cap;
     int grab;           // chunks a tile takes with its first atomic, twice as many with each later one: the
@@ -62,7 +62,7 @@ struct CutPool {
 
 // The pool's memory, kept between launches.
 struct CutPoolMem {
-    DevBuf entries, meta, part, tiles;
+    DevBuf buf;
     int* seen = nullptr;
     int cap = 0;
 };
