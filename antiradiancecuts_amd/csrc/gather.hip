@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kThreads) void k_finalize_f64(const double* __restr
 // Decision arithmetic of kernel_bvh (cudaGather.cu:405-414) in FP32 with IEEE
 // division and square root and no fused multiply-add, so every traversal
 // decision equals the oracle's REF32 decision.
-__device__ __attribute__((noinline)) bool cluster_visible(f3 n, f3 p, f3 bmin, f3 bmax) {
+__device__ inline bool cluster_visible(f3 n, f3 p, f3 bmin, f3 bmax) {
 #pragma clang fp contract(off)
     const float ax = bmax.x - p.x, ay = bmax.y - p.y, az = bmax.z - p.z;
     const float sa = 1.0f / sqrtf(ax * ax + ay * ay + az * az);
@@ -235,7 +235,7 @@ __device__ __attribute__((noinline)) bool cluster_visible(f3 n, f3 p, f3 bmin, f
     return (c1 > 0.f) || (c2 > 0.f);
 }
 
-__device__ __attribute__((noinline)) bool solid_angle_below(f3 p, f3 rep, f3 bmin, f3 bmax, float thresh) {
+__device__ inline bool solid_angle_below(f3 p, f3 rep, f3 bmin, f3 bmax, float thresh) {
 #pragma clang fp contract(off)
     const float ex = bmax.x - bmin.x, ey = bmax.y - bmin.y, ez = bmax.z - bmin.z;
     const float radius = 0.5f * sqrtf(ex * ex + ey * ey + ez * ez);
@@ -255,7 +255,90 @@ struct CutTree {
     int n;  // leaves
 };
 
-__global__ __launch_bounds__(kThreads) void k_cut_sa(CutTree t, const float4* __restrict__ gpos,
+// The cut's records: a leaf's (position, 0), (unit normal, 0), (radiance times
+// the AVPL's Lambertian reflectance, 0) and an inner node's (box lo, left),
+// (box hi, right), (position, far), (unit normal, near), (radiance, 0) of its
+// representative.  With squared distance d2 from a pixel to the
+// representative, d2 > far is certainly below the threshold, d2 < near
+// certainly not (SaBand).
+constexpr int kSaLeaf = 3, kSaNode = 5;
+
+// Omega = 2 pi (1 - d / sqrt(r^2 + d^2)) < thresh is d2 > ratio(thresh) r2; its
+// FP32 value carries at most 2.3e-6 of rounding (4 ulp of 1 in the quotient),
+// so it is certain where the threshold moved by 4e-6 either way gives the same
+// answer (far, near: the ratios of the moved thresholds).
+struct SaBand {
+    float far, near;
+};
+
+SaBand sa_band(float thresh) {
+    auto ratio = [](double t) {
+        const double q = 1.0 - t / (2.0 * M_PI);
+        if (q >= 1.0) return (double)INFINITY;
+        if (q <= 0.0) return -1.0;
+        return q * q / (1.0 - q * q);
+    };
+    const double lo = ratio((double)thresh - 4e-6), hi = ratio((double)thresh + 4e-6);
+    return SaBand{(float)(lo * (1.0 + 2e-6)), (float)(hi * (1.0 - 2e-6))};
+}
+
+__global__ __launch_bounds__(kThreads) void k_sa_records(CutTree t, const arc_material* __restrict__ mats, SaBand band,
+                                                         float4* __restrict__ rec) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= 2 * t.n - 1) return;
+    const V<float> p = ld3<float>(t.pos[i]), nrm = normalize(ld3<float>(t.nrm[i])), w = ld3<float>(t.dir[i]);
+    V<float> c = ld3<float>(t.rad[i]);
+    if (length(w) != 0.f) c = c * (kOneOverPi * material<float>(mats, t.mat[i]).diffuse);
+    float far = 0.f, near = 0.f;
+    float4* r = rec + kSaLeaf * (size_t)i;
+    if (i >= t.n) {
+        const arc_bvh_node b = t.nodes[i - t.n];
+        const float ex = b.bbMax.x - b.bbMin.x, ey = b.bbMax.y - b.bbMin.y, ez = b.bbMax.z - b.bbMin.z;
+        const float r2 = 0.25f * (ex * ex + ey * ey + ez * ez);
+        // below 1e-30 the squares lose their accuracy: neither
+        far = band.far * r2 + 1e-30f;
+        near = band.near * r2 - 1e-30f;
+        r = rec + kSaLeaf * (size_t)t.n + kSaNode * (size_t)(i - t.n);
+        r[0] = make_float4(b.bbMin.x, b.bbMin.y, b.bbMin.z, __int_as_float(b.left));
+        r[1] = make_float4(b.bbMax.x, b.bbMax.y, b.bbMax.z, __int_as_float(b.right));
+        r += 2;
+    }
+    r[0] = make_float4(p.x, p.y, p.z, far);
+    r[1] = make_float4(nrm.x, nrm.y, nrm.z, near);
+    r[2] = make_float4(c.x, c.y, c.z, 0.f);
+}
+
+// kernel_bvh (cudaGather.cu:375-433): each pixel's depth-first cut, the right
+// child first.
+//
+// A wave walks the union of its 8x8 pixels' cuts: an entry of the stack is a
+// node and the set of pixels that reach it, so the records are read by scalar
+// loads, the stack is one for the wave, and no lane waits for another's branch.
+// Neighbouring pixels' cuts are nearly equal.  A pixel sees the nodes in the
+// order of its own traversal, and it is in every entry above which its node
+// lies: the stack's height is its own stack's, which may overflow
+// (stack_size; the pixel is then an error, as in kernel_bvh).
+//
+// The decisions are made without square roots and divisions wherever the FP32
+// formulas' rounding cannot change them, and by these formulas elsewhere.  A
+// corner's test is the sign of n . (corner - p), here n . corner - n . p: both
+// carry at most 4 ulp of the terms' absolute sums, against a guard of 1e-6 of
+// these sums at the scene's largest coordinates (and 1e-12, below which the
+// formula's squares may underflow).
+//
+// Bound: vector and scalar instructions, about 40 of each per visited node
+// (half of them its share of the evaluations), and the reads' latency where
+// few waves hide it.  1280x720 pixels over 65536 AVPLs: 3.64 ms where each lane
+// walked its own tree with the formulas (a wave then waits for its longest
+// lane and runs every branch of each step), 0.95 here; 1.33 with the corners'
+// differences taken before the products and the stack in LDS.  Fetching the
+// right child's record ahead made it 1.1, and a 160x120 image 5 % faster.
+constexpr float kSaGuard = 1e-6f;
+constexpr int kSaStack = 64;  // entries: a pixel's stack is at most that high
+
+template <bool GENERAL>
+__global__ __launch_bounds__(kThreads) void k_cut_sa(CutTree t, const float4* __restrict__ rec,
+                                                     const float4* __restrict__ gpos,
                                                      const float4* __restrict__ gnrm,
                                                      const float4* __restrict__ galb,
                                                      const arc_material* __restrict__ mats, int W, int H,
@@ -263,80 +346,135 @@ __global__ __launch_bounds__(kThreads) void k_cut_sa(CutTree t, const float4* __
                                                      int stack_size, int sentinel,
                                                      float4* __restrict__ out_rad,
                                                      unsigned long long* __restrict__ counters) {
-    extern __shared__ int stk[];  // [stack_size][kThreads]
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int x = blockIdx.x * 16 + (wave & 1) * 8 + (lane & 7);
-    const int y = blockIdx.y * 16 + (wave >> 1) * 8 + (lane >> 3);
+    static_assert(kSaStack == 64, "the stack is a register's lanes");
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int tw = (W + 15) / 16, b = xcd_block(blockIdx.x, tw * ((H + 15) / 16));
+    const int x = (b % tw) * 16 + (wave & 1) * 8 + (lane & 7);
+    const int y = (b / tw) * 16 + (wave >> 1) * 8 + (lane >> 3);
     const bool live = x < W && y < H;
-    unsigned long long nvis = 0, neval = 0, nerr = 0;
-    if (live) {
-        using V3 = V<float>;
-        const int pix = y * W + x;
-        const float4 p4 = gpos[pix], n4 = gnrm[pix];
-        const f3 p = f3of(p4), nraw = f3of(n4);
-        const V3 pos = mk(p4.x, p4.y, p4.z), nrm = mk(n4.x, n4.y, n4.z);
-        Mat<float> pm = material<float>(mats, (int)n4.w);
-        if (galb) pm.diffuse = mk(galb[pix].x, galb[pix].y, galb[pix].z);
-        const V3 cam = mk(camx, camy, camz);
-        auto eval = [&](int idx) {
-            const Mat<float> am = material<float>(mats, t.mat[idx]);
-            return radiance(pos, nrm, pm, ld3<float>(t.pos[idx]), ld3<float>(t.nrm[idx]), ld3<float>(t.dir[idx]),
-                            ld3<float>(t.rad[idx]), am, cam);
-        };
-        V3 R = mk(0.f, 0.f, 0.f);
-        int sp = 0;
-        stk[sp * kThreads + tid] = -1;
-        sp = 1;
-        bool error = false;
-        while (sp > 0) {
-            const int node = stk[(--sp) * kThreads + tid];
-            if (node >= 0) {
-                R = R + eval(node);
-                neval++;
-                continue;
-            }
+    const int pix = live ? y * W + x : 0;
+    const PixelF P = load_pixel(gpos, gnrm, galb, mats, pix);
+    const f3 p = f3{P.px, P.py, P.pz}, nraw = f3of(gnrm[pix]);
+    ufloat* const root = uptr(rec + kSaLeaf * (size_t)t.n);
+    const float np = nraw.x * p.x + nraw.y * p.y + nraw.z * p.z;
+    const float scale = fabsf(nraw.x) * (fabsf(p.x) + fmaxf(fabsf(root[0]), fabsf(root[4]))) +
+                        fabsf(nraw.y) * (fabsf(p.y) + fmaxf(fabsf(root[1]), fabsf(root[5]))) +
+                        fabsf(nraw.z) * (fabsf(p.z) + fmaxf(fabsf(root[2]), fabsf(root[6])));
+    const float guard = kSaGuard * scale + 1e-12f;
+    // the guards hold for magnitudes whose squares stay finite and for numbers;
+    // a pixel outside them is decided by the formulas throughout
+    const float far_out = fabsf(p.x) + fabsf(p.y) + fabsf(p.z) + fabsf(root[0]) + fabsf(root[1]) + fabsf(root[2]) +
+                          fabsf(root[4]) + fabsf(root[5]) + fabsf(root[6]);
+    const bool plain = far_out < 1e15f && fabsf(nraw.x) + fabsf(nraw.y) + fabsf(nraw.z) < 1e3f;
+    const uint64_t odd = __ballot(!plain);
+    uint64_t alive = __ballot(live), erred = 0;
+    unsigned nvis = 0, neval = 0;
+    V<float> R = mk(0.f, 0.f, 0.f);
+    // the sum is taken without the Lambertian pixel's reflectance
+    auto eval = [&](ufloat* r, int idx, uint64_t m) {
+        neval += __popcll(m);
+        if (!__builtin_amdgcn_inverse_ballot_w64(m)) return;
+        if constexpr (GENERAL) {
+            Mat<float> pm = material<float>(mats, P.mat);
+            if (galb) pm.diffuse = mk(galb[pix].x, galb[pix].y, galb[pix].z);
+            const float4 n4 = gnrm[pix];
+            R = R + radiance(mk(P.px, P.py, P.pz), mk(n4.x, n4.y, n4.z), pm, ld3<float>(t.pos[idx]),
+                             ld3<float>(t.nrm[idx]), ld3<float>(t.dir[idx]), ld3<float>(t.rad[idx]),
+                             material<float>(mats, t.mat[idx]), mk(camx, camy, camz));
+        } else {
+            const float dx = r[0] - P.px, dy = r[1] - P.py, dz = r[2] - P.pz;
+            const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
+            const float c1 = clamp01((P.nx * dx + P.ny * dy + P.nz * dz) * inv);
+            const float c2 = clamp01(-(r[4] * dx + r[5] * dy + r[6] * dz) * inv);
+            const float gg = (c1 * c2) * (inv * inv);
+            R.x += r[8] * gg;
+            R.y += r[9] * gg;
+            R.z += r[10] * gg;
+        }
+    };
+    // the stack: entry j in lane j
+    int snode = 0, slo = 0, shi = 0;
+    int sp = 0, node = -1;
+    uint64_t m = alive;
+    while (m) {
+        while (node < 0) {
             const int k = -(node + 1);
             if (k >= t.n - 1) {
-                error = true;
+                erred |= m;
+                alive &= ~m;
                 break;
             }
-            nvis++;
-            const arc_bvh_node b = t.nodes[k];
-            const f3 bmin = f3{b.bbMin.x, b.bbMin.y, b.bbMin.z}, bmax = f3{b.bbMax.x, b.bbMax.y, b.bbMax.z};
-            if (!cluster_visible(nraw, p, bmin, bmax)) continue;
-            const int idx = t.n + k;
-            if (solid_angle_below(p, t.pos[idx], bmin, bmax, thresh)) {
-                R = R + eval(idx);
-                neval++;
-            } else {
-                stk[sp * kThreads + tid] = b.left;
-                stk[(sp + 1) * kThreads + tid] = b.right;
-                sp += 2;
-                if (sp >= stack_size) {
-                    error = true;
-                    break;
+            nvis += __popcll(m);
+            ufloat* r = root + 4 * kSaNode * (size_t)k;
+            const float r0 = r[0], r1 = r[1], r2 = r[2], r4 = r[4], r5 = r[5], r6 = r[6], r8 = r[8], r9 = r[9],
+                        r10 = r[10], far = r[11], near = r[15];
+            const int left = __float_as_int(r[3]), right = __float_as_int(r[7]);
+            const float sa = __builtin_fmaf(nraw.x, r4, __builtin_fmaf(nraw.y, r5, __builtin_fmaf(nraw.z, r6, -np)));
+            const float sb = __builtin_fmaf(nraw.x, r0, __builtin_fmaf(nraw.y, r1, __builtin_fmaf(nraw.z, r2, -np)));
+            uint64_t visible = __ballot(sa > guard) | __ballot(sb > guard);
+            uint64_t unsure = m & (odd | ~(visible | (__ballot(sa < -guard) & __ballot(sb < -guard))));
+            if (unsure) {
+                bool v = false;
+                if (__builtin_amdgcn_inverse_ballot_w64(unsure)) {
+                    // most often the box lies in the pixel's plane, a corner not above it to the last bit
+                    const float ax = r4 - p.x, ay = r5 - p.y, az = r6 - p.z, bx = r0 - p.x, by = r1 - p.y, bz = r2 - p.z;
+                    const bool ha = sa < -guard || (nraw.x * ax == 0.f && nraw.y * ay == 0.f && nraw.z * az == 0.f &&
+                                                    fabsf(ax) + fabsf(ay) + fabsf(az) > 1e-12f);
+                    const bool hb = sb < -guard || (nraw.x * bx == 0.f && nraw.y * by == 0.f && nraw.z * bz == 0.f &&
+                                                    fabsf(bx) + fabsf(by) + fabsf(bz) > 1e-12f);
+                    v = !(plain && ha && hb) && cluster_visible(nraw, p, f3{r0, r1, r2}, f3{r4, r5, r6});
                 }
+                visible = (visible & ~unsure) | __ballot(v);
             }
+            visible &= m;
+            const float dx = r8 - p.x, dy = r9 - p.y, dz = r10 - p.z;
+            const float d2 = dx * dx + dy * dy + dz * dz;
+            uint64_t below = __ballot(d2 > far);
+            unsure = visible & (odd | ~(below | __ballot(d2 < near)));
+            if (unsure) {
+                bool v = false;
+                if (__builtin_amdgcn_inverse_ballot_w64(unsure))
+                    v = solid_angle_below(p, f3{r8, r9, r10}, f3{r0, r1, r2}, f3{r4, r5, r6}, thresh);
+                below = (below & ~unsure) | __ballot(v);
+            }
+            below &= visible;
+            if (below) eval(r + 8, t.n + k, below);
+            m = visible & ~below;
+            if (!m) break;
+            if (sp + 2 >= stack_size) {
+                erred |= m;
+                alive &= ~m;
+                break;
+            }
+            if (__builtin_amdgcn_inverse_ballot_w64(1ull << sp)) {
+                snode = left;
+                slo = (int)(uint32_t)m;
+                shi = (int)(uint32_t)(m >> 32);
+            }
+            ++sp;
+            node = right;
         }
-        float4 o = make_float4(R.x, R.y, R.z, 1.f);
-        if (error) {
-            nerr = 1;
-            if (sentinel) o = make_float4(100000.f, 0.f, 100000.f, 1.f);
-        }
+        if (node >= 0) eval(uptr(rec + kSaLeaf * (size_t)node), node, m);
+        do {  // the next entry; pixels that erred are in none any more
+            if (sp == 0) {
+                m = 0;
+                break;
+            }
+            --sp;
+            node = __builtin_amdgcn_readlane(snode, sp);
+            m = alive & ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(slo, sp) |
+                         (uint64_t)(uint32_t)__builtin_amdgcn_readlane(shi, sp) << 32);
+        } while (!m);
+    }
+    if (live) {
+        float4 o = GENERAL ? make_float4(R.x, R.y, R.z, 1.f) : make_float4(R.x * P.br, R.y * P.bg, R.z * P.bb, 1.f);
+        if (sentinel && __builtin_amdgcn_inverse_ballot_w64(erred)) o = make_float4(100000.f, 0.f, 100000.f, 1.f);
         out_rad[pix] = o;
     }
-    if (counters) {
-        // one atomic per wave
-        for (int off = 32; off > 0; off >>= 1) {
-            nvis += __shfl_down(nvis, off);
-            neval += __shfl_down(neval, off);
-            nerr += __shfl_down(nerr, off);
-        }
-        if (lane == 0) {
-            atomicAdd(&counters[C_VISITED], nvis);
-            atomicAdd(&counters[C_EVALUATED], neval);
-            atomicAdd(&counters[C_ERRORS], nerr);
-        }
+    if (counters && lane == 0) {  // one atomic per wave
+        atomicAdd(&counters[C_VISITED], (unsigned long long)nvis);
+        atomicAdd(&counters[C_EVALUATED], (unsigned long long)neval);
+        atomicAdd(&counters[C_ERRORS], (unsigned long long)__popcll(erred));
     }
 }
 
@@ -712,11 +850,18 @@ int arc_gather_run(arc_gather* g, const arc_avpls* avpls, arc_float3 camPos, flo
             if (profile) ARC_HIP(ctx, hipEventRecord(ev[6], ctx->stream));
             CutTree t{b->nodes.as<arc_bvh_node>(), b->nd_mat.as<int>(), b->nd_pos.as<f3>(), b->nd_nrm.as<f3>(),
                       b->nd_rad.as<f3>(), b->nd_dir.as<f3>(), b->n};
-            dim3 grid((g->width + 15) / 16, (g->height + 15) / 16);
-            const size_t lds = sizeof(int) * (size_t)p->stackSize * kThreads;
-            hipLaunchKernelGGL(k_cut_sa, grid, dim3(kThreads), lds, ctx->stream, t, g->gpos, g->gnrm, g->galb,
-                               g->mats.as<arc_material>(), g->width, g->height, cam.x, cam.y, cam.z,
-                               p->clusterRefinementThreshold, p->stackSize, p->writeSentinel, rad, counters);
+            ARC_TRY(arc::ensure(ctx, g->crec, sizeof(float4) * ((kSaLeaf + kSaNode) * (size_t)t.n)));
+            float4* rec = g->crec.as<float4>();
+            hipLaunchKernelGGL(k_sa_records, dim3(blocks(2LL * t.n - 1)), dim3(kThreads), 0, ctx->stream, t,
+                               g->mats.as<arc_material>(), sa_band(p->clusterRefinementThreshold), rec);
+            const dim3 grid(((g->width + 15) / 16) * ((g->height + 15) / 16));
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, ctx->stream, t, rec, g->gpos, g->gnrm, g->galb,
+                                   g->mats.as<arc_material>(), g->width, g->height, cam.x, cam.y, cam.z,
+                                   p->clusterRefinementThreshold, p->stackSize, p->writeSentinel, rad, counters);
+            };
+            if (g->general) launch(k_cut_sa<true>);
+            else launch(k_cut_sa<false>);
         }
         ARC_LAUNCHED(ctx);
         if (profile) ARC_HIP(ctx, hipEventRecord(ev[3], ctx->stream));

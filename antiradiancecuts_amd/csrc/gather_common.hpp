@@ -87,7 +87,7 @@ struct arc_gather {
     // clustered antiradiance: compacted AVPL indices (+ block offsets and
     // count), cluster boxes, list lengths and lists
     arc::DevBuf anti_idx, cbox, ccount, clist;
-    arc::DevBuf crec;  // error-bound cut: packed node records
+    arc::DevBuf crec;  // error-bound cut: packed node records; solid-angle cut: its records
     arc::DevBuf cest;  // error-bound cut: per-pixel estimates and their sum
     // moment estimator: per-internal-node records, and the FP64 prefix sums
     // over the sorted leaves (with per-block offsets) they are made from
@@ -169,6 +169,22 @@ struct Kahan {
 
 __device__ inline f3 f3of(float4 v) { return f3{v.x, v.y, v.z}; }
 
+
+// Wave-uniform record reads (the nodes' boxes and moment records, one
+// address for the whole wave) go through the constant address space in the
+// device pass: a uniform load from it is a scalar load (one request for the
+// wave, the values in scalar registers) whatever the compiler can prove
+// about aliasing stores.  The reads are of scalars, so no vector type's
+// constructor meets the address space.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define ARC_UNIFORM_AS __attribute__((address_space(4)))
+#else
+#define ARC_UNIFORM_AS
+#endif
+using ufloat = const ARC_UNIFORM_AS float;
+using uint_ = const ARC_UNIFORM_AS int;
+__device__ inline ufloat* uptr(const void* p) { return (ufloat*)p; }
+__device__ inline float4 uload4(ufloat* p) { return make_float4(p[0], p[1], p[2], p[3]); }
 
 // ----------------------------------------------------------- pixels ----
 struct PixelF {
