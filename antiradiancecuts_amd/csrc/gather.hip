@@ -6,17 +6,18 @@
 //                 unit normal, raw and unit incident direction, radiance with
 //                 the AVPL-side Lambertian BRDF folded in, antiradiance with
 //                 the disk normalisation 1/(pi r^2) folded in.
-//   k_exact       exact gather (kernel_radiance_simple :269-314 and
-//                 kernel_antiradiance :446-557 fused): one pixel per lane,
-//                 AVPL records read with wave-uniform (scalar) loads, runs of
-//                 64 pairs summed in FP32 and added to the pixel total with
-//                 Kahan compensation; optional split over AVPL ranges.
+//   k_exact_*     exact gather (kernel_radiance_simple :269-314 and
+//                 kernel_antiradiance :446-557 fused), Lambertian (two pixels
+//                 per lane) and with specular lobes: 64 records at a time in
+//                 LDS, runs summed in FP32 and added to the pixel total with
+//                 Kahan compensation; split over AVPL ranges.
 //   k_exact_f64   the same sums in FP64 with the reference's formulas (the
 //                 reference image for error metrics).
 //   k_finalize    sums the splits (Kahan), writes radiance, antiradiance and
 //                 result = radiance - antiradiance (kernel_combine :782-803).
 //   k_cut_sa      light-cut radiance with the solid-angle criterion
-//                 (kernel_bvh :316-444): per-pixel DFS, stack in LDS.
+//                 (kernel_bvh :316-444): an 8x8 tile's pixels walk the tree
+//                 together.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -61,84 +62,360 @@ __global__ __launch_bounds__(kThreads) void k_pack(arc::AvplsDev a, const arc_ma
 
 // ------------------------------------------------------------ exact ----
 // part layout: [split][6][npix] = radiance rgb, antiradiance rgb.
-template <int MODEL, bool GENERAL, bool DO_RAD, bool DO_ANTI>
-__global__ __launch_bounds__(kThreads) void k_exact(const float4* __restrict__ rec, arc::AvplsDev raw, int chunk,
-                                                    const float4* __restrict__ gpos,
-                                                    const float4* __restrict__ gnrm,
-                                                    const float4* __restrict__ galb,
-                                                    const arc_material* __restrict__ mats, int npix,
-                                                    float camx, float camy, float camz, AntiParams ap,
-                                                    float* __restrict__ part) {
-    const int pix = blockIdx.x * kThreads + threadIdx.x;
-    const bool live = pix < npix;
-    const int q = live ? pix : 0;
+
+// c^e for finite c >= 0 and e > 0, rounded once: log2 by the atanh series of
+// (m - 1) / (m + 1) and 2^x by its Taylor series, in double (their errors are
+// 1e-10 and 5e-9 relative), which issues at half the single rate: powf, which
+// carries its logarithm in pairs of floats, takes about twice as long.
+__device__ inline float pow_pos(float c, float e) {
+    float m = __builtin_amdgcn_frexp_mantf(c);
+    int k = __builtin_amdgcn_frexp_expf(c);
+    if (m < 0.70710678f) {
+        m += m;
+        --k;
+    }
+    const double den = (double)m + 1.0;
+    double r = (double)__builtin_amdgcn_rcpf((float)den);
+    r = __builtin_fma(r, __builtin_fma(-den, r, 1.0), r);
+    const double f = (double)(m - 1.0f) * r, s = f * f;
+    double p = 1.0 / 11.0;
+    p = __builtin_fma(p, s, 1.0 / 9.0);
+    p = __builtin_fma(p, s, 1.0 / 7.0);
+    p = __builtin_fma(p, s, 1.0 / 5.0);
+    p = __builtin_fma(p, s, 1.0 / 3.0);
+    p = __builtin_fma(p, s, 1.0);
+    const double log2 = __builtin_fma(f * p, 2.0 / M_LN2, (double)k);
+    const double y = fmin(fmax((double)e * log2, -200.0), 200.0);  // beyond: 0 and infinity in float
+    const double n = rint(y), x = (y - n) * M_LN2;
+    double q = 1.0 / 5040.0;
+    q = __builtin_fma(q, x, 1.0 / 720.0);
+    q = __builtin_fma(q, x, 1.0 / 120.0);
+    q = __builtin_fma(q, x, 1.0 / 24.0);
+    q = __builtin_fma(q, x, 1.0 / 6.0);
+    q = __builtin_fma(q, x, 0.5);
+    q = __builtin_fma(q, x, 1.0);
+    q = __builtin_fma(q, x, 1.0);
+    return c == 0.f ? 0.f : (float)ldexp(q, (int)n);
+}
+
+// A lobe's value: powf where pow_pos does not hold.
+__device__ inline float lobe(float c, float e, bool odd) { return odd ? powf(c, e) : pow_pos(c, e); }
+__device__ inline bool odd_lobe(float e, float x, float y, float z) {
+    return !(e > 0.f && e < 1e5f && fabsf(x) + fabsf(y) + fabsf(z) < 1e15f);
+}
+
+// Materials with specular lobes: a wave stages 64 AVPLs at a time in LDS with
+// the mirrored incident direction and the two factors of its material, so that
+// a pair's BRDFs (cudaGather.cu:59-68) are a dot product and a power each, and
+// the powers are left out for AVPLs without a lobe (a branch of the wave) and
+// for waves without a pixel that has one.  The pixel's lobe max(0, reflect(-wi,
+// n) . wo) is max(0, wi . m) with m = 2 n (n . wo) - wo, one vector per pixel;
+// both mirrored vectors are made in double, since their rounding would be in
+// every pair alike, times the exponent.
+//
+// Bound: vector instructions, half of them the powers.  331x247 pixels, 3001
+// AVPLs, every other material glossy: 1.97 ms with the BRDFs written out and
+// powf, 0.68 here.
+constexpr int kPlain = 32;  // pairs summed plainly before a compensated add
+
+struct GlossyLds {
+    float4 a[64], b[64];  // position, normal.x; normal.yz, radiance x diffuse / pi .rg
+    float4 c[64], d[64];  // .b, radiance x lobe factor; mirrored direction, exponent
+};
+
+template <int MODEL, bool DO_RAD, bool DO_ANTI>
+__global__ __launch_bounds__(kThreads) void k_exact_glossy(const float4* __restrict__ rec, arc::AvplsDev raw, int chunk,
+                                                           const float4* __restrict__ gpos,
+                                                           const float4* __restrict__ gnrm,
+                                                           const float4* __restrict__ galb,
+                                                           const arc_material* __restrict__ mats, int npix,
+                                                           float camx, float camy, float camz, AntiParams ap,
+                                                           float* __restrict__ part) {
+    using V3 = V<float>;
+    __shared__ GlossyLds lds[kThreads / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    GlossyLds& S = lds[wave];
+    const int first = (blockIdx.x * (kThreads / 64) + wave) * 64;
+    if (first >= npix) return;
+    const int q = first + lane < npix ? first + lane : 0;
     const PixelF P = load_pixel(gpos, gnrm, galb, mats, q);
-    const int n_avpl = raw.n;
-    const int a0 = blockIdx.y * chunk;
-    const int a1 = min(n_avpl, a0 + chunk);
+    // the pixel's lobe
+    const Mat<float> pm = material<float>(mats, P.mat);
+    const bool pglossy = length(pm.specular) > 0.f;
+    V3 mirror;
+    {
+        const float4 p4 = gpos[q], n4 = gnrm[q];
+        const V<double> n = mk<double>(n4.x, n4.y, n4.z);
+        const V<double> wo = normalize(mk<double>(camx, camy, camz) - mk<double>(p4.x, p4.y, p4.z));
+        const V<double> m = 2.0 * n * dot(n, wo) - wo;
+        mirror = mk((float)m.x, (float)m.y, (float)m.z);
+    }
+    const V3 pspec = (0.5f * kOneOverPi * (pm.exponent + 2.f)) * pm.specular;
+    const bool any_glossy = __ballot(pglossy) != 0;
+    const bool podd = __ballot(pglossy && odd_lobe(pm.exponent, mirror.x, mirror.y, mirror.z)) != 0;
+    auto pixel_brdf = [&](float cm) {  // cm = wi . mirror
+        V3 b = mk(P.br, P.bg, P.bb);
+        if (any_glossy) {
+            const float l = lobe(fmaxf(0.f, cm), pm.exponent, podd);
+            if (pglossy) b = b + l * pspec;
+        }
+        return b;
+    };
+    const int a0 = blockIdx.y * chunk, a1 = min(raw.n, a0 + chunk);
     Kahan kr[3], ka[3];
-    for (int base = a0; base < a1; base += kRun) {
-        const int end = min(a1, base + kRun);
-        float sr0 = 0.f, sr1 = 0.f, sr2 = 0.f, sa0 = 0.f, sa1 = 0.f, sa2 = 0.f;
-#pragma unroll 2
-        for (int i = base; i < end; ++i) {
-            const float4* r = rec + (size_t)kRecF4 * i;
-            const float4 r0 = r[0], r1 = r[1], r2v = r[2], r3 = r[3], r4 = r[4];
-            // d = a - p, from pixel to AVPL
-            const float dx = r0.x - P.px, dy = r0.y - P.py, dz = r0.z - P.pz;
-            const float dd = dx * dx + dy * dy + dz * dz;
-            const float inv = rsq(dd);
-            const float cn = P.nx * dx + P.ny * dy + P.nz * dz;        // |d| cos at the pixel
-            const float ca = -(r1.x * dx + r1.y * dy + r1.z * dz);     // |d| cos at the AVPL
-            // antiradiance decision and weight
-            const float m =
-                DO_ANTI ? anti_weight<MODEL>(P, r0, r1, r2v, r4.w, dx, dy, dz, dd, inv, cn, ca, ap, gpos, gnrm, q, raw, i)
-                        : 0.f;
-            if (GENERAL) {
-                using V3 = V<float>;
-                const V3 pos = mk(P.px, P.py, P.pz), nrm = mk(P.nx, P.ny, P.nz);
-                const V3 apos = mk(r0.x, r0.y, r0.z), anrm = mk(r1.x, r1.y, r1.z);
-                const V3 aw = mk(r2v.x, r2v.y, r2v.z);
-                const V3 cam = mk(camx, camy, camz);
-                Mat<float> pm = material<float>(mats, P.mat);
-                if (galb) pm.diffuse = mk(P.br / kOneOverPi, P.bg / kOneOverPi, P.bb / kOneOverPi);
-                if (DO_RAD) {
-                    const Mat<float> am = material<float>(mats, (int)r3.w);
-                    const V3 v = radiance(pos, nrm, pm, apos, anrm, aw, mk(r3.x, r3.y, r3.z), am, cam);
-                    sr0 += v.x; sr1 += v.y; sr2 += v.z;
+    for (int base = a0; base < a1; base += 64) {
+        const int cnt = min(64, a1 - base);
+        const int mine = lane < cnt ? base + lane : base;
+        const float4* r = rec + (size_t)kRecF4 * mine;
+        const float4 r4 = r[4];
+        uint64_t has_anti = 0;
+        if (DO_ANTI) has_anti = __ballot(lane < cnt && !(r4.x == 0.f && r4.y == 0.f && r4.z == 0.f));
+        if (DO_RAD) {
+            const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+            const Mat<float> am = material<float>(mats, (int)r3.w);
+            const V3 w = mk(r2.x, r2.y, r2.z), L = mk(r3.x, r3.y, r3.z), an = mk(r1.x, r1.y, r1.z);
+            const bool flat = length(w) == 0.f;  // no incident direction: a reflectance of 1
+            const bool glossy = !flat && length(am.specular) > 0.f;
+            const V<double> rd = reflect(ld3<double>(raw.dir[mine]), ld3<double>(raw.nrm[mine]));
+            const V3 refl = mk((float)rd.x, (float)rd.y, (float)rd.z);
+            const V3 ld = flat ? L : L * (kOneOverPi * am.diffuse);
+            const V3 ls = L * ((0.5f * kOneOverPi * (am.exponent + 2.f)) * am.specular);
+            const uint64_t gm = __ballot(glossy);
+            const uint64_t om = __ballot(glossy && odd_lobe(am.exponent, refl.x, refl.y, refl.z));
+            __builtin_amdgcn_wave_barrier();  // the last run's reads come first
+            S.a[lane] = make_float4(r0.x, r0.y, r0.z, an.x);
+            S.b[lane] = make_float4(an.y, an.z, ld.x, ld.y);
+            S.c[lane] = make_float4(ld.z, ls.x, ls.y, ls.z);
+            S.d[lane] = make_float4(refl.x, refl.y, refl.z, am.exponent);
+            __builtin_amdgcn_wave_barrier();  // before the reads of other lanes' writes
+            for (int from = 0; from < cnt; from += kPlain) {
+                float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+                for (int j = from; j < min(cnt, from + kPlain); ++j) {
+                    const float4 a = S.a[j], b = S.b[j], c = S.c[j];
+                    const float dx = a.x - P.px, dy = a.y - P.py, dz = a.z - P.pz;
+                    const float dd = dx * dx + dy * dy + dz * dz, inv = __builtin_amdgcn_rsqf(dd);
+                    const float c1 = clamp01((P.nx * dx + P.ny * dy + P.nz * dz) * inv);
+                    const float c2 = clamp01(-(a.w * dx + b.x * dy + b.y * dz) * inv);
+                    const float gg = c1 * c2 * __builtin_amdgcn_rcpf(dd);
+                    if (!__ballot(!(gg == 0.f))) continue;  // no pixel of the wave sees it
+                    V3 l = mk(b.z, b.w, c.x);
+                    if (gm >> j & 1) {
+                        const float4 d = S.d[j];
+                        const float p = lobe(fmaxf(0.f, -(d.x * dx + d.y * dy + d.z * dz) * inv), d.w, (om >> j & 1) != 0);
+                        l.x += c.y * p;
+                        l.y += c.z * p;
+                        l.z += c.w * p;
+                    }
+                    const V3 f = pixel_brdf((mirror.x * dx + mirror.y * dy + mirror.z * dz) * inv);
+                    s0 += l.x * f.x * gg;
+                    s1 += l.y * f.y * gg;
+                    s2 += l.z * f.z * gg;
                 }
-                if (DO_ANTI && m != 0.f) {
-                    // record holds A / (pi r^2) (disk) or A (cone); the pixel BRDF varies per pair
-                    const V3 b = f_r3(apos, pos, cam, nrm, pm) * m;
-                    sa0 += r4.x * b.x; sa1 += r4.y * b.y; sa2 += r4.z * b.z;
-                }
-            } else {
-                if (DO_RAD) {
-                    const float c1 = fminf(fmaxf(cn * inv, 0.f), 1.f);
-                    const float c2 = fminf(fmaxf(ca * inv, 0.f), 1.f);
-                    const float gg = c1 * c2 * (inv * inv);
-                    sr0 += r3.x * gg; sr1 += r3.y * gg; sr2 += r3.z * gg;
-                }
-                if (DO_ANTI) { sa0 += r4.x * m; sa1 += r4.y * m; sa2 += r4.z * m; }
+                kr[0].add(s0);
+                kr[1].add(s1);
+                kr[2].add(s2);
             }
         }
-        if (DO_RAD) { kr[0].add(sr0); kr[1].add(sr1); kr[2].add(sr2); }
-        if (DO_ANTI) { ka[0].add(sa0); ka[1].add(sa1); ka[2].add(sa2); }
+        if (DO_ANTI && has_anti) {
+            float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+            for (uint64_t m = has_anti; m; m &= m - 1) {
+                const int i = base + __builtin_ctzll(m);
+                const float4* r = rec + (size_t)kRecF4 * i;
+                const float4 r0 = r[0], r1 = r[1], r2 = r[2], A = r[4];
+                const float dx = r0.x - P.px, dy = r0.y - P.py, dz = r0.z - P.pz;
+                const float dd = dx * dx + dy * dy + dz * dz;
+                const float inv = rsq(dd);
+                const float cn = P.nx * dx + P.ny * dy + P.nz * dz;
+                const float ca = -(r1.x * dx + r1.y * dy + r1.z * dz);
+                const float wgt = anti_weight<MODEL>(P, r0, r1, r2, A.w, dx, dy, dz, dd, inv, cn, ca, ap, gpos, gnrm, q, raw, i);
+                if (!__ballot(wgt != 0.f)) continue;
+                const V3 f = pixel_brdf((mirror.x * dx + mirror.y * dy + mirror.z * dz) * inv);
+                if (wgt != 0.f) {
+                    s0 += A.x * (f.x * wgt);
+                    s1 += A.y * (f.y * wgt);
+                    s2 += A.z * (f.z * wgt);
+                }
+            }
+            ka[0].add(s0);
+            ka[1].add(s1);
+            ka[2].add(s2);
+        }
     }
-    if (!live) return;
-    float* o = part + (size_t)blockIdx.y * 6 * npix + pix;
-    if (!GENERAL) {  // the Lambertian pixel BRDF is constant per pixel
+    if (first + lane >= npix) return;
+    float* o = part + (size_t)blockIdx.y * 6 * npix + first + lane;
+    if (DO_RAD) { o[0] = kr[0].s; o[(size_t)npix] = kr[1].s; o[2 * (size_t)npix] = kr[2].s; }
+    if (DO_ANTI) { o[3 * (size_t)npix] = ka[0].s; o[4 * (size_t)npix] = ka[1].s; o[5 * (size_t)npix] = ka[2].s; }
+}
+
+// Lambertian materials: the BRDFs are factors of the record and of the pixel.
+//
+// A lane sums two pixels.  Each wave stages 64 AVPLs at a time in LDS, those
+// with antiradiance in a list of their own, so that the others (two thirds of
+// a scene's AVPLs: a path's antiradiance leaves only where it is blocked) pay
+// nothing for it, and reads a record for both pixels as vector operands: an
+// instruction with a scalar operand issues at half the rate, and read by scalar
+// loads the records made every first operation on them one.  A wave needs no
+// other wave's lists: no barrier.
+//
+// Bound: vector instructions, 20 per pair for the radiance and 25 (cone) per
+// pair with antiradiance.  256x256 pixels, 4096 AVPLs, cone: 387 us with a
+// pixel per lane and scalar loads, 160 here; one pixel per lane 170.
+constexpr int kExactSlots = 2;
+
+template <int MODEL>
+struct ExactLds {
+    float4 a[64], b[64];                  // position and normal.x; normal.yz, radiance.rg
+    float c[64];                          // radiance.b
+    float4 u[64], v[64], w[MODEL == ARC_ANTIRAD_DISK ? 64 : 1];
+    float4 A[64];                         // antiradiance, guard of |w . n|
+    int i[64];
+};
+
+template <int MODEL, bool DO_RAD, bool DO_ANTI>
+__global__ __launch_bounds__(kThreads) void k_exact_lambert(const float4* __restrict__ rec, arc::AvplsDev raw, int chunk,
+                                                            const float4* __restrict__ gpos,
+                                                            const float4* __restrict__ gnrm,
+                                                            const float4* __restrict__ galb,
+                                                            const arc_material* __restrict__ mats, int npix,
+                                                            AntiParams ap, float* __restrict__ part) {
+    __shared__ ExactLds<MODEL> lds[kThreads / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    ExactLds<MODEL>& S = lds[wave];
+    const int first = (blockIdx.x * (kThreads / 64) + wave) * 64 * kExactSlots;
+    if (first >= npix) return;
+    PixelF P[kExactSlots];
+    int q[kExactSlots];
+#pragma unroll
+    for (int s = 0; s < kExactSlots; ++s) {
+        q[s] = first + 64 * s + lane < npix ? first + 64 * s + lane : 0;
+        P[s] = load_pixel(gpos, gnrm, galb, mats, q[s]);
+        // a pixel without a normal accepts no pair of the cone model
+        if (MODEL == ARC_ANTIRAD_CONE && !(P[s].nx == P[s].nx && P[s].ny == P[s].ny && P[s].nz == P[s].nz))
+            P[s].nx = P[s].ny = P[s].nz = 0.f;
+    }
+    const float edge = fmaxf(kConeEps, ap.cos_half);  // c above both
+    const int a0 = blockIdx.y * chunk, a1 = min(raw.n, a0 + chunk);
+    Kahan kr[kExactSlots][3], ka[kExactSlots][3];
+    for (int base = a0; base < a1; base += 64) {
+        const int cnt = min(64, a1 - base);
+        int na = 0;
+        {
+            const bool in = lane < cnt;
+            const float4* r = rec + (size_t)kRecF4 * (in ? base + lane : base);
+            const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4];
+            __builtin_amdgcn_wave_barrier();  // the last run's reads come first
+            if (DO_RAD) {
+                S.a[lane] = make_float4(r0.x, r0.y, r0.z, r1.x);
+                S.b[lane] = make_float4(r1.y, r1.z, r3.x, r3.y);
+                S.c[lane] = r3.z;
+            }
+            if (DO_ANTI) {
+                const bool has = in && !(r4.x == 0.f && r4.y == 0.f && r4.z == 0.f);
+                const uint64_t m = __ballot(has);
+                if (has) {
+                    const int k = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    // a direction that is no number accepts no pair
+                    const bool num = r0.w == r0.w && r1.w == r1.w && r2.w == r2.w;
+                    S.u[k] = make_float4(r0.x, r0.y, r0.z, num || MODEL == ARC_ANTIRAD_DISK ? r0.w : 0.f);
+                    if (MODEL == ARC_ANTIRAD_DISK) {
+                        S.v[k] = make_float4(r1.x, r1.y, r1.z, r1.w);
+                        S.w[k] = make_float4(r2.x, r2.y, r2.z, r2.w);
+                        S.A[k] = r4;
+                    } else {
+                        S.v[k] = make_float4(num ? r1.w : 0.f, num ? r2.w : 0.f, r4.x, r4.y);
+                        S.A[k].x = r4.z;
+                    }
+                    S.i[k] = base + lane;
+                }
+                na = __popcll(m);
+            }
+            __builtin_amdgcn_wave_barrier();  // before the reads of other lanes' writes
+        }
         if (DO_RAD) {
-            o[0] = kr[0].s * P.br; o[(size_t)npix] = kr[1].s * P.bg; o[2 * (size_t)npix] = kr[2].s * P.bb;
+            for (int from = 0; from < cnt; from += kPlain) {
+                float sum[kExactSlots][3] = {};
+#pragma unroll 2
+                for (int j = from; j < min(cnt, from + kPlain); ++j) {
+                    const float4 a = S.a[j], b = S.b[j];
+                    const float lz = S.c[j];
+#pragma unroll
+                    for (int s = 0; s < kExactSlots; ++s) {
+                        const float dx = a.x - P[s].px, dy = a.y - P[s].py, dz = a.z - P[s].pz;
+                        const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
+                        const float cn = P[s].nx * dx + P[s].ny * dy + P[s].nz * dz;
+                        const float ca = -(a.w * dx + b.x * dy + b.y * dz);
+                        const float c1 = fminf(fmaxf(cn * inv, 0.f), 1.f), c2 = fminf(fmaxf(ca * inv, 0.f), 1.f);
+                        const float gg = c1 * c2 * (inv * inv);
+                        sum[s][0] += b.z * gg;
+                        sum[s][1] += b.w * gg;
+                        sum[s][2] += lz * gg;
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < kExactSlots; ++s)
+                    for (int c = 0; c < 3; ++c) kr[s][c].add(sum[s][c]);
+            }
         }
-        if (DO_ANTI) {
-            o[3 * (size_t)npix] = ka[0].s * P.br; o[4 * (size_t)npix] = ka[1].s * P.bg;
-            o[5 * (size_t)npix] = ka[2].s * P.bb;
+        if (DO_ANTI && na > 0) {
+            float sum[kExactSlots][3] = {};
+            for (int j = 0; j < na; ++j) {
+                const float4 u = S.u[j], v = S.v[j];
+                if constexpr (MODEL == ARC_ANTIRAD_DISK) {
+                    const float4 w = S.w[j], A = S.A[j];
+                    bool may = false;  // some pixel faces the AVPL's direction
+#pragma unroll
+                    for (int s = 0; s < kExactSlots; ++s)
+                        may = may || w.x * P[s].nx + w.y * P[s].ny + w.z * P[s].nz < A.w;
+                    if (!__ballot(may)) continue;
+#pragma unroll
+                    for (int s = 0; s < kExactSlots; ++s) {
+                        const float dx = u.x - P[s].px, dy = u.y - P[s].py, dz = u.z - P[s].pz;
+                        const float dd = dx * dx + dy * dy + dz * dz;
+                        const float inv = __builtin_amdgcn_rsqf(dd);
+                        const float cn = P[s].nx * dx + P[s].ny * dy + P[s].nz * dz;
+                        const float ca = -(v.x * dx + v.y * dy + v.z * dz);
+                        const float m = anti_weight<MODEL>(P[s], u, v, w, A.w, dx, dy, dz, dd, inv, cn, ca, ap, gpos, gnrm,
+                                                           q[s], raw, S.i[j]);
+                        sum[s][0] += A.x * m;
+                        sum[s][1] += A.y * m;
+                        sum[s][2] += A.z * m;
+                    }
+                } else {
+                    const float az = S.A[j].x;
+#pragma unroll
+                    for (int s = 0; s < kExactSlots; ++s) {
+                        const float dx = u.x - P[s].px, dy = u.y - P[s].py, dz = u.z - P[s].pz;
+                        const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
+                        const float cn = P[s].nx * dx + P[s].ny * dy + P[s].nz * dz;
+                        const float cw = u.w * dx + v.x * dy + v.y * dz;
+                        const float cp = cn * inv;
+                        // the smaller distance from the thresholds decides, in FP64 inside the guard band
+                        const float least = fminf(-(cw * inv) - edge, cp - kConeEps);
+                        bool in = least > 0.f;
+                        if (fabsf(least) <= kGuard)
+                            in = cone_accept_f64(gpos[q[s]], gnrm[q[s]], raw.pos[S.i[j]], raw.dir[S.i[j]], ap.cos_half_d);
+                        const float m = in ? cp * (inv * inv) : 0.f;
+                        sum[s][0] += v.z * m;
+                        sum[s][1] += v.w * m;
+                        sum[s][2] += az * m;
+                    }
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < kExactSlots; ++s)
+                for (int c = 0; c < 3; ++c) ka[s][c].add(sum[s][c]);
         }
-    } else {
-        if (DO_RAD) { o[0] = kr[0].s; o[(size_t)npix] = kr[1].s; o[2 * (size_t)npix] = kr[2].s; }
-        if (DO_ANTI) {
-            o[3 * (size_t)npix] = ka[0].s; o[4 * (size_t)npix] = ka[1].s; o[5 * (size_t)npix] = ka[2].s;
+    }
+#pragma unroll
+    for (int s = 0; s < kExactSlots; ++s) {
+        const int pix = first + 64 * s + lane;
+        if (pix >= npix) continue;
+        float* o = part + (size_t)blockIdx.y * 6 * npix + pix;
+        const float b[3] = {P[s].br, P[s].bg, P[s].bb};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (DO_RAD) o[c * (size_t)npix] = kr[s][c].s * b[c];
+            if (DO_ANTI) o[(3 + c) * (size_t)npix] = ka[s][c].s * b[c];
         }
     }
 }
@@ -147,20 +424,33 @@ __global__ __launch_bounds__(kThreads) void k_exact(const float4* __restrict__ r
 // result = radiance - antiradiance including w, i.e. 1 - 1 = 0).
 // Radiance comes from rad_splits splits of `part`, or from rad_in when
 // rad_splits < 0 (the cut kernel wrote it); antiradiance from anti_splits
-// splits (0: none).
+// splits (0: none).  A pixel's splits are summed by kSlices threads: one chain
+// of 313 (48x32 pixels, 5000 AVPLs) took 180 us.
+template <int kSlices>
 __global__ __launch_bounds__(kThreads) void k_finalize(const float* __restrict__ part, int rad_splits,
                                                        int anti_splits, int npix,
                                                        const float4* __restrict__ rad_in,
                                                        float4* __restrict__ out_rad,
                                                        float4* __restrict__ out_anti,
                                                        float4* __restrict__ out_res) {
-    const int pix = blockIdx.x * kThreads + threadIdx.x;
-    if (pix >= npix) return;
+    constexpr int kPix = kThreads / kSlices;
+    const int pix = blockIdx.x * kPix + threadIdx.x % kPix, slice = threadIdx.x / kPix;
     Kahan k[6];
-    for (int s = 0; s < rad_splits; ++s)
-        for (int c = 0; c < 3; ++c) k[c].add(part[((size_t)s * 6 + c) * npix + pix]);
-    for (int s = 0; s < anti_splits; ++s)
-        for (int c = 3; c < 6; ++c) k[c].add(part[((size_t)s * 6 + c) * npix + pix]);
+    if (pix < npix) {
+        for (int s = slice; s < rad_splits; s += kSlices)
+            for (int c = 0; c < 3; ++c) k[c].add(part[((size_t)s * 6 + c) * npix + pix]);
+        for (int s = slice; s < anti_splits; s += kSlices)
+            for (int c = 3; c < 6; ++c) k[c].add(part[((size_t)s * 6 + c) * npix + pix]);
+    }
+    if constexpr (kSlices > 1) {
+        __shared__ float sum[kSlices][6][kPix];
+        for (int c = 0; c < 6; ++c) sum[slice][c][threadIdx.x % kPix] = k[c].s;
+        __syncthreads();
+        if (slice > 0) return;
+        for (int s = 1; s < kSlices; ++s)
+            for (int c = 0; c < 6; ++c) k[c].add(sum[s][c][threadIdx.x]);
+    }
+    if (pix >= npix) return;
     const float4 rad = rad_splits >= 0 ? make_float4(k[0].s, k[1].s, k[2].s, 1.f) : rad_in[pix];
     const float4 anti = make_float4(k[3].s, k[4].s, k[5].s, 1.f);
     if (rad_splits >= 0 && out_rad) out_rad[pix] = rad;
@@ -488,26 +778,48 @@ int pick_splits(int npix, int n_avpl) {
     return s;
 }
 
-template <int MODEL, bool GENERAL, bool DO_RAD, bool DO_ANTI>
+// The exact kernels' waves cost alike, so their number should fill the chip
+// (two to three blocks of each CU's four are resident) and no more, each split
+// being written and read once; a split of less than 32 AVPLs costs more to
+// start than it saves.  At least 256 per split left a 64x48 image with 500
+// AVPLs at 24 blocks, 138 us; 18 us here.
+int exact_splits(const arc_gather* g, int npix, int n_avpl) {
+    const int per = g->general ? kThreads : kThreads * kExactSlots, pblocks = (npix + per - 1) / per;
+    return std::max(1, std::min(2048 / pblocks, (n_avpl + 31) / 32));
+}
+
+template <int MODEL, bool DO_RAD, bool DO_ANTI>
 void launch_exact(arc_gather* g, const arc::AvplsDev& a, int chunk, int splits, float3 cam, float radius,
                   double cos_half) {
     const int npix = g->width * g->height;
-    hipLaunchKernelGGL((k_exact<MODEL, GENERAL, DO_RAD, DO_ANTI>), dim3(blocks(npix), splits), dim3(kThreads), 0,
-                       g->ctx->stream, g->rec.as<float4>(), a, chunk, g->gpos, g->gnrm, g->galb,
-                       g->mats.as<arc_material>(), npix, cam.x, cam.y, cam.z, anti_params(radius, cos_half),
-                       g->part.as<float>());
+    if (g->general)
+        hipLaunchKernelGGL((k_exact_glossy<MODEL, DO_RAD, DO_ANTI>), dim3(blocks(npix), splits), dim3(kThreads), 0,
+                           g->ctx->stream, g->rec.as<float4>(), a, chunk, g->gpos, g->gnrm, g->galb,
+                           g->mats.as<arc_material>(), npix, cam.x, cam.y, cam.z, anti_params(radius, cos_half),
+                           g->part.as<float>());
+    else
+        hipLaunchKernelGGL((k_exact_lambert<MODEL, DO_RAD, DO_ANTI>),
+                           dim3((npix + kThreads * kExactSlots - 1) / (kThreads * kExactSlots), splits), dim3(kThreads),
+                           0, g->ctx->stream, g->rec.as<float4>(), a, chunk, g->gpos, g->gnrm, g->galb,
+                           g->mats.as<arc_material>(), npix, anti_params(radius, cos_half), g->part.as<float>());
 }
 
 template <bool DO_RAD, bool DO_ANTI>
 void dispatch_exact(arc_gather* g, int model, const arc::AvplsDev& a, int chunk, int splits, float3 cam,
                     float radius, double cos_half) {
-    if (model == ARC_ANTIRAD_DISK) {
-        if (g->general) launch_exact<ARC_ANTIRAD_DISK, true, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
-        else launch_exact<ARC_ANTIRAD_DISK, false, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
-    } else {
-        if (g->general) launch_exact<ARC_ANTIRAD_CONE, true, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
-        else launch_exact<ARC_ANTIRAD_CONE, false, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
-    }
+    if (model == ARC_ANTIRAD_DISK) launch_exact<ARC_ANTIRAD_DISK, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
+    else launch_exact<ARC_ANTIRAD_CONE, DO_RAD, DO_ANTI>(g, a, chunk, splits, cam, radius, cos_half);
+}
+
+// Eight threads per pixel where there are splits for them.
+void finalize(arc_gather* g, int rad_splits, int anti_splits, int npix, float4* rad, float4* anti, float4* res) {
+    auto launch = [&](auto kernel, int slices) {
+        const int per = kThreads / slices;
+        hipLaunchKernelGGL(kernel, dim3((npix + per - 1) / per), dim3(kThreads), 0, g->ctx->stream, g->part.as<float>(),
+                           rad_splits, anti_splits, npix, rad, rad, anti, res);
+    };
+    if (std::max(rad_splits, anti_splits) > 8) launch(k_finalize<8>, 8);
+    else launch(k_finalize<1>, 1);
 }
 
 // This frame's LBVH for the error-bound and learned cuts, with their node
@@ -762,7 +1074,7 @@ int arc_gather_run(arc_gather* g, const arc_avpls* avpls, arc_float3 camPos, flo
     }
     if (profile) ARC_HIP(ctx, hipEventRecord(ev[1], ctx->stream));
 
-    const int splits = pick_splits(npix, std::max(n, 1));
+    const int splits = exact_splits(g, npix, std::max(n, 1));
     const int chunk = (std::max(n, 1) + splits - 1) / splits;
     ARC_TRY(arc::ensure(ctx, g->part, sizeof(float) * 6 * (size_t)splits * npix));
     unsigned long long* counters = count ? g->counters.as<unsigned long long>() : nullptr;
@@ -907,8 +1219,7 @@ int arc_gather_run(arc_gather* g, const arc_avpls* avpls, arc_float3 camPos, flo
         return ARC_OK;
     }
     if (profile) ARC_HIP(ctx, hipEventRecord(ev[4], ctx->stream));
-    hipLaunchKernelGGL(k_finalize, dim3(blocks(npix)), dim3(kThreads), 0, ctx->stream, g->part.as<float>(),
-                       rad_splits, anti_splits, npix, rad, rad, anti, res);
+    finalize(g, rad_splits, anti_splits, npix, rad, anti, res);
     ARC_LAUNCHED(ctx);
     if (profile) ARC_HIP(ctx, hipEventRecord(ev[5], ctx->stream));
     if (stats) {
@@ -954,8 +1265,7 @@ int gather_finish(arc_gather* g) {
     if (!g || !g->deferred) return ARC_E_STATE;
     arc_ctx* ctx = g->ctx;
     const int npix = g->width * g->height;
-    hipLaunchKernelGGL(k_finalize, dim3(blocks(npix)), dim3(kThreads), 0, ctx->stream, g->part.as<float>(),
-                       g->def_rad_splits, g->def_anti_splits, npix, g->def_rad, g->def_rad, g->out_anti, g->out_res);
+    finalize(g, g->def_rad_splits, g->def_anti_splits, npix, g->def_rad, g->out_anti, g->out_res);
     ARC_LAUNCHED(ctx);
     g->deferred = false;
     return ARC_OK;
