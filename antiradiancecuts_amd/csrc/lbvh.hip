@@ -120,28 +120,30 @@ __device__ inline uint32_t interleave6_lo32(uint32_t a, uint32_t b, uint32_t c, 
     return (uint32_t)r;
 }
 
+__device__ inline uint32_t morton_code(const f3* __restrict__ pos, const f3* __restrict__ nrm, int i,
+                                       const float* __restrict__ bounds, int consider_normals) {
+    const f3 p = pos[i];
+    // Normalize functor (bvh.cu:73-81): component-wise IEEE division
+    const float x = (p.x - bounds[0]) / (bounds[3] - bounds[0]);
+    const float y = (p.y - bounds[1]) / (bounds[4] - bounds[1]);
+    const float z = (p.z - bounds[2]) / (bounds[5] - bounds[2]);
+    if (consider_normals) {
+        const f3 q = nrm[i];
+        const float u = (q.x - bounds[6]) / (bounds[9] - bounds[6]);
+        const float v = (q.y - bounds[7]) / (bounds[10] - bounds[7]);
+        const float w = (q.z - bounds[8]) / (bounds[11] - bounds[8]);
+        return interleave6_lo32(quant10(x), quant10(y), quant10(z), quant10(u), quant10(v), quant10(w));
+    }
+    return (expand2(quant10(z)) << 2) + (expand2(quant10(y)) << 1) + expand2(quant10(x));
+}
+
 __global__ __launch_bounds__(kBlock) void k_encode(const f3* __restrict__ pos, const f3* __restrict__ nrm,
                                                    int n, const float* __restrict__ bounds,
                                                    int consider_normals, uint32_t* __restrict__ keys,
                                                    int* __restrict__ vals) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const f3 p = pos[i];
-    // Normalize functor (bvh.cu:73-81): component-wise IEEE division
-    const float x = (p.x - bounds[0]) / (bounds[3] - bounds[0]);
-    const float y = (p.y - bounds[1]) / (bounds[4] - bounds[1]);
-    const float z = (p.z - bounds[2]) / (bounds[5] - bounds[2]);
-    uint32_t code;
-    if (consider_normals) {
-        const f3 q = nrm[i];
-        const float u = (q.x - bounds[6]) / (bounds[9] - bounds[6]);
-        const float v = (q.y - bounds[7]) / (bounds[10] - bounds[7]);
-        const float w = (q.z - bounds[8]) / (bounds[11] - bounds[8]);
-        code = interleave6_lo32(quant10(x), quant10(y), quant10(z), quant10(u), quant10(v), quant10(w));
-    } else {
-        code = (expand2(quant10(z)) << 2) + (expand2(quant10(y)) << 1) + expand2(quant10(x));
-    }
-    keys[i] = code;
+    keys[i] = morton_code(pos, nrm, i, bounds, consider_normals);
     vals[i] = i;
 }
 
@@ -254,31 +256,16 @@ __global__ __launch_bounds__(kBlock) void k_random(uint64_t seed, int count, flo
 }
 
 // ---------------------------------------------------------- Karras ----
-__global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ m, int num_nodes,
-                                                   arc_bvh_node* __restrict__ nodes,
-                                                   int* __restrict__ parents, int* __restrict__ ranges,
-                                                   int* __restrict__ nready) {
-    // The searches of most nodes stay within 128 slots of the node (the first
-    // l_max): the block's codes and 256 on each side are read once into LDS,
-    // and a probe outside that window reads global memory.
-    constexpr int kWin = 3 * kBlock;
-    __shared__ uint32_t win[kWin];
-    const int wbase = (int)(blockIdx.x * blockDim.x) - kBlock;
-    for (int k = threadIdx.x; k < kWin; k += blockDim.x) {
-        const int j = wbase + k;
-        win[k] = (j >= 0 && j <= num_nodes) ? m[j] : 0u;
-    }
-    __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) nready[0] = nready[1] = nready[2] = 0;  // the refits' list lengths
-    if (i >= num_nodes) return;             // no barrier follows
-    const uint32_t mi = win[i - wbase];
+// Node i's range, split and children; code(j): sorted code j, 0 <= j <= num_nodes.
+template <class Code>
+__device__ inline void karras_node(int i, int num_nodes, Code code, arc_bvh_node* __restrict__ nodes,
+                                   int* __restrict__ parents, int* __restrict__ ranges) {
+    const uint32_t mi = code(i);
     // delta(i, j) (bvh.cu:124-135): -1 outside [0, num_nodes]; on equal codes
     // the common prefix continues into the slot indices
     auto dl = [&](int j) -> int {
         if (j < 0 || j > num_nodes) return -1;
-        const int k = j - wbase;
-        const uint32_t x = mi ^ ((k >= 0 && k < kWin) ? win[k] : m[j]);
+        const uint32_t x = mi ^ code(j);
         return x ? __clz(x) : 32 + __clz((uint32_t)(i ^ j));
     };
     const int root_slot = num_nodes + 1;
@@ -314,6 +301,125 @@ __global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ 
     ranges[2 * i] = lo;
     ranges[2 * i + 1] = hi;
     if (i == 0) parents[root_slot] = -1;
+}
+
+__global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ m, int num_nodes,
+                                                   arc_bvh_node* __restrict__ nodes,
+                                                   int* __restrict__ parents, int* __restrict__ ranges,
+                                                   int* __restrict__ nready) {
+    // The searches of most nodes stay within 128 slots of the node (the first
+    // l_max): the block's codes and 256 on each side are read once into LDS,
+    // and a probe outside that window reads global memory.
+    constexpr int kWin = 3 * kBlock;
+    __shared__ uint32_t win[kWin];
+    const int wbase = (int)(blockIdx.x * blockDim.x) - kBlock;
+    for (int k = threadIdx.x; k < kWin; k += blockDim.x) {
+        const int j = wbase + k;
+        win[k] = (j >= 0 && j <= num_nodes) ? m[j] : 0u;
+    }
+    __syncthreads();
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) nready[0] = nready[1] = nready[2] = 0;  // the refits' list lengths
+    if (i >= num_nodes) return;             // no barrier follows
+    karras_node(i, num_nodes, [&](int j) {
+        const int k = j - wbase;
+        return (k >= 0 && k < kWin) ? win[k] : m[j];
+    }, nodes, parents, ranges);
+}
+
+// ------------------------------------------------------- small trees ----
+// Bounds, codes, sort, sorted points and Karras nodes of at most kSmallTree
+// points in one workgroup: what a small build spends is launches (17 of them, 55 us for 1000
+// points), not work.  The sort is bitonic over code << 32 | index in LDS, so
+// equal codes keep their input order as the radix sort's do; strides of up to
+// 64 stay inside a wave's 128 keys and need no barrier.  1000 points: 74 us, 25 here;
+// 4096: 94 and 69, and beyond it one CU takes as long as the launches.
+constexpr int kSmallTree = 4096, kSmallThreads = 1024;
+
+__global__ __launch_bounds__(kSmallThreads) void k_small_tree(const f3* __restrict__ pos, const f3* __restrict__ nrm,
+                                                              int n, int consider_normals, float* __restrict__ bounds,
+                                                              uint32_t* __restrict__ codes, int* __restrict__ perm,
+                                                              arc_bvh_node* __restrict__ nodes,
+                                                              int* __restrict__ parents, int* __restrict__ ranges,
+                                                              int* __restrict__ nready, f3* __restrict__ spos,
+                                                              f3* __restrict__ snrm) {
+    __shared__ uint64_t key[kSmallTree];
+    __shared__ float sbounds[12];
+    __shared__ float partial[kSmallThreads / 64][12];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    {
+        float v[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) v[k] = ((k / 3) & 1) ? FLT_MIN : FLT_MAX;  // as k_bounds_partial
+        for (int i = tid; i < n; i += kSmallThreads) {
+            const f3 p = pos[i];
+            v[0] = fminf(v[0], p.x); v[1] = fminf(v[1], p.y); v[2] = fminf(v[2], p.z);
+            v[3] = fmaxf(v[3], p.x); v[4] = fmaxf(v[4], p.y); v[5] = fmaxf(v[5], p.z);
+            if (nrm) {
+                const f3 q = nrm[i];
+                v[6] = fminf(v[6], q.x); v[7] = fminf(v[7], q.y); v[8] = fminf(v[8], q.z);
+                v[9] = fmaxf(v[9], q.x); v[10] = fmaxf(v[10], q.y); v[11] = fmaxf(v[11], q.z);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+            for (int off = 32; off > 0; off >>= 1) {
+                const float o = __shfl_xor(v[k], off);
+                v[k] = ((k / 3) & 1) ? fmaxf(v[k], o) : fminf(v[k], o);
+            }
+            if (lane == 0) partial[wave][k] = v[k];
+        }
+    }
+    __syncthreads();
+    if (tid < 12) {
+        float r = partial[0][tid];
+        for (int w = 1; w < kSmallThreads / 64; ++w)
+            r = ((tid / 3) & 1) ? fmaxf(r, partial[w][tid]) : fminf(r, partial[w][tid]);
+        sbounds[tid] = r;
+        bounds[tid] = r;
+    }
+    if (tid == 0) nready[0] = nready[1] = nready[2] = 0;
+    __syncthreads();
+    int size = 128;
+    while (size < n) size *= 2;
+    for (int i = tid; i < size; i += kSmallThreads)
+        key[i] = i < n ? (uint64_t)morton_code(pos, nrm, i, sbounds, consider_normals) << 32 | (uint32_t)i : ~0ull;
+    __syncthreads();
+    auto step = [&](int pair, int k, int j) {  // j a power of two
+        const int a = 2 * pair - (pair & (j - 1)), b = a + j;
+        const uint64_t x = key[a], y = key[b];
+        if ((x > y) == ((a & k) == 0)) {
+            key[a] = y;
+            key[b] = x;
+        }
+    };
+    const int pairs = size / 2;
+    for (int k = 2; k <= size; k *= 2) {
+        for (int j = k / 2; j > 64; j /= 2) {
+            for (int t = tid; t < pairs; t += kSmallThreads) step(t, k, j);
+            __syncthreads();
+        }
+        for (int t = tid; t < pairs; t += kSmallThreads) {  // whole waves: 64 pairs, 128 keys each
+            for (int j = min(k / 2, 64); j > 0; j /= 2) {
+                step(t, k, j);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        if (k >= 128) __syncthreads();  // the next stage may leave the wave's keys
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kSmallThreads) {
+        const uint64_t x = key[i];
+        codes[i] = (uint32_t)(x >> 32);
+        const int o = (int)(uint32_t)x;
+        perm[i] = o;
+        spos[i] = pos[o];
+        if (nrm) snrm[i] = nrm[o];
+    }
+    const uint32_t* half = reinterpret_cast<const uint32_t*>(key);
+    for (int i = tid; i < n - 1; i += kSmallThreads)
+        karras_node(i, n - 1, [&](int j) { return half[2 * j + 1]; }, nodes, parents, ranges);
 }
 
 // ----------------------------------------------------------- refit ----
@@ -787,6 +893,7 @@ void launch_range_boxes(arc_bvh* b, int n, In in, Out out, int* crossing, int* n
     f3* block_box = chunk_box + 2 * (((size_t)n + kChunk - 1) / kChunk);
     hipLaunchKernelGGL((k_refit_points_local<In, Out>), dim3(rblocks), dim3(kRefitLeaves), 0, b->ctx->stream, out,
                        b->ranges.as<int>(), in, n, chunk_box, block_box, crossing, ncross);
+    if (rblocks == 1) return;  // no node crosses blocks
     // about ten nodes per block cross blocks; a wave takes one at a time
     const int cblocks = std::max(1, std::min(1024, 2 * rblocks));
     hipLaunchKernelGGL((k_refit_points_crossing<In, Out>), dim3(cblocks), dim3(kCrossThreads), 0, b->ctx->stream,
@@ -815,11 +922,20 @@ int ensure_tree(arc_bvh* b, int n) {
     return ARC_OK;
 }
 
-// Bounds + encode + sort (Bvh::create up to sort(), bvh.cu:346-374).
+// Bounds + encode + sort (Bvh::create up to sort(), bvh.cu:346-374); for small
+// trees the sorted points and the Karras nodes too.
 int encode_and_sort(arc_bvh* b, const f3* pos, const f3* nrm, int n) {
     arc_ctx* ctx = b->ctx;
     const int nparts = std::min(kReduceBlocks, std::max(1, blocks_for(n)));
     float* bounds = b->bounds.as<float>();
+    if (n <= kSmallTree) {
+        hipLaunchKernelGGL(k_small_tree, dim3(1), dim3(kSmallThreads), 0, ctx->stream, pos, nrm, n,
+                           b->consider_normals && nrm ? 1 : 0, bounds, b->codes.as<uint32_t>(), b->perm.as<int>(),
+                           b->nodes.as<arc_bvh_node>(), b->parents.as<int>(), b->ranges.as<int>(),
+                           reinterpret_cast<int*>(bounds + 13), b->positions.as<f3>(), b->normals.as<f3>());
+        ARC_LAUNCHED(ctx);
+        return ARC_OK;
+    }
     hipLaunchKernelGGL(k_bounds_partial, dim3(nparts), dim3(kBlock), 0, ctx->stream, pos, nrm, n,
                        b->partials.as<float>());
     hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(768), 0, ctx->stream, b->partials.as<float>(),
@@ -838,9 +954,11 @@ void launch_refit(arc_bvh* b, int n, const NodeData& nd, const CutRecs& cr, int*
     auto* nodes = b->nodes.as<arc_bvh_node>();
     hipLaunchKernelGGL(k_refit_local<kMode>, dim3(rblocks), dim3(kRefitLeaves), 0, b->ctx->stream, nodes,
                        b->parents.as<int>(), b->ranges.as<int>(), b->positions.as<f3>(), n, nd, cr, ready, nready);
+    if (rblocks == 1) return;  // no node crosses blocks
     hipLaunchKernelGGL(k_refit_mid<kMode>, dim3((n + kMidLeaves - 1) / kMidLeaves), dim3(kMidThreads), 0,
                        b->ctx->stream, nodes, b->parents.as<int>(), b->ranges.as<int>(), b->positions.as<f3>(), n, nd,
                        cr, ready, nready, ready + n, nready + 1);
+    if (n <= kMidLeaves) return;  // no node crosses spans
     hipLaunchKernelGGL(k_refit_top<kMode>, dim3(1), dim3(b->refit_top_threads), 0, b->ctx->stream, nodes,
                        b->parents.as<int>(), b->positions.as<f3>(), n, nd, cr, ready + n, nready + 1);
 }
@@ -849,9 +967,10 @@ void launch_refit(arc_bvh* b, int n, const NodeData& nd, const CutRecs& cr, int*
 // neither (boxes only).
 int build_tree(arc_bvh* b, int n, const NodeData* nd, const CutRecs* cr) {
     arc_ctx* ctx = b->ctx;
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kBlock), 0, ctx->stream,
-                       b->codes.as<uint32_t>(), n - 1, b->nodes.as<arc_bvh_node>(), b->parents.as<int>(),
-                       b->ranges.as<int>(), reinterpret_cast<int*>(b->bounds.as<float>() + 13));
+    if (n > kSmallTree)
+        hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kBlock), 0, ctx->stream,
+                           b->codes.as<uint32_t>(), n - 1, b->nodes.as<arc_bvh_node>(), b->parents.as<int>(),
+                           b->ranges.as<int>(), reinterpret_cast<int*>(b->bounds.as<float>() + 13));
     int* nready = reinterpret_cast<int*>(b->bounds.as<float>() + 13);  // two counters, zeroed by k_karras
     int* ready = b->ready.as<int>();
     const NodeData d = nd ? *nd : NodeData{};
@@ -892,8 +1011,9 @@ int bvh_build_points(arc_bvh* b, const f3* pos, const f3* nrm, int n) {
     if (b->consider_normals && !nrm) return fail(b->ctx, ARC_E_INVALID, "normals required");
     ARC_TRY(ensure_tree(b, n));
     ARC_TRY(encode_and_sort(b, pos, nrm, n));
-    hipLaunchKernelGGL(k_permute_points, dim3(blocks_for(n)), dim3(kBlock), 0, b->ctx->stream,
-                       b->perm.as<int>(), pos, nrm, n, b->positions.as<f3>(), b->normals.as<f3>());
+    if (n > kSmallTree)
+        hipLaunchKernelGGL(k_permute_points, dim3(blocks_for(n)), dim3(kBlock), 0, b->ctx->stream,
+                           b->perm.as<int>(), pos, nrm, n, b->positions.as<f3>(), b->normals.as<f3>());
     ARC_LAUNCHED(b->ctx);
     ARC_TRY(build_tree(b, n, nullptr, nullptr));
     b->n = n;
