@@ -32,6 +32,10 @@ using arc::write_cut_record;
 
 constexpr int kBlock = 256;
 constexpr int kReduceBlocks = 512;
+// arc_bvh::bounds: 12 bounds, the bounce check's flag, and the lengths of the
+// range queries' lists, the points' and the normals' (zeroed by the kernel that
+// makes the Karras nodes)
+constexpr int kCounters = 13, kNumCounters = 2, kNormalList = 1;
 
 __device__ inline f3 ldf3(const f3* p, size_t i) { return p[i]; }
 
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ 
     }
     __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) nready[0] = nready[1] = nready[2] = 0;  // the refits' list lengths
+    if (blockIdx.x == 0 && threadIdx.x < kNumCounters) nready[threadIdx.x] = 0;
     if (i >= num_nodes) return;             // no barrier follows
     karras_node(i, num_nodes, [&](int j) {
         const int k = j - wbase;
@@ -378,7 +382,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_tree(const f3* __restri
         sbounds[tid] = r;
         bounds[tid] = r;
     }
-    if (tid == 0) nready[0] = nready[1] = nready[2] = 0;
+    if (tid < kNumCounters) nready[tid] = 0;
     __syncthreads();
     int size = 128;
     while (size < n) size *= 2;
@@ -428,23 +432,6 @@ __device__ inline float len3(f3 v) {
     return sqrtf(v.x * v.x + v.y * v.y + v.z * v.z);
 }
 
-// cluster() (bvh.cu:726-744)
-__device__ inline void cluster(int target, int left, int right, int n, const NodeData& nd) {
-    const int tid = n + target;
-    const int lid = left < 0 ? n - (left + 1) : left;
-    const int rid = right < 0 ? n - (right + 1) : right;
-    const f3 rl = nd.rad[lid], rr = nd.rad[rid];
-    const float i1 = len3(rl), i2 = len3(rr);
-    int repr = lid;
-    if (nd.rnd[tid] > (i1 / (i1 + i2))) repr = rid;  // NaN ratio keeps the left child
-    nd.size[tid] = nd.size[lid] + nd.size[rid];
-    nd.mat[tid] = nd.mat[repr];
-    nd.rad[tid] = f3{rl.x + rr.x, rl.y + rr.y, rl.z + rr.z};
-    nd.dir[tid] = nd.dir[repr];
-    nd.pos[tid] = nd.pos[repr];
-    nd.nrm[tid] = nd.nrm[repr];
-}
-
 // The cut's merge sums of an internal node from its children's, a (left) +
 // b (right) in that order: (I, count), (sum w x, sum w), (sum w n, -).
 __device__ inline void add_cut_sums(const float4 (&a)[kMrec], const float4 (&b)[kMrec], float4 (&m)[kMrec]) {
@@ -470,230 +457,325 @@ __device__ inline void store_merge(int target, int n, const float4 (&m)[kMrec], 
     for (int q = 0; q < kMrec; ++q) mg[q] = m[q];
 }
 
-// The cut's sums of an internal node from its children's merge records in
-// HBM, and its node record; lo / hi: the node's box.
-__device__ inline void merge_cut(int target, int left, int right, int n, f3 lo, f3 hi, const CutRecs& cr) {
-    const size_t lid = left < 0 ? (size_t)n - (left + 1) : (size_t)left;
-    const size_t rid = right < 0 ? (size_t)n - (right + 1) : (size_t)right;
-    float4 a[kMrec], b[kMrec], m[kMrec];
-#pragma unroll
-    for (int q = 0; q < kMrec; ++q) {
-        a[q] = cr.merge[kMrec * lid + q];
-        b[q] = cr.merge[kMrec * rid + q];
-    }
-    add_cut_sums(a, b, m);
-    store_merge(target, n, m, cr);
-    write_cut_node(target, n, lo, hi, m, cr);
-}
-
-// kernel_innerNodes (bvh.cu:280-316).  One thread per leaf walks up; the
-// second thread to arrive at a node merges both children.  The reference
-// reads the sibling's box without ordering (quirk Q3); here the arrival
-// counters inside one kernel's workgroup are acq_rel RMWs at workgroup
-// scope, so the first arrival's writes are visible to the second arrival
-// before it reads them, and the arrivals that cross workgroups (blocks,
-// spans) are relaxed: the kernel boundary publishes their writes before the
-// next kernel reads them.
-//
-// Three kernels, no cross-XCD fence:
+// kernel_innerNodes (bvh.cu:280-316).  The reference walks up from every
+// leaf, the second thread to arrive at a node merging both children, and reads
+// the sibling's box without ordering (quirk Q3).  Here, without a cross-XCD
+// fence or a global counter:
 //   k_refit_local: a block owns kRefitLeaves consecutive leaves.  Karras node
 //     k has k at one end of its leaf range, so a node whose range lies inside
 //     the block's leaves has its index there too and both of its subtrees are
-//     merged by this block: its counter lives in LDS (workgroup scope).  At a
-//     node whose range crosses a block boundary the walk stops after a
-//     relaxed increment of the node's `visited`; the thread that makes it 2
-//     appends the node to the ready list.
-//   k_refit_mid: one workgroup per kMidLeaves-leaf span, after the kernel
-//     boundary, climbs from the ready nodes inside its span through the
-//     crossing nodes inside it, with workgroup-scope counters on `visited`;
-//     at a node that spans two of them it stops as k_refit_local does at a
-//     block boundary, and the second arrival appends the node to a second
-//     ready list.  One workgroup merging all ~10000 crossing nodes of 1M
-//     points is bound by its CU's rate of scattered memory requests (about
-//     20 per merge); the spans share them over tens of CUs.
-//   k_refit_top: one workgroup, after the kernel boundary has published every
-//     span's result, climbs from the second ready list through the remaining
-//     nodes with workgroup-scope counters on `visited`.  Its width
-//     is the tree's refit_top_threads: 1024 threads climb the most chains at
-//     once, but a 16-wave workgroup needs 16 free wave slots on one CU, and
-//     beside a kernel that fills the CUs (the gather's antiradiance on its
-//     second stream) it waited for them up to 0.8 ms; the gather's trees use
-//     four waves.
+//     merged by this block, one thread per leaf walking up: the arrival
+//     counters, the links and the merged values that a walk reads are in LDS,
+//     so that a level costs LDS reads and not a chain of reads from HBM.  The
+//     block's other nodes, which cross its ends, go to its list.
+//   k_refit_span, for spans of 8 blocks, 64, 512 and so on until one holds
+//     all leaves: one workgroup per span takes the lists of its 8 blocks (or
+//     smaller spans).  Nodes that cross the span's ends go to its own list; of
+//     the others each thread takes one, reads the children that an earlier
+//     kernel merged, and merges once its other children, in LDS, are there: a
+//     round and a barrier per level.  Three dependent reads from L2 in all;
+//     walking up with counters and both children's records read at each
+//     level, the crossing nodes of 131071 leaves took 110 us, 55 here.
+// The attributes that a reference node copies from its representative do not
+// depend on the order: each kernel copies them at its end, from the slot that
+// the merged values carry along.
 // Every internal node ends with visited == 2, as the reference's counters do.
 constexpr int kRefitLeaves = 1024;
-constexpr int kMidLeaves = 32 * kRefitLeaves, kMidThreads = 256;
+constexpr int kSpanFactor = 8, kSpanThreads = 512;
+// A node that crosses a boundary contains the leaves on both sides, and each
+// longer range that does has a shorter common prefix: at most 63 (32 code
+// bits, 31 index bits) per boundary.  A list holds the nodes across its two
+// ends, after their number; a span's own nodes cross one of 7 boundaries.
+constexpr int kListSize = 128, kSpanNodes = 63 * (kSpanFactor - 1), kSpanSlots = 1024;
+static_assert(2 * 63 < kListSize && kSpanNodes <= kSpanThreads, "the lists and a thread per node");
 
 // What a refit merges besides the boxes.
-enum RefitMode { kBoxes = 0, kReference = 1, kCut = 2 };
+enum RefitMode { kReference = 1, kCut = 2 };
 
+// A subtree's merged values: its box and, in kReference, the cluster's size,
+// radiance and the slot whose attributes represent it; in kCut the merge sums.
 template <int kMode>
-__device__ inline void merge_node(int parent, arc_bvh_node* nodes, const f3* spos, int n, const NodeData& nd,
-                                  const CutRecs& cr) {
-    const int l = nodes[parent].left, r = nodes[parent].right;
-    f3 lmin, lmax, rmin, rmax;
-    if (l < 0) {
-        const arc_bvh_node& c = nodes[-(l + 1)];
-        lmin = f3{c.bbMin.x, c.bbMin.y, c.bbMin.z};
-        lmax = f3{c.bbMax.x, c.bbMax.y, c.bbMax.z};
+struct Merged;
+template <>
+struct Merged<kReference> {
+    f3 lo, hi, rad;
+    int size, rep;
+};
+template <>
+struct Merged<kCut> {
+    f3 lo, hi;
+    float4 m[kMrec];
+};
+
+// The values of a child that an earlier kernel merged, or of a leaf.
+template <int kMode>
+__device__ inline Merged<kMode> child_values(int c, const arc_bvh_node* nodes, const f3* spos, int n, const NodeData& nd,
+                                             const CutRecs& cr) {
+    Merged<kMode> v;
+    if (c < 0) {
+        const arc_bvh_node& b = nodes[-(c + 1)];
+        v.lo = f3{b.bbMin.x, b.bbMin.y, b.bbMin.z};
+        v.hi = f3{b.bbMax.x, b.bbMax.y, b.bbMax.z};
     } else {
-        lmin = lmax = spos[l];
+        v.lo = v.hi = spos[c];
     }
-    if (r < 0) {
-        const arc_bvh_node& c = nodes[-(r + 1)];
-        rmin = f3{c.bbMin.x, c.bbMin.y, c.bbMin.z};
-        rmax = f3{c.bbMax.x, c.bbMax.y, c.bbMax.z};
+    const int slot = c < 0 ? n - (c + 1) : c;
+    if constexpr (kMode == kReference) {
+        v.rad = nd.rad[slot];
+        v.size = nd.size[slot];
+        v.rep = slot;
     } else {
-        rmin = rmax = spos[r];
+#pragma unroll
+        for (int q = 0; q < kMrec; ++q) v.m[q] = cr.merge[kMrec * (size_t)slot + q];
     }
-    const f3 lo{fminf(lmin.x, rmin.x), fminf(lmin.y, rmin.y), fminf(lmin.z, rmin.z)};
-    const f3 hi{fmaxf(lmax.x, rmax.x), fmaxf(lmax.y, rmax.y), fmaxf(lmax.z, rmax.z)};
-    nodes[parent].bbMin = arc_float3{lo.x, lo.y, lo.z};
-    nodes[parent].bbMax = arc_float3{hi.x, hi.y, hi.z};
-    if (kMode == kReference) cluster(parent, l, r, n, nd);
-    if (kMode == kCut) merge_cut(parent, l, r, n, lo, hi, cr);
+    return v;
 }
 
-// A child of a block-local node: a leaf (its point, and for the light cuts'
-// rebuild its merge record, from HBM) or a local node merged earlier in this
-// block (from LDS).
+// A node's values from its children's; rnd: its random number (kReference).
 template <int kMode>
-__device__ inline void local_child(int c, int lo, const f3* spos, const CutRecs& cr, const f3* sbmin,
-                                   const f3* sbmax, const float4* smerge, f3& bmin, f3& bmax, float4 (&m)[kMrec]) {
-    if (c >= 0) {
-        bmin = bmax = spos[c];
-        if (kMode == kCut) {
-#pragma unroll
-            for (int q = 0; q < kMrec; ++q) m[q] = cr.merge[kMrec * (size_t)c + q];
-        }
+__device__ inline Merged<kMode> merge(const Merged<kMode>& l, const Merged<kMode>& r, float rnd) {
+    Merged<kMode> v;
+    v.lo = f3{fminf(l.lo.x, r.lo.x), fminf(l.lo.y, r.lo.y), fminf(l.lo.z, r.lo.z)};
+    v.hi = f3{fmaxf(l.hi.x, r.hi.x), fmaxf(l.hi.y, r.hi.y), fmaxf(l.hi.z, r.hi.z)};
+    if constexpr (kMode == kReference) {  // cluster() (bvh.cu:726-744)
+        const float i1 = len3(l.rad), i2 = len3(r.rad);
+        v.rep = rnd > (i1 / (i1 + i2)) ? r.rep : l.rep;  // NaN ratio keeps the left child
+        v.size = l.size + r.size;
+        v.rad = f3{l.rad.x + r.rad.x, l.rad.y + r.rad.y, l.rad.z + r.rad.z};
     } else {
-        const int s = -(c + 1) - lo;
-        bmin = sbmin[s];
-        bmax = sbmax[s];
-        if (kMode == kCut) {
-#pragma unroll
-            for (int q = 0; q < kMrec; ++q) m[q] = smerge[kMrec * s + q];
-        }
+        add_cut_sums(l.m, r.m, v.m);
+    }
+    return v;
+}
+
+// Writes a node's box and values; the attributes of a reference node's
+// representative come later (copy_representative).  keep: a later kernel
+// merges it (kCut).
+template <int kMode>
+__device__ inline void store_values(int k, const Merged<kMode>& v, bool keep, arc_bvh_node* nodes, int n,
+                                    const NodeData& nd, const CutRecs& cr) {
+    nodes[k].bbMin = arc_float3{v.lo.x, v.lo.y, v.lo.z};
+    nodes[k].bbMax = arc_float3{v.hi.x, v.hi.y, v.hi.z};
+    nodes[k].visited = 2;
+    if constexpr (kMode == kReference) {
+        nd.size[n + k] = v.size;
+        nd.rad[n + k] = v.rad;
+    } else {
+        if (keep) store_merge(k, n, v.m, cr);
+        write_cut_node(k, n, v.lo, v.hi, v.m, cr);
     }
 }
+
+__device__ inline void copy_representative(int k, int rep, int n, const NodeData& nd) {
+    nd.mat[n + k] = nd.mat[rep];
+    nd.dir[n + k] = nd.dir[rep];
+    nd.pos[n + k] = nd.pos[rep];
+    nd.nrm[n + k] = nd.nrm[rep];
+}
+
+// The block's local nodes, by index - lo.
+template <int kMode>
+struct LocalLds {
+    // left, right (leaf or node of the block: index - lo, 1024 added to a
+    // node's) and parent (its own index: not local), 11 + 11 + 10 bits; all
+    // ones: not a local node
+    uint32_t links[kRefitLeaves];
+    uint32_t arrivals[kRefitLeaves / 4];  // a byte each: two blocks fit a CU's LDS in kCut
+    f3 lo[kRefitLeaves], hi[kRefitLeaves];
+    float4 m[kMode == kCut ? kMrec * kRefitLeaves : 1];
+    f3 rad[kMode == kReference ? kRefitLeaves : 1];
+    int size[kMode == kReference ? kRefitLeaves : 1];
+    int rep[kMode == kReference ? kRefitLeaves : 1];
+    float rnd[kMode == kReference ? kRefitLeaves : 1];
+};
 
 template <int kMode>
 __global__ __launch_bounds__(kRefitLeaves) void k_refit_local(arc_bvh_node* __restrict__ nodes,
                                                               const int* __restrict__ parents,
                                                               const int* __restrict__ ranges,
                                                               const f3* __restrict__ spos, int n, NodeData nd,
-                                                              CutRecs cr, int* __restrict__ ready,
-                                                              int* __restrict__ nready) {
-    // The block's local nodes, by index - lo: arrival counters, boxes and, for
-    // the light cuts' rebuild, merge sums.  A local node's children are
-    // leaves or local nodes, so its merge reads HBM only for leaves.
-    __shared__ int arrivals[kRefitLeaves];
-    __shared__ f3 sbmin[kRefitLeaves], sbmax[kRefitLeaves];
-    __shared__ float4 smerge[kMode == kCut ? kMrec * kRefitLeaves : 1];
-    arrivals[threadIdx.x] = 0;
-    __syncthreads();
+                                                              CutRecs cr, int* __restrict__ list) {
+    static_assert(kRefitLeaves == 1024, "links");
+    constexpr uint32_t kNotLocal = ~0u;
+    __shared__ LocalLds<kMode> S;
+    __shared__ int crossing;
+    const int tid = threadIdx.x;
     const int lo = blockIdx.x * kRefitLeaves;
     const int hi = min(n, lo + kRefitLeaves) - 1;
-    const int i = lo + threadIdx.x;
-    if (i >= n) return;  // no barrier follows
-    int parent = parents[i];
-    bool local = parent >= 0 && ranges[2 * parent] >= lo && ranges[2 * parent + 1] <= hi;
-    while (parent >= 0) {
-        if (!local) {
-            const int old = __hip_atomic_fetch_add(&nodes[parent].visited, 1, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-            if (old == 1) ready[atomicAdd(nready, 1)] = parent;
-            return;
+    const int i = lo + tid;
+    list += (size_t)kListSize * blockIdx.x;
+    if (tid == 0) crossing = 0;
+    {
+        uint32_t w = kNotLocal;
+        if (i < n - 1 && ranges[2 * i] >= lo && ranges[2 * i + 1] <= hi) {
+            const int l = nodes[i].left, r = nodes[i].right, p = parents[n + i];
+            const uint32_t wl = l < 0 ? 1024 - (l + 1) - lo : l - lo, wr = r < 0 ? 1024 - (r + 1) - lo : r - lo;
+            const bool up = p >= 0 && ranges[2 * p] >= lo && ranges[2 * p + 1] <= hi;
+            w = wl | wr << 11 | (uint32_t)(up ? p - lo : tid) << 22;
         }
-        if (__hip_atomic_fetch_add(&arrivals[parent - lo], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
-            return;
-        const int l = nodes[parent].left, r = nodes[parent].right;
-        f3 lmin, lmax, rmin, rmax;
-        float4 a[kMrec], b[kMrec];
-        local_child<kMode>(l, lo, spos, cr, sbmin, sbmax, smerge, lmin, lmax, a);
-        local_child<kMode>(r, lo, spos, cr, sbmin, sbmax, smerge, rmin, rmax, b);
-        const f3 blo{fminf(lmin.x, rmin.x), fminf(lmin.y, rmin.y), fminf(lmin.z, rmin.z)};
-        const f3 bhi{fmaxf(lmax.x, rmax.x), fmaxf(lmax.y, rmax.y), fmaxf(lmax.z, rmax.z)};
-        const int s = parent - lo;
-        sbmin[s] = blo;
-        sbmax[s] = bhi;
-        nodes[parent].bbMin = arc_float3{blo.x, blo.y, blo.z};
-        nodes[parent].bbMax = arc_float3{bhi.x, bhi.y, bhi.z};
-        if (kMode == kReference) cluster(parent, l, r, n, nd);
-        const int next = parents[n + parent];
-        const bool next_local = next >= 0 && ranges[2 * next] >= lo && ranges[2 * next + 1] <= hi;
-        if (kMode == kCut) {
-            float4 m[kMrec];
-            add_cut_sums(a, b, m);
+        S.links[tid] = w;
+        if (tid < kRefitLeaves / 4) S.arrivals[tid] = 0;
+        if (kMode == kReference && i < n - 1) S.rnd[tid] = nd.rnd[n + i];
+    }
+    __syncthreads();
+    if (i < n - 1 && S.links[tid] == kNotLocal) list[1 + atomicAdd(&crossing, 1)] = i;
+    auto child = [&](uint32_t c) -> Merged<kMode> {
+        if (c < 1024) return child_values<kMode>(lo + (int)c, nodes, spos, n, nd, cr);
+        const int k = c - 1024;
+        Merged<kMode> v;
+        v.lo = S.lo[k];
+        v.hi = S.hi[k];
+        if constexpr (kMode == kReference) {
+            v.rad = S.rad[k];
+            v.size = S.size[k];
+            v.rep = S.rep[k];
+        } else {
 #pragma unroll
-            for (int q = 0; q < kMrec; ++q) smerge[kMrec * s + q] = m[q];
-            // HBM holds the merge sums the top refit reads: those of a node
-            // whose parent spans blocks (and the root's)
-            if (!next_local) store_merge(parent, n, m, cr);
-            write_cut_node(parent, n, blo, bhi, m, cr);
+            for (int q = 0; q < kMrec; ++q) v.m[q] = S.m[kMrec * k + q];
         }
-        nodes[parent].visited = 2;
-        parent = next;
-        local = next_local;
+        return v;
+    };
+    int parent = i < n ? parents[i] : -1;
+    bool local = parent >= lo && parent <= hi && S.links[parent - lo] != kNotLocal;
+    while (local) {
+        const int s = parent - lo;
+        const int byte = 8 * (s & 3);
+        if ((__hip_atomic_fetch_add(&S.arrivals[s >> 2], 1u << byte, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) >> byte & 255) == 0)
+            break;
+        const uint32_t w = S.links[s];
+        const float rnd = kMode == kReference ? S.rnd[s] : 0.f;
+        const Merged<kMode> v = merge<kMode>(child(w & 2047), child(w >> 11 & 2047), rnd);
+        S.lo[s] = v.lo;
+        S.hi[s] = v.hi;
+        if constexpr (kMode == kReference) {
+            S.rad[s] = v.rad;
+            S.size[s] = v.size;
+            S.rep[s] = v.rep;
+        } else {
+#pragma unroll
+            for (int q = 0; q < kMrec; ++q) S.m[kMrec * s + q] = v.m[q];
+        }
+        const int up = (int)(w >> 22);
+        local = up != s;
+        // HBM holds the merge sums of a node whose parent spans blocks (and the root's)
+        store_values<kMode>(parent, v, !local, nodes, n, nd, cr);
+        parent = lo + up;
+    }
+    __syncthreads();
+    if (tid == 0) list[0] = crossing;
+    if constexpr (kMode == kReference) {
+        if (S.links[tid] != kNotLocal) copy_representative(i, S.rep[tid], n, nd);
     }
 }
 
+// A span's nodes, one per thread, found by their index (slot), and their merged
+// values.
 template <int kMode>
-__global__ __launch_bounds__(kMidThreads) void k_refit_mid(arc_bvh_node* __restrict__ nodes,
-                                                           const int* __restrict__ parents,
-                                                           const int* __restrict__ ranges,
-                                                           const f3* __restrict__ spos, int n, NodeData nd,
-                                                           CutRecs cr, const int* __restrict__ ready,
-                                                           const int* __restrict__ nready, int* __restrict__ ready2,
-                                                           int* __restrict__ nready2) {
-    const int count = *nready;
-    const int lo = blockIdx.x * kMidLeaves;
-    const int hi = min(n, lo + kMidLeaves) - 1;
-    for (int j = threadIdx.x; j < count; j += kMidThreads) {
-        int node = ready[j];
+struct SpanLds {
+    static constexpr int kWords = sizeof(Merged<kMode>) / 4;
+    int key[kSpanSlots], entry[kSpanSlots];
+    int node[kSpanNodes], first[kSpanNodes], last[kSpanNodes], left[kSpanNodes], right[kSpanNodes];
+    int done[kSpanNodes];  // the round that merged it
+    uint32_t value[kWords][kSpanNodes];
+    int count, crossing, merged[3];
+};
+
+// units: the lists of the kSpanFactor last spans (blocks) in each span.
+template <int kMode>
+__global__ __launch_bounds__(kSpanThreads) void k_refit_span(arc_bvh_node* __restrict__ nodes,
+                                                             const int* __restrict__ ranges,
+                                                             const f3* __restrict__ spos, int n, NodeData nd,
+                                                             CutRecs cr, long long span, int units,
+                                                             const int* __restrict__ lists, int* __restrict__ list2) {
+    __shared__ SpanLds<kMode> S;
+    constexpr int kWords = SpanLds<kMode>::kWords;
+    const int tid = threadIdx.x;
+    for (int k = tid; k < kSpanSlots; k += kSpanThreads) S.key[k] = -1;
+    if (tid < kSpanNodes) S.done[tid] = 0;
+    if (tid == 0) S.count = S.crossing = S.merged[1] = 0;
+    __syncthreads();
+    auto slot_of = [](int k) { return (int)((unsigned)k * 0x9E3779B1u >> 22); };
+    const int lo = (int)(blockIdx.x * span);
+    const int hi = (int)min((long long)n, lo + span) - 1;
+    const int unit = blockIdx.x * kSpanFactor;
+    list2 += (size_t)kListSize * blockIdx.x;
+    for (int k = tid; k < kSpanFactor * kListSize; k += kSpanThreads) {
+        const int u = unit + k / kListSize, j = k % kListSize;
+        if (u >= units || j == 0) continue;
+        const int* list = lists + (size_t)kListSize * u;
+        const int count = list[0], node = list[j];
+        if (j > count) continue;
         const int first = ranges[2 * node], last = ranges[2 * node + 1];
-        if (first < lo || first > hi) continue;  // the span holding its first leaf takes it
-        if (last > hi) {                         // spans two spans: the top refit's
-            ready2[atomicAdd(nready2, 1)] = node;
+        if (first < lo || last > hi) {
+            list2[1 + atomicAdd(&S.crossing, 1)] = node;
             continue;
         }
-        while (true) {
-            merge_node<kMode>(node, nodes, spos, n, nd, cr);
-            const int parent = parents[n + node];
-            if (parent < 0) break;
-            if (ranges[2 * parent] >= lo && ranges[2 * parent + 1] <= hi) {
-                // 0: the sibling subtree is still pending and will climb on; 1: both done
-                if (__hip_atomic_fetch_add(&nodes[parent].visited, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) != 1)
-                    break;
-                node = parent;
+        const int e = atomicAdd(&S.count, 1);
+        S.node[e] = node;
+        S.first[e] = first;
+        S.last[e] = last;
+        S.left[e] = nodes[node].left;
+        S.right[e] = nodes[node].right;
+        int slot = slot_of(node);
+        while (atomicCAS(&S.key[slot], -1, node) != -1) slot = (slot + 1) & (kSpanSlots - 1);
+        S.entry[slot] = e;
+    }
+    __syncthreads();
+    if (tid == 0) list2[0] = S.crossing;
+    const bool mine = tid < S.count;
+    const long long unit_leaves = span / kSpanFactor;
+    int wait[2] = {-1, -1}, node = 0;  // the entries of the children merged here
+    Merged<kMode> child[2];
+    float rnd = 0.f;
+    if (mine) {
+        node = S.node[tid];
+        if (kMode == kReference) rnd = nd.rnd[n + node];
+        const int c[2] = {S.left[tid], S.right[tid]};
+        const int split = c[0] < 0 ? -(c[0] + 1) : c[0];  // the left child's last leaf
+        const int from[2] = {S.first[tid], split + 1}, to[2] = {split, S.last[tid]};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (c[s] < 0 && from[s] / unit_leaves != to[s] / unit_leaves) {
+                const int k = -(c[s] + 1);
+                int slot = slot_of(k);
+                while (S.key[slot] != k) slot = (slot + 1) & (kSpanSlots - 1);
+                wait[s] = S.entry[slot];
             } else {
-                const int old = __hip_atomic_fetch_add(&nodes[parent].visited, 1, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT);
-                if (old == 1) ready2[atomicAdd(nready2, 1)] = parent;
-                break;
+                child[s] = child_values<kMode>(c[s], nodes, spos, n, nd, cr);
             }
         }
     }
-}
-
-template <int kMode>
-__global__ __launch_bounds__(kRefitLeaves) void k_refit_top(arc_bvh_node* __restrict__ nodes,
-                                                            const int* __restrict__ parents,
-                                                            const f3* __restrict__ spos, int n, NodeData nd,
-                                                            CutRecs cr, const int* __restrict__ ready,
-                                                            const int* __restrict__ nready) {
-    const int count = *nready;
-    for (int j = threadIdx.x; j < count; j += blockDim.x) {
-        int node = ready[j];
-        while (true) {
-            merge_node<kMode>(node, nodes, spos, n, nd, cr);
-            const int parent = parents[n + node];
-            if (parent < 0) break;
-            // 0: the sibling subtree is still pending and will climb on; 1: both done
-            if (__hip_atomic_fetch_add(&nodes[parent].visited, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) != 1)
-                break;
-            node = parent;
+    // A round merges the nodes whose children earlier rounds merged.  How many
+    // it merges is counted in one of three counters: in a round one is added
+    // to, the next is cleared and the last one may still be read.
+    const int total = S.count;
+    bool todo = mine;
+    for (int round = 1, merged = 0; merged < total; ++round) {
+        auto there = [&](int e) { return e < 0 || (unsigned)(S.done[e] - 1) < (unsigned)(round - 1); };
+        if (tid == 0) S.merged[(round + 1) % 3] = 0;
+        if (todo && there(wait[0]) && there(wait[1])) {
+            uint32_t words[kWords];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if (wait[s] < 0) continue;
+#pragma unroll
+                for (int q = 0; q < kWords; ++q) words[q] = S.value[q][wait[s]];
+                __builtin_memcpy(&child[s], words, sizeof child[s]);
+            }
+            child[0] = merge<kMode>(child[0], child[1], rnd);
+            __builtin_memcpy(words, &child[0], sizeof child[0]);
+#pragma unroll
+            for (int q = 0; q < kWords; ++q) S.value[q][tid] = words[q];
+            S.done[tid] = round;
+            todo = false;
+            atomicAdd(&S.merged[round % 3], 1);
         }
+        __syncthreads();
+        merged += S.merged[round % 3];
     }
+    if (!mine) return;
+    store_values<kMode>(node, child[0], true, nodes, n, nd, cr);
+    if constexpr (kMode == kReference) copy_representative(node, child[0].rep, n, nd);
 }
 
 inline int blocks_for(int n) { return (n + kBlock - 1) / kBlock; }
@@ -916,7 +998,9 @@ int ensure_tree(arc_bvh* b, int n) {
     ARC_TRY(arc::ensure(ctx, b->positions, sizeof(f3) * (size_t)n));
     ARC_TRY(arc::ensure(ctx, b->normals, sizeof(f3) * (size_t)n));
     ARC_TRY(arc::ensure(ctx, b->bounds, sizeof(float) * 16));
-    ARC_TRY(arc::ensure(ctx, b->ready, sizeof(int) * 2 * (size_t)n));  // two ready lists
+    // the refits' lists of nodes: all that cross blocks (points), or per block and per span
+    const size_t rblocks = ((size_t)n + kRefitLeaves - 1) / kRefitLeaves;
+    ARC_TRY(arc::ensure(ctx, b->ready, sizeof(int) * std::max((size_t)n, 2 * kListSize * rblocks)));
     ARC_TRY(arc::ensure(ctx, b->partials, sizeof(float) * 12 * kReduceBlocks));
     ARC_TRY(arc::ensure(ctx, b->boxes, point_boxes_bytes(n)));
     return ARC_OK;
@@ -932,7 +1016,7 @@ int encode_and_sort(arc_bvh* b, const f3* pos, const f3* nrm, int n) {
         hipLaunchKernelGGL(k_small_tree, dim3(1), dim3(kSmallThreads), 0, ctx->stream, pos, nrm, n,
                            b->consider_normals && nrm ? 1 : 0, bounds, b->codes.as<uint32_t>(), b->perm.as<int>(),
                            b->nodes.as<arc_bvh_node>(), b->parents.as<int>(), b->ranges.as<int>(),
-                           reinterpret_cast<int*>(bounds + 13), b->positions.as<f3>(), b->normals.as<f3>());
+                           reinterpret_cast<int*>(bounds + kCounters), b->positions.as<f3>(), b->normals.as<f3>());
         ARC_LAUNCHED(ctx);
         return ARC_OK;
     }
@@ -949,18 +1033,23 @@ int encode_and_sort(arc_bvh* b, const f3* pos, const f3* nrm, int n) {
 }
 
 template <int kMode>
-void launch_refit(arc_bvh* b, int n, const NodeData& nd, const CutRecs& cr, int* ready, int* nready) {
+void launch_refit(arc_bvh* b, int n, const NodeData& nd, const CutRecs& cr, int* lists) {
     const int rblocks = (n + kRefitLeaves - 1) / kRefitLeaves;
     auto* nodes = b->nodes.as<arc_bvh_node>();
     hipLaunchKernelGGL(k_refit_local<kMode>, dim3(rblocks), dim3(kRefitLeaves), 0, b->ctx->stream, nodes,
-                       b->parents.as<int>(), b->ranges.as<int>(), b->positions.as<f3>(), n, nd, cr, ready, nready);
-    if (rblocks == 1) return;  // no node crosses blocks
-    hipLaunchKernelGGL(k_refit_mid<kMode>, dim3((n + kMidLeaves - 1) / kMidLeaves), dim3(kMidThreads), 0,
-                       b->ctx->stream, nodes, b->parents.as<int>(), b->ranges.as<int>(), b->positions.as<f3>(), n, nd,
-                       cr, ready, nready, ready + n, nready + 1);
-    if (n <= kMidLeaves) return;  // no node crosses spans
-    hipLaunchKernelGGL(k_refit_top<kMode>, dim3(1), dim3(b->refit_top_threads), 0, b->ctx->stream, nodes,
-                       b->parents.as<int>(), b->positions.as<f3>(), n, nd, cr, ready + n, nready + 1);
+                       b->parents.as<int>(), b->ranges.as<int>(), b->positions.as<f3>(), n, nd, cr, lists);
+    // spans of kSpanFactor of the last ones, the lists in turn
+    int units = rblocks;
+    int* from = lists;
+    int* to = lists + (size_t)kListSize * rblocks;
+    for (long long span = kRefitLeaves; span < n;) {
+        span *= kSpanFactor;
+        const int spans = (int)((n + span - 1) / span);
+        hipLaunchKernelGGL(k_refit_span<kMode>, dim3(spans), dim3(kSpanThreads), 0, b->ctx->stream, nodes,
+                           b->ranges.as<int>(), b->positions.as<f3>(), n, nd, cr, span, units, from, to);
+        std::swap(from, to);
+        units = spans;
+    }
 }
 
 // Karras tree and refit; nd (reference node data) or cr (cut records) or
@@ -970,14 +1059,14 @@ int build_tree(arc_bvh* b, int n, const NodeData* nd, const CutRecs* cr) {
     if (n > kSmallTree)
         hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kBlock), 0, ctx->stream,
                            b->codes.as<uint32_t>(), n - 1, b->nodes.as<arc_bvh_node>(), b->parents.as<int>(),
-                           b->ranges.as<int>(), reinterpret_cast<int*>(b->bounds.as<float>() + 13));
-    int* nready = reinterpret_cast<int*>(b->bounds.as<float>() + 13);  // two counters, zeroed by k_karras
-    int* ready = b->ready.as<int>();
+                           b->ranges.as<int>(), reinterpret_cast<int*>(b->bounds.as<float>() + kCounters));
+    int* ncross = reinterpret_cast<int*>(b->bounds.as<float>() + kCounters);  // zeroed with the Karras nodes
+    int* lists = b->ready.as<int>();
     const NodeData d = nd ? *nd : NodeData{};
     const CutRecs c = cr ? *cr : CutRecs{};
-    if (nd) launch_refit<kReference>(b, n, d, c, ready, nready);
-    else if (cr) launch_refit<kCut>(b, n, d, c, ready, nready);
-    else launch_refit_points(b, n, ready, nready);
+    if (nd) launch_refit<kReference>(b, n, d, c, lists);
+    else if (cr) launch_refit<kCut>(b, n, d, c, lists);
+    else launch_refit_points(b, n, lists, ncross);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }
@@ -997,7 +1086,7 @@ int node_normal_boxes(arc_bvh* b, const float4* crec, float4* nbox) {
     const int n = b->n;
     if (n < 2) return ARC_OK;
     // the list and its counter of the range queries: the refit is done with them
-    int* ncross = reinterpret_cast<int*>(b->bounds.as<float>() + 15);  // zeroed by k_karras
+    int* ncross = reinterpret_cast<int*>(b->bounds.as<float>() + kCounters) + kNormalList;  // zeroed with the Karras nodes
     launch_range_boxes(b, n, NormalsIn{crec}, BoxOut{nbox}, b->ready.as<int>(), ncross);
     ARC_LAUNCHED(b->ctx);
     return ARC_OK;
