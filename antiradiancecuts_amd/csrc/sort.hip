@@ -12,9 +12,11 @@
 //             out: the tile's keys of one digit go to one contiguous run of
 //             the output, so consecutive threads write consecutive
 //             addresses.  A key's place in its digit's run: keys of that
-//             digit in earlier rounds + earlier waves + earlier lanes of
-//             its wave (ballot match), so equal digits keep their input
-//             order and the sort is stable.
+//             digit in earlier waves + earlier in its wave + in earlier
+//             lanes (ballot match), so equal digits keep their input order
+//             and the sort is stable.  With the tile's keys read a round of
+//             512 at a time, three barriers each and two scans of 16, the
+//             scatter of 1M pairs took 15.4 us and of 131071 11.4, 10.4 and 6.2 here.
 #include "arc_internal.hpp"
 
 namespace {
@@ -59,28 +61,21 @@ __global__ __launch_bounds__(kThreads) void k_hist(const uint32_t* __restrict__ 
     if (tid < kRadix) counts[(size_t)tid * num_tiles + blockIdx.x] = h[tid];
 }
 
-// Exclusive scan of sh[0, kRadix) in place, by the whole block
-// (Hillis-Steele over the first kRadix threads; every thread reaches every
-// barrier).  Returns the total.
-__device__ inline uint32_t radix_exclusive_scan(uint32_t* sh, uint32_t* tmp) {
-    const int tid = threadIdx.x;
-    uint32_t v = 0;
-    if (tid < kRadix) {
-        v = sh[tid];
-        tmp[tid] = v;
+// Exclusive scan of one value per thread over the first kRadix threads (whole
+// waves; all the block's threads call it).  sums: one word per wave of them.
+__device__ inline uint32_t radix_exclusive_scan(uint32_t v, uint32_t* sums) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t u = __shfl_up(x, off);
+        if (lane >= off) x += u;
     }
+    if (lane == 63 && wave < kRadix / 64) sums[wave] = x;
     __syncthreads();
-    for (int off = 1; off < kRadix; off <<= 1) {
-        uint32_t u = 0;
-        if (tid < kRadix && tid >= off) u = tmp[tid - off];
-        __syncthreads();
-        if (tid < kRadix) tmp[tid] += u;
-        __syncthreads();
-    }
-    const uint32_t total = tmp[kRadix - 1];
-    if (tid < kRadix) sh[tid] = tmp[tid] - v;
-    __syncthreads();
-    return total;
+    uint32_t before = 0;
+    for (int w = 0; w < min(wave, kRadix / 64); ++w) before += sums[w];
+    return before + x - v;
 }
 
 // Block d scans row d of the digit-major count table (exclusive, in place)
@@ -117,69 +112,82 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict
                                                       const uint32_t* __restrict__ totals, int num_tiles) {
     __shared__ uint32_t s_keys[kTile];
     __shared__ int s_vals[kTile];
-    __shared__ uint32_t local_start[kRadix];  // the tile's digit counts, then their exclusive scan
-    __shared__ uint32_t out_start[kRadix];    // where the tile's run of each digit starts in the output
-    __shared__ uint32_t run[kRadix];          // keys of each digit placed in earlier rounds
-    __shared__ uint32_t wcount[kWaves][kRadix];
-    __shared__ uint32_t tmp[kRadix];
+    __shared__ uint32_t out_start[kRadix];      // output place of a digit's keys minus their place in the tile
+    __shared__ uint32_t wcount[kWaves][kRadix];  // keys of each digit per wave, then where the wave's start in the tile
+    __shared__ uint32_t sums[2][kRadix / 64];
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
     const int tile = blockIdx.x;
     const int base = tile * kTile;
     const int tile_n = min(kTile, n - base);
-    // digit bases: the exclusive scan of the digit totals, plus this tile's
-    // offset within each digit (the scanned count table); the tile's own
-    // count of digit d is the next tile's offset minus its own
-    if (tid < kRadix) {
-        const uint32_t off = offsets[(size_t)tid * num_tiles + tile];
-        const uint32_t next = tile + 1 < num_tiles ? offsets[(size_t)tid * num_tiles + tile + 1] : totals[tid];
-        local_start[tid] = next - off;
-        out_start[tid] = totals[tid];
-        run[tid] = off;
-    }
-    __syncthreads();
-    radix_exclusive_scan(out_start, tmp);  // out_start = digit bases
-    radix_exclusive_scan(local_start, tmp);
-    if (tid < kRadix) {
-        out_start[tid] += run[tid];
-        run[tid] = 0;
-    }
-    // 1. the tile sorted by digit into LDS, stably, a round of kThreads keys at a time
-    for (int j = 0; j < kItems; ++j) {
+    // 1. the tile sorted by digit into LDS, stably: a wave's keys are kItems
+    // times 64 consecutive ones, all read before the first is ranked, and
+    // ranked within the wave without a barrier
+    const int first = wave * 64 * kItems + lane;
+    uint32_t key[kItems], rank[kItems];
+    int val[kItems];
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w)
-            if (tid < kRadix) wcount[w][tid] = 0;
-        __syncthreads();
-        const int i = j * kThreads + tid;
-        const bool valid = i < tile_n;
-        const uint32_t key = valid ? keys_in[base + i] : 0u;
-        const int val = valid ? vals_in[base + i] : 0;
-        const uint32_t digit = (key >> shift) & 0xffu;
+    for (int j = 0; j < kItems; ++j) {
+        const int i = first + 64 * j;
+        key[j] = i < tile_n ? keys_in[base + i] : 0u;
+        val[j] = i < tile_n ? vals_in[base + i] : 0;
+    }
+    uint32_t off = 0, total = 0;
+    if (tid < kRadix) {
+        // the tile's place within each digit (the scanned count table)
+        off = offsets[(size_t)tid * num_tiles + tile];
+        total = totals[tid];
+    }
+    for (int d = lane; d < kRadix; d += 64) wcount[wave][d] = 0;
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        const bool valid = first + 64 * j < tile_n;
+        const uint32_t digit = (key[j] >> shift) & 0xffu;
         const uint64_t m = match_digit(__ballot(valid), digit);
         const uint64_t lower = m & ((1ull << lane) - 1ull);
-        if (valid && lower == 0ull) wcount[wave][digit] = (uint32_t)__popcll(m);
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = local_start[digit] + run[digit] + (uint32_t)__popcll(lower);
-            for (int w = 0; w < wave; ++w) pos += wcount[w][digit];
-            s_keys[pos] = key;
-            s_vals[pos] = val;
-        }
-        __syncthreads();
-        if (tid < kRadix) {
-            uint32_t add = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t before = wcount[wave][digit];
+        rank[j] = before + (uint32_t)__popcll(lower);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && lower == 0ull) wcount[wave][digit] = before + (uint32_t)__popcll(m);
+    }
+    __syncthreads();
+    uint32_t mine = 0, count[kWaves];
+    if (tid < kRadix) {
 #pragma unroll
-            for (int w = 0; w < kWaves; ++w) add += wcount[w][tid];
-            run[tid] += add;
+        for (int w = 0; w < kWaves; ++w) {
+            count[w] = wcount[w][tid];
+            mine += count[w];
         }
+    }
+    const uint32_t digit_base = radix_exclusive_scan(total, sums[0]);
+    const uint32_t local = radix_exclusive_scan(mine, sums[1]);
+    if (tid < kRadix) {
+        out_start[tid] = digit_base + off - local;
+        uint32_t at = local;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            wcount[w][tid] = at;
+            at += count[w];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+        if (first + 64 * j >= tile_n) continue;
+        const uint32_t pos = wcount[wave][(key[j] >> shift) & 0xffu] + rank[j];
+        s_keys[pos] = key[j];
+        s_vals[pos] = val[j];
     }
     __syncthreads();
     // 2. out in LDS order: consecutive threads, consecutive places of one run
     for (int i = tid; i < tile_n; i += kThreads) {
         const uint32_t key = s_keys[i];
         const uint32_t digit = (key >> shift) & 0xffu;
-        const uint32_t pos = out_start[digit] + (uint32_t)i - local_start[digit];
+        const uint32_t pos = out_start[digit] + (uint32_t)i;
         keys_out[pos] = key;
         vals_out[pos] = s_vals[i];
     }
