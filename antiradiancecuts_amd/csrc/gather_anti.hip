@@ -325,15 +325,24 @@ __global__ __launch_bounds__(kListThreads) void k_cluster_lists_tree(arc::AvplsD
     }
 }
 
+struct ConeLds {  // a run's records: position, unit direction, antiradiance, index
+    float4 u[64], v[64];
+    float z[64];
+    int i[64];
+};
+
 // Four blocks per 32x32 cluster (its rows of 32x8 pixels), one wave per 8x8
 // tile.  A block reads the cluster's list once: each thread takes an entry
 // and tests its ray against the block's 4 tile boxes (the same conservative
 // test as the lists, on smaller boxes), appending hits to the tile's
-// sub-list in LDS.  Each wave then walks its tile's sub-list with
-// wave-uniform (scalar) loads of the packed records.
-// LDS at 25 KB per block, so the occupancy is set by the registers (at least 5 waves
-// per SIMD) and the blocks share the CUs with the cut kernel that runs
-// beside them on the other stream.
+// sub-list in LDS.  Each wave then walks its tile's sub-list: for the
+// Lambertian cone with 64 records at a time staged in LDS, 25 vector
+// instructions a pair; else with wave-uniform (scalar) loads of the packed
+// records.  1920x1080 pixels, 1M AVPLs, cone, beside the cut: 7.5 ms with
+// scalar loads, whose operands halve the issue rate, 5.2 staged.
+// LDS at 25 KB per block at most, so the occupancy is set by the registers (at
+// least 5 waves per SIMD) and the blocks share the CUs with the cut kernel that
+// runs beside them on the other stream.
 template <int MODEL, bool GENERAL, int kChunk>
 __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_anti_clustered(
     const float4* __restrict__ rec, arc::AvplsDev raw, const float4* __restrict__ gpos,
@@ -345,7 +354,8 @@ __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5)
     __shared__ float tface[kBlockTiles][8];  // cone: m xyz, h, s, box centre xyz
     __shared__ int tlive[kBlockTiles];
     __shared__ int tcount[kBlockTiles];
-    __shared__ int sub[kBlockTiles][kChunk];
+    __shared__ unsigned short sub[kBlockTiles][kChunk];  // places in the chunk of the list
+    __shared__ ConeLds cone[MODEL == ARC_ANTIRAD_CONE && !GENERAL ? kBlockTiles : 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int c = b / kParts, half = b % kParts;
@@ -408,12 +418,11 @@ __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5)
     const bool overflow = listed > kCap;
     const int count = overflow ? *n_anti_ptr : listed;
     const int* list = overflow ? idx : lists + (size_t)c * kCap;
-    // Entries are fetched 64 at a time, one per lane, and broadcast with
-    // readlane.  Their records are read with scalar loads four entries at a
-    // time: scalar loads complete out of order, so one wait covers a batch
-    // and the four loads overlap.  Each chunk of 64 is one plain FP32 run,
-    // Kahan-added.  (Staging each chunk's records in LDS instead measured
-    // slower: 3.8 -> 49 ms for the disk model on the 1080p x 1M frame.)
+    // Entries are fetched 64 at a time, one per lane, and (but for the
+    // Lambertian cone) broadcast with readlane.  Their records are read with
+    // scalar loads four entries at a time: scalar loads complete out of order,
+    // so one wait covers a batch and the four loads overlap.  Each chunk of 64
+    // is one plain FP32 run, Kahan-added.
     static_assert(kRun == 64, "one compensated add per 64-entry chunk");
     auto pair = [&](int i, const float4& r0, const float4& r1, const float4& r2v, const float4& r4, float& s0,
                     float& s1, float& s2) {
@@ -442,6 +451,11 @@ __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5)
     // each chunk into the tiles' sub-lists (a chunk cannot overflow them),
     // then each wave walks its tile's sub-list, so a tile never walks entries
     // its own box test rejected.
+    // The Lambertian cone's wave stages its next 64 records in LDS and reads
+    // them as vector operands, which issue at twice the rate of scalar ones.
+    const bool bare = !(P.nx == P.nx && P.ny == P.ny && P.nz == P.nz);  // a pixel without a normal accepts no pair
+    const float nx = bare ? 0.f : P.nx, ny = bare ? 0.f : P.ny, nz = bare ? 0.f : P.nz;
+    const float edge = fmaxf(kConeEps, ap.cos_half);
     Kahan ka[3];
     unsigned long long walked = 0;
     for (int cbase = 0; cbase < count; cbase += kChunk) {
@@ -464,17 +478,58 @@ __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5)
                 }
                 if (tlive[t] && ray_box_hit<MODEL>(p, w, na, ix, iy, iz, tbox[t], grow, cos_t, sin_t)) {
                     const int slot = atomicAdd(&tcount[t], 1);
-                    sub[t][slot] = i;  // slot < cend - cbase <= kChunk
+                    sub[t][slot] = (unsigned short)(j - cbase);  // slot < cend - cbase <= kChunk
                 }
             }
         }
         __syncthreads();
         const int walk = tlive[wave] ? tcount[wave] : 0;
         walked += walk;
-        for (int base = 0; base < walk; base += 64) {
+        if constexpr (MODEL == ARC_ANTIRAD_CONE && !GENERAL) {
+            ConeLds& S = cone[wave];
+            for (int base = 0; base < walk; base += 64) {
+                const int cnt = min(64, walk - base);
+                if (lane < cnt) {
+                    const int i = list[cbase + sub[wave][base + lane]];
+                    const float4* r = rec + (size_t)kRecF4 * i;
+                    const float4 r0 = r[0], r4 = r[4];
+                    const float wy = r[1].w, wz = r[2].w;
+                    // a direction that is no number accepts no pair
+                    const bool num = r0.w == r0.w && wy == wy && wz == wz;
+                    __builtin_amdgcn_wave_barrier();  // the last run's reads come first
+                    S.u[lane] = make_float4(r0.x, r0.y, r0.z, num ? r0.w : 0.f);
+                    S.v[lane] = make_float4(num ? wy : 0.f, num ? wz : 0.f, r4.x, r4.y);
+                    S.z[lane] = r4.z;
+                    S.i[lane] = i;
+                }
+                __builtin_amdgcn_wave_barrier();  // before the reads of other lanes' writes
+                float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+#pragma unroll 2
+                for (int j = 0; j < cnt; ++j) {
+                    const float4 u = S.u[j], v = S.v[j];
+                    const float az = S.z[j];
+                    const float dx = u.x - P.px, dy = u.y - P.py, dz = u.z - P.pz;
+                    const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
+                    const float cp = (nx * dx + ny * dy + nz * dz) * inv;
+                    const float c = (u.w * dx + v.x * dy + v.y * dz) * -inv;
+                    // the smaller distance from the thresholds decides, in FP64 inside the guard band
+                    const float least = fminf(c - edge, cp - kConeEps);
+                    bool in = least > 0.f;
+                    if (fabsf(least) <= kGuard) {
+                        const int i = S.i[j];
+                        in = cone_accept_f64(gpos[q], gnrm[q], raw.pos[i], raw.dir[i], ap.cos_half_d);
+                    }
+                    const float m = in ? cp * (inv * inv) : 0.f;
+                    s0 += v.z * m;
+                    s1 += v.w * m;
+                    s2 += az * m;
+                }
+                ka[0].add(s0); ka[1].add(s1); ka[2].add(s2);
+            }
+        } else for (int base = 0; base < walk; base += 64) {
             const int jj = base + lane;
             // lanes past the end hold the chunk's first entry (a valid index)
-            const int mine = jj < walk ? sub[wave][jj] : sub[wave][base];
+            const int mine = list[cbase + sub[wave][jj < walk ? jj : base]];
             const int cnt = __builtin_amdgcn_readfirstlane(min(64, walk - base));
             float s0 = 0.f, s1 = 0.f, s2 = 0.f;
             for (int u = 0; u < cnt; u += 4) {

@@ -1,0 +1,48 @@
+"""The clustered cone antiradiance's staged lists: lists shorter than a run,
+of one run and one more, images that do not fill a tile or a cluster, pixels
+without a normal, AVPLs without a direction and the guard band (pixels on
+cones' edges).  Against the exact gather, which sums the same pairs."""
+import math
+
+import numpy as np
+import pytest
+
+from antiradiancecuts_amd import ffi
+from antiradiancecuts_amd import scene as S
+from antiradiancecuts_amd.runtime import DeviceAvpls, Gather, default_params, device_array
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("w,h,n", [(1, 1, 5), (9, 7, 64), (33, 31, 65), (70, 45, 400), (130, 66, 3000)])
+@pytest.mark.parametrize("specular", [0, 12])
+@pytest.mark.parametrize("half", [math.pi / 18, 1.2])
+def test_clustered_cone_equals_exact(gpu_ctx, w, h, n, specular, half):
+    sc = S.cornell_256(seed=n, width=w, height=h, num_avpls=n)
+    sc.materials[::2, 6:9] = [0.3, 0.25, 0.2] if specular else 0
+    sc.materials[::2, 9] = specular
+    sc.avpl_anti[::2] = np.random.RandomState(n).uniform(0.1, 1, sc.avpl_anti[::2].shape).astype(np.float32)
+    sc.avpl_dir[3::7] = 0
+    sc.nrm4[5::11, :3] = 0
+    on = np.arange(0, n, 3)  # cones whose edge passes through a pixel
+    d = sc.pos4[on % sc.npix, :3] - sc.avpl_pos[on]
+    d /= np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-20)
+    side = np.cross(d, np.roll(d, 1, axis=1))
+    side /= np.maximum(np.linalg.norm(side, axis=1, keepdims=True), 1e-20)
+    sc.avpl_dir[on] = (math.cos(half) * d + math.sin(half) * side).astype(np.float32)
+    g = Gather(gpu_ctx, sc.width, sc.height, sc.materials)
+    g.set_gbuffer(device_array(sc.pos4), device_array(sc.nrm4), device_array(sc.albedo4))
+    av = DeviceAvpls.from_scene(sc)
+    out = []
+    for mode in (ffi.ARC_ANTI_EXACT, ffi.ARC_ANTI_CLUSTERED):
+        g.run(av, sc.cam, sc.extent, default_params(useLightCuts=0, antiradianceMode=mode, coneHalfAngle=half,
+                                                    antiradianceModel=ffi.ARC_ANTIRAD_CONE))
+        gpu_ctx.sync()
+        out.append(g.antiradiance[:, :3].double().cpu().numpy())
+    g.close()
+    exact, clustered = out
+    bare = ~sc.nrm4[:, :3].any(1)
+    if not specular:
+        assert not exact[bare].any() and not clustered[bare].any()
+    # both sum FP32 pairs of one sign with the same decisions: 64 plain additions at most between compensated ones
+    np.testing.assert_allclose(clustered[~bare], exact[~bare], rtol=2e-5, atol=1e-6 * np.abs(exact[~bare]).max(initial=1e-30))
