@@ -12,6 +12,7 @@ struct arc_ctx {
     int device = 0;
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
+    int* host_flag = nullptr;  // pinned: a kernel's verdict on a call's input, read after a synchronisation
     std::string last_error;
 };
 

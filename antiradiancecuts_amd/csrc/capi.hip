@@ -79,6 +79,11 @@ int arc_ctx_create(int device, arc_ctx** out) {
         return ARC_E_HIP;
     }
     c->stream = c->own_stream;
+    if (hipHostMalloc(reinterpret_cast<void**>(&c->host_flag), sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        (void)hipStreamDestroy(c->own_stream);
+        delete c;
+        return ARC_E_HIP;
+    }
     *out = c;
     return ARC_OK;
 }
@@ -90,6 +95,7 @@ void arc_ctx_destroy(arc_ctx* ctx) {
         (void)hipStreamSynchronize(ctx->own_stream);
         (void)hipStreamDestroy(ctx->own_stream);
     }
+    if (ctx->host_flag) (void)hipHostFree(ctx->host_flag);
     delete ctx;
 }
 

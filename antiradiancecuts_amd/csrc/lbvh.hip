@@ -32,7 +32,7 @@ using arc::write_cut_record;
 
 constexpr int kBlock = 256;
 constexpr int kReduceBlocks = 512;
-// arc_bvh::bounds: 12 bounds, the bounce check's flag, and the lengths of the
+// arc_bvh::bounds: 12 bounds and, from the 14th on, the lengths of the
 // range queries' lists, the points' and the normals' (zeroed by the kernel that
 // makes the Karras nodes)
 constexpr int kCounters = 13, kNumCounters = 2, kNormalList = 1;
@@ -151,11 +151,13 @@ __global__ __launch_bounds__(kBlock) void k_encode(const f3* __restrict__ pos, c
     vals[i] = i;
 }
 
-// Flags AVPLs with bounce <= 0 (they would misalign leaves and node data).
+// Flags AVPLs with bounce <= 0 (they would misalign leaves and node data) in
+// pinned host memory: a flag on the device costs a clear before and a copy
+// after, 10 us of a build.
 __global__ __launch_bounds__(kBlock) void k_check_bounce(const int* __restrict__ bounce, int n,
                                                          int* __restrict__ flag) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && bounce[i] <= 0) atomicOr(flag, 1);
+    if (i < n && bounce[i] <= 0) *flag = 1;
 }
 
 // --------------------------------------------------------- permute ----
@@ -1117,14 +1119,12 @@ namespace {
 // against the node data).
 int check_bounces(arc_bvh* b, const AvplsDev& a) {
     arc_ctx* ctx = b->ctx;
-    int* flag = reinterpret_cast<int*>(b->bounds.as<float>() + 12);
-    ARC_HIP(ctx, hipMemsetAsync(flag, 0, sizeof(int), ctx->stream));
-    hipLaunchKernelGGL(k_check_bounce, dim3(blocks_for(a.n)), dim3(kBlock), 0, ctx->stream, a.bounce, a.n, flag);
+    volatile int* flag = ctx->host_flag;
+    *flag = 0;
+    hipLaunchKernelGGL(k_check_bounce, dim3(blocks_for(a.n)), dim3(kBlock), 0, ctx->stream, a.bounce, a.n, ctx->host_flag);
     ARC_LAUNCHED(ctx);
-    int host_flag = 0;
-    ARC_HIP(ctx, hipMemcpyAsync(&host_flag, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (host_flag) {
+    if (*flag) {
         b->n = 0;
         return fail(ctx, ARC_E_INVALID, "AVPL with bounce <= 0: leaves would not match node data");
     }
