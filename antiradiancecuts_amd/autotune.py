@@ -2,13 +2,14 @@
 
 A view's frame time depends on knobs that leave its image alone (to
 rounding):
-  * launch shapes (Gather.set_launch_shape): the moment cut's traversal
-    stack, 64, 96 or 128 nodes per 8x8 tile (the deepest cut a tile can
-    refine to), and the clustered antiradiance's list entries filed into LDS
-    per pass, 768, 1536 or 3072 (the AVPL block of a pass);
-  * where the moment cut's kept nodes are estimated: in the traversal, or
-    handed to the matrix-core pass (Gather.set_estimate_pool, 0 or 32
-    chunks per tile);
+  * launch shapes (Gather.set_launch_shape): a traversal stack of 64, 96 or
+    128 nodes (kept for callers that name one: the moment cut's traversal
+    needs no depth any more, so these candidates time the same), and the
+    clustered antiradiance's list entries filed into LDS per pass, 768, 1536
+    or 3072 (the AVPL block of a pass);
+  * the moment cut's pool of kept nodes (Gather.set_estimate_pool): sized to
+    what the frames ask for, or held to 32 chunks per tile (less memory;
+    tiles that find it full are cut node by node);
   * for the centroid estimator, the cut per 8x8 tile or per pixel and the
     depth of the estimate cut that sets each pixel's threshold (these move
     the cut a little).

@@ -79,11 +79,6 @@ int arc_ctx_create(int device, arc_ctx** out) {
         return ARC_E_HIP;
     }
     c->stream = c->own_stream;
-    if (hipHostMalloc(reinterpret_cast<void**>(&c->host_flag), sizeof(int), hipHostMallocDefault) != hipSuccess) {
-        (void)hipStreamDestroy(c->own_stream);
-        delete c;
-        return ARC_E_HIP;
-    }
     *out = c;
     return ARC_OK;
 }

@@ -340,9 +340,8 @@ struct ConeLds {  // a run's records: position, unit direction, antiradiance, in
 // instructions a pair; else with wave-uniform (scalar) loads of the packed
 // records.  1920x1080 pixels, 1M AVPLs, cone, beside the cut: 7.5 ms with
 // scalar loads, whose operands halve the issue rate, 5.2 staged.
-// LDS at 25 KB per block at most, so the occupancy is set by the registers (at
-// least 5 waves per SIMD) and the blocks share the CUs with the cut kernel that
-// runs beside them on the other stream.
+// The blocks share the CUs with the cut kernel that runs beside them on the
+// other stream.
 template <int MODEL, bool GENERAL, int kChunk>
 __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_anti_clustered(
     const float4* __restrict__ rec, arc::AvplsDev raw, const float4* __restrict__ gpos,
@@ -576,9 +575,13 @@ void launch_pixels(arc_gather* g, const arc::AvplsDev& a, int cw, int C, float3 
                            cam.y, cam.z, ap, g->ccount.as<int>(), g->clist.as<int>(), g->anti_idx.as<int>(),
                            n_anti_ptr, grow, cos_t, sin_t, part, counters);
     };
-    // list entries filed per pass: a launch-shape setting (LDS against passes)
-    if (g->anti_chunk == 768) launch(k_anti_clustered<MODEL, GENERAL, 768>);
-    else if (g->anti_chunk == 3072) launch(k_anti_clustered<MODEL, GENERAL, 3072>);
+    // list entries filed per pass: a launch-shape setting (LDS against passes).
+    // Beside the cut's kernels the Lambertian cone's blocks do best at 34 KB,
+    // with half of the CU's waves (1080p, 1M AVPLs: 26.2 ms a frame with 3072
+    // entries, 28.0 with 1536); alone and for the disk model they cost alike.
+    const int chunk = g->anti_chunk ? g->anti_chunk : MODEL == ARC_ANTIRAD_CONE && !GENERAL ? 3072 : kSub;
+    if (chunk == 768) launch(k_anti_clustered<MODEL, GENERAL, 768>);
+    else if (chunk == 3072) launch(k_anti_clustered<MODEL, GENERAL, 3072>);
     else launch(k_anti_clustered<MODEL, GENERAL, kSub>);
 }
 

@@ -101,7 +101,7 @@ struct arc_gather {
     arc::CutPoolMem pool;
     // a launch shape the results do not depend on: the clustered
     // antiradiance's list entries filed per pass (768, 1536 or 3072)
-    int anti_chunk = 1536;
+    int anti_chunk = 0;  // list entries filed per pass; 0: the kernel's own choice
     arc_cutnet* net = nullptr;  // learned cut: the predictor (borrowed)
     arc_bvh* bvh = nullptr;
     // per-frame phase events: frame slot, then 9 marks (start, upload done,

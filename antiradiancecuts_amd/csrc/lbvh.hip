@@ -1119,6 +1119,8 @@ namespace {
 // against the node data).
 int check_bounces(arc_bvh* b, const AvplsDev& a) {
     arc_ctx* ctx = b->ctx;
+    if (!ctx->host_flag)
+        ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocDefault));
     volatile int* flag = ctx->host_flag;
     *flag = 0;
     hipLaunchKernelGGL(k_check_bounce, dim3(blocks_for(a.n)), dim3(kBlock), 0, ctx->stream, a.bounce, a.n, ctx->host_flag);

@@ -243,14 +243,14 @@ class Gather:
         self._net = net
 
     def set_estimate_pool(self, chunks_per_tile: int) -> None:
-        """The moment cut's pool of kept nodes for the matrix-core pass, in
-        chunks of 128 per tile (0: every node estimated in the traversal)."""
+        """The moment cut's pool of kept nodes, in chunks of 128 per 8x8 tile
+        (0: sized from the tree, grown to what the last frame asked for)."""
         check(self.lib.arc_gather_set_estimate_pool(self.h, int(chunks_per_tile)), "arc_gather_set_estimate_pool",
               self.ctx.h)
 
     def set_launch_shape(self, cut_stack: int = 96, anti_chunk: int = 1536) -> None:
-        """The moment cut's traversal stack (64, 96, 128 nodes) and the
-        clustered antiradiance's list entries filed per pass (768, 1536,
+        """A traversal stack (64, 96, 128 nodes: accepted, without effect) and
+        the clustered antiradiance's list entries filed per pass (768, 1536,
         3072); neither changes the image beyond rounding."""
         check(self.lib.arc_gather_set_launch_shape(self.h, int(cut_stack), int(anti_chunk)),
               "arc_gather_set_launch_shape", self.ctx.h)

@@ -119,7 +119,7 @@ def parse(argv=None):
                     help="autotune the frame's (or each batched view's) schedule before timing (1) or not (0)")
     ap.add_argument("--schedule", default="",
                     help="cut_stack,anti_chunk,estimate_pool: a fixed schedule instead of the tuner's "
-                         "(e.g. 96,1536,32 estimates the kept nodes on the matrix cores)")
+                         "(e.g. 96,1536,32 holds the moment cut to a pool of 32 chunks per tile)")
     return ap.parse_args(argv)
 
 
@@ -177,7 +177,7 @@ def main() -> int:
     cone = args.antiradiance == "cone"
     params = frame_params(args)
     flags = ffi.ARC_RUN_TIMELINE | ffi.ARC_TRUST_INPUT
-    # the schedule: launch shapes and estimate pool, fixed or tuned on the frame (untimed)
+    # the schedule: launch shapes and the cut's pool, fixed or tuned on the frame (untimed)
     from antiradiancecuts_amd import autotune
     tune_table = None
     if args.schedule:
@@ -256,7 +256,7 @@ def main() -> int:
         exact = float(st.exactLeaves)
         flop_rad = float(st.testedNodes) * (FLOP_MOM_TEST_EXP if args.criterion == "expansion" else FLOP_MOM_TEST) \
             + (float(st.evaluatedNodes) - exact) * FLOP_MOM_EST + exact * FLOP_RAD_PAIR
-        rad_name = "k_cut_mom_tile"
+        rad_name = "k_cut_decide + k_cut_eval"
     elif eb:
         flop_rad = float(st.testedNodes) * FLOP_EB_TEST + float(st.evaluatedNodes) * FLOP_EB_EST
         rad_name = "k_cut_eb_tile" if args.per_tile else "k_cut_eb_px"
@@ -400,10 +400,10 @@ def main() -> int:
 
 # the PMC summary of the benchmark frame (moment estimates, cone antiradiance)
 TRAFFIC_PROFILE = ROOT / "profiles" / "frame_1080p_1M_cone_moments_traffic.txt"
-# LBVH kernels of one rebuild, with their dispatch counts (4 radix passes)
+# LBVH kernels of one rebuild, with their dispatch counts (4 radix passes; spans of 8K, 64K, 512K and 4M leaves)
 BVH_KERNELS = {"k_bounds_partial": 1, "k_bounds_final": 1, "k_encode": 1, "k_hist": 4, "k_scan_digit": 4,
                "k_scatter": 4, "k_stage_avpls": 1, "k_permute_cut": 1, "k_karras": 1,
-               "k_refit_local<2>": 1, "k_refit_mid<2>": 1, "k_refit_top<2>": 1}
+               "k_refit_local<2>": 1, "k_refit_span<2>": 4}
 
 
 def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mom: bool = False, cone: bool = False):
@@ -423,13 +423,11 @@ def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mo
         stem = f"k_anti_clustered<{1 if cone else 0}, false"
         names = {next((k for k in table if k.startswith(stem)), stem + ">"): 1}
     elif dom == "radiance":
-        name = "k_cut_mom_tile" if mom else ("k_cut_eb_tile" if per_tile else "k_cut_eb_px") if eb else "k_cut_sa"
-        own = next((k for k in table if k.startswith(f"{name}<false")), None) if mom else None
-        if own:  # the traversal that estimates its kept nodes itself (any stack depth)
-            name = own
-        elif eb and per_tile and f"{name}<{eval_depth}>" in table:
+        name = ("k_cut_eb_tile" if per_tile else "k_cut_eb_px") if eb else "k_cut_sa<false>"
+        if eb and per_tile and f"{name}<{eval_depth}>" in table:
             name = f"{name}<{eval_depth}>"
-        names = {name: 1}
+        names = {k: 1 for k in ("k_cut_decide<false, false>", "k_cut_eval<false>", "k_cut_combine<false>")} if mom \
+            else {name: 1}
     else:
         names = BVH_KERNELS
     if not all(k in table for k in names if names[k] == 1 and k != "k_bounds_final"):
@@ -692,7 +690,7 @@ def bench_exact(args) -> int:
             "vs_baseline": None, "dtype": "f32", "data": "synthetic",
             "config": {"workload": "cornell_256: 256x256 G-buffer, 4096 AVPLs (seed 0), exact radiance + exact "
                                    "cone antiradiance, Kahan-compensated", "rel_l2_vs_f64": err},
-            "roofline": {"kernel": "k_exact (radiance and antiradiance pairs)", "bound": COMPUTE_BOUND,
+            "roofline": {"kernel": "k_exact_lambert (radiance and antiradiance pairs)", "bound": COMPUTE_BOUND,
                          "engine": "VALU",
                          "achieved": round(ach, 3), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(ach / PEAK_FP32_TFLOPS, 4), "traffic": None, "ms": round(ms, 4)},

@@ -385,8 +385,9 @@ int arc_gather_set_estimate_pool(arc_gather* g, int chunks_per_tile);
  * searched by its autotuner).  cut_stack: 64, 96 or 128 (accepted; the moment
  * cut's traversal needs no depth setting any more).  anti_chunk: the clustered
  * antiradiance's list entries filed into the tiles' LDS sub-lists per pass
- * (768, 1536 or 3072; default 1536): more per pass is fewer passes and more
- * LDS per workgroup.  Neither changes the image beyond rounding.  Read by the
+ * (768, 1536 or 3072; until it is set, 3072 for the cone model over Lambertian
+ * materials and else 1536): more per pass is fewer passes and more LDS per
+ * workgroup.  Neither changes the image beyond rounding.  Read by the
  * next frame.  ARC_E_INVALID for other values. */
 int arc_gather_set_launch_shape(arc_gather* g, int cut_stack, int anti_chunk);
 /* Training rows of one frame: builds the frame's AvplBvh and thresholds as
@@ -426,7 +427,7 @@ arc_ctx* arc_batch_lane(arc_batch* b, int lane);
 int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews);
 /* When every view's radiance is the moment cut (ARC_ESTIMATOR_MOMENTS), the
  * captured graph runs the views' cuts as one launch over all views' tiles,
- * heaviest first (on = 1), or one launch per view (on = 0, the default).  No
+ * in view order (on = 1), or one launch per view (on = 0, the default).  No
  * counterpart in the reference, which renders one view per run; read at the
  * next arc_batch_capture. */
 int arc_batch_set_one_cut_launch(arc_batch* b, int on);
