@@ -1531,7 +1531,7 @@ int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, lo
     }
     // a small image's tiles can hold 512 chunks each (a budget of 65536): no small pools
     want = std::max(want, std::min((long long)kMinChunks, 512LL * nitems));
-    if (want > INT_MAX / kKeep) want = INT_MAX / kKeep;
+    want = std::min(want, (long long)(INT_MAX >> kPartBits));  // a chunk's entries and part share a word (67M: 87 GB)
     // one allocation: a new gather's first frame pays for each
     const size_t chunk = (size_t)want, part = sizeof(float) * 192 * chunk, entries = sizeof(uint32_t) * kKeep * chunk,
                  meta = sizeof(int4) * chunk;
