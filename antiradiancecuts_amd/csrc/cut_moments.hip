@@ -1261,7 +1261,13 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_combine(Views<kMany> views,
     const int lane = threadIdx.x & 63;
     const int item = uniform(blockIdx.x * (kCutThreads / 64) + (threadIdx.x >> 6));
     if (item >= nitems) return;
-    if (item == 0 && lane == 0) *pool.seen = *pool.taken;  // what the next frame's pool should hold
+    if (item == 0 && lane == 0) {
+        // what the next frame's pool should hold: the tiles that found it full
+        // need as much as the others, as far as is known (the count alone grows
+        // by what is asked for until it is full, a quarter per frame)
+        const int taken = *pool.taken, rest = max(1, nitems - *pool.nserial);
+        *pool.seen = (int)fminf((float)taken * fminf((float)nitems / (float)rest, 8.f), 1e9f);
+    }
     const CutView v = views.of(item);
     const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
     const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
