@@ -576,9 +576,10 @@ void launch_pixels(arc_gather* g, const arc::AvplsDev& a, int cw, int C, float3 
                            n_anti_ptr, grow, cos_t, sin_t, part, counters);
     };
     // list entries filed per pass: a launch-shape setting (LDS against passes).
-    // Beside the cut's kernels the Lambertian cone's blocks do best at 34 KB,
-    // with half of the CU's waves (1080p, 1M AVPLs: 26.2 ms a frame with 3072
-    // entries, 28.0 with 1536); alone and for the disk model they cost alike.
+    // The Lambertian cone's kernel wants 110 registers: with 3072 entries, 34 KB,
+    // four waves per SIMD are what the LDS allows and it gets them; with fewer it
+    // is held to 96 and spills 17 (1080p, 1M AVPLs: 0.9 GB of traffic and 26.2 ms
+    // a frame against 2.0 GB and 28.0 with 1536).  The other models cost alike.
     const int chunk = g->anti_chunk ? g->anti_chunk : MODEL == ARC_ANTIRAD_CONE && !GENERAL ? 3072 : kSub;
     if (chunk == 768) launch(k_anti_clustered<MODEL, GENERAL, 768>);
     else if (chunk == 3072) launch(k_anti_clustered<MODEL, GENERAL, 3072>);

@@ -286,11 +286,13 @@ def main() -> int:
         roof = {"kernel": name, "bound": COMPUTE_BOUND, "engine": "VALU", "achieved": round(ach, 3),
                 "peak": PEAK_FP32_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(ach / PEAK_FP32_TFLOPS, 4),
-                "traffic": profiled_traffic(dom, eb, bool(args.per_tile), args.eval_depth, mom, cone), "ms": round(t_dom, 4),
+                "traffic": profiled_traffic(dom, eb, bool(args.per_tile), args.eval_depth, mom, cone, sched.anti_chunk),
+                "ms": round(t_dom, 4),
                 "kernels": per_kernel}
     elif t_pair >= t_bvh and t_pair > 0.0:
         ach = (flop_rad + flop_anti) / (t_pair * 1e-3) / 1e12
-        tr = [profiled_traffic(k, eb, bool(args.per_tile), args.eval_depth, mom, cone) for k in ("radiance", "antiradiance")]
+        tr = [profiled_traffic(k, eb, bool(args.per_tile), args.eval_depth, mom, cone, sched.anti_chunk)
+              for k in ("radiance", "antiradiance")]
         roof = {"kernel": f"{rad_name} + k_anti_clustered (concurrent on two streams)", "bound": COMPUTE_BOUND,
                 "engine": "VALU",
                 "achieved": round(ach, 3), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
@@ -406,7 +408,8 @@ BVH_KERNELS = {"k_bounds_partial": 1, "k_bounds_final": 1, "k_encode": 1, "k_his
                "k_refit_local<2>": 1, "k_refit_span<2>": 4}
 
 
-def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mom: bool = False, cone: bool = False):
+def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mom: bool = False, cone: bool = False,
+                     anti_chunk: int = 1536):
     """HBM bytes per launch of the dominant kernel on the 1080p x 1M frame,
     from the committed rocprofv3 PMC summary (FETCH_SIZE + WRITE_SIZE scaled
     by a plain copy's readings); None when the summary does not cover it."""
@@ -421,7 +424,8 @@ def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mo
     if dom == "antiradiance":
         # the kernel's name, with or without its list-block template argument
         stem = f"k_anti_clustered<{1 if cone else 0}, false"
-        names = {next((k for k in table if k.startswith(stem)), stem + ">"): 1}
+        own = f"{stem}, {anti_chunk}>"
+        names = {own if own in table else next((k for k in table if k.startswith(stem)), stem + ">"): 1}
     elif dom == "radiance":
         name = ("k_cut_eb_tile" if per_tile else "k_cut_eb_px") if eb else "k_cut_sa<false>"
         if eb and per_tile and f"{name}<{eval_depth}>" in table:
