@@ -1,8 +1,8 @@
 // Stable LSD radix sort of (uint32 key, int32 value) pairs for the LBVH key
 // sort (replaces thrust::sort_by_key, bvh.cu:795-807 / 888-894).
 //
-// One pass per 8-bit digit, three kernels per pass, over tiles of
-// kSortTile keys:
+// One pass per 8-bit digit, three kernels per pass (two over few tiles), over
+// tiles of kSortTile keys:
 //   hist    — each 512-thread block counts the digits of its tile; lanes
 //             with equal digits are found with 8 wave ballots, so only one
 //             lane per (wave, digit) touches LDS.
@@ -26,8 +26,15 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kTile = arc::kSortTile;
 constexpr int kItems = kTile / kThreads;
 constexpr int kRadix = arc::kSortRadix;
-constexpr int kScanThreads = 256;
-static_assert(kTile % kThreads == 0 && kRadix <= kThreads, "sort tile shape");
+constexpr int kScanThreads = 512;
+static_assert(kTile % kThreads == 0 && 2 * kRadix == kThreads, "sort tile shape");
+
+// Up to this many tiles the scatter adds the tiles' counts up itself, a row of
+// 256 per tile, instead of a scan kernel between: tiles loads per digit and
+// block against a launch.  Builds over random points, with the sums and with
+// the scan: 5000 points 68 us and 78, 65536 78 and 87, 131072 (64 tiles) 88 and
+// 92, 196608 97 and 98, 262144 105 and 103, 1M 221 and 174.
+constexpr int kFewTiles = 64;
 
 __device__ inline uint64_t match_digit(uint64_t active, uint32_t digit) {
     uint64_t m = active;
@@ -40,6 +47,7 @@ __device__ inline uint64_t match_digit(uint64_t active, uint32_t digit) {
     return m;
 }
 
+template <bool kFew>
 __global__ __launch_bounds__(kThreads) void k_hist(const uint32_t* __restrict__ keys, int n, int shift,
                                                    uint32_t* __restrict__ counts, int num_tiles) {
     __shared__ uint32_t h[kRadix];
@@ -58,7 +66,7 @@ __global__ __launch_bounds__(kThreads) void k_hist(const uint32_t* __restrict__ 
         if (valid && lower == 0ull) atomicAdd(&h[digit], (uint32_t)__popcll(m));
     }
     __syncthreads();
-    if (tid < kRadix) counts[(size_t)tid * num_tiles + blockIdx.x] = h[tid];
+    if (tid < kRadix) counts[kFew ? (size_t)blockIdx.x * kRadix + tid : (size_t)tid * num_tiles + blockIdx.x] = h[tid];
 }
 
 // Exclusive scan of one value per thread over the first kRadix threads (whole
@@ -78,32 +86,63 @@ __device__ inline uint32_t radix_exclusive_scan(uint32_t v, uint32_t* sums) {
     return before + x - v;
 }
 
+// Thread tid's digit tid % kRadix in every second tile from tid / kRadix on:
+// the digit's keys in those before `tile` and in all of them.  Sixteen loads
+// are in flight at a time.
+__device__ inline void sum_tiles(const uint32_t* __restrict__ counts, int tile, int num_tiles, uint32_t& before,
+                                 uint32_t& all) {
+    const int d = threadIdx.x % kRadix;
+    before = all = 0;
+    for (int t0 = threadIdx.x / kRadix; t0 < num_tiles; t0 += 32) {
+        uint32_t c[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) c[j] = t0 + 2 * j < num_tiles ? counts[(size_t)(t0 + 2 * j) * kRadix + d] : 0u;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            all += c[j];
+            before += t0 + 2 * j < tile ? c[j] : 0u;
+        }
+    }
+}
+
 // Block d scans row d of the digit-major count table (exclusive, in place)
-// and writes the digit's total count.
+// and writes the digit's total count.  Bound by latency: the scan is in
+// registers per wave and one barrier per 512 tiles joins the waves (with a
+// scan in LDS of 16 barriers per 256 tiles a build over 1M points took 173.6
+// us, 168.2 here).
 __global__ __launch_bounds__(kScanThreads) void k_scan_digit(uint32_t* __restrict__ counts, int num_tiles,
                                                             uint32_t* __restrict__ totals) {
-    __shared__ uint32_t sh[kScanThreads];
-    const int tid = threadIdx.x;
+    __shared__ uint32_t sums[2][kScanThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint32_t* row = counts + (size_t)blockIdx.x * num_tiles;
     uint32_t run = 0;
-    for (int base = 0; base < num_tiles; base += kScanThreads) {
+    for (int base = 0, k = 0; base < num_tiles; base += kScanThreads, k ^= 1) {
         const int t = base + tid;
         const uint32_t v = t < num_tiles ? row[t] : 0u;
-        sh[tid] = v;
-        __syncthreads();
-        for (int off = 1; off < kScanThreads; off <<= 1) {
-            const uint32_t u = tid >= off ? sh[tid - off] : 0u;
-            __syncthreads();
-            sh[tid] += u;
-            __syncthreads();
+        uint32_t x = v;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t u = __shfl_up(x, off);
+            if (lane >= off) x += u;
         }
-        if (t < num_tiles) row[t] = run + sh[tid] - v;
-        run += sh[kScanThreads - 1];
-        __syncthreads();
+        if (lane == 63) sums[k][wave] = x;
+        __syncthreads();  // two sets of sums: the next round's writes are a barrier behind this one's reads
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < kScanThreads / 64; ++w) {
+            const uint32_t c = sums[k][w];
+            before += w < wave ? c : 0u;
+            all += c;
+        }
+        if (t < num_tiles) row[t] = run + before + x - v;
+        run += all;
     }
     if (tid == 0) totals[blockIdx.x] = run;
 }
 
+// kFew: offsets are k_hist's counts, a row per tile; else the scanned table, a
+// row per digit, and totals.
+template <bool kFew>
 __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict__ keys_in,
                                                       const int* __restrict__ vals_in,
                                                       uint32_t* __restrict__ keys_out,
@@ -115,6 +154,7 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict
     __shared__ uint32_t out_start[kRadix];      // output place of a digit's keys minus their place in the tile
     __shared__ uint32_t wcount[kWaves][kRadix];  // keys of each digit per wave, then where the wave's start in the tile
     __shared__ uint32_t sums[2][kRadix / 64];
+    __shared__ uint2 odd[kFew ? kRadix : 1];  // the second half's sums of sum_tiles
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
@@ -134,7 +174,10 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict
         val[j] = i < tile_n ? vals_in[base + i] : 0;
     }
     uint32_t off = 0, total = 0;
-    if (tid < kRadix) {
+    if constexpr (kFew) {
+        sum_tiles(offsets, tile, num_tiles, off, total);
+        if (tid >= kRadix) odd[tid - kRadix] = make_uint2(off, total);
+    } else if (tid < kRadix) {
         // the tile's place within each digit (the scanned count table)
         off = offsets[(size_t)tid * num_tiles + tile];
         total = totals[tid];
@@ -161,6 +204,10 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict
         for (int w = 0; w < kWaves; ++w) {
             count[w] = wcount[w][tid];
             mine += count[w];
+        }
+        if constexpr (kFew) {
+            off += odd[tid].x;
+            total += odd[tid].y;
         }
     }
     const uint32_t digit_base = radix_exclusive_scan(total, sums[0]);
@@ -212,12 +259,19 @@ int sort_pairs(arc_ctx* ctx, SortScratch& s, uint32_t* keys, int* vals, int n, i
     uint32_t* totals = counts + (size_t)kRadix * num_tiles;
     for (int p = 0; p < passes; ++p) {
         const int shift = 8 * p;
-        hipLaunchKernelGGL(k_hist, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, n, shift,
-                           counts, num_tiles);
-        hipLaunchKernelGGL(k_scan_digit, dim3(kRadix), dim3(kScanThreads), 0, ctx->stream, counts, num_tiles,
-                           totals);
-        hipLaunchKernelGGL(k_scatter, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, vin,
-                           kout, vout, n, shift, counts, totals, num_tiles);
+        if (num_tiles <= kFewTiles) {
+            hipLaunchKernelGGL(k_hist<true>, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, n, shift,
+                               counts, num_tiles);
+            hipLaunchKernelGGL(k_scatter<true>, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, vin,
+                               kout, vout, n, shift, counts, totals, num_tiles);
+        } else {
+            hipLaunchKernelGGL(k_hist<false>, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, n, shift,
+                               counts, num_tiles);
+            hipLaunchKernelGGL(k_scan_digit, dim3(kRadix), dim3(kScanThreads), 0, ctx->stream, counts, num_tiles,
+                               totals);
+            hipLaunchKernelGGL(k_scatter<false>, dim3(num_tiles), dim3(kThreads), 0, ctx->stream, kin, vin,
+                               kout, vout, n, shift, counts, totals, num_tiles);
+        }
         ARC_LAUNCHED(ctx);
         std::swap(kin, kout);
         std::swap(vin, vout);

@@ -434,9 +434,10 @@ def profiled_traffic(dom: str, eb: bool, per_tile: bool, eval_depth: int = 0, mo
             else {name: 1}
     else:
         names = BVH_KERNELS
-    if not all(k in table for k in names if names[k] == 1 and k != "k_bounds_final"):
+    if not all(k in table or f"{k}<false>" in table for k in names if names[k] == 1 and k != "k_bounds_final"):
         return None
-    return float(sum(table.get(k, 0.0) * c for k, c in names.items()))
+    # (the sort's kernels with or without their template argument)
+    return float(sum(table.get(k, table.get(f"{k}<false>", 0.0)) * c for k, c in names.items()))
 
 
 def bench_trace(args) -> int:

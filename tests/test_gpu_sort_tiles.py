@@ -32,3 +32,25 @@ def test_sorted_and_stable(gpu_ctx, orc, n, kind):
     np.testing.assert_array_equal(g["perm"], order)
     np.testing.assert_array_equal(g["codes"], code[order])
     np.testing.assert_array_equal(g["codes"], orc.lbvh_build(p)["codes"])
+
+
+@pytest.mark.parametrize("kind", ["random", "two"])
+@pytest.mark.parametrize("n", [129_025, 131_071, 131_072, 131_073, 133_121, 1_048_576, 1_048_577, 2_097_153])
+def test_tile_counts(gpu_ctx, n, kind):
+    """At 64 tiles, the most whose counts the scatter sums itself, and at 512
+    and 1024, a block's width of the scan once and twice."""
+    rng = np.random.RandomState(n)
+    p = rng.rand(n, 3).astype(np.float32)
+    if kind == "two":
+        p[:] = p[rng.randint(0, 2, n)]
+    b = Bvh(gpu_ctx)
+    try:
+        b.build_points(device_array(p))
+        g = b.to_host()
+    finally:
+        b.close()
+    assert np.array_equal(np.bincount(g["perm"], minlength=n), np.ones(n, np.int64))
+    code = np.empty(n, np.uint32)
+    code[g["perm"]] = g["codes"]
+    np.testing.assert_array_equal(g["perm"], np.argsort(code, kind="stable"))
+    assert np.all(np.diff(g["codes"].astype(np.int64)) >= 0)
