@@ -23,6 +23,7 @@
 // combine.  A small view then adds its tiles to the launch instead of leaving
 // the GPU to a short kernel of its own.
 #include <algorithm>
+#include <memory>
 #include <vector>
 
 #include "gather_common.hpp"
@@ -43,6 +44,9 @@ struct arc_batch {
     std::vector<arc::CutView> views;       // the views' descriptors
     arc::DevBuf views_dev;                 // the same on the device
     arc::CutPoolMem pool;
+    // the pools' blocks whose addresses the graph has: an eager frame of a
+    // view's gather may grow the gather's pool into another block meanwhile
+    std::vector<std::shared_ptr<void>> held;
 };
 
 namespace {
@@ -50,10 +54,14 @@ namespace {
 constexpr int kMaxLanes = 8;
 
 void drop_graph(arc_batch* b) {
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->exec) {
+        (void)hipStreamSynchronize(b->ctx->stream);  // a replay still running uses the blocks held
+        (void)hipGraphExecDestroy(b->exec);
+    }
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->exec = nullptr;
     b->graph = nullptr;
+    b->held.clear();
     b->nviews = 0;
 }
 
@@ -205,7 +213,10 @@ int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews) {
     if (!one_cut) {
         for (int i = 0; st == ARC_OK && i < nviews; ++i) {
             const arc_batch_view& v = views[i];
+            v.gather->batch_capture = true;
             st = arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr);
+            v.gather->batch_capture = false;
+            b->held.push_back(v.gather->pool.mem.hold());
         }
         if (st == ARC_OK) st = join_lanes(b, b->origin, b->join);
     } else {
@@ -223,6 +234,7 @@ int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews) {
     if (st == ARC_OK && ee != hipSuccess) st = arc::hip_fail(ctx, ee, "hipStreamEndCapture", __FILE__, __LINE__);
     if (st != ARC_OK) {
         if (g) (void)hipGraphDestroy(g);
+        b->held.clear();
         for (int i = 0; i < nviews; ++i) views[i].gather->deferred = false;
         return st;
     }

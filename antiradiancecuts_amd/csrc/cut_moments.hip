@@ -1522,15 +1522,17 @@ constexpr int kMinChunks = 16384;  // 21 MB
 // Readies `mem` for nitems tiles: the chunks of `per_tile` per tile, or as
 // many as the last frame asked for when that was more (read from pinned
 // memory that k_cut_combine writes: a frame still running counts at the next
-// one).  Nothing grows while the stream is captured.
-int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, long long want, bool grow, CutPool& p) {
+// one).  Nothing grows while the stream is captured; held: the caller keeps
+// the memory with the graph.
+int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, long long want, bool grow, bool held,
+               CutPool& p) {
     if (!mem.seen) {
         ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&mem.seen), sizeof(int), hipHostMallocDefault));
         *mem.seen = 0;
     }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
     if (grow) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
         const int seen = *static_cast<volatile int*>(mem.seen);
         want = std::max(want, (long long)mem.cap);
         if (capture == hipStreamCaptureStatusNone && seen > want) want = (long long)seen + seen / 4;
@@ -1541,10 +1543,14 @@ int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, lo
     // one allocation: a new gather's first frame pays for each
     const size_t chunk = (size_t)want, part = sizeof(float) * 192 * chunk, entries = sizeof(uint32_t) * kKeep * chunk,
                  meta = sizeof(int4) * chunk;
-    ARC_TRY(ensure(ctx, mem.buf, part + entries + meta +
-                                     sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1))));
+    const size_t bytes = part + entries + meta + sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1));
+    hipError_t e = hipSuccess;
+    const bool got = mem.mem.reserve(bytes, [&] { e = hipStreamSynchronize(ctx->stream); });
+    if (!got) return fail(ctx, ARC_E_NOMEM, "out of device memory for the moment cut's pool");
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize", __FILE__, __LINE__);
+    if (capture != hipStreamCaptureStatusNone && !held) mem.mem.keep();
     mem.cap = (int)want;
-    char* at = mem.buf.as<char>();
+    char* at = static_cast<char*>(mem.mem.data());
     float* tbox = reinterpret_cast<float*>(at + part + entries + meta);
     int* head = reinterpret_cast<int*>(tbox + 8 * (size_t)nitems);
     p = CutPool{reinterpret_cast<uint32_t*>(at + part), reinterpret_cast<int4*>(at + part + entries),
@@ -1583,8 +1589,15 @@ void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool 
 
 }  // namespace
 
+void* PoolDevice::alloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+void PoolDevice::free(void* p) { (void)hipFree(p); }
+
 void release_pool(CutPoolMem& mem) {
-    release(mem.buf);
     if (mem.seen) (void)hipHostFree(mem.seen);
     mem = CutPoolMem{};
 }
@@ -1615,7 +1628,7 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
     CutPool pool{};
     if (!serial) {
         const long long per_tile = g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);
-        ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, pool));
+        ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, g->batch_capture, pool));
     }
     if (mark) ARC_HIP(ctx, hipEventRecord(mark, ctx->stream));
     launch_cut<false>(ctx->stream, Views<false>{v}, nitems, cp.criterion == ARC_CRITERION_EXPANSION, serial, pool);
@@ -1636,7 +1649,7 @@ int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_view
         expansion = expansion || host_views[i].criterion == ARC_CRITERION_EXPANSION;
     }
     CutPool pool{};
-    ARC_TRY(ready_pool(ctx, stream, mem, nitems, want, true, pool));
+    ARC_TRY(ready_pool(ctx, stream, mem, nitems, want, true, true, pool));
     launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, serial, pool);
     ARC_LAUNCHED(ctx);
     return ARC_OK;

@@ -822,11 +822,18 @@ void finalize(arc_gather* g, int rad_splits, int anti_splits, int npix, float4* 
     else launch(k_finalize<1>, 1);
 }
 
+// g->crec for n AVPLs: one size for every cut's records, so that a frame of
+// another cut does not move the buffer from under a captured graph.
+int ensure_records(arc_gather* g, int n) {
+    static_assert(kSaLeaf + kSaNode <= 2 * arc::kCrec, "the solid-angle cut's records fit");
+    return arc::ensure(g->ctx, g->crec, sizeof(float4) * 2 * arc::kCrec * (size_t)n);
+}
+
 // This frame's LBVH for the error-bound and learned cuts, with their node
 // records in g->crec.
 int build_cut_tree(arc_gather* g, const arc::AvplsDev& a, bool validate) {
     g->mom_ready = false;
-    if (a.n > 1) ARC_TRY(arc::ensure(g->ctx, g->crec, sizeof(float4) * arc::kCrec * (size_t)(2 * a.n - 1)));
+    if (a.n > 1) ARC_TRY(ensure_records(g, a.n));
     return arc::bvh_build_cut(g->bvh, a, validate, g->mats.as<arc_material>(), g->crec.as<float4>());
 }
 
@@ -1161,7 +1168,7 @@ int arc_gather_run(arc_gather* g, const arc_avpls* avpls, arc_float3 camPos, flo
             if (profile) ARC_HIP(ctx, hipEventRecord(ev[6], ctx->stream));
             CutTree t{b->nodes.as<arc_bvh_node>(), b->nd_mat.as<int>(), b->nd_pos.as<f3>(), b->nd_nrm.as<f3>(),
                       b->nd_rad.as<f3>(), b->nd_dir.as<f3>(), b->n};
-            ARC_TRY(arc::ensure(ctx, g->crec, sizeof(float4) * ((kSaLeaf + kSaNode) * (size_t)t.n)));
+            ARC_TRY(ensure_records(g, t.n));
             float4* rec = g->crec.as<float4>();
             hipLaunchKernelGGL(k_sa_records, dim3(blocks(2LL * t.n - 1)), dim3(kThreads), 0, ctx->stream, t,
                                g->mats.as<arc_material>(), sa_band(p->clusterRefinementThreshold), rec);

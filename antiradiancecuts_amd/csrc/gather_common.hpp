@@ -8,6 +8,7 @@
 #include <algorithm>
 
 #include "arc_internal.hpp"
+#include "cut_pool.hpp"
 #include "gather_math.hpp"
 
 namespace arc {
@@ -60,9 +61,12 @@ struct CutPool {
                         // some unused, which the evaluation has to pass over
 };
 
-// The pool's memory, kept between launches.
+struct PoolDevice {
+    static void* alloc(size_t bytes);
+    static void free(void* p);
+};
 struct CutPoolMem {
-    DevBuf buf;
+    PoolMemory<PoolDevice> mem;
     int* seen = nullptr;
     int cap = 0;
 };
@@ -99,6 +103,7 @@ struct arc_gather {
     // sets its chunks per tile, 0 sizes it from the tree and the last frame
     int est_chunks = 0;
     arc::CutPoolMem pool;
+    bool batch_capture = false;  // the frame is being captured by arc_batch, which holds the pool's memory itself
     // a launch shape the results do not depend on: the clustered
     // antiradiance's list entries filed per pass (768, 1536 or 3072)
     int anti_chunk = 0;  // list entries filed per pass; 0: the kernel's own choice
@@ -348,7 +353,7 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
 // The moment cuts of many views in one set of launches (host_views and its
 // device copy `views`).
 int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_views, const CutView* views, int nviews,
-                      CutPoolMem& mem);
+                      CutPoolMem& mem);  // the caller holds mem's block with a graph it captures this into
 // Whether the last frame asked for more chunks than the gather's pool holds
 // (its remaining tiles were cut serially; the next eager frame grows it).
 // The frame must have ended.
