@@ -1523,40 +1523,44 @@ constexpr int kMinChunks = 16384;  // 21 MB
 // many as the last frame asked for when that was more (read from pinned
 // memory that k_cut_combine writes: a frame still running counts at the next
 // one).  Nothing grows while the stream is captured; held: the caller keeps
-// the memory with the graph.
+// the memory with the graph.  p.cap is 0 when there is no memory for a pool: the
+// tiles are cut serially then.
 int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, long long want, bool grow, bool held,
                CutPool& p) {
+    p = CutPool{};
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
+    const bool captured = capture != hipStreamCaptureStatusNone;
     if (!mem.seen) {
+        if (captured) return ARC_OK;
         ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&mem.seen), sizeof(int), hipHostMallocDefault));
         *mem.seen = 0;
     }
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
     if (grow) {
         const int seen = *static_cast<volatile int*>(mem.seen);
         want = std::max(want, (long long)mem.cap);
-        if (capture == hipStreamCaptureStatusNone && seen > want) want = (long long)seen + seen / 4;
+        if (!captured && seen > want) want = (long long)seen + seen / 4;
     }
     // a small image's tiles can hold 512 chunks each (a budget of 65536): no small pools
     want = std::max(want, std::min((long long)kMinChunks, 512LL * nitems));
     want = std::min(want, (long long)(INT_MAX >> kPartBits));  // a chunk's entries and part share a word (67M: 87 GB)
     // one allocation: a new gather's first frame pays for each
-    const size_t chunk = (size_t)want, part = sizeof(float) * 192 * chunk, entries = sizeof(uint32_t) * kKeep * chunk,
-                 meta = sizeof(int4) * chunk;
-    const size_t bytes = part + entries + meta + sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1));
     hipError_t e = hipSuccess;
-    const bool got = mem.mem.reserve(bytes, [&] { e = hipStreamSynchronize(ctx->stream); });
-    if (!got) return fail(ctx, ARC_E_NOMEM, "out of device memory for the moment cut's pool");
+    const size_t chunk = mem.mem.fit((size_t)want, sizeof(float) * 192 + sizeof(uint32_t) * kKeep + sizeof(int4),
+                                     sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1)), grow,
+                                     !captured, [&] { e = hipStreamSynchronize(ctx->stream); });
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize", __FILE__, __LINE__);
-    if (capture != hipStreamCaptureStatusNone && !held) mem.mem.keep();
-    mem.cap = (int)want;
+    mem.cap = (int)chunk;
+    if (chunk == 0) return ARC_OK;
+    if (captured && !held) mem.mem.keep();
+    const size_t part = sizeof(float) * 192 * chunk, entries = sizeof(uint32_t) * kKeep * chunk, meta = sizeof(int4) * chunk;
     char* at = static_cast<char*>(mem.mem.data());
     float* tbox = reinterpret_cast<float*>(at + part + entries + meta);
     int* head = reinterpret_cast<int*>(tbox + 8 * (size_t)nitems);
     p = CutPool{reinterpret_cast<uint32_t*>(at + part), reinterpret_cast<int4*>(at + part + entries),
                 reinterpret_cast<float*>(at), tbox, head, head + nitems,
                 head + 2 * (size_t)nitems, head + 3 * (size_t)nitems, head + 3 * (size_t)nitems + 1,
-                head + 3 * (size_t)nitems + 2 + kNextStride, mem.seen, (int)want, nitems < 4096 ? 4 : 8};
+                head + 3 * (size_t)nitems + 2 + kNextStride, mem.seen, (int)chunk, nitems < 4096 ? 4 : 8};
     return ARC_OK;
 }
 
@@ -1597,13 +1601,24 @@ void* PoolDevice::alloc(size_t bytes) {
 }
 void PoolDevice::free(void* p) { (void)hipFree(p); }
 
+// What is free but a sixteenth of the device, left to other objects' buffers.
+size_t PoolDevice::room() {
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return SIZE_MAX;
+    }
+    return free > total / 16 ? free - total / 16 : 0;
+}
+
 void release_pool(CutPoolMem& mem) {
     if (mem.seen) (void)hipHostFree(mem.seen);
     mem = CutPoolMem{};
 }
 
 bool cut_pool_short(arc_gather* g) {
-    return g->est_chunks == 0 && g->pool.seen && *static_cast<volatile int*>(g->pool.seen) > g->pool.cap;
+    return g->est_chunks == 0 && g->pool.seen && !g->pool.mem.refused() &&
+           *static_cast<volatile int*>(g->pool.seen) > g->pool.cap;
 }
 
 int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, unsigned long long* counters,
@@ -1624,11 +1639,12 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
         *defer = v;
         return ARC_OK;
     }
-    const bool serial = cp.budget < kSerialBudget;
+    bool serial = cp.budget < kSerialBudget;
     CutPool pool{};
     if (!serial) {
         const long long per_tile = g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);
         ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, g->batch_capture, pool));
+        serial = pool.cap == 0;
     }
     if (mark) ARC_HIP(ctx, hipEventRecord(mark, ctx->stream));
     launch_cut<false>(ctx->stream, Views<false>{v}, nitems, cp.criterion == ARC_CRITERION_EXPANSION, serial, pool);
@@ -1650,7 +1666,7 @@ int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_view
     }
     CutPool pool{};
     ARC_TRY(ready_pool(ctx, stream, mem, nitems, want, true, true, pool));
-    launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, serial, pool);
+    launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, serial || pool.cap == 0, pool);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }

@@ -64,6 +64,7 @@ struct CutPool {
 struct PoolDevice {
     static void* alloc(size_t bytes);
     static void free(void* p);
+    static size_t room();
 };
 struct CutPoolMem {
     PoolMemory<PoolDevice> mem;

@@ -378,8 +378,11 @@ int arc_gather_set_cutnet(arc_gather* g, arc_cutnet* net);
  * sets the pool's chunks per 8x8 tile; 0 (the default) sizes it from the tree
  * and grows it to what the last frame asked for.  A tile that finds the pool
  * full is cut and summed node by node, so the setting changes the speed and
- * the memory, and the image only by rounding.  Read by the next frame.
- * ARC_E_INVALID for a negative count or more than 256. */
+ * the memory, and the image only by rounding.  A pool that the device has no
+ * memory for is smaller, down to none, and asked for again after the next call
+ * here; one sized by itself leaves a sixteenth of the device's memory free.
+ * Read by the next frame.  ARC_E_INVALID for a negative count or more than
+ * 256. */
 int arc_gather_set_estimate_pool(arc_gather* g, int chunks_per_tile);
 /* No counterpart in the reference (launch shapes of this library's kernels,
  * searched by its autotuner).  cut_stack: 64, 96 or 128 (accepted; the moment
