@@ -430,7 +430,7 @@ __device__ inline int lane_below(uint64_t m) {  // set bits of m below this lane
 // r2) gets each lane's leaf record and whether it can face some pixel.
 template <class Take>
 __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32_t* X, int nx, int from, int most,
-                                   int* pfx, int* mark, const float* tb, Take take) {
+                                   int* pfx, unsigned char* mark, const float* tb, Take take) {
     const int lane = threadIdx.x & 63;
     const int c0 = lane < nx ? (int)(X[lane] & 127u) + 1 : 0;
     const int c1 = lane + 64 < nx ? (int)(X[lane + 64] & 127u) + 1 : 0;
@@ -1076,7 +1076,8 @@ struct Pixels {  // a lane's pixels
 struct EvalLds {
     uint32_t ex[kKeep];  // a chunk's kept nodes or exact ranges
     int pfx[kKeep];      // the ranges' leaves' prefix counts
-    int mark[64];        // where ranges start among 64 leaves
+    unsigned char mark[64];       // where ranges start among 64 leaves
+    float sum[kSlots][3][64];     // the lanes' sums of a range chunk
     union {
         struct {
             float4 a[64 + 2 * kSlots];  // (x, y, z, nx) of the leaves that face the tile
@@ -1098,8 +1099,14 @@ __device__ inline float leaf_cos2(const Pixels& P, int b, float x, float y, floa
     return (c1 * c2) * (inv * inv);
 }
 
-// n staged leaves, n a multiple of 2 kSlots.
-__device__ inline void sum_leaves(const EvalLds& S, int n, const Pixels& P, float (&tot)[kSlots][3]) {
+// n staged leaves, n a multiple of 2 kSlots and at most 64 + kSlots, in a plain
+// run of their own, added to S.sum: a chunk's sum is plain runs of at most 34
+// terms, 16 or 17 of them added plainly, and compensated per chunk, no worse than
+// plain runs of 64 (all of a chunk's 512 terms in one run lost 6e-6 of equal
+// terms).  S.sum is in LDS since six more registers here are spills.
+__device__ inline void sum_leaves(EvalLds& S, int n, const Pixels& P) {
+    float run[kSlots][3] = {};
+    const int lane = threadIdx.x & 63;
     const int r = (threadIdx.x & 63) / kGroupLanes;
     const float4 *pa = S.leaf.a + r, *pq = S.leaf.b + r;
     const float* pc = S.leaf.c + r;
@@ -1111,19 +1118,27 @@ __device__ inline void sum_leaves(const EvalLds& S, int n, const Pixels& P, floa
 #pragma unroll
             for (int b = 0; b < kSlots; ++b) {
                 const float g = leaf_cos2(P, b, a.x, a.y, a.z, a.w, q.x, q.y);
-                tot[b][0] = fmaf(q.z, g, tot[b][0]);
-                tot[b][1] = fmaf(q.w, g, tot[b][1]);
-                tot[b][2] = fmaf(c, g, tot[b][2]);
+                run[b][0] = fmaf(q.z, g, run[b][0]);
+                run[b][1] = fmaf(q.w, g, run[b][1]);
+                run[b][2] = fmaf(c, g, run[b][2]);
             }
         }
     }
+#pragma unroll
+    for (int b = 0; b < kSlots; ++b)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) S.sum[b][c][lane] += run[b][c];
 }
 
 // A chunk's exact ranges: the kChunkLeaves leaves from `from` on that face the tile.
 __device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, int nx, int from, const float* tb,
-                                  const Pixels& P, float (&tot)[kSlots][3]) {
+                                  const Pixels& P) {
     const int lane = threadIdx.x & 63;
     int n = 0;
+#pragma unroll
+    for (int b = 0; b < kSlots; ++b)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) S.sum[b][c][lane] = 0.f;
     walk_ranges(crec, S.ex, nx, from, kChunkLeaves, S.pfx, S.mark, tb, [&](bool facing, const float4& r0, const float4& r1, const float4& r2) {
         const uint64_t m = __ballot(facing);
         if (facing) {
@@ -1135,7 +1150,7 @@ __device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, i
         n += __popcll(m);
         __builtin_amdgcn_wave_barrier();  // before the wave's reads of other lanes' writes
         const int whole = n & ~(2 * kSlots - 1), rest = n - whole;
-        sum_leaves(S, whole, P, tot);
+        sum_leaves(S, whole, P);
         if (rest && whole) {  // the rest waits for the next 64 leaves
             float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
             float c = 0.f;
@@ -1161,7 +1176,7 @@ __device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, i
             S.leaf.c[lane] = 0.f;
         }
         __builtin_amdgcn_wave_barrier();
-        sum_leaves(S, 2 * kSlots, P, tot);
+        sum_leaves(S, 2 * kSlots, P);
     }
 }
 
@@ -1234,18 +1249,15 @@ __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))
             P.nx[b] = p.w; P.ny[b] = q.x; P.nz[b] = q.y;
         }
         __builtin_amdgcn_wave_barrier();  // read before the leaves are written over them
-        float tot[kSlots][3];
-#pragma unroll
-        for (int b = 0; b < kSlots; ++b) tot[b][0] = tot[b][1] = tot[b][2] = 0.f;
         ufloat* box = uptr(pool.tbox + 8 * (size_t)item);
         const float tb[6] = {box[0], box[1], box[2], box[3], box[4], box[5]};
-        sum_ranges(v.crec, S, cnt, (uniform(m.w) & ((1 << kPartBits) - 1)) * kChunkLeaves, tb, P, tot);
+        sum_ranges(v.crec, S, cnt, (uniform(m.w) & ((1 << kPartBits) - 1)) * kChunkLeaves, tb, P);
 #pragma unroll
         for (int ch = 0; ch < 3; ++ch) {
             float out = 0.f;
 #pragma unroll
             for (int b = 0; b < kSlots; ++b) {
-                float s = tot[b][ch];
+                float s = S.sum[b][ch][lane];
 #pragma unroll
                 for (int off = kGroupLanes; off < 64; off <<= 1) s += __shfl_xor(s, off);
                 if (lane / kGroupLanes == b) out = s;  // lane l keeps pixel l
@@ -1293,7 +1305,7 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_combine(Views<kMany> views,
 // of their own when a queue fills, so the traversal carries no sums across
 // its branches.
 __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int* E, uint32_t* X, int* pfx,
-                                            int* mark, float4 (*stage)[3], float* tb) {
+                                            unsigned char* mark, float4 (*stage)[3], float* tb) {
     const int lane = threadIdx.x & 63, tw = tiles_wide(v.W);
     const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
     const bool live = x < v.W && y < v.H;
@@ -1454,7 +1466,7 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_serial(Views<kMany> views, 
     __shared__ int qest[kCutThreads / 64][kKeep];       // internal nodes to estimate
     __shared__ uint32_t qex[kCutThreads / 64][kKeep];   // exact ranges: first << 7 | (count - 1)
     __shared__ int qpfx[kCutThreads / 64][kKeep];       // their leaves' prefix counts
-    __shared__ int qmark[kCutThreads / 64][64];         // where ranges start among 64 leaves
+    __shared__ unsigned char qmark[kCutThreads / 64][64];  // where ranges start among 64 leaves
     __shared__ float4 lstage[kCutThreads / 64][64][3];  // leaves that face the tile
     __shared__ float tbox[kCutThreads / 64][8];         // the tile's box: centre, half extent
     const int wave = threadIdx.x >> 6;
