@@ -142,14 +142,14 @@ __global__ __launch_bounds__(kThreads) void k_exact_glossy(const float4* __restr
     // the pixel's lobe
     const Mat<float> pm = material<float>(mats, P.mat);
     const bool pglossy = length(pm.specular) > 0.f;
-    V3 mirror;
+    V<double> mirror_d;
     {
         const float4 p4 = gpos[q], n4 = gnrm[q];
         const V<double> n = mk<double>(n4.x, n4.y, n4.z);
         const V<double> wo = normalize(mk<double>(camx, camy, camz) - mk<double>(p4.x, p4.y, p4.z));
-        const V<double> m = 2.0 * n * dot(n, wo) - wo;
-        mirror = mk((float)m.x, (float)m.y, (float)m.z);
+        mirror_d = 2.0 * n * dot(n, wo) - wo;
     }
+    const V3 mirror = mk((float)mirror_d.x, (float)mirror_d.y, (float)mirror_d.z);
     const V3 pspec = (0.5f * kOneOverPi * (pm.exponent + 2.f)) * pm.specular;
     const bool any_glossy = __ballot(pglossy) != 0;
     const bool podd = __ballot(pglossy && odd_lobe(pm.exponent, mirror.x, mirror.y, mirror.z)) != 0;
@@ -229,7 +229,11 @@ __global__ __launch_bounds__(kThreads) void k_exact_glossy(const float4* __restr
                 const float ca = -(r1.x * dx + r1.y * dy + r1.z * dz);
                 const float wgt = anti_weight<MODEL>(P, r0, r1, r2, A.w, dx, dy, dz, dd, inv, cn, ca, ap, gpos, gnrm, q, raw, i);
                 if (!__ballot(wgt != 0.f)) continue;
-                const V3 f = pixel_brdf((mirror.x * dx + mirror.y * dy + mirror.z * dz) * inv);
+                // a pixel accepts a few of thousands, so the cosine's rounding, times
+                // the exponent, is not averaged out as in the radiance: in double
+                const V<double> d = mk<double>(r0.x, r0.y, r0.z) - mk<double>(P.px, P.py, P.pz);
+                const double d2 = dot(d, d), ri = inv;
+                const V3 f = pixel_brdf((float)(dot(mirror_d, d) * (ri * (1.5 - 0.5 * d2 * ri * ri))));
                 if (wgt != 0.f) {
                     s0 += A.x * (f.x * wgt);
                     s1 += A.y * (f.y * wgt);

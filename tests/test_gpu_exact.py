@@ -76,3 +76,33 @@ def test_lobes(gpu_ctx, exponent):
     sc.materials[1, 6:9] = 0
     sc.materials[3, 9] = 40.0
     _check(gpu_ctx, sc, ffi.ARC_ANTIRAD_CONE, 1e-5 + 2e-7 * max(exponent, 40.0))
+
+
+@pytest.mark.parametrize("model", [ffi.ARC_ANTIRAD_DISK, ffi.ARC_ANTIRAD_CONE])
+@pytest.mark.parametrize("exponent", [12.0, 80.0])
+def test_antiradiance_of_lobes(gpu_ctx, model, exponent):
+    """A pixel's antiradiance is a few AVPLs', all of one sign: each pair's
+    relative error is the cosine's rounding (half a unit u = 2^-24) times the
+    exponent and 13 u of products (lobe, reflectance, disk or distance,
+    antiradiance), and up to 64 of them are added plainly, 20 u for the at most
+    20 a pixel has here."""
+    sc = S.cornell_256(seed=0, width=64, height=48, num_avpls=500)
+    sc.materials[:, 6:9] = [0.3, 0.25, 0.2]
+    sc.materials[:, 3:6] = 0
+    sc.materials[:, 9] = exponent
+    sc.albedo4[:] = 0
+    print(f"[exact] antiradiance lobes model {model} exponent {exponent}", flush=True)
+    g = Gather(gpu_ctx, sc.width, sc.height, sc.materials)
+    g.set_gbuffer(device_array(sc.pos4), device_array(sc.nrm4), device_array(sc.albedo4))
+    av = DeviceAvpls.from_scene(sc)
+    p = default_params(useLightCuts=0, antiradianceMode=0, antiradianceModel=model, coneHalfAngle=math.pi / 18)
+    g.run(av, sc.cam, sc.extent, p)
+    _, a64 = g.exact_f64(av, sc.cam, sc.extent, p)
+    gpu_ctx.sync()
+    anti, a64 = g.antiradiance[:, :3].double().cpu().numpy(), a64.cpu().numpy()
+    g.close()
+    lit = a64 > 1e-20 * a64.max()
+    assert lit.any()
+    e = np.abs(anti[lit] / a64[lit] - 1).max() * 2.0 ** 24
+    print(f"[exact] largest error {e:.1f} u", flush=True)
+    assert e <= 0.5 * exponent + 13 + 20
