@@ -393,8 +393,8 @@ __global__ __launch_bounds__(kThreads) void k_exact_lambert(const float4* __rest
                         const float cn = P[s].nx * dx + P[s].ny * dy + P[s].nz * dz;
                         const float cw = u.w * dx + v.x * dy + v.y * dz;
                         const float cp = cn * inv;
-                        // the smaller distance from the thresholds decides, in FP64 inside the guard band
-                        const float least = fminf(-(cw * inv) - edge, cp - kConeEps);
+                        // the smaller distance from the thresholds decides (no number if either is none), in FP64 inside the guard band
+                        const float least = __builtin_elementwise_minimum(-(cw * inv) - edge, cp - kConeEps);
                         bool in = least > 0.f;
                         if (fabsf(least) <= kGuard)
                             in = cone_accept_f64(gpos[q[s]], gnrm[q[s]], raw.pos[S.i[j]], raw.dir[S.i[j]], ap.cos_half_d);

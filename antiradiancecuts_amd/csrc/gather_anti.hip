@@ -511,8 +511,8 @@ __global__ __launch_bounds__(kAntiThreads) __attribute__((amdgpu_waves_per_eu(5)
                     const float inv = __builtin_amdgcn_rsqf(dx * dx + dy * dy + dz * dz);
                     const float cp = (nx * dx + ny * dy + nz * dz) * inv;
                     const float c = (u.w * dx + v.x * dy + v.y * dz) * -inv;
-                    // the smaller distance from the thresholds decides, in FP64 inside the guard band
-                    const float least = fminf(c - edge, cp - kConeEps);
+                    // the smaller distance from the thresholds decides (no number if either is none), in FP64 inside the guard band
+                    const float least = __builtin_elementwise_minimum(c - edge, cp - kConeEps);
                     bool in = least > 0.f;
                     if (fabsf(least) <= kGuard) {
                         const int i = S.i[j];

@@ -46,3 +46,36 @@ def test_clustered_cone_equals_exact(gpu_ctx, w, h, n, specular, half):
         assert not exact[bare].any() and not clustered[bare].any()
     # both sum FP32 pairs of one sign with the same decisions: 64 plain additions at most between compensated ones
     np.testing.assert_allclose(clustered[~bare], exact[~bare], rtol=2e-5, atol=1e-6 * np.abs(exact[~bare]).max(initial=1e-30))
+
+
+@pytest.mark.parametrize("mode", [ffi.ARC_ANTI_EXACT, ffi.ARC_ANTI_CLUSTERED])
+def test_points_whose_squared_distance_underflows(gpu_ctx, mode):
+    """AVPLs 1e-25 from the pixels, where 1/|d| is infinite and a cosine at a
+    right angle is 0 times infinity: one in the pixels' plane (the pixel's
+    cosine is no number, the cone's is infinite), one along the normal with its
+    direction across (the other way round).  Both cosines of a pair must pass,
+    so both AVPLs are rejected as in FP64; a third one is accepted."""
+    n = 3
+    pos = np.zeros((64, 4), np.float32)
+    pos[:, 3] = 1
+    nrm = np.zeros((64, 4), np.float32)
+    nrm[:, 2:] = 1
+    alb = np.full((64, 4), 0.5, np.float32)
+    a = np.array([[1e-25, 0, 0], [0, 0, 1e-25], [0, 0, 1]], np.float32)
+    w = np.array([[-1, 0, 0], [1, 0, 0], [0, 0, -1]], np.float32)
+    mats = np.array([[0] * 10, [0, 0, 0, 0.5, 0.5, 0.5, 0, 0, 0, 0]], np.float32)
+    ones = np.ones(n, np.int32)
+    sc = S.Scene(8, 8, pos, nrm, alb, mats, np.array([0, 0, 10], np.float32), 4.0, a, w, w,
+                 np.zeros((n, 3), np.float32), np.ones((n, 3), np.float32), ones, ones)
+    print(f"[anti] underflow mode {mode}", flush=True)
+    g = Gather(gpu_ctx, 8, 8, mats)
+    g.set_gbuffer(device_array(pos), device_array(nrm), device_array(alb))
+    av = DeviceAvpls.from_scene(sc)
+    p = default_params(useLightCuts=0, antiradianceMode=mode, antiradianceModel=ffi.ARC_ANTIRAD_CONE)
+    g.run(av, sc.cam, sc.extent, p)
+    _, a64 = g.exact_f64(av, sc.cam, sc.extent, p)
+    gpu_ctx.sync()
+    anti, a64 = g.antiradiance[:, :3].double().cpu().numpy(), a64.cpu().numpy()
+    g.close()
+    assert a64.min() > 0 and np.isfinite(a64).all()
+    np.testing.assert_allclose(anti, a64, rtol=1e-5)
