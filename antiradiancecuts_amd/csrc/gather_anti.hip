@@ -46,6 +46,7 @@
 #include <cmath>
 
 #include "gather_common.hpp"
+#include "launch_rules.hpp"
 
 using arc::f3;
 using namespace arc::gm;
@@ -60,8 +61,6 @@ constexpr int kTiles = (kClusterPx / 8) * (kClusterPx / 8);  // 8x8 tiles per cl
 constexpr int kParts = 4;                                      // blocks per cluster (rows of 32 x 8 px)
 constexpr int kBlockTiles = kTiles / kParts;                   // tiles per block
 constexpr int kAntiThreads = 64 * kBlockTiles;                 // one wave per tile
-constexpr int kSub = 1536;       // tile sub-list entries in LDS: list entries filed per chunk (default;
-                                 // 768 and 3072 also built)
 constexpr int kTreeMaxLevels = 10;  // cluster quadtree levels: up to 512 x 512 clusters
 
 __device__ inline bool has_anti(const arc::AvplsDev& a, int i) {
@@ -575,15 +574,12 @@ void launch_pixels(arc_gather* g, const arc::AvplsDev& a, int cw, int C, float3 
                            cam.y, cam.z, ap, g->ccount.as<int>(), g->clist.as<int>(), g->anti_idx.as<int>(),
                            n_anti_ptr, grow, cos_t, sin_t, part, counters);
     };
-    // list entries filed per pass: a launch-shape setting (LDS against passes).
-    // The Lambertian cone's kernel wants 110 registers: with 3072 entries, 34 KB,
-    // four waves per SIMD are what the LDS allows and it gets them; with fewer it
-    // is held to 96 and spills 17 (1080p, 1M AVPLs: 0.9 GB of traffic and 26.2 ms
-    // a frame against 2.0 GB and 28.0 with 1536).  The other models cost alike.
-    const int chunk = g->anti_chunk ? g->anti_chunk : MODEL == ARC_ANTIRAD_CONE && !GENERAL ? 3072 : kSub;
+    // list entries filed per pass: a launch-shape setting (LDS against passes)
+    constexpr bool staged = MODEL == ARC_ANTIRAD_CONE && !GENERAL;
+    const int chunk = arc::anti_block(g->anti_chunk, staged);
     if (chunk == 768) launch(k_anti_clustered<MODEL, GENERAL, 768>);
-    else if (chunk == 3072) launch(k_anti_clustered<MODEL, GENERAL, 3072>);
-    else launch(k_anti_clustered<MODEL, GENERAL, kSub>);
+    else if (staged || chunk == 3072) launch(k_anti_clustered<MODEL, GENERAL, 3072>);
+    else if constexpr (!staged) launch(k_anti_clustered<MODEL, GENERAL, arc::kAntiBlock>);
 }
 
 }  // namespace

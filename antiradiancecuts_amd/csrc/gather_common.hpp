@@ -10,6 +10,7 @@
 #include "arc_internal.hpp"
 #include "cut_pool.hpp"
 #include "gather_math.hpp"
+#include "launch_rules.hpp"
 
 namespace arc {
 // One view's moment cut, as its kernels read it (by value, or from an array
@@ -107,7 +108,7 @@ struct arc_gather {
     bool batch_capture = false;  // the frame is being captured by arc_batch, which holds the pool's memory itself
     // a launch shape the results do not depend on: the clustered
     // antiradiance's list entries filed per pass (768, 1536 or 3072)
-    int anti_chunk = 0;  // list entries filed per pass; 0: the kernel's own choice
+    int anti_chunk = arc::kAntiBlock;  // 1536: the kernel's own choice
     arc_cutnet* net = nullptr;  // learned cut: the predictor (borrowed)
     arc_bvh* bvh = nullptr;
     // per-frame phase events: frame slot, then 9 marks (start, upload done,

@@ -250,8 +250,9 @@ class Gather:
 
     def set_launch_shape(self, cut_stack: int = 96, anti_chunk: int = 1536) -> None:
         """A traversal stack (64, 96, 128 nodes: accepted, without effect) and
-        the clustered antiradiance's list entries filed per pass (768, 1536,
-        3072); neither changes the image beyond rounding."""
+        the clustered antiradiance's list entries filed per pass (768, 3072, or
+        1536: the library's own choice); neither changes the image beyond
+        rounding."""
         check(self.lib.arc_gather_set_launch_shape(self.h, int(cut_stack), int(anti_chunk)),
               "arc_gather_set_launch_shape", self.ctx.h)
 

@@ -277,6 +277,7 @@ def main() -> int:
     # the pair is one unit when each kernel spends a good part of its time
     # beside the other; otherwise the longer of the two is the unit alone
     paired = t_overlap > 0.25 * min(t_rad, t_anti)
+    anti_chunk = 3072 if cone and sched.anti_chunk == 1536 else sched.anti_chunk  # 1536: the library's choice
     per_kernel = {rad_name: {**rate(flop_rad, t_rad), "flop": flop_rad, "overlap_ms": round(t_overlap, 4)},
                   "k_anti_clustered": {**rate(flop_anti, t_anti), "flop": flop_anti}}
     if not paired and max(t_rad, t_anti) >= t_bvh and max(t_rad, t_anti) > 0.0:
@@ -286,12 +287,12 @@ def main() -> int:
         roof = {"kernel": name, "bound": COMPUTE_BOUND, "engine": "VALU", "achieved": round(ach, 3),
                 "peak": PEAK_FP32_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(ach / PEAK_FP32_TFLOPS, 4),
-                "traffic": profiled_traffic(dom, eb, bool(args.per_tile), args.eval_depth, mom, cone, sched.anti_chunk),
+                "traffic": profiled_traffic(dom, eb, bool(args.per_tile), args.eval_depth, mom, cone, anti_chunk),
                 "ms": round(t_dom, 4),
                 "kernels": per_kernel}
     elif t_pair >= t_bvh and t_pair > 0.0:
         ach = (flop_rad + flop_anti) / (t_pair * 1e-3) / 1e12
-        tr = [profiled_traffic(k, eb, bool(args.per_tile), args.eval_depth, mom, cone, sched.anti_chunk)
+        tr = [profiled_traffic(k, eb, bool(args.per_tile), args.eval_depth, mom, cone, anti_chunk)
               for k in ("radiance", "antiradiance")]
         roof = {"kernel": f"{rad_name} + k_anti_clustered (concurrent on two streams)", "bound": COMPUTE_BOUND,
                 "engine": "VALU",

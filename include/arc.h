@@ -387,11 +387,11 @@ int arc_gather_set_estimate_pool(arc_gather* g, int chunks_per_tile);
 /* No counterpart in the reference (launch shapes of this library's kernels,
  * searched by its autotuner).  cut_stack: 64, 96 or 128 (accepted; the moment
  * cut's traversal needs no depth setting any more).  anti_chunk: the clustered
- * antiradiance's list entries filed into the tiles' LDS sub-lists per pass
- * (768, 1536 or 3072; until it is set, 3072 for the cone model over Lambertian
- * materials and else 1536): more per pass is fewer passes and more LDS per
- * workgroup.  Neither changes the image beyond rounding.  Read by the
- * next frame.  ARC_E_INVALID for other values. */
+ * antiradiance's list entries filed into the tiles' LDS sub-lists per pass: 768
+ * or 3072, or 1536, the default, which leaves it to the library (3072 for the
+ * cone model over Lambertian materials, else 1536): more per pass is fewer
+ * passes and more LDS per workgroup.  Neither changes the image beyond
+ * rounding.  Read by the next frame.  ARC_E_INVALID for other values. */
 int arc_gather_set_launch_shape(arc_gather* g, int cut_stack, int anti_chunk);
 /* Training rows of one frame: builds the frame's AvplBvh and thresholds as
  * arc_gather_run does with params (cutMode is ignored), then walks each tile's
