@@ -57,7 +57,7 @@ constexpr int kMom = 13;
 // float4 per internal node of the traversal's record, one 48-byte gather per
 // node: (box min, max_c I_c), (box max, first leaf), (left, right, count, -)
 constexpr int kTrav = 3;
-constexpr int kMomStack = 128;   // per-wave stack of the serial traversal (deeper than any tree: 32 code bits + 25 index bits)
+constexpr int kMomStack = 64;    // per-wave stack of the serial traversal (deeper than any tree: 32 code bits + 25 index bits)
 
 // Terms of leaf i of the sorted order (crec leaf record: r0 = position,
 // r1 = unit normal, r2 = I), in four groups of ten:
@@ -426,11 +426,13 @@ __device__ inline int lane_below(uint64_t m) {  // set bits of m below this lane
 // every sum (its cosine max(0, n_a . (p - x_a)) is 0), and about half of the
 // leaves do (a surface's AVPLs seen from behind).  tb = (centre, half extent)
 // of the tile's box: the largest n_a . (p - x_a) over it is n_a . (c - x_a) +
-// |n_a| . e, compared with a margin above FP32 rounding.  take(facing, r0, r1,
-// r2) gets each lane's leaf record and whether it can face some pixel.
-template <class Take>
+// |n_a| . e, compared with a margin above FP32 rounding.  stage(facing, r0, r1,
+// r2) gets each lane's leaf record and whether it can face some pixel, sum()
+// follows: the next 64 records are fetched between them, into the registers that
+// stage has read.
+template <class Stage, class Sum>
 __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32_t* X, int nx, int from, int most,
-                                   int* pfx, unsigned char* mark, const float* tb, Take take) {
+                                   int* pfx, unsigned char* mark, const float* tb, Stage stage, Sum sum) {
     const int lane = threadIdx.x & 63;
     const int c0 = lane < nx ? (int)(X[lane] & 127u) + 1 : 0;
     const int c1 = lane + 64 < nx ? (int)(X[lane + 64] & 127u) + 1 : 0;
@@ -441,16 +443,17 @@ __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32
     const int total = leaves - from > most ? from + most : leaves;
     s0 = lane < nx ? s0 - c0 : INT_MAX;       // where the range in X[lane] starts
     s1 = lane + 64 < nx ? s1 - c1 : INT_MAX;  // and the one in X[lane + 64]
-    if (lane < nx) pfx[lane] = s0;
-    if (lane + 64 < nx) pfx[lane + 64] = s1;
+    pfx[lane] = s0;  // kept in LDS: registers are short
+    pfx[lane + 64] = s1;
     const float scale = fabsf(tb[0]) + fabsf(tb[1]) + fabsf(tb[2]) + tb[3] + tb[4] + tb[5];
     float4 b0 = make_float4(0.f, 0.f, 0.f, 0.f), b1 = b0, b2 = b0;
     int before = __popcll(__ballot(s0 < from)) + __popcll(__ballot(s1 < from));  // ranges that start before the batch
     auto fetch = [&](int base) {
         mark[lane] = 0;
         __builtin_amdgcn_wave_barrier();  // the wave's LDS writes come before its reads of other lanes' slots
-        if ((unsigned)(s0 - base) < 64u) mark[s0 - base] = 1;
-        if ((unsigned)(s1 - base) < 64u) mark[s1 - base] = 1;
+        const unsigned at0 = (unsigned)(pfx[lane] - base), at1 = (unsigned)(pfx[lane + 64] - base);
+        if (at0 < 64u) mark[at0] = 1;
+        if (at1 < 64u) mark[at1] = 1;
         __builtin_amdgcn_wave_barrier();
         const uint64_t m = __ballot(mark[lane] != 0);
         const int g = base + lane;
@@ -464,15 +467,16 @@ __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32
         before += __popcll(m);
     };
     fetch(from);
+#pragma unroll 1
     for (int base = from; base < total; base += 64) {
         const float dx = tb[0] - b0.x, dy = tb[1] - b0.y, dz = tb[2] - b0.z;
         const float reach = b1.x * dx + b1.y * dy + b1.z * dz + fabsf(b1.x) * tb[3] + fabsf(b1.y) * tb[4] +
                             fabsf(b1.z) * tb[5];
         const float margin = 1e-5f * (scale + fabsf(b0.x) + fabsf(b0.y) + fabsf(b0.z));
         const bool facing = base + lane < total && reach > -margin;
-        const float4 r0 = b0, r1 = b1, r2 = b2;
+        stage(facing, b0, b1, b2);
         if (base + 64 < total) fetch(base + 64);  // in flight while these are summed
-        take(facing, r0, r1, r2);
+        sum();
     }
 }
 
@@ -489,7 +493,8 @@ __device__ inline void walk_ranges(const float4* __restrict__ crec, const uint32
 //                  chunks as they hold times kChunkLeaves leaves;
 //   k_cut_eval     sums the chunks, a wave per chunk whatever tile it belongs
 //                  to, into 64 x 3 partial sums each;
-//   k_cut_serial   the tiles that found the pool full: the depth-first cut of
+//   k_cut_serial   the tiles that found the pool full, and all tiles where most
+//                  would meet their budget (serial_cut): the depth-first cut of
 //                  one node at a time, summed as it goes;
 //   k_cut_combine  adds each tile's partial sums in the order of its chunks.
 //
@@ -539,6 +544,20 @@ struct Views<true> {
         return v;
     }
 };
+
+// The view of an item, read again from the kernel's arguments (its first one is a
+// Views): what a tile needs only at its start and end is then not held in
+// between, where scalar registers are short and spill.
+template <bool kMany>
+__device__ inline CutView view_again(int item) {
+    auto* args = (const ARC_UNIFORM_AS uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    Views<kMany> w;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(&w);
+#pragma unroll
+    for (size_t i = 0; i < sizeof(w) / 4; ++i) dst[i] = args[i];
+    return w.of(item);
+}
 
 __device__ inline Threshold view_threshold(const CutView& v) {
     Threshold th;
@@ -607,6 +626,26 @@ __device__ inline bool node_faces(const float* tb, const float4& lo, const float
     return reach > -1e-5f * scale;
 }
 
+// A tile's cost where it is cut serially, in vector instructions: a bound test
+// is about 30, an estimate 130, a queued exact leaf 18 (26 a pair for the half
+// that face the tile, a few for the rest), and the pixel's own loads and stores.
+__device__ inline float tile_cost(int tested, int kept, int leaves) {
+    return 300.f + 30.f * (float)tested + 130.f * (float)kept + 18.f * (float)leaves;
+}
+
+// The k-th tile of a launch in no order: of one view's a block's four are a 16x16-pixel
+// block, neighbouring blocks on one XCD.
+template <bool kMany>
+__device__ inline int unordered_item(const Views<kMany>& views, int wave, int k) {
+    if constexpr (kMany) {
+        return k;
+    } else {
+        const int gx = (views.one.W + 15) / 16, gy = (views.one.H + 15) / 16;
+        const int b = xcd_block(blockIdx.x, gx * gy);
+        return uniform(((b / gx) * 2 + (wave >> 1)) * 2 * gx + (b % gx) * 2 + (wave & 1));
+    }
+}
+
 // One wave's working memory of k_cut_decide.
 struct DecideLds {
     int stack[kDecideStack];  // pending internal nodes
@@ -644,9 +683,7 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
         item = uniform(blockIdx.x * (kCutThreads / 64) + wave);
         if (item >= nitems) return;  // the whole wave: no block barrier below
     } else {  // a block's four tiles are one 16x16-pixel block, neighbouring blocks on one XCD
-        const int gx = (views.one.W + 15) / 16, gy = (views.one.H + 15) / 16;
-        const int b = xcd_block(blockIdx.x, gx * gy);
-        item = uniform(((b / gx) * 2 + (wave >> 1)) * 2 * gx + (b % gx) * 2 + (wave & 1));
+        item = unordered_item(views, wave, 0);
     }
     const CutView v = views.of(item);
     const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
@@ -719,7 +756,7 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
         if (nspare == 0) {
             nspare = head < 0 ? pool.grab : 2 * pool.grab;
             int got = 0;
-            if (lane == 0) got = atomicAdd(pool.taken, nspare);
+            if (lane == 0) got = atomicAdd(pool.count + arc::kTaken, nspare);
             spare = uniform(got);
         }
         c = spare;
@@ -1035,7 +1072,8 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
         if (lane == 0) {
             for (int c = head; c >= 0; c = pool.meta[c].z) pool.meta[c].y = 0;
             pool.head[item] = -1;
-            pool.serial[atomicAdd(pool.nserial, 1)] = item;
+            pool.serial[atomicAdd(pool.count + arc::kSerialTiles, 1)] = item;
+            atomicAdd(pool.count + arc::kFullTiles, 1);
             pool.evaluated[item] = -1;
         }
         return;
@@ -1044,6 +1082,8 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
     if (lane == 0) {
         pool.head[item] = head;
         pool.evaluated[item] = total;
+        pool.tbox[8 * (size_t)item + 6] = tile_cost(ntest, nkeep, total - nkeep);
+        if (nbud > 0) atomicAdd(pool.count + arc::kSpentTiles, 1);
         if (v.counters) {
             const unsigned long long n = (unsigned long long)__popcll(alive);
             atomicAdd(&v.counters[C_TESTED], n * ntest);
@@ -1149,6 +1189,7 @@ __device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, i
         }
         n += __popcll(m);
         __builtin_amdgcn_wave_barrier();  // before the wave's reads of other lanes' writes
+    }, [&]() {
         const int whole = n & ~(2 * kSlots - 1), rest = n - whole;
         sum_leaves(S, whole, P);
         if (rest && whole) {  // the rest waits for the next 64 leaves
@@ -1186,10 +1227,10 @@ __device__ inline void sum_ranges(const float4* __restrict__ crec, EvalLds& S, i
 template <bool kMany>
 __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_cut_eval(Views<kMany> views, CutPool pool) {
     __shared__ EvalLds lds[kCutThreads / 64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     EvalLds& S = lds[wave];
     const int waves = gridDim.x * (kCutThreads / 64);
-    const int n = uniform(min(*pool.taken, pool.cap));
+    const int n = uniform(min(pool.count[arc::kTaken], pool.cap));
     // A wave starts with the chunk of its number and then takes groups of
     // chunks, a fraction of its share, from one of eight counters: a counter
     // serves about 100 atomics per microsecond (one for all took 230 us for 23K
@@ -1277,15 +1318,20 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_combine(Views<kMany> views,
         // what the next frame's pool should hold: the tiles that found it full
         // need as much as the others, as far as is known (the count alone grows
         // by what is asked for until it is full, a quarter per frame)
-        const int taken = *pool.taken, rest = max(1, nitems - *pool.nserial);
-        *pool.seen = (int)fminf((float)taken * fminf((float)nitems / (float)rest, 8.f), 1e9f);
+        const int taken = pool.count[arc::kTaken], rest = max(1, nitems - pool.count[arc::kFullTiles]);
+        pool.seen[0] = (int)fminf((float)taken * fminf((float)nitems / (float)rest, 8.f), 1e9f);
+        pool.seen[1] = pool.count[arc::kSpentTiles] + (pool.fixed ? pool.count[arc::kFullTiles] : 0);
     }
     const CutView v = views.of(item);
     const int t = item - (kMany ? v.tile_base : 0), tw = tiles_wide(v.W);
     const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
-    if (!__ballot(x < v.W && y < v.H)) return;
+    if (!__ballot(x < v.W && y < v.H)) {
+        if (lane == 0) pool.cost[item] = 0.f;
+        return;
+    }
     const int evaluated = uniform(pool.evaluated[item]);
     if (evaluated < 0) return;  // k_cut_serial writes it
+    if (lane == 0) pool.cost[item] = pool.tbox[8 * (size_t)item + 6];
     Kahan k[3];
     for (int c = uniform(pool.head[item]); c >= 0;) {
         const float* s = pool.part + (size_t)c * 192 + lane;
@@ -1300,18 +1346,35 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_combine(Views<kMany> views,
     v.out_rad[q] = make_float4(k[0].s * P.br, k[1].s * P.bg, k[2].s * P.bb, v.counters ? (float)evaluated : 1.f);
 }
 
-// One depth-first cut, a node at a time, summed as it goes: the tiles that
-// found the pool full.  Kept nodes and exact ranges are queued in LDS and summed in passes
-// of their own when a queue fills, so the traversal carries no sums across
-// its branches.
-__device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int* E, uint32_t* X, int* pfx,
-                                            unsigned char* mark, float4 (*stage)[3], float* tb) {
-    const int lane = threadIdx.x & 63, tw = tiles_wide(v.W);
-    const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
-    const bool live = x < v.W && y < v.H;
-    const int q = live ? y * v.W + x : 0;
-    const PixelF P = load_pixel(v.gpos, v.gnrm, v.galb, v.mats, q);
-    const float thr = live ? view_threshold(v).at(q) : INFINITY;
+// One depth-first cut, a node at a time, summed as it goes.  Kept nodes and exact
+// ranges are queued in LDS and summed in passes of their own when a queue fills,
+// so the traversal carries no sums across its branches.
+//
+// Bound by vector and scalar issue and by each node's dependent record load.  With
+// the tile's set-up held in registers throughout, arguments read again per node
+// and records read in two loads, a budget of 8191 at 1283x719 pixels over 250001
+// AVPLs took 9.1 ms a frame; 6.8 here and with the tiles in order.
+template <bool kMany>
+__device__ __forceinline__ void serial_tile(const CutView& v, float* cost, int item, int* S, int* E,
+                                            uint32_t* X, int* pfx, unsigned char* mark, float4 (*stage)[3], float* tb) {
+    const int lane = threadIdx.x & 63;
+    PixelF P;
+    float thr;
+    bool live;
+    {
+        const CutView w = view_again<kMany>(item);
+        const int t = item - (kMany ? w.tile_base : 0), tw = tiles_wide(w.W);
+        const int x = (t % tw) * 8 + (lane & 7), y = (t / tw) * 8 + (lane >> 3);
+        live = x < w.W && y < w.H;
+        const int q = live ? y * w.W + x : 0;
+        P = load_pixel(w.gpos, w.gnrm, w.galb, w.mats, q);
+        thr = live ? view_threshold(w).at(q) : INFINITY;
+    }
+    // what each node needs stays in registers: left to itself the compiler reads
+    // some of it from the arguments again per node, a load's latency each
+    const float4 *trav = v.trav, *mom = v.mom, *nbox = v.nbox, *crec = v.crec;
+    int exact_count = v.exact_count, budget = v.budget;
+    asm volatile("" : "+s"(trav), "+s"(mom), "+s"(exact_count), "+s"(budget));
     const float delta2 = v.delta * v.delta;
     {  // the box of the tile's live pixels, as centre and half extent
         const float lx = wave_fmin(live ? P.px : INFINITY), hx = wave_fmax(live ? P.px : -INFINITY);
@@ -1328,6 +1391,7 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
         __builtin_amdgcn_wave_barrier();  // lane 0's writes before the wave's reads
     }
     const bool expansion = v.criterion == ARC_CRITERION_EXPANSION;
+    auto load = [](const float4* r) { return uload4(uptr(r)); };
     Acc acc;
     unsigned nvis = 0, nev = 0, nerr = 0, nbud = 0, ntest = 0, nexact = 0;  // wave-uniform
     int ne = 0, nx = 0;                                                     // queued, wave-uniform
@@ -1341,8 +1405,8 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
             int k = 0;
             if (j < ne) {
                 k = E[j];
-                const float4* r = v.trav + (size_t)kTrav * k;
-                facing = node_faces(tb, r[0], r[1], v.nbox[2 * (size_t)k], v.nbox[2 * (size_t)k + 1]);
+                const float4* r = trav + (size_t)kTrav * k;
+                facing = node_faces(tb, r[0], r[1], nbox[2 * (size_t)k], nbox[2 * (size_t)k + 1]);
             }
             const uint64_t fm = __ballot(facing);
             // every lane has read its entry before any is overwritten (kept <= base)
@@ -1353,14 +1417,15 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
         }
         nev -= (unsigned)(ne - kept);
         for (int j = 0; j < kept; ++j) {
-            add_moments<true>(P, v.mom + kMom * (size_t)uniform(E[j]), acc);
+            add_moments<true>(P, mom + kMom * (size_t)uniform(E[j]), acc);
             acc.maybe_flush();
         }
         ne = 0;
     };
     auto drain_exact = [&]() {
+        int cnt = 0;  // staged leaves
         if (nx > 0)
-            walk_ranges(v.crec, X, nx, 0, INT_MAX, pfx, mark, tb, [&](bool facing, const float4& r0, const float4& r1, const float4& r2) {
+            walk_ranges(crec, X, nx, 0, INT_MAX, pfx, mark, tb, [&](bool facing, const float4& r0, const float4& r1, const float4& r2) {
                 const uint64_t fm = __ballot(facing);
                 if (facing) {
                     const int j = lane_below(fm);
@@ -1368,8 +1433,9 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
                     stage[j][1] = r1;
                     stage[j][2] = r2;
                 }
+                cnt = __popcll(fm);
                 __builtin_amdgcn_wave_barrier();
-                const int cnt = __popcll(fm);
+            }, [&]() {
 #pragma unroll 1
                 for (int j = 0; j < cnt; ++j) acc.add_run(stage[j][2], leaf_g(P, stage[j][0], stage[j][1]));
                 acc.maybe_flush();
@@ -1383,29 +1449,32 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
         bool pop = true;  // take the next node from the stack (not a refined node's left child)
         if (node < 0) {
             const int k = -(node + 1);
-            ufloat* r = uptr(v.trav + (size_t)kTrav * k);
-            const float4 r0 = uload4(r), r1 = uload4(r + 4), r2 = uload4(r + 8);
+            const float4* r = trav + (size_t)kTrav * k;
+            const float4 r0 = load(r), r1 = load(r + 1), r2 = load(r + 2);
             arc_bvh_node b;
             b.left = __float_as_int(r2.x);
             b.right = __float_as_int(r2.y);
+            int count = __float_as_int(r2.z);
+            asm volatile("" : "+s"(b.left), "+s"(b.right), "+s"(count));  // the whole record in one wait
             b.bbMin = arc_float3{r0.x, r0.y, r0.z};
             b.bbMax = arc_float3{r1.x, r1.y, r1.z};
             b.visited = 0;  // not read
-            const int first = __float_as_int(r1.w), count = __float_as_int(r2.z);
+            const int first = __float_as_int(r1.w);
             const float bound = node_bound1(P, b, r0.w, delta2);
             if (!__ballot(bound > 0.f)) {
                 // behind every pixel's tangent plane: contributes exactly 0
-            } else if (count <= v.exact_count) {
+            } else if (count <= exact_count) {
                 // small node: its AVPLs exactly (refining it would end in the same sum)
                 X[nx++] = ((uint32_t)first << 7) | (uint32_t)(count - 1);
                 nexact += count;
             } else {
                 bool refine;
                 if (expansion) {
-                    ufloat* m = uptr(v.mom + kMom * (size_t)k);
-                    const float dx = m[0] - P.px, dy = m[1] - P.py, dz = m[2] - P.pz;
+                    const float4* m = mom + kMom * (size_t)k;
+                    const float4 c = load(m), size = load(m + 1);
+                    const float dx = c.x - P.px, dy = c.y - P.py, dz = c.z - P.pz;
                     const float dc2 = dx * dx + dy * dy + dz * dz;
-                    const float s2 = m[4] * m[4];
+                    const float s2 = size.x * size.x;
                     refine = bound > 0.f && (s2 > v.open2 * dc2 || bound * s2 > thr * dc2);
                 } else {
                     refine = bound > thr;
@@ -1413,7 +1482,7 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
                 ++ntest;
                 bool keep = true;
                 if (__ballot(refine)) {
-                    if ((int)(nev + nexact) >= v.budget) {
+                    if ((int)(nev + nexact) >= budget) {
                         ++nbud;  // cut budget spent: keep the cluster
                     } else if (sp < kMomStack) {
                         S[sp++] = b.right;
@@ -1445,22 +1514,29 @@ __device__ __forceinline__ void serial_tile(const CutView& v, int t, int* S, int
     drain_exact();
     acc.flush();
     const int alive = __popcll(__ballot(live));  // all lanes take part in the ballot
-    if (v.counters && lane == 0) {
-        atomicAdd(&v.counters[C_TESTED], (unsigned long long)ntest * alive);
-        atomicAdd(&v.counters[C_VISITED], (unsigned long long)nvis * alive);
-        atomicAdd(&v.counters[C_EVALUATED], (unsigned long long)(nev + nexact) * alive);
-        atomicAdd(&v.counters[C_EXACT], (unsigned long long)nexact * alive);
-        atomicAdd(&v.counters[C_ERRORS], (unsigned long long)nerr);
-        atomicAdd(&v.counters[C_BUDGET], (unsigned long long)nbud);
+    const CutView w = view_again<kMany>(item);
+    if (cost && lane == 0) *cost = tile_cost(ntest, nev, nexact);
+    if (w.counters && lane == 0) {
+        atomicAdd(&w.counters[C_TESTED], (unsigned long long)ntest * alive);
+        atomicAdd(&w.counters[C_VISITED], (unsigned long long)nvis * alive);
+        atomicAdd(&w.counters[C_EVALUATED], (unsigned long long)(nev + nexact) * alive);
+        atomicAdd(&w.counters[C_EXACT], (unsigned long long)nexact * alive);
+        atomicAdd(&w.counters[C_ERRORS], (unsigned long long)nerr);
+        atomicAdd(&w.counters[C_BUDGET], (unsigned long long)nbud);
     }
-    if (live)
-        v.out_rad[q] = make_float4(acc.k[0].s * P.br, acc.k[1].s * P.bg, acc.k[2].s * P.bb,
-                                   v.counters ? (float)(nev + nexact) : 1.f);
+    if (live) {
+        const int t = item - (kMany ? w.tile_base : 0), tw = tiles_wide(w.W);
+        const int q = ((t / tw) * 8 + (lane >> 3)) * w.W + (t % tw) * 8 + (lane & 7);
+        const PixelF L = load_pixel(w.gpos, w.gnrm, w.galb, w.mats, q);  // again: its reflectance is not held meanwhile
+        w.out_rad[q] = make_float4(acc.k[0].s * L.br, acc.k[1].s * L.bg, acc.k[2].s * L.bb,
+                                   w.counters ? (float)(nev + nexact) : 1.f);
+    }
 }
 
-// The tiles of pool.serial; with `all`, every tile of the launch.
-template <bool kMany>
-__global__ __launch_bounds__(kCutThreads) void k_cut_serial(Views<kMany> views, int nitems, int all,
+// The tiles of pool.serial, more than the launch's waves as these come free; with
+// `all`, every tile of the launch, a wave each.
+template <bool kMany, int kWaves>
+__global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_cut_serial(Views<kMany> views, int nitems, int all,
                                                            CutPool pool) {
     __shared__ int stk[kCutThreads / 64][kMomStack];
     __shared__ int qest[kCutThreads / 64][kKeep];       // internal nodes to estimate
@@ -1469,22 +1545,61 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_serial(Views<kMany> views, 
     __shared__ unsigned char qmark[kCutThreads / 64][64];  // where ranges start among 64 leaves
     __shared__ float4 lstage[kCutThreads / 64][64][3];  // leaves that face the tile
     __shared__ float tbox[kCutThreads / 64][8];         // the tile's box: centre, half extent
-    const int wave = threadIdx.x >> 6;
+    const int wave = uniform(threadIdx.x >> 6);
     const int waves = gridDim.x * (kCutThreads / 64);
-    const int n = all ? nitems : uniform(*pool.nserial);
-    for (int k = uniform(blockIdx.x * (kCutThreads / 64) + wave); k < n; k += waves) {
-        const int item = all ? k : uniform(pool.serial[k]);
-        const CutView v = views.of(item);
-        serial_tile(v, item - (kMany ? v.tile_base : 0), stk[wave], qest[wave], qex[wave], qpfx[wave], qmark[wave], lstage[wave],
-                    tbox[wave]);
+    const int n = all ? nitems : uniform(pool.count[arc::kSerialTiles]);
+    const int id = blockIdx.x * (kCutThreads / 64) + wave;
+    const bool queue = n > waves;
+    auto next = [&]() {
+        int got = 0;
+        if ((threadIdx.x & 63) == 0) got = atomicAdd(pool.count + arc::kSerialNext, 1);
+        return uniform(got);
+    };
+    for (int k = queue ? next() : uniform(id); k < n; k = next()) {
+        const int item = !all ? uniform(pool.serial[k]) : pool.ordered ? uniform(pool.order[k]) : unordered_item(views, wave, k);
+        serial_tile<kMany>(views.of(item), pool.cost ? pool.cost + item : nullptr, item, stk[wave], qest[wave], qex[wave],
+                           qpfx[wave], qmark[wave], lstage[wave], tbox[wave]);
+        if (!queue) break;
     }
+}
+
+// The order of the tiles from their costs in the last cut, heaviest first: the
+// costs spread over two orders of magnitude, and a heavy tile started last runs
+// alone at the end of the launch (1283x719 pixels, 250001 AVPLs, a budget of
+// 8191: 8.4 ms in no order, 6.8 so).  A bucket sort on eight buckets per octave of cost, in one
+// workgroup; the order within a bucket is that of the LDS atomics.  A tile's
+// result does not depend on the order.
+constexpr int kOrderBins = 256;
+constexpr int kOrderThreads = 1024;
+
+__device__ inline int order_bin(float c) {
+    const int b = (int)(__log2f(fmaxf(c, 1.f)) * 8.f);
+    return kOrderBins - 1 - min(max(b, 0), kOrderBins - 1);
+}
+
+__global__ __launch_bounds__(kOrderThreads) void k_tile_order(const float* __restrict__ cost, int n,
+                                                              int* __restrict__ order) {
+    __shared__ int hist[kOrderBins];
+    __shared__ int off[kOrderBins];
+    for (int i = threadIdx.x; i < kOrderBins; i += kOrderThreads) hist[i] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kOrderThreads) atomicAdd(&hist[order_bin(cost[i])], 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int s = 0;
+        for (int b = 0; b < kOrderBins; ++b) {
+            off[b] = s;
+            s += hist[b];
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kOrderThreads) order[atomicAdd(&off[order_bin(cost[i])], 1)] = i;
 }
 
 // A frame's pool: no chunk taken, no tile handed back.
 __global__ void k_pool_reset(CutPool p) {
     if (threadIdx.x == 0) {
-        *p.taken = 0;
-        *p.nserial = 0;
+        for (int k = 0; k < arc::kPoolCounters; ++k) p.count[k] = 0;
     }
     p.next[kNextStride * threadIdx.x] = 0;
 }
@@ -1536,17 +1651,27 @@ constexpr int kMinChunks = 16384;  // 21 MB
 // memory that k_cut_combine writes: a frame still running counts at the next
 // one).  Nothing grows while the stream is captured; held: the caller keeps
 // the memory with the graph.  p.cap is 0 when there is no memory for a pool: the
-// tiles are cut serially then.
+// tiles are cut serially then, as with `want` 0.
 int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, long long want, bool grow, bool held,
                CutPool& p) {
     p = CutPool{};
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     ARC_HIP(ctx, hipStreamIsCapturing(stream, &capture));
     const bool captured = capture != hipStreamCaptureStatusNone;
+    const size_t serial = sizeof(int) * 2 * (size_t)nitems;
+    if (captured && mem.serial.bytes < serial) return ARC_OK;  // not run before: nothing is allocated now
+    ARC_TRY(ensure(ctx, mem.serial, serial));
+    if (mem.tiles != nitems) mem.costs = false;
+    mem.tiles = nitems;
+    p.cost = mem.serial.as<float>();
+    p.order = mem.serial.as<int>() + nitems;
+    p.ordered = mem.costs ? 1 : 0;
+    mem.costs = true;  // the cut that follows writes them
+    if (want == 0) return ARC_OK;
     if (!mem.seen) {
         if (captured) return ARC_OK;
-        ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&mem.seen), sizeof(int), hipHostMallocDefault));
-        *mem.seen = 0;
+        ARC_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&mem.seen), 2 * sizeof(int), hipHostMallocDefault));
+        mem.seen[0] = mem.seen[1] = 0;
     }
     if (grow) {
         const int seen = *static_cast<volatile int*>(mem.seen);
@@ -1559,7 +1684,7 @@ int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, lo
     // one allocation: a new gather's first frame pays for each
     hipError_t e = hipSuccess;
     const size_t chunk = mem.mem.fit((size_t)want, sizeof(float) * 192 + sizeof(uint32_t) * kKeep + sizeof(int4),
-                                     sizeof(int) * ((size_t)11 * nitems + 2 + kNextStride * (kNextCounters + 1)), grow,
+                                     sizeof(int) * ((size_t)11 * nitems + arc::kPoolCounters + kNextStride * (kNextCounters + 1)), grow,
                                      !captured, [&] { e = hipStreamSynchronize(ctx->stream); });
     if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize", __FILE__, __LINE__);
     mem.cap = (int)chunk;
@@ -1569,28 +1694,40 @@ int ready_pool(arc_ctx* ctx, hipStream_t stream, CutPoolMem& mem, int nitems, lo
     char* at = static_cast<char*>(mem.mem.data());
     float* tbox = reinterpret_cast<float*>(at + part + entries + meta);
     int* head = reinterpret_cast<int*>(tbox + 8 * (size_t)nitems);
-    p = CutPool{reinterpret_cast<uint32_t*>(at + part), reinterpret_cast<int4*>(at + part + entries),
-                reinterpret_cast<float*>(at), tbox, head, head + nitems,
-                head + 2 * (size_t)nitems, head + 3 * (size_t)nitems, head + 3 * (size_t)nitems + 1,
-                head + 3 * (size_t)nitems + 2 + kNextStride, mem.seen, (int)chunk, nitems < 4096 ? 4 : 8};
+    int* counters = head + 3 * (size_t)nitems;
+    p.entries = reinterpret_cast<uint32_t*>(at + part);
+    p.meta = reinterpret_cast<int4*>(at + part + entries);
+    p.part = reinterpret_cast<float*>(at);
+    p.tbox = tbox;
+    p.head = head;
+    p.evaluated = head + nitems;
+    p.serial = head + 2 * (size_t)nitems;
+    p.count = counters;
+    p.next = counters + arc::kPoolCounters + kNextStride;
+    p.seen = mem.seen;
+    p.cap = (int)chunk;
+    p.fixed = !grow || mem.mem.refused();
+    p.grab = nitems < 4096 ? 4 : 8;
     return ARC_OK;
 }
 
 // Resident waves of k_cut_eval: eight per SIMD.
 constexpr int kEvalBlocks = 2048;
 
-// Below this budget the serial cut takes every tile: most would reach their
-// budget, and entering subtrees that are then taken back costs more than it
-// saves (1283x719 pixels, 250001 AVPLs: 2.9 ms against 4.0 at a budget of 4096,
-// 7.6 against 7.7 at 15000; 200x120 pixels, 20000 AVPLs: 1.0 against 1.2 and
-// 2.0 against 0.7).
-constexpr int kSerialBudget = 8192;
+// Tiles that leave at most four waves per SIMD: k_cut_serial built for four has
+// registers for everything.
+constexpr int kFewTiles = 4096;
 
 template <bool kMany>
 void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool expansion, bool serial, const CutPool& p) {
     const int blocks = (nitems + 3) / 4;
     if (serial) {
-        hipLaunchKernelGGL(k_cut_serial<kMany>, dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, 1, p);
+        if (p.ordered)
+            hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderThreads), 0, stream, p.cost, nitems, p.order);
+        if (nitems <= kFewTiles)
+            hipLaunchKernelGGL((k_cut_serial<kMany, 4>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, 1, p);
+        else
+            hipLaunchKernelGGL((k_cut_serial<kMany, 8>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, 1, p);
         return;
     }
     hipLaunchKernelGGL(k_pool_reset, dim3(1), dim3(kNextCounters), 0, stream, p);
@@ -1599,7 +1736,7 @@ void launch_cut(hipStream_t stream, const Views<kMany>& views, int nitems, bool 
     else
         hipLaunchKernelGGL((k_cut_decide<kMany, false>), dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
     hipLaunchKernelGGL(k_cut_eval<kMany>, dim3(std::min(8 * blocks, kEvalBlocks)), dim3(kCutThreads), 0, stream, views, p);
-    hipLaunchKernelGGL(k_cut_serial<kMany>, dim3(std::min(blocks, 256)), dim3(kCutThreads), 0, stream, views, nitems, 0, p);
+    hipLaunchKernelGGL((k_cut_serial<kMany, 8>), dim3(std::min(blocks, kEvalBlocks)), dim3(kCutThreads), 0, stream, views, nitems, 0, p);
     hipLaunchKernelGGL(k_cut_combine<kMany>, dim3(blocks), dim3(kCutThreads), 0, stream, views, nitems, p);
 }
 
@@ -1624,6 +1761,8 @@ size_t PoolDevice::room() {
 }
 
 void release_pool(CutPoolMem& mem) {
+    mem.mem.release();
+    release(mem.serial);
     if (mem.seen) (void)hipHostFree(mem.seen);
     mem = CutPoolMem{};
 }
@@ -1651,15 +1790,17 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
         *defer = v;
         return ARC_OK;
     }
-    bool serial = cp.budget < kSerialBudget;
+    // what the last cut of this setting says: how many tiles met their budget, or found a pool full that does not grow
+    CutPoolMem& mem = g->pool;
+    const CutSetting now{nitems, cp.budget, cp.exact_count, cp.criterion, g->est_chunks, cp.eps, cp.image_floor};
+    if (mem.seen && !(mem.last == now)) mem.seen[1] = 0;
+    const bool serial = serial_cut(cp.budget, nitems, mem.seen ? static_cast<volatile int*>(mem.seen)[1] : 0);
+    mem.last = now;
     CutPool pool{};
-    if (!serial) {
-        const long long per_tile = g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);
-        ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, g->batch_capture, pool));
-        serial = pool.cap == 0;
-    }
+    const long long per_tile = serial ? 0 : g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);
+    ARC_TRY(ready_pool(ctx, ctx->stream, g->pool, nitems, per_tile * nitems, g->est_chunks == 0, g->batch_capture, pool));
     if (mark) ARC_HIP(ctx, hipEventRecord(mark, ctx->stream));
-    launch_cut<false>(ctx->stream, Views<false>{v}, nitems, cp.criterion == ARC_CRITERION_EXPANSION, serial, pool);
+    launch_cut<false>(ctx->stream, Views<false>{v}, nitems, cp.criterion == ARC_CRITERION_EXPANSION, pool.cap == 0, pool);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }
@@ -1673,7 +1814,7 @@ int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_view
     for (int i = 0; i < nviews; ++i) {
         nitems += host_views[i].ntiles;
         want += (long long)host_views[i].ntiles * default_chunks(host_views[i].n, host_views[i].exact_count);
-        serial = serial || host_views[i].budget < kSerialBudget;
+        serial = serial || serial_cut(host_views[i].budget, 0, 0);
         expansion = expansion || host_views[i].criterion == ARC_CRITERION_EXPANSION;
     }
     CutPool pool{};

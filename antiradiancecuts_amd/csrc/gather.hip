@@ -1345,6 +1345,7 @@ int arc_gather_set_estimate_pool(arc_gather* g, int chunks_per_tile) {
         return arc::fail(g->ctx, ARC_E_INVALID, "estimate pool: 0..256 chunks per tile");
     g->est_chunks = chunks_per_tile;
     g->pool.mem.retry();  // the device may have the memory by now that it refused
+    g->pool.last = arc::CutSetting{};
     return ARC_OK;
 }
 

@@ -43,20 +43,31 @@ struct CutView {
 
 // The chunks of a moment cut's launch: kept nodes and exact ranges found by
 // the decision kernel, summed by the evaluation kernel (cut_moments.hip).
+enum PoolCount {
+    kTaken,        // chunks asked for (may pass cap)
+    kSerialTiles,  // tiles to cut serially
+    kFullTiles,    // of these, tiles that found the pool full
+    kSpentTiles,   // tiles that met their budget
+    kSerialNext,   // k_cut_serial's next tile
+    kPoolCounters
+};
 struct CutPool {
     uint32_t* entries;  // cap chunks of 128 entries
     int4* meta;         // per chunk: (tile, kind | entries << 8, the tile's next chunk or -1, the chunk that holds
                         // its entries and which part of them)
     float* part;        // per chunk: 3 x 64 partial sums
-    float* tbox;        // per tile: its box, centre and half extent (8 floats)
+    float* tbox;        // per tile: its box, centre and half extent, and its cost (8 floats)
     int* head;          // per tile: its first chunk or -1
     int* evaluated;     // per tile: nodes and leaves its cut sums, -1 when it is cut serially
     int* serial;        // the tiles to cut serially
-    int* taken;         // chunks asked for (may pass cap)
-    int* nserial;
+    int* count;         // a frame's counts (PoolCount)
+    float* cost;        // per tile: its cost in vector instructions in the last cut, estimated from its counts
+    int* order;         // the tiles by the last cut's costs
+    int ordered;        // whether there are any
     int* next;          // the evaluation's counters of chunks
-    int* seen;          // pinned host memory: chunks the frame asked for
+    int* seen;          // pinned host memory: chunks the frame asked for, tiles better cut serially
     int cap;
+    int fixed;          // the pool does not grow: tiles that find it full are better cut serially
     int grab;           // chunks a tile takes with its first atomic, twice as many with each later one: the
                         // counter serves about 100 atomics per microsecond, and a tile's last grab leaves
                         // some unused, which the evaluation has to pass over
@@ -67,10 +78,25 @@ struct PoolDevice {
     static void free(void* p);
     static size_t room();
 };
+// What the tiles' cuts depend on besides the scene.
+struct CutSetting {
+    int tiles = 0, budget = 0, exact_count = 0, criterion = 0, chunks = 0;
+    float eps = 0.f, floor = 0.f;
+    bool operator==(const CutSetting& o) const {
+        return tiles == o.tiles && budget == o.budget && exact_count == o.exact_count && criterion == o.criterion &&
+               chunks == o.chunks && eps == o.eps && floor == o.floor;
+    }
+};
 struct CutPoolMem {
     PoolMemory<PoolDevice> mem;
+    // the tiles' costs in the last cut and the order made from them, for `tiles`
+    // tiles (costs: whether there are any)
+    DevBuf serial;
+    int tiles = 0;
+    bool costs = false;
     int* seen = nullptr;
     int cap = 0;
+    CutSetting last;  // of the last cut that was decided 64 nodes at a time
 };
 void release_pool(CutPoolMem& mem);
 }  // namespace arc

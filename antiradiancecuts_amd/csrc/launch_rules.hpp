@@ -15,4 +15,22 @@ constexpr int anti_block(int setting, bool staged) {
     return setting == kAntiBlock && staged ? kAntiBlockStaged : setting;
 }
 
+// Whether a moment cut's tiles are all cut serially, a node at a time, with the
+// sums in the same wave, the heaviest first by the last cut's costs.  A tile that
+// meets its budget is decided twice by the kernel that takes 64 nodes at a time,
+// so the line lies where most tiles would: at budgets below 8192, and, where the
+// last cut of this setting says so (`bad`: tiles that met their budget, or found
+// a pool full that does not grow), from a quarter of the tiles on.  Below 2048
+// tiles a serial wave's latency is what counts, and the other kernel's is shorter.
+// Milliseconds a frame, serial and decided, over 20000, 60000 and 250001 AVPLs:
+//                 200x120        640x360        1283x719
+//   budget  4096  0.91   1.12    1.63   2.02     4.49    6.41
+//           8192  1.63   1.30    2.22   2.83     6.82    8.65
+//          12000  1.94   0.66    2.82   3.88     8.5    10.0   (a quarter and 30 % of the tiles, none of 200x120)
+//          16384  1.94   0.66    3.30   2.83     9.2     9.2   (1.5 % and 13 %)
+constexpr int kSerialBudget = 8192, kSerialMinTiles = 2048;
+constexpr bool serial_cut(int budget, int tiles, int bad) {
+    return budget < kSerialBudget || (tiles >= kSerialMinTiles && 4LL * bad >= tiles);
+}
+
 }  // namespace arc

@@ -18,6 +18,10 @@ int main() {
     check(arc::anti_block(1536, false) == 1536, "the default block of the others");
     for (int staged = 0; staged < 2; ++staged)
         for (int set : {768, 3072}) check(arc::anti_block(set, staged) == set, "a block that was set");
+    check(arc::serial_cut(8191, 100, 0) && !arc::serial_cut(8192, 100, 0), "the budget's line");
+    check(!arc::serial_cut(65536, 2047, 2047), "few tiles are not cut serially");
+    check(arc::serial_cut(65536, 2048, 512) && !arc::serial_cut(65536, 2048, 511), "the tiles' line");
+    check(arc::serial_cut(65536, 2000000000, 2000000000), "many tiles");
     if (!failures) std::printf("launch rules hold\n");
     return failures ? 1 : 0;
 }
