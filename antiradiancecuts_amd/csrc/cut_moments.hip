@@ -694,6 +694,14 @@ __global__ __launch_bounds__(kCutThreads) void k_cut_decide(Views<kMany> views, 
         if (lane == 0) pool.head[item] = -1;
         return;
     }
+    if (kMany && v.budget < arc::kSerialBudget) {  // a view whose tiles are cut serially among others whose are not
+        if (lane == 0) {
+            pool.head[item] = -1;
+            pool.serial[atomicAdd(pool.count + arc::kSerialTiles, 1)] = item;
+            pool.evaluated[item] = -1;
+        }
+        return;
+    }
     DecideLds& S = lds[wave];
     const bool outside = !((alive >> 63) & 1);  // some lane is outside the image
     const bool expansion = kExpansion && v.criterion == ARC_CRITERION_EXPANSION;
@@ -1810,16 +1818,16 @@ int cut_moments_views(arc_ctx* ctx, hipStream_t stream, const CutView* host_view
     if (nviews < 1) return ARC_OK;
     int nitems = 0;
     long long want = 0;
-    bool serial = false, expansion = false;
+    bool expansion = false;
     for (int i = 0; i < nviews; ++i) {
         nitems += host_views[i].ntiles;
-        want += (long long)host_views[i].ntiles * default_chunks(host_views[i].n, host_views[i].exact_count);
-        serial = serial || serial_cut(host_views[i].budget, 0, 0);
+        if (!serial_cut(host_views[i].budget, 0, 0))
+            want += (long long)host_views[i].ntiles * default_chunks(host_views[i].n, host_views[i].exact_count);
         expansion = expansion || host_views[i].criterion == ARC_CRITERION_EXPANSION;
     }
     CutPool pool{};
     ARC_TRY(ready_pool(ctx, stream, mem, nitems, want, true, true, pool));
-    launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, serial || pool.cap == 0, pool);
+    launch_cut<true>(stream, Views<true>{views, nviews}, nitems, expansion, pool.cap == 0, pool);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }

@@ -10,7 +10,7 @@ import pytest
 
 from antiradiancecuts_amd import ffi
 from antiradiancecuts_amd import scene as S
-from antiradiancecuts_amd.runtime import DeviceAvpls, Gather, default_params, device_array
+from antiradiancecuts_amd.runtime import Batch, DeviceAvpls, Gather, default_params, device_array
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +97,36 @@ def test_frames_repeat(gpu_ctx, w, h, n, bound, budget):
     assert np.array_equal(images[2], images[3])
     if budget != 9_000:
         assert np.array_equal(images[0], images[2])
+
+
+@pytest.mark.parametrize("budgets", [(512, 65_536, 65_536), (512, 512, 512), (65_536, 4096, 9_000)])
+def test_one_launch_of_uneven_budgets(gpu_ctx, budgets):
+    """Views whose tiles are cut serially in one launch with views whose are
+    not: each replay gives every view's eager image."""
+    shapes = [(203, 117, 20_000), (320, 200, 9_000), (96, 64, 30_000)]
+    b = Batch(gpu_ctx, lanes=2)
+    views, ref = [], []
+    try:
+        for k, ((w, h, n), budget) in enumerate(zip(shapes, budgets)):
+            sc, g, av = rig(b.lane(k), w, h, n, seed=40 + k)
+            p = params(errorBound=1e-3, cutBudget=budget)
+            g.run(av, sc.cam, sc.extent, p)
+            b.lane(k).sync()
+            ref.append(g.radiance[:, :3].cpu().numpy())
+            views.append((g, av, sc.cam, sc.extent, p))
+        print(f"[serial] one launch, budgets {budgets}", flush=True)
+        b.set_one_cut_launch(True)
+        b.capture(views)
+        for rep in range(3):
+            for g, *_ in views:
+                g.radiance.fill_(-1.0)
+            b.launch()
+            gpu_ctx.sync()
+            for k, (g, *_rest) in enumerate(views):
+                e = rel(g.radiance[:, :3].cpu().numpy(), ref[k])
+                print(f"[serial] replay {rep} view {k}: rel-L2 {e:.2e}", flush=True)
+                assert e <= 1e-5
+    finally:
+        for g, *_ in views:
+            g.close()
+        b.close()
