@@ -188,23 +188,28 @@ int arc_batch_capture(arc_batch* b, const arc_batch_view* views, int nviews) {
     }
     drop_graph(b);
     const bool one_cut = b->one_cut && all_moment_cuts(views, nviews);
-    // 1. every view once, eagerly: buffers reach their final sizes.  The
-    // lanes first wait for the caller's stream, which produced the inputs.
-    ARC_TRY(fork_lanes(b, ctx->stream, b->fork));
-    for (int i = 0; i < nviews; ++i) {
-        const arc_batch_view& v = views[i];
-        ARC_TRY(arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr));
+    // 1. every view once, eagerly: buffers reach their final sizes (in one cut
+    // launch the batch's own pool, and the views need none).  The lanes first
+    // wait for the caller's stream, which produced the inputs.
+    if (one_cut) {
+        ARC_TRY(prepare_one_cut(b, views, nviews));
+        ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    } else {
+        ARC_TRY(fork_lanes(b, ctx->stream, b->fork));
+        for (int i = 0; i < nviews; ++i) {
+            const arc_batch_view& v = views[i];
+            ARC_TRY(arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr));
+        }
+        for (arc_ctx* c : b->lanes) ARC_HIP(ctx, hipStreamSynchronize(c->stream));
+        ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        // a view whose cut's pool was too small runs again: the pool grows, which it cannot in the graph
+        for (int i = 0; i < nviews; ++i) {
+            const arc_batch_view& v = views[i];
+            if (!arc::cut_pool_short(v.gather)) continue;
+            ARC_TRY(arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr));
+            ARC_HIP(ctx, hipStreamSynchronize(arc_gather_ctx(v.gather)->stream));
+        }
     }
-    for (arc_ctx* c : b->lanes) ARC_HIP(ctx, hipStreamSynchronize(c->stream));
-    ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    // a view whose cut's pool was too small runs again: the pool grows, which it cannot in the graph
-    for (int i = 0; i < nviews; ++i) {
-        const arc_batch_view& v = views[i];
-        if (!arc::cut_pool_short(v.gather)) continue;
-        ARC_TRY(arc_gather_run(v.gather, &v.avpls, v.camPos, v.sceneExtent, &v.params, ARC_TRUST_INPUT, nullptr));
-        ARC_HIP(ctx, hipStreamSynchronize(arc_gather_ctx(v.gather)->stream));
-    }
-    if (one_cut) ARC_TRY(prepare_one_cut(b, views, nviews));
     // 2. capture on the batch's own stream (the legacy null stream cannot be
     // captured): fork the lanes from it, run the views on their lanes, join
     // back.  The launch orders the whole graph on the caller's stream.

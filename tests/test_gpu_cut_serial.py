@@ -108,11 +108,11 @@ def test_one_launch_of_uneven_budgets(gpu_ctx, budgets):
     views, ref = [], []
     try:
         for k, ((w, h, n), budget) in enumerate(zip(shapes, budgets)):
-            sc, g, av = rig(b.lane(k), w, h, n, seed=40 + k)
             p = params(errorBound=1e-3, cutBudget=budget)
-            g.run(av, sc.cam, sc.extent, p)
-            b.lane(k).sync()
-            ref.append(g.radiance[:, :3].cpu().numpy())
+            sc, g, av = rig(gpu_ctx, w, h, n, seed=40 + k)
+            ref.append(frame(gpu_ctx, sc, g, av, p)[0])
+            g.close()
+            sc, g, av = rig(b.lane(k), w, h, n, seed=40 + k)  # has run no frame before the capture
             views.append((g, av, sc.cam, sc.extent, p))
         print(f"[serial] one launch, budgets {budgets}", flush=True)
         b.set_one_cut_launch(True)
