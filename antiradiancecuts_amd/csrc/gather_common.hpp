@@ -202,22 +202,10 @@ struct Kahan {
 
 __device__ inline f3 f3of(float4 v) { return f3{v.x, v.y, v.z}; }
 
-
-// Wave-uniform record reads (the nodes' boxes and moment records, one
-// address for the whole wave) go through the constant address space in the
-// device pass: a uniform load from it is a scalar load (one request for the
-// wave, the values in scalar registers) whatever the compiler can prove
-// about aliasing stores.  The reads are of scalars, so no vector type's
-// constructor meets the address space.
-#if defined(__HIP_DEVICE_COMPILE__)
-#define ARC_UNIFORM_AS __attribute__((address_space(4)))
-#else
-#define ARC_UNIFORM_AS
-#endif
-using ufloat = const ARC_UNIFORM_AS float;
-using uint_ = const ARC_UNIFORM_AS int;
-__device__ inline ufloat* uptr(const void* p) { return (ufloat*)p; }
-__device__ inline float4 uload4(ufloat* p) { return make_float4(p[0], p[1], p[2], p[3]); }
+using arc::ufloat;
+using arc::uint_;
+using arc::uptr;
+using arc::uload4;
 
 // ----------------------------------------------------------- pixels ----
 struct PixelF {

@@ -33,4 +33,29 @@ constexpr bool serial_cut(int budget, int tiles, int bad) {
     return budget < kSerialBudget || (tiles >= kSerialMinTiles && 4LL * bad >= tiles);
 }
 
+// Whether a wave's 64 rays go through the triangle tree together, one ray a lane,
+// or eight by eight, each ray in eight lanes of its own.  Together a node costs
+// the wave 14 instructions a child however few of the rays enter it, so that pays
+// where a tree has few nodes for the rays, and with fewer rays the chip is not
+// full.  A camera's rays enter much the same nodes; a path's go everywhere, but
+// those that leave one light start alike and a long shoot takes many; rays from
+// the caller may be in any order.  Microseconds, together and in groups of eight:
+//   nodes                  5          31           100           413          1058
+//   pixels  640x360     10   13    18    26     22    29     43     55     62     86
+//         3840x2160     74  325   231   710    266   783    554   1510    854   2427
+//   paths      1e5     388  693   570   733   1046   813   2691    992   4311   1074
+//              5e5     995 2589  1123  2778   1640  3121   4012   3663   6918   3924
+//              2e6    2786 9825  2922 10538   4039 11554  10999  13792  19540  14744
+//   rays, at random
+//              1e5      12   11    54    22    124    34    356     54    705     75
+//              1e6      36   79   181   156    413   253   1162    386   2271    514
+// A picture of more nodes than that would gain too as long as its neighbouring
+// pixels see the same triangles; where they do not, it is the rays at random.
+enum class Rays { kCamera, kPaths, kAny };
+constexpr int kTogetherRays = 200000, kTogetherPaths = 100000, kPathsPerNode = 1600;
+constexpr bool rays_together(Rays kind, long long rays, int nodes) {
+    if (kind == Rays::kPaths) return rays >= kTogetherPaths && rays >= (long long)kPathsPerNode * nodes && nodes <= 512;
+    return rays >= kTogetherRays && nodes <= (kind == Rays::kCamera ? 512 : 16);
+}
+
 }  // namespace arc

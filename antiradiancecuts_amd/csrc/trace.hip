@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "arc_internal.hpp"
+#include "launch_rules.hpp"
 
 using arc::f3;
 
@@ -52,6 +53,7 @@ struct arc_trace_scene {
     arc::DevBuf tri;                  // 4 float4 per triangle, input order
     arc::DevBuf nodes;                // the tree's eight-wide nodes, 16 float4 each (wide_nodes)
     int stack = 1;                    // most nodes a traversal keeps pending
+    int nnodes = 0;                   // eight-wide nodes
     arc::DevBuf mats;                 // material table, 256 entries
     arc::DevBuf emissive;             // per material: emissive != 0
     int max_depth = 0;                // deepest internal node of the binary tree (root = 1)
@@ -327,6 +329,72 @@ __device__ inline void ray_wide(const SceneDev& S, Ray& mine, int from, int2* st
     }
 }
 
+// The rays of a wave, one per lane, through the tree together: an entry of the
+// stack is a node and the rays that enter it, its records are read once for the
+// wave as scalars, and each child is tested by all of the node's rays.  For trees
+// of a few nodes and many rays (rays_together): there a ray in eight lanes of its
+// own spends its steps on nodes that its neighbours visit too, and the blocks are
+// eight times as many.  Bound by vector instructions, about 14 per child and 40 per
+// triangle.  12 triangles, 5 nodes: 1920x1080 pixels 85 -> 23 us, a million rays 79
+// -> 36, two million paths 9.8 -> 2.8 ms.  The tests are those of ray_step, so the
+// hits are the same bits.  The pending nodes are at most those of one ray that
+// enters every box, which S.stack counts.
+__device__ inline void packet_trace(const SceneDev& S, Ray& r, int4* stk) {
+    using namespace arc;
+    uint64_t m = __ballot(r.on);
+    int sp = 0, node = 0;
+    while (m) {
+        ufloat* c = uptr(S.nodes + 16 * (size_t)node);
+        for (int k = 0; k < kGroup; ++k, c += 8) {
+            const float4 lo = uload4(c), hi = uload4(c + 4);
+            const int child = __float_as_int(lo.w);
+            if (child == kNoChild) break;  // the children come first
+            const float tx0 = (lo.x - r.o.x) * r.inv.x, tx1 = (hi.x - r.o.x) * r.inv.x;
+            const float ty0 = (lo.y - r.o.y) * r.inv.y, ty1 = (hi.y - r.o.y) * r.inv.y;
+            const float tz0 = (lo.z - r.o.z) * r.inv.z, tz1 = (hi.z - r.o.z) * r.inv.z;
+            const float t0 = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.f));
+            const float t1 = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), r.t));
+            const bool in = t0 <= t1 * kBoxSlack && t0 != INFINITY;
+            const uint64_t enter = __ballot(in) & m;
+            if (!enter) continue;
+            if (child < 0) {
+                if (threadIdx.x == 0) stk[sp] = make_int4(-(child + 1), (int)(uint32_t)enter, (int)(uint32_t)(enter >> 32), 0);
+                ++sp;
+                continue;
+            }
+            ufloat* p = uptr(S.tri + 4 * (size_t)child);
+            const Tri T{uload4(p), uload4(p + 4), uload4(p + 8), make_float4(0.f, 0.f, 0.f, 0.f)};
+            float d;
+            if ((enter >> threadIdx.x & 1) && tri_hit(T, r.o, r.d, r.det_eps, d) && d > 0.f &&
+                (d < r.t || (d == r.t && child < r.tri))) {
+                r.t = d;
+                r.tri = child;
+            }
+        }
+        m = 0;
+        if (sp > 0) {
+            __builtin_amdgcn_wave_barrier();  // lane 0's writes before the wave's reads
+            const int4 e = stk[--sp];
+            node = __builtin_amdgcn_readfirstlane(e.x);
+            m = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(e.y) |
+                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(e.z) << 32;
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    r.on = false;
+}
+
+// Each ray to its end: kLanes lanes of the wave per ray, 8 or 1.
+template <int kLanes>
+__device__ inline void trace_rays(const SceneDev& S, Ray& r, int4* stacks) {
+    if constexpr (kLanes == 1) {
+        packet_trace(S, r, stacks);
+    } else {
+        int2* stk = reinterpret_cast<int2*>(stacks) + (size_t)(threadIdx.x / kGroup) * S.stack;
+        while (__ballot(r.on)) ray_step(S, r, stk);
+    }
+}
+
 // Scene::IntersectRayScene: a hit on an emissive triangle is no hit.
 __device__ inline int scene_hit(const SceneDev& S, const Ray& r) {
     if (r.tri < 0) return -1;
@@ -446,15 +514,17 @@ struct Staged {  // AVPLs in the order they were created; path -1: no AVPL
 constexpr int kWideRays = 4;   // most rays of a wave that it takes one by one
 constexpr int kSlotGrab = 64;  // staging slots a wave takes with one atomic
 
+template <int kLanes>
 __global__ __launch_bounds__(kWave) void k_paths(SceneDev S, Light L, uint64_t seed, int paths, int explicit_direct,
                                                     int* __restrict__ next_path, unsigned* __restrict__ n_staged, int cap,
                                                     int* __restrict__ count, Staged st) {
-    extern __shared__ int2 stacks[];
-    const int grp = threadIdx.x / kGroup, lane = threadIdx.x & 63;
-    const bool lead = (threadIdx.x & (kGroup - 1)) == 0;
+    extern __shared__ int4 lds[];
+    int2* stacks = reinterpret_cast<int2*>(lds);
+    const int grp = threadIdx.x / kLanes, lane = threadIdx.x & 63;
+    const bool lead = (threadIdx.x & (kLanes - 1)) == 0;
     int2* stk = stacks + (size_t)grp * S.stack;
     int slots = 0, nslots = 0;  // the wave's staging slots
-    int path = (int)blockIdx.x * kGroups + grp;
+    int path = (int)blockIdx.x * (kWave / kLanes) + grp;
     bool wide = false;          // so few paths are left that the wave traces each ray as a whole
     bool fresh = true, done = false;  // the group starts a path; has none left
     V pos{}, nrm{}, rad0{}, in_dir{}, direction{};
@@ -534,7 +604,7 @@ __global__ __launch_bounds__(kWave) void k_paths(SceneDev S, Light L, uint64_t s
             if (lane == 0) got = atomicAdd(next_path, __popcll(me));
             got = __builtin_amdgcn_readfirstlane(got);
             // the group's leader's place among the wave's leaders
-            const int mine = got + __popcll(me & ((1ull << (lane & ~(kGroup - 1))) - 1ull));
+            const int mine = got + __popcll(me & ((1ull << (lane & ~(kLanes - 1))) - 1ull));
             if (shade && ended && !fresh) path = mine;
         }
         if (shade && ended) {
@@ -559,6 +629,10 @@ __global__ __launch_bounds__(kWave) void k_paths(SceneDev S, Light L, uint64_t s
         if (shade && !done) ray_start(r, pos + kEps * nrm, direction, kEps);
         const uint64_t live = __ballot(!done);
         if (live == 0) break;
+        if constexpr (kLanes == 1) {
+            packet_trace(S, r, lds);
+            continue;
+        }
         if (wide) {  // every live ray starts here
             for (uint64_t m = live & 0x0101010101010101ull; m; m &= m - 1) ray_wide(S, r, __builtin_ctzll(m), stacks);
             continue;
@@ -645,12 +719,14 @@ struct Camera {
     V pos, right, up, fwd;  // right and up scaled by tan(fovy / 2) (and the aspect)
 };
 
+template <int kLanes>
 __global__ __launch_bounds__(kWave) void k_gbuffer(SceneDev S, Camera cam, int W, int H,
                                                       float4* __restrict__ pos4, float4* __restrict__ nrm4) {
-    extern __shared__ int2 stacks[];
-    // a block's rays are 4 x 2 pixels
-    const int grp = threadIdx.x / kGroup, bw = (W + 3) / 4;
-    const int px = (int)(blockIdx.x % bw) * 4 + (grp & 3), py = (int)(blockIdx.x / bw) * 2 + (grp >> 2);
+    extern __shared__ int4 lds[];
+    // a block's rays are 4 x 2 pixels, or 8 x 8
+    constexpr int bx = kLanes == 1 ? 8 : 4, by = kWave / kLanes / bx;
+    const int grp = threadIdx.x / kLanes, bw = (W + bx - 1) / bx;
+    const int px = (int)(blockIdx.x % bw) * bx + grp % bx, py = (int)(blockIdx.x / bw) * by + grp / bx;
     const bool live = px < W && py < H;
     const int i = py * W + px;
     const float sx = 2.f * ((float)px + 0.5f) / (float)W - 1.f;
@@ -659,8 +735,8 @@ __global__ __launch_bounds__(kWave) void k_gbuffer(SceneDev S, Camera cam, int W
     Ray r;
     ray_start(r, cam.pos, dir, 0.f);  // a rasteriser has no |det| floor: any front face counts
     r.on = live;
-    while (__ballot(r.on)) ray_step(S, r, stacks + (size_t)grp * S.stack);
-    if (!live || (threadIdx.x & (kGroup - 1)) != 0) return;
+    trace_rays<kLanes>(S, r, lds);
+    if (!live || (threadIdx.x & (kLanes - 1)) != 0) return;
     const int s = r.tri;
     const float t = r.t;
     if (s < 0) {
@@ -702,17 +778,18 @@ __global__ void k_paths_reset(int* __restrict__ counters, int first) {
     counters[1] = 0;
 }
 
+template <int kLanes>
 __global__ __launch_bounds__(kWave) void k_intersect(SceneDev S, const f3* __restrict__ org,
-                                                        const f3* __restrict__ dir, int n, float* __restrict__ t,
-                                                        int* __restrict__ tri_index) {
-    extern __shared__ int2 stacks[];
-    const int grp = threadIdx.x / kGroup, i = blockIdx.x * kGroups + grp;
+                                                     const f3* __restrict__ dir, int n, float* __restrict__ t,
+                                                     int* __restrict__ tri_index) {
+    extern __shared__ int4 lds[];
+    const int grp = threadIdx.x / kLanes, i = blockIdx.x * (kWave / kLanes) + grp;
     const bool live = i < n;
     Ray r;
     ray_start(r, ld(org[live ? i : 0]), ld(dir[live ? i : 0]), kEps);
     r.on = live;
-    while (__ballot(r.on)) ray_step(S, r, stacks + (size_t)grp * S.stack);
-    if (!live || (threadIdx.x & (kGroup - 1)) != 0) return;
+    trace_rays<kLanes>(S, r, lds);
+    if (!live || (threadIdx.x & (kLanes - 1)) != 0) return;
     const int s = scene_hit(S, r);
     t[i] = s < 0 ? -1.f : r.t;
     tri_index[i] = s;
@@ -1132,6 +1209,7 @@ int arc_trace_scene_create(arc_ctx* ctx, const arc_float3* p0, const arc_float3*
     if (st == ARC_OK) {
         std::vector<float4> wide;
         wide_nodes(hn, order, plo, phi, ptri, wide, sc->stack);
+        sc->nnodes = (int)(wide.size() / 16);
         st = arc::ensure(ctx, sc->nodes, sizeof(float4) * wide.size());
         if (st == ARC_OK) {
             e = hipMemcpy(sc->nodes.p, wide.data(), sizeof(float4) * wide.size(), hipMemcpyHostToDevice);
@@ -1168,8 +1246,14 @@ int arc_trace_intersect(arc_trace_scene* sc, const arc_float3* org, const arc_fl
     if (!sc || n < 0 || (n > 0 && (!org || !dir || !t || !tri_index))) return ARC_E_INVALID;
     if (n == 0) return ARC_OK;
     arc_ctx* ctx = sc->ctx;
-    hipLaunchKernelGGL(k_intersect, dim3((n + kGroups - 1) / kGroups), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc),
-                       reinterpret_cast<const f3*>(org), reinterpret_cast<const f3*>(dir), n, t, tri_index);
+    const bool together = arc::rays_together(arc::Rays::kAny, n, sc->nnodes);
+    const int per = together ? kWave : kGroups;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((n + per - 1) / per), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc),
+                           reinterpret_cast<const f3*>(org), reinterpret_cast<const f3*>(dir), n, t, tri_index);
+    };
+    if (together) launch(k_intersect<1>);
+    else launch(k_intersect<kGroup>);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }
@@ -1225,7 +1309,9 @@ int arc_trace_shoot(arc_trace_scene* sc, const arc_area_light* light, int num_pa
         return r;
     };
     const size_t slot_bytes = 5 * sizeof(f3) + 3 * sizeof(int);
-    const int pblocks = std::min((num_paths + kGroups - 1) / kGroups, kPathBlocks);
+    const bool together = arc::rays_together(arc::Rays::kPaths, num_paths, sc->nnodes);
+    const int per = together ? kWave : kGroups;  // paths of a wave
+    const int pblocks = std::min((num_paths + per - 1) / per, kPathBlocks);
     // a path makes 5 AVPLs at most on average (roulette at 0.8), and a wave
     // may leave a grab's rest unused
     size_t cap = std::min(std::max(8 * np + (size_t)kSlotGrab * pblocks, sc->stage.bytes / slot_bytes), (size_t)INT_MAX);
@@ -1234,9 +1320,13 @@ int arc_trace_shoot(arc_trace_scene* sc, const arc_area_light* light, int num_pa
     for (;;) {  // a second time when the paths made more AVPLs than that
         ARC_TRY(arc::ensure(ctx, sc->stage, cap * slot_bytes));
         st = stage_at(sc->stage, cap);
-        hipLaunchKernelGGL(k_paths_reset, dim3(1), dim3(1), 0, ctx->stream, counters, pblocks * kGroups);
-        hipLaunchKernelGGL(k_paths, dim3(pblocks), dim3(kWave), stack_bytes(sc), ctx->stream, S, L, seed, num_paths,
-                           explicit_direct, counters, reinterpret_cast<unsigned*>(counters + 1), (int)cap, count, st);
+        hipLaunchKernelGGL(k_paths_reset, dim3(1), dim3(1), 0, ctx->stream, counters, pblocks * per);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(pblocks), dim3(kWave), stack_bytes(sc), ctx->stream, S, L, seed, num_paths,
+                               explicit_direct, counters, reinterpret_cast<unsigned*>(counters + 1), (int)cap, count, st);
+        };
+        if (together) launch(k_paths<1>);
+        else launch(k_paths<kGroup>);
         ARC_LAUNCHED(ctx);
         ARC_HIP(ctx, hipMemcpyAsync(&staged, counters + 1, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         ARC_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1298,9 +1388,14 @@ int arc_trace_gbuffer(arc_trace_scene* sc, arc_float3 camPos, arc_float3 forward
     const float th = std::tan(0.5f * fovy), aspect = (float)width / (float)height;
     Camera cam{mk(camPos.x, camPos.y, camPos.z), mk(rx * th * aspect, ry * th * aspect, rz * th * aspect),
                mk(ux * th, uy * th, uz * th), mk(fx, fy, fz)};
-    const int gblocks = ((width + 3) / 4) * ((height + 1) / 2);
-    hipLaunchKernelGGL(k_gbuffer, dim3(gblocks), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc), cam, width,
-                       height, reinterpret_cast<float4*>(pos4), reinterpret_cast<float4*>(nrm4));
+    const bool together = arc::rays_together(arc::Rays::kCamera, (long long)width * height, sc->nnodes);
+    const int gblocks = together ? ((width + 7) / 8) * ((height + 7) / 8) : ((width + 3) / 4) * ((height + 1) / 2);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gblocks), dim3(kWave), stack_bytes(sc), ctx->stream, scene_dev(sc), cam, width, height,
+                           reinterpret_cast<float4*>(pos4), reinterpret_cast<float4*>(nrm4));
+    };
+    if (together) launch(k_gbuffer<1>);
+    else launch(k_gbuffer<kGroup>);
     ARC_LAUNCHED(ctx);
     return ARC_OK;
 }

@@ -22,6 +22,17 @@ int main() {
     check(!arc::serial_cut(65536, 2047, 2047), "few tiles are not cut serially");
     check(arc::serial_cut(65536, 2048, 512) && !arc::serial_cut(65536, 2048, 511), "the tiles' line");
     check(arc::serial_cut(65536, 2000000000, 2000000000), "many tiles");
+    using arc::Rays;
+    check(arc::rays_together(Rays::kCamera, 200000, 512) && !arc::rays_together(Rays::kCamera, 199999, 512) &&
+              !arc::rays_together(Rays::kCamera, 33177600, 513),
+          "the lines of a camera's rays");
+    check(arc::rays_together(Rays::kAny, 200000, 16) && !arc::rays_together(Rays::kAny, 199999, 16) &&
+              !arc::rays_together(Rays::kAny, 2147483647, 17),
+          "the lines of the caller's rays");
+    check(arc::rays_together(Rays::kPaths, 100000, 62) && !arc::rays_together(Rays::kPaths, 100000, 63) &&
+              !arc::rays_together(Rays::kPaths, 99999, 1) && !arc::rays_together(Rays::kPaths, 2147483647, 513) &&
+              arc::rays_together(Rays::kPaths, 819200, 512) && !arc::rays_together(Rays::kPaths, 2147483647, 2147483647),
+          "the lines of a shoot's paths");
     if (!failures) std::printf("launch rules hold\n");
     return failures ? 1 : 0;
 }
