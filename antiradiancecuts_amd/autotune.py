@@ -2,11 +2,9 @@
 
 A view's frame time depends on knobs that leave its image alone (to
 rounding):
-  * launch shapes (Gather.set_launch_shape): a traversal stack of 64, 96 or
-    128 nodes (kept for callers that name one: the moment cut's traversal
-    needs no depth any more, so these candidates time the same), and the
-    clustered antiradiance's list entries filed into LDS per pass, 768, 1536
-    or 3072 (the AVPL block of a pass);
+  * a launch shape (Gather.set_launch_shape): the clustered antiradiance's
+    list entries filed into LDS per pass (the AVPL block of a pass), 1536, the
+    library's own choice for the kernel at hand, or 768 or 3072;
   * the moment cut's pool of kept nodes (Gather.set_estimate_pool): sized to
     what the frames ask for, or held to 32 chunks per tile (less memory;
     tiles that find it full are cut node by node);
@@ -31,7 +29,7 @@ import numpy as np
 from . import ffi
 from .runtime import default_params
 
-STACKS = (96, 64, 128)
+STACKS = (96, 64, 128)  # valid, but no kernel's speed depends on it: tune() leaves the default
 CHUNKS = (1536, 768, 3072)
 POOLS = (0, 32)
 
@@ -64,7 +62,7 @@ def candidates(base: ffi.arc_gather_params):
 
 
 def schedule_axes(base: ffi.arc_gather_params):
-    """The launch-shape knobs that apply to `base`: (name, values), the
+    """The launch-shape knobs that `base` accepts: (name, values), the
     current default first."""
     moments = (base.useLightCuts and base.cutMode == ffi.ARC_CUT_ERROR_BOUND
                and base.cutEstimator == ffi.ARC_ESTIMATOR_MOMENTS)
@@ -108,6 +106,8 @@ def tune(gather, avpls, cam, extent, base: ffi.arc_gather_params | None = None, 
     if best is None:  # every candidate reported error pixels: the default schedule stands
         return _copy(base), sched, table
     for name, values in schedule_axes(best):
+        if name == "cut_stack":  # the same kernels at every depth: noise would choose
+            continue
         current = getattr(sched, name)  # timed already: best_ms
         for v in values:
             if v == current:
