@@ -304,19 +304,6 @@ __global__ __launch_bounds__(kScanBlock) void k_mom_nodes(const int* __restrict_
     t[2] = make_float4(__int_as_float(b.left), __int_as_float(b.right), __int_as_float(last - first + 1), 0.f);
 }
 
-// A node's box and children (BvhNode layout: left, right, bbMin, bbMax, visited).
-__device__ inline arc_bvh_node uload_node(const arc_bvh_node* n) {
-    ufloat* f = uptr(n);
-    uint_* i = (uint_*)n;
-    arc_bvh_node b;
-    b.left = i[0];
-    b.right = i[1];
-    b.bbMin = arc_float3{f[2], f[3], f[4]};
-    b.bbMax = arc_float3{f[5], f[6], f[7]};
-    b.visited = 0;  // not read
-    return b;
-}
-
 // Squared distances carry 1e-24 (the first addend of their FMA chain) before
 // their reciprocal square root: 1e36 bounds the cube of the result, at a
 // point that coincides with the pixel the numerators (a cosine times |d|, or
@@ -339,14 +326,10 @@ __device__ inline float pixel_g(const PixelF& P, const float4& x) {
 }
 
 // The node's estimate for the pixel, per channel, added to the pixel's sums.
-template <bool kUniformAs>
 __device__ inline void add_moments(const PixelF& P, const float4* __restrict__ r, Acc& acc) {
     // Records are read in three groups, each just before its use: fewer of
     // them are live at once in scalar registers.
-    auto ld = [&](int i) -> float4 {
-        if constexpr (kUniformAs) return uload4(uptr(r + i));
-        else return r[i];
-    };
+    auto ld = [&](int i) { return uload4(uptr(r + i)); };
     const float4 m0 = ld(0), p01 = ld(2), p12 = ld(3), p23 = ld(4);
     const float K = pixel_g(P, make_float4(p01.x, p01.y, p01.z, 0.f)) +
                     pixel_g(P, make_float4(p01.w, p12.x, p12.y, 0.f)) +
@@ -1274,10 +1257,10 @@ __global__ __launch_bounds__(kCutThreads) __attribute__((amdgpu_waves_per_eu(8))
             Acc acc;
             const int half = min(cnt, 64);
             for (int j = 0; j < half; ++j)
-                add_moments<true>(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e0, j), acc);
+                add_moments(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e0, j), acc);
             acc.flush();
             for (int j = 64; j < cnt; ++j)
-                add_moments<true>(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e1, j - 64), acc);
+                add_moments(F, v.mom + kMom * (size_t)__builtin_amdgcn_readlane(e1, j - 64), acc);
             acc.flush();
             o[0] = acc.k[0].s;
             o[64] = acc.k[1].s;
@@ -1425,7 +1408,7 @@ __device__ __forceinline__ void serial_tile(const CutView& v, float* cost, int i
         }
         nev -= (unsigned)(ne - kept);
         for (int j = 0; j < kept; ++j) {
-            add_moments<true>(P, mom + kMom * (size_t)uniform(E[j]), acc);
+            add_moments(P, mom + kMom * (size_t)uniform(E[j]), acc);
             acc.maybe_flush();
         }
         ne = 0;

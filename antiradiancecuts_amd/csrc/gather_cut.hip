@@ -109,8 +109,6 @@ __device__ inline int add_desc(const CutEB& t, const PixelF& P, int v, Acc& acc)
     return add_desc<(D > 0 ? D - 1 : 0)>(t, P, l, acc) + add_desc<(D > 0 ? D - 1 : 0)>(t, P, r, acc);
 }
 
-constexpr int kMaxEvalDepth = 4;
-
 __device__ inline int add_kept(const CutEB& t, const PixelF& P, int node, int depth, Acc& acc) {
     switch (depth) {
         case 1: return add_desc<1>(t, P, node, acc);

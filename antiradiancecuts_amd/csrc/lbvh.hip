@@ -37,8 +37,6 @@ constexpr int kReduceBlocks = 512;
 // makes the Karras nodes)
 constexpr int kCounters = 13, kNumCounters = 2, kNormalList = 1;
 
-__device__ inline f3 ldf3(const f3* p, size_t i) { return p[i]; }
-
 // ------------------------------------------------------------ bounds ----
 // partials: [block][12] = pos min xyz, pos max xyz, nrm min xyz, nrm max xyz
 __global__ __launch_bounds__(kBlock) void k_bounds_partial(const f3* __restrict__ pos,
