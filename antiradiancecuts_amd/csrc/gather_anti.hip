@@ -35,9 +35,11 @@
 //                  one wave per 8x8 tile; a block reads the cluster's list
 //                  once and sorts its
 //                  entries into per-tile sub-lists in LDS (ray against the
-//                  tile's own box), then each wave walks its sub-list with
-//                  wave-uniform (scalar) loads of the packed records and
-//                  evaluates the guarded pair test per pixel; the list is
+//                  tile's own box), then each wave walks its sub-list,
+//                  64 records at a time staged in LDS for the Lambertian
+//                  cone, with wave-uniform (scalar) loads of the packed
+//                  records otherwise, and evaluates the guarded pair test
+//                  per pixel; the list is
 //                  filed and walked in chunks of the sub-lists' size, so no
 //                  sub-list overflows.  A cluster whose list overflowed
 //                  files every antiradiance AVPL the same way; the

@@ -497,17 +497,17 @@ struct Staged {  // AVPLs in the order they were created; path -1: no AVPL
     int* path;
 };
 
-// createPath (AvplShooter.h:77-142), a path per group of lanes from its first
-// ray to its last: traced, its AVPL staged, continued or replaced by the next
-// path without leaving the kernel.  (With a launch per bounce, the host waits
-// for the count of live paths 47 times per 100K paths, and a bounce of a
-// handful of rays takes as long as its longest ray: 100K paths over 100K
-// triangles took 33 ms, 2.1 here.)  A wave shades when at
-// most half of its rays are still in the tree, so that few lanes wait for the
-// longest one.  What bounds it is the longest path, up to 47 rays one after the
-// other (5.4 ms with eight lanes for each ray to the end); so a wave with no
-// more than four paths left takes their rays one by one with all its lanes
-// (ray_wide).  Draw order per path as in createPath: light position (2),
+// createPath (AvplShooter.h:77-142), a path per group of kLanes lanes (eight, or
+// one where a wave's rays are traced together) from its first ray to its last:
+// traced, its AVPL staged, continued or replaced by the next path without
+// leaving the kernel.  (With a launch per bounce, the host waits for the count
+// of live paths 47 times per 100K paths, and a bounce of a handful of rays takes
+// as long as its longest ray: 100K paths over 100K triangles took 33 ms, 2.1
+// here.)  With eight lanes a ray, a wave shades when at most a third of its live
+// rays are still in the tree, so that few lanes wait for the longest one.  What
+// bounds it is the longest path, up to 47 rays one after the other (5.4 ms with
+// eight lanes for each ray to the end); so a wave with no more than four paths
+// left takes their rays one by one with all its lanes (ray_wide).  Draw order per path as in createPath: light position (2),
 // first direction (2), then per bounce roulette (1) and the next direction
 // (2).  Writes each path's AVPL count; a final scatter puts every path's AVPLs
 // together in path order.  AVPLs past `cap` are counted, not staged.
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(kWave) void k_paths(SceneDev S, Light L, uint64_t s
             continue;
         }
         wide = __popcll(live) <= kWideRays * kGroup;
-        // trace until at most half of the live rays are in the tree; to the
+        // trace until at most a third of the live rays are in the tree; to the
         // end before the wave takes its last rays one by one
         for (;;) {
             const uint64_t on = __ballot(r.on);
