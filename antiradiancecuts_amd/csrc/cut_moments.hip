@@ -1785,7 +1785,8 @@ int cut_moments(arc_gather* g, arc_bvh* b, const CutEBParams& cp, float4* rad, u
     CutPoolMem& mem = g->pool;
     const CutSetting now{nitems, cp.budget, cp.exact_count, cp.criterion, g->est_chunks, cp.eps, cp.image_floor};
     if (mem.seen && !(mem.last == now)) mem.seen[1] = 0;
-    const bool serial = serial_cut(cp.budget, nitems, mem.seen ? static_cast<volatile int*>(mem.seen)[1] : 0);
+    const bool serial = serial_cut(cp.budget, nitems, mem.seen ? static_cast<volatile int*>(mem.seen)[1] : 0,
+                                   cp.criterion == ARC_CRITERION_EXPANSION);
     mem.last = now;
     CutPool pool{};
     const long long per_tile = serial ? 0 : g->est_chunks > 0 ? g->est_chunks : default_chunks(n, cp.exact_count);

@@ -18,19 +18,29 @@ constexpr int anti_block(int setting, bool staged) {
 // Whether a moment cut's tiles are all cut serially, a node at a time, with the
 // sums in the same wave, the heaviest first by the last cut's costs.  A tile that
 // meets its budget is decided twice by the kernel that takes 64 nodes at a time,
-// so the line lies where most tiles would: at budgets below 8192, and, where the
+// so the line lies where many tiles would: at budgets below 8192, and, where the
 // last cut of this setting says so (`bad`: tiles that met their budget, or found
-// a pool full that does not grow), from a quarter of the tiles on.  Below 2048
-// tiles a serial wave's latency is what counts, and the other kernel's is shorter.
-// Milliseconds a frame, serial and decided, over 20000, 60000 and 250001 AVPLs:
-//                 200x120        640x360        1283x719
-//   budget  4096  0.91   1.12    1.63   2.02     4.49    6.41
-//           8192  1.63   1.30    2.22   2.83     6.82    8.65
-//          12000  1.94   0.66    2.82   3.88     8.5    10.0   (a quarter and 30 % of the tiles, none of 200x120)
-//          16384  1.94   0.66    3.30   2.83     9.2     9.2   (1.5 % and 13 %)
-constexpr int kSerialBudget = 8192, kSerialMinTiles = 2048;
-constexpr bool serial_cut(int budget, int tiles, int bad) {
-    return budget < kSerialBudget || (tiles >= kSerialMinTiles && 4LL * bad >= tiles);
+// a pool full that does not grow), from a third of the tiles on, or from a fifth
+// where there are fewer than 16384, four rounds of the chip's waves: such tiles
+// are then the end of the launch, and with the expansion criterion, whose few
+// large tiles stand out more, from a 30th.  Below 2048 tiles a serial wave's latency is what
+// counts, and the other kernel's is shorter.  Milliseconds a frame, serial and
+// decided, and the share of such tiles, over 20000, 60000, 250001 and 1000000 AVPLs:
+//                 200x120       640x360             1283x719            1920x1080
+//   budget  4096  0.86  1.12    1.53  2.02          4.50  6.41
+//           8192  1.53  1.27    2.08  2.83  0.65    6.84  8.67  0.44    22.3  23.6  0.37
+//          12000  1.94  0.65    2.50  3.73  0.24    8.25  9.95  0.30    25.4  24.5  0.33
+//          14000                2.65  3.03  0.10    8.64  9.83  0.21    26.4  24.1  0.25
+//          16384                2.93  2.76  0.01    9.10  9.49  0.13    27.3  25.0  0.21
+// expansion  8192               (30 tiles: 2.49)    6.24  6.95  0.068   19.9  17.9  0.14
+//           10000                                   6.32  7.07  0.038   20.3  17.0  0.11
+//           14000                                   6.39  6.11  0.010
+// and at 65536 with nodes of up to 128 exact (bound 0.0045, floor 4)
+//                                                  15.7  15.2   0.16
+constexpr int kSerialBudget = 8192, kSerialMinTiles = 2048, kSerialFewTiles = 16384;
+constexpr bool serial_cut(int budget, int tiles, int bad, bool expansion = false) {
+    const long long line = tiles >= kSerialFewTiles ? 3 : expansion ? 30 : 5;
+    return budget < kSerialBudget || (tiles >= kSerialMinTiles && line * bad >= tiles);
 }
 
 // Whether a wave's 64 rays go through the triangle tree together, one ray a lane,

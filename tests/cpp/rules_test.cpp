@@ -20,7 +20,11 @@ int main() {
         for (int set : {768, 3072}) check(arc::anti_block(set, staged) == set, "a block that was set");
     check(arc::serial_cut(8191, 100, 0) && !arc::serial_cut(8192, 100, 0), "the budget's line");
     check(!arc::serial_cut(65536, 2047, 2047), "few tiles are not cut serially");
-    check(arc::serial_cut(65536, 2048, 512) && !arc::serial_cut(65536, 2048, 511), "the tiles' line");
+    check(arc::serial_cut(65536, 2048, 410) && !arc::serial_cut(65536, 2048, 409) && arc::serial_cut(65536, 16383, 3277) &&
+              !arc::serial_cut(65536, 16384, 5461) && arc::serial_cut(65536, 16384, 5462) &&
+              arc::serial_cut(65536, 16383, 547, true) && !arc::serial_cut(65536, 16383, 546, true) &&
+              !arc::serial_cut(65536, 16384, 5461, true) && !arc::serial_cut(65536, 2047, 2047, true),
+          "the tiles' line");
     check(arc::serial_cut(65536, 2000000000, 2000000000), "many tiles");
     using arc::Rays;
     check(arc::rays_together(Rays::kCamera, 200000, 512) && !arc::rays_together(Rays::kCamera, 199999, 512) &&
